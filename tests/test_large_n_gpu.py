@@ -104,21 +104,20 @@ def test_bias_gradient_with_few_head_groups(n, h):
 # (the last pass runs with 2, 8, 4, 6, 2 and 2 key tiles per wave)
 @pytest.mark.parametrize("n,h,dtype", [(1030, 2, torch.bfloat16), (2048, 1, torch.bfloat16), (1500, 1, torch.float16), (1700, 1, torch.bfloat16), (2100, 1, torch.bfloat16), (4200, 1, torch.bfloat16)],
                          ids=["n1030_two_passes_ragged", "n2048_two_passes", "n1500_f16", "n1700", "n2100_three_passes", "n4200_five_passes"])
-def test_row_resident_backward_in_several_passes(n, h, dtype, monkeypatch):
+def test_row_resident_backward_in_several_passes(n, h, dtype, forced_tiles):
     """Rows longer than the row-resident kernel holds at once run it once per 1024 keys: dk, dv
     of each pass's keys and the dq summed over the passes are checked on a few pair rows, among
     them a fully masked one, one whose attended keys all lie in the last pass and one whose
     attended keys all lie in the first; db (from the db kernel, which reads the planes the first
     pass leaves) through the rows that carry the upstream gradient.  Two runs give the same bits."""
-    from trifast_amd import _lib, tuner
+    from trifast_amd import _lib
 
     lib = _lib.load()
     code = _lib.BF16 if dtype == torch.bfloat16 else _lib.F16
     nt = lib.trifast_num_tiles(_lib.KERNEL_BWD_KV)
     tile = nt - 1
     assert lib.trifast_bwd_kv_tile_writes_dq(tile) and lib.trifast_supports(_lib.KERNEL_BWD_KV, tile, n, h, D, code)
-    real_pick = tuner.pick
-    monkeypatch.setattr(tuner, "pick", lambda kern, *a, **kw: tile if kern == _lib.KERNEL_BWD_KV else real_pick(kern, *a, **kw))
+    forced_tiles({_lib.KERNEL_BWD_KV: tile})
     dev = "cuda"
     rows = (0, 3, 4, 5, n // 2, n - 1)
     g = torch.Generator(device=dev).manual_seed(n)

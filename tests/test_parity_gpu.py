@@ -19,7 +19,7 @@ import torch
 import bench
 import trifast_amd
 from oracle import triangle_oracle as orc
-from trifast_amd import _lib, tuner
+from trifast_amd import _lib
 from trifast_amd import torch as tt
 
 pytestmark = pytest.mark.gpu
@@ -126,7 +126,7 @@ def test_values_and_vectors(n, h, d, mask, bs, dtype, std):
 # ---------------------------------------------------------------------------
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "f32"])
 @pytest.mark.parametrize("n,h,d", [(70, 2, 32), (130, 1, 64), (40, 1, 16), (33, 1, 128)])
-def test_every_tile(n, h, d, dtype, monkeypatch):
+def test_every_tile(n, h, d, dtype, forced_tiles):
     lib = _lib.load()
     code = tt._DTYPE_CODE[dtype]
     g = torch.Generator().manual_seed(n)
@@ -137,17 +137,26 @@ def test_every_tile(n, h, d, dtype, monkeypatch):
     low = [t.to(dtype) for t in (q, k, v, b)]
     ref = orc.forward_backward(*(t.float() for t in low), m, do.to(dtype).float())
     pt = orc.forward_backward(*low, m, do.to(dtype))
-    ran = 0
-    for tile in range(max(lib.trifast_num_tiles(kern) for kern in range(4))):
-        tiles = {kern: tile if lib.trifast_supports(kern, tile, n, h, d, code) else None for kern in range(4)}
-        if all(t is None for t in tiles.values()):
-            continue
-        monkeypatch.setattr(tuner, "pick", lambda kern, n_, h_, d_, dt, launch, extra_cost=None, tiles=tiles: tiles[kern] if tiles[kern] is not None else lib.trifast_default_tile(kern, n_, h_, d_, code))
+    supported = {kern: [t for t in range(lib.trifast_num_tiles(kern)) if lib.trifast_supports(kern, t, n, h, d, code)] for kern in range(4)}
+    # (the dq kernel runs with the dk/dv tiles that do not write dq themselves: tile 0 stands in for the others)
+    streaming = [t for t in supported[_lib.KERNEL_BWD_KV] if not lib.trifast_bwd_kv_tile_writes_dq(t)]
+    for x in range(max(map(len, supported.values()))):
+        tiles = {kern: ts[x] for kern, ts in supported.items() if x < len(ts)}
+        if _lib.KERNEL_BWD_Q in tiles:
+            tiles[_lib.KERNEL_BWD_KV] = streaming[min(x, len(streaming) - 1)]
+        else:
+            tiles[_lib.KERNEL_BWD_KV] = supported[_lib.KERNEL_BWD_KV][min(x, len(supported[_lib.KERNEL_BWD_KV]) - 1)]
+        forced_tiles(tiles)
         kern_out = kernel_fwd_bwd(*low, m, do.to(dtype))
-        check_all(kern_out, pt, ref, dtype, f"tile {tile} n={n} d={d} {dtype}", directions=False)
-        ran += 1
+        check_all(kern_out, pt, ref, dtype, f"tiles {tiles} n={n} d={d} {dtype}", directions=False)
+    for tile in supported[_lib.KERNEL_BWD_KV]:
+        forced_tiles({_lib.KERNEL_BWD_KV: tile})
+        kern_out = kernel_fwd_bwd(*low, m, do.to(dtype))
+        check_all(kern_out, pt, ref, dtype, f"dk/dv tile {tile} n={n} d={d} {dtype}", directions=False)
+    forced_tiles({})
+    assert forced_tiles.launched >= {(kern, t) for kern, ts in supported.items() for t in ts}
     # large head dims in fp32 leave few tiles that fit the register file and LDS
-    assert ran >= (3 if d * (4 if dtype == torch.float32 else 2) <= 128 else 1)
+    assert len(set().union(*supported.values())) >= (3 if d * (4 if dtype == torch.float32 else 2) <= 128 else 1)
 
 
 # ---------------------------------------------------------------------------
@@ -160,7 +169,7 @@ def test_every_tile(n, h, d, dtype, monkeypatch):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
 @pytest.mark.parametrize("pattern", ["random", "padding", "first_dead", "middle_dead", "one_key"])
 @pytest.mark.parametrize("n,h,d", [(256, 2, 32), (128, 1, 16), (160, 1, 32)])
-def test_forward_scheduled_loop_masked(n, h, d, pattern, dtype, monkeypatch):
+def test_forward_scheduled_loop_masked(n, h, d, pattern, dtype, forced_tiles):
     lib = _lib.load()
     code = tt._DTYPE_CODE[dtype]
     g = torch.Generator().manual_seed(3 * n + d)
@@ -187,8 +196,7 @@ def test_forward_scheduled_loop_masked(n, h, d, pattern, dtype, monkeypatch):
     scheduled = [t for t in range(lib.trifast_num_tiles(_lib.KERNEL_FWD)) if t >= 6 and lib.trifast_supports(_lib.KERNEL_FWD, t, n, h, d, code)]
     assert len(scheduled) == 2, "tiles 6 and 7 are the forward's scheduled loop"
     for tile in scheduled:
-        monkeypatch.setattr(tuner, "pick", lambda kern, n_, h_, d_, dt, launch, extra_cost=None, tile=tile:
-                            tile if kern == _lib.KERNEL_FWD else lib.trifast_default_tile(kern, n_, h_, d_, code))
+        forced_tiles({_lib.KERNEL_FWD: tile})
         out = kernel_fwd_bwd(*low, m, do.to(dtype))
         tag = f"fwd tile {tile} n={n} d={d} {pattern} {dtype}"
         check_all(out, pt, ref, dtype, tag, directions=False)
@@ -304,7 +312,7 @@ def test_seeded_mixtures(seed):
 # forced in the second pass) read those bitmaps.  At n = 2112 a bitmap is two words.
 # ---------------------------------------------------------------------------
 @pytest.mark.parametrize("n,valid", [(1088, 1060), (2112, 2090)], ids=["34_tiles", "66_tiles"])
-def test_key_tile_bitmaps_past_32_tiles(n, valid, monkeypatch):
+def test_key_tile_bitmaps_past_32_tiles(n, valid, forced_tiles):
     lib = _lib.load()
     h, d, dtype = 1, 32, torch.bfloat16
     code = tt._DTYPE_CODE[dtype]
@@ -328,8 +336,7 @@ def test_key_tile_bitmaps_past_32_tiles(n, valid, monkeypatch):
     # the same with the dq and dk/dv kernels instead of the row-resident one
     kv = next(t for t in range(lib.trifast_num_tiles(_lib.KERNEL_BWD_KV))
               if not lib.trifast_bwd_kv_tile_writes_dq(t) and lib.trifast_supports(_lib.KERNEL_BWD_KV, t, n, h, d, code))
-    real_pick = tuner.pick
-    monkeypatch.setattr(tuner, "pick", lambda kern, *a, **kw: kv if kern == _lib.KERNEL_BWD_KV else real_pick(kern, *a, **kw))
+    forced_tiles({_lib.KERNEL_BWD_KV: kv})
     out = kernel_fwd_bwd(*low, m, do.to(dtype))
     check_all(out, pt, ref, dtype, f"n={n} padding to {valid}, three-kernel backward", directions=False)
 
@@ -346,7 +353,7 @@ def test_key_tile_bitmaps_past_32_tiles(n, valid, monkeypatch):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
 @pytest.mark.parametrize("pattern", ["none", "padding", "middle", "early"])
 @pytest.mark.parametrize("n,h,d", [(300, 2, 32), (256, 1, 16), (200, 1, 32)])
-def test_db_pipelined_rows(n, h, d, pattern, dtype, monkeypatch):
+def test_db_pipelined_rows(n, h, d, pattern, dtype, forced_tiles):
     lib = _lib.load()
     code = tt._DTYPE_CODE[dtype]
     g = torch.Generator().manual_seed(n + d)
@@ -372,8 +379,7 @@ def test_db_pipelined_rows(n, h, d, pattern, dtype, monkeypatch):
     assert len(two_key_tiles) >= 2, infos
     results = {}
     for tile in [plain_tile] + two_key_tiles:
-        monkeypatch.setattr(tuner, "pick", lambda kern, n_, h_, d_, dt, launch, extra_cost=None, tile=tile:
-                            tile if kern == _lib.KERNEL_BWD_B else lib.trifast_default_tile(kern, n_, h_, d_, code))
+        forced_tiles({_lib.KERNEL_BWD_B: tile})
         out = kernel_fwd_bwd(*low, m, do.to(dtype))
         check_all(out, pt, ref, dtype, f"db tile {tile} n={n} d={d} {pattern} {dtype}", directions=False)
         results[tile] = out[NAMES.index("db")] if "db" in NAMES else out[-1]
@@ -393,7 +399,7 @@ def test_db_pipelined_rows(n, h, d, pattern, dtype, monkeypatch):
 # ---------------------------------------------------------------------------
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
 @pytest.mark.parametrize("n,h,d", [(131, 2, 32), (300, 1, 32), (450, 1, 32), (520, 1, 32), (700, 1, 32), (800, 1, 32), (1000, 1, 32), (300, 1, 64), (450, 1, 64), (190, 1, 16), (330, 1, 16)])
-def test_row_resident_backward_size_classes(n, h, d, dtype, monkeypatch):
+def test_row_resident_backward_size_classes(n, h, d, dtype, forced_tiles):
     lib = _lib.load()
     code = tt._DTYPE_CODE[dtype]
     row_tiles = [t for t in range(lib.trifast_num_tiles(_lib.KERNEL_BWD_KV))
@@ -411,8 +417,7 @@ def test_row_resident_backward_size_classes(n, h, d, dtype, monkeypatch):
     chunk = 64 if n > 400 else None
     ref = oracle_fwd_bwd(*(t.float() for t in low), m, do.to(dtype).float(), chunk)
     pt = oracle_fwd_bwd(*low, m, do.to(dtype), chunk)
-    real_pick = tuner.pick
-    monkeypatch.setattr(tuner, "pick", lambda kern, *a, **kw: tile if kern == _lib.KERNEL_BWD_KV else real_pick(kern, *a, **kw))
+    forced_tiles({_lib.KERNEL_BWD_KV: tile})
     kern_out = kernel_fwd_bwd(*low, m, do.to(dtype))
     check_all(kern_out, pt, ref, dtype, f"row-resident tile {tile} n={n} d={d} {dtype}", directions=False)
     again = kernel_fwd_bwd(*low, m, do.to(dtype))
