@@ -200,7 +200,8 @@ constexpr int bwd_uniform_lds_bytes(int D, int es) {
 //   dk_k = s / n (M2 V_k - sQ),            M2 = sum_j Q_j dO_j^T, sQ = sum_j delta_j Q_j
 //   dv_k = sO / n,                          sO = sum_j dO_j
 // The sums run on the matrix pipe over 32-row tiles (wave w takes tiles w, w + 4, ...; every
-// wave's part is added in wave order), in fp32; M1 and M2 go into the second products as hi + lo parts.
+// wave's part is added in wave order), in fp32; M1 and M2 go into the second products as hi + lo parts
+// (scaled for fp16, see there).
 // What is left is the memory traffic of the row and its latency.  A training step over n = 512 with
 // 397 valid positions (bf16, h = 4, d = 32), with the same rule in db and the rows dealt evenly:
 // 605 -> 543 us.
@@ -349,6 +350,29 @@ TRI_DEV void bwd_uniform_row(const BwdArgs& a, int bh, int i, unsigned char* sme
     }
     __syncthreads();
   }
+  // fp16 ends at 65504, which sums over a row of coherent numbers pass (768 keys with K = V = 10 in a
+  // channel give 76800): M1 and M2 go in times a power of two that brings their largest entry to
+  // 2^13 .. 2^14, which costs no bits, and the factor comes off with the store.
+  int up1 = 0, up2 = 0;
+  if constexpr (std::is_same_v<T, _Float16>) {
+    float x1 = 0.f, x2 = 0.f;
+#pragma unroll
+    for (int mt = 0; mt < DM; ++mt) {
+      const int row = min(32 * mt + jl, D - 1);
+#pragma unroll
+      for (int e = 0; e < D / 2; ++e) {
+        x1 = fmaxf(x1, __builtin_fabsf(m1[row * D + D / 2 * g + e]));
+        x2 = fmaxf(x2, __builtin_fabsf(m2[row * D + D / 2 * g + e]));
+      }
+    }
+#pragma unroll
+    for (int m = 1; m < 64; m *= 2) {
+      x1 = fmaxf(x1, __shfl_xor(x1, m));
+      x2 = fmaxf(x2, __shfl_xor(x2, m));
+    }
+    up1 = 14 - __builtin_amdgcn_frexp_expf(x1);
+    up2 = 14 - __builtin_amdgcn_frexp_expf(x2);
+  }
   // second products: row jl of M1, M2 as hi + lo parts; the vectors at this lane's rows of the result
   frag h1[DM][DS], l1[DM][DS], h2[DM][DS], l2[DM][DS];
   f32x16 vk[DM], vq[DM], vo[DM];
@@ -359,7 +383,7 @@ TRI_DEV void bwd_uniform_row(const BwdArgs& a, int bh, int i, unsigned char* sme
     for (int s = 0; s < DS; ++s)
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        const float x1 = m1[row * D + 16 * s + 8 * g + e], x2 = m2[row * D + 16 * s + 8 * g + e];
+        const float x1 = ldexpf(m1[row * D + 16 * s + 8 * g + e], up1), x2 = ldexpf(m2[row * D + 16 * s + 8 * g + e], up2);
         h1[mt][s][e] = (T)x1;
         l1[mt][s][e] = (T)(x1 - (float)h1[mt][s][e]);
         h2[mt][s][e] = (T)x2;
@@ -368,12 +392,12 @@ TRI_DEV void bwd_uniform_row(const BwdArgs& a, int bh, int i, unsigned char* sme
 #pragma unroll
     for (int v = 0; v < 16; ++v) {
       const int r = min(32 * mt + crow(v, g), D - 1);
-      vk[mt][v] = sk[r];
-      vq[mt][v] = -sq[r];
+      vk[mt][v] = ldexpf(sk[r], up1);
+      vq[mt][v] = ldexpf(-sq[r], up2);
       vo[mt][v] = so[r];
     }
   }
-  const float inv = 1.0f / (float)N, mul = a.scale * inv;
+  const float inv = 1.0f / (float)N, mulq = ldexpf(a.scale * inv, -up1), mulk = ldexpf(a.scale * inv, -up2);
   T* const dqrow = reinterpret_cast<T*>(a.dq) + b * a.sdq.b + h * a.sdq.h + i * a.sdq.i;
   T* const dkrow = reinterpret_cast<T*>(a.dk) + b * a.sdk.b + h * a.sdk.h + i * a.sdk.i;
   T* const dvrow = reinterpret_cast<T*>(a.dv) + b * a.sdv.b + h * a.sdv.h + i * a.sdv.i;
@@ -417,8 +441,8 @@ TRI_DEV void bwd_uniform_row(const BwdArgs& a, int bh, int i, unsigned char* sme
         k[mt] = E::mfma(h2[mt][s], vf[s], k[mt]);
       }
     }
-    store_rows_wide<T, D, DM>(dqrow + (int64_t)j * a.sdq.j, q, mul, g, j < N);
-    store_rows_wide<T, D, DM>(dkrow + (int64_t)j * a.sdk.j, k, mul, g, j < N);
+    store_rows_wide<T, D, DM>(dqrow + (int64_t)j * a.sdq.j, q, mulq, g, j < N);
+    store_rows_wide<T, D, DM>(dkrow + (int64_t)j * a.sdk.j, k, mulk, g, j < N);
     store_rows_wide<T, D, DM>(dvrow + (int64_t)j * a.sdv.j, vo, inv, g, j < N);
   }
 }
