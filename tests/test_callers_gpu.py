@@ -13,6 +13,7 @@ import torch
 
 import trifast_amd
 from oracle import triangle_oracle as orc
+from trifast_amd.torch import triangle_attention_ending_node
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -241,3 +242,49 @@ def test_empty_inputs_give_empty_outputs(shape):
     o.sum().backward()
     for t in (q, k, v, bias):
         assert t.grad is not None and t.grad.shape == t.shape
+
+
+# ---------------------------------------------------------------------------
+# calls that are not ordinary eager ones: nothing is computed with a part of them left out
+# ---------------------------------------------------------------------------
+def _entries():
+    """Every public entry as (function, floating-point tensors, the rest): the operator around both
+    nodes and under a batch dim, the gate, the block."""
+    from trifast_amd import nn
+
+    torch.manual_seed(5)
+    n, h, d, c, dtype = 24, 2, 32, 64, torch.bfloat16
+    q, k, v = (torch.randn(1, h, n, n, d, device=DEV, dtype=dtype) for _ in range(3))
+    b = torch.randn(1, h, n, n, device=DEV, dtype=dtype)
+    m = torch.rand(1, n, n, device=DEV) < 0.2
+    x, g = torch.randn(1, n, n, c, device=DEV, dtype=dtype), torch.randn(1, n, n, h * d, device=DEV, dtype=dtype)
+    block = nn.TriangleAttention(c, h, d).to(DEV, dtype)
+    return {
+        "starting": (lambda *t: trifast_amd.triangle_attention(*t, m), (q, k, v, b)),
+        "ending": (lambda *t: triangle_attention_ending_node(*t, m), (q, k, v, b)),
+        "leading dims": (lambda *t: trifast_amd.triangle_attention(*t, m[0]), (q[0], k[0], v[0], b[0])),
+        "gate": (nn.gated_output, (q, g)),
+        "block": (lambda t: block(t, m), (x,)),
+        "frozen block": (lambda t, frozen=nn.TriangleAttention(c, h, d).to(DEV, dtype).requires_grad_(False): frozen(t, m), (x,)),
+    }
+
+
+ENTRIES = ("starting", "ending", "leading dims", "gate", "block", "frozen block")
+
+
+@pytest.mark.parametrize("wants_grad", [False, True], ids=["plain", "with_grad"])
+@pytest.mark.parametrize("name", ENTRIES)
+def test_forward_mode_raises(name, wants_grad):
+    """The kernels have no forward-mode rule: a call with a tangent raises, also where no input
+    requires grad, instead of returning a result without its tangent."""
+    import torch.autograd.forward_ad as fwad
+
+    fn, tensors = _entries()[name]
+    for x in range(len(tensors)):
+        with fwad.dual_level():
+            args = [t.requires_grad_(wants_grad) for t in tensors]
+            args[x] = fwad.make_dual(args[x], torch.ones_like(args[x]))
+            with pytest.raises(NotImplementedError, match="jvp"):
+                fn(*args)
+    with pytest.raises((NotImplementedError, RuntimeError), match="jvp"):
+        torch.func.jvp(fn, tuple(t.detach() for t in tensors), tuple(torch.ones_like(t) for t in tensors))

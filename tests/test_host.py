@@ -254,3 +254,16 @@ def test_equiv_simple_takes_any_number_of_batch_dims():
     parts = torch.stack([equiv.attention_reference(q[x], k[x], v[x], b[x], m[x]) for x in range(2)])
     assert torch.allclose(whole, parts, atol=1e-6)
     assert torch.allclose(equiv.triangle_attention_simple(q[0, 0], k[0, 0], v[0, 0], b[0, 0], m[0, 0]), whole[0, 0], atol=1e-6)
+
+
+def test_tensors_with_a_tangent_do_not_take_the_native_path():
+    """The native path launches the kernels without the dispatcher: a forward-mode tangent would be
+    dropped there, so such tensors are declined."""
+    import torch.autograd.forward_ad as fwad
+
+    native = tt._native()
+    x = torch.randn(3)
+    assert native.plain_eager([x, x.clone().requires_grad_(True)])
+    with fwad.dual_level():
+        assert native.plain_eager([x])
+        assert not native.plain_eager([x, fwad.make_dual(x, torch.ones_like(x))])

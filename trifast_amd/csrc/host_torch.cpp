@@ -242,7 +242,8 @@ struct Attention : torch::autograd::Function<Attention> {
   }
 };
 
-// Ordinary eager execution: no function transforms, no dispatch modes, no autocast, plain tensors.
+// Ordinary eager execution: no function transforms, no dispatch modes, no autocast, plain tensors
+// without a forward-mode tangent (the kernels have no rule for it, and the launches here would drop it).
 bool plain_eager(std::initializer_list<const Tensor*> tensors) {
   using c10::DispatchKey;
   if (at::autocast::is_autocast_enabled(at::kCUDA)) return false;
@@ -251,7 +252,7 @@ bool plain_eager(std::initializer_list<const Tensor*> tensors) {
   if (c10::impl::TorchDispatchModeTLS::stack_len() > 0) return false;
   for (const Tensor* t : tensors)
     if (!t->defined() || t->key_set().has_any(c10::DispatchKeySet({DispatchKey::Python, DispatchKey::FuncTorchGradWrapper, DispatchKey::FuncTorchBatched})) ||
-        t->layout() != at::kStrided || t->is_neg() || t->is_conj())
+        t->layout() != at::kStrided || t->is_neg() || t->is_conj() || t->_fw_grad(/*level=*/0).defined())
       return false;
   return true;
 }
@@ -519,6 +520,11 @@ OptTensor gate(const Tensor& o, const Tensor& g) {
 
 PYBIND11_MODULE(_host, m) {
   using release = py::call_guard<py::gil_scoped_release>;
+  m.def("plain_eager", [](const std::vector<Tensor>& tensors) {
+    for (const Tensor& t : tensors)
+      if (!plain_eager({&t})) return false;
+    return true;
+  });
   m.def("attention", &attention, release());
   m.def("forward", [](const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& b, const Tensor& mask) {
     Forward f = forward(q, k, v, b, mask);

@@ -33,7 +33,7 @@ from typing import Optional, Sequence
 import torch
 
 from trifast_amd import _lib
-from trifast_amd.torch import _dtype_code, _native, triangle_attention, triangle_attention_ending_node
+from trifast_amd.torch import _dtype_code, _native, _no_forward_mode, triangle_attention, triangle_attention_ending_node
 
 
 def _gate_shapes(o: torch.Tensor, g: torch.Tensor) -> tuple[int, int, int, int]:
@@ -96,6 +96,7 @@ def gated_output(o: torch.Tensor, g: torch.Tensor) -> torch.Tensor:
         y = _native().gate(o, g)  # (None where the call has to go through the registered operators)
         if y is not None:
             return y
+        _no_forward_mode(o, g)
     return _gated_output(o, g)
 
 

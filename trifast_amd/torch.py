@@ -276,6 +276,14 @@ def setup_context(ctx, inputs, output) -> None:
 _triangle_attention.register_autograd(backwards, setup_context=setup_context)
 
 
+def _no_forward_mode(*tensors: torch.Tensor) -> None:
+    """Raises for tensors with a forward-mode tangent: a registered operator called without an input
+    that requires grad would return a result without one."""
+    for t in tensors:
+        if torch.autograd.forward_ad.unpack_dual(t).tangent is not None:
+            raise NotImplementedError("the triangle attention kernels have no forward-mode derivative (jvp)")
+
+
 def _attend(q, k, v, b, mask, ending: bool) -> torch.Tensor:
     """The operator (``ending``: on the pair-transposed problem) on 5-D inputs.  Ordinary eager
     calls on plain GPU tensors run natively, with an autograd node of their own over the same
@@ -283,11 +291,12 @@ def _attend(q, k, v, b, mask, ending: bool) -> torch.Tensor:
     the backward's trips through the interpreter took 0.2 ms of a step, twice what its kernels
     take at n = 256.  The native path declines (None) anything else -- tracing, transforms,
     autocast, other devices, shapes that do not fit -- which goes through the registered
-    operators."""
+    operators; forward-mode differentiation raises."""
     if not torch.compiler.is_compiling():
         o = _native().attention(q, k, v, b, mask, ending)
         if o is not None:
             return o
+        _no_forward_mode(q, k, v, b)
     if ending:
         t = lambda x: x.transpose(-3, -2)
         return t(_triangle_attention(t(q), t(k), t(v), b.transpose(-1, -2), mask.transpose(-1, -2))[0])
