@@ -288,3 +288,30 @@ def test_forward_mode_raises(name, wants_grad):
                 fn(*args)
     with pytest.raises((NotImplementedError, RuntimeError), match="jvp"):
         torch.func.jvp(fn, tuple(t.detach() for t in tensors), tuple(torch.ones_like(t) for t in tensors))
+
+
+@pytest.mark.parametrize("wants_grad", [False, True], ids=["plain", "with_grad"])
+@pytest.mark.parametrize("name", ENTRIES[:4])
+def test_torch_jit_trace_replays(name, wants_grad):
+    """A traced call replays on new numbers, twice, with the gradients of the eager call."""
+    fn, tensors = _entries()[name]
+    traced = torch.jit.trace(fn, tuple(t.requires_grad_(wants_grad) for t in tensors), check_trace=False)
+    for _ in range(2):
+        new = [torch.randn_like(t).requires_grad_(wants_grad) for t in tensors]
+        got, want = traced(*new), fn(*new)
+        assert torch.equal(got, want)
+        if wants_grad:
+            dy = torch.randn_like(want)
+            for a, r in zip(torch.autograd.grad(got, new, dy), torch.autograd.grad(want, new, dy)):
+                assert torch.equal(a, r)
+
+
+def test_torch_jit_trace_of_the_block_raises():
+    """Its projections are operators over lists of optional tensors, which a trace cannot hold: it
+    says so rather than recording the block without its launches."""
+    from trifast_amd import nn
+
+    block = nn.TriangleAttention(64, 2, 32).to(DEV, torch.bfloat16)
+    x, m = torch.randn(1, 24, 24, 64, device=DEV, dtype=torch.bfloat16), torch.zeros(1, 24, 24, device=DEV, dtype=torch.bool)
+    with pytest.raises(RuntimeError, match="list type"):
+        torch.jit.trace(block, (x, m), check_trace=False)

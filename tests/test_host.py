@@ -267,3 +267,15 @@ def test_tensors_with_a_tangent_do_not_take_the_native_path():
     with fwad.dual_level():
         assert native.plain_eager([x])
         assert not native.plain_eager([x, fwad.make_dual(x, torch.ones_like(x))])
+
+
+def test_nothing_takes_the_native_path_while_torch_jit_traces():
+    """A tracer under the native path records the allocation of the output and no launch."""
+    seen = []
+
+    def fn(x):
+        seen.append(tt._native().plain_eager([x]))
+        return x + 1
+
+    torch.jit.trace(fn, (torch.randn(3),), check_trace=False)
+    assert seen == [False] and tt._native().plain_eager([torch.randn(3)])

@@ -17,6 +17,7 @@
 #include <torch/extension.h>
 
 #include <ATen/FuncTorchTLS.h>
+#include <ATen/TracerMode.h>
 #include <ATen/autocast_mode.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
@@ -242,11 +243,11 @@ struct Attention : torch::autograd::Function<Attention> {
   }
 };
 
-// Ordinary eager execution: no function transforms, no dispatch modes, no autocast, plain tensors
-// without a forward-mode tangent (the kernels have no rule for it, and the launches here would drop it).
+// Ordinary eager execution: no function transforms, no dispatch modes, no autocast, no tracer (which
+// would record the allocations made here and none of the launches), plain tensors without a forward-mode tangent (the kernels have no rule for it, and the launches here would drop it).
 bool plain_eager(std::initializer_list<const Tensor*> tensors) {
   using c10::DispatchKey;
-  if (at::autocast::is_autocast_enabled(at::kCUDA)) return false;
+  if (at::autocast::is_autocast_enabled(at::kCUDA) || at::tracer::impl::is_dispatch_enabled()) return false;
   const auto tls = c10::impl::tls_local_dispatch_key_set();
   if (tls.included_.has(DispatchKey::Python) || tls.included_.has(DispatchKey::FuncTorchDynamicLayerFrontMode)) return false;
   if (c10::impl::TorchDispatchModeTLS::stack_len() > 0) return false;
