@@ -315,3 +315,20 @@ def test_torch_jit_trace_of_the_block_raises():
     x, m = torch.randn(1, 24, 24, 64, device=DEV, dtype=torch.bfloat16), torch.zeros(1, 24, 24, device=DEV, dtype=torch.bool)
     with pytest.raises(RuntimeError, match="list type"):
         torch.jit.trace(block, (x, m), check_trace=False)
+
+
+@pytest.mark.parametrize("name", ENTRIES)
+def test_second_derivatives_raise(name):
+    """create_graph gives the same first gradients; differentiating them raises."""
+    fn, tensors = _entries()[name]
+    leaves = [t.requires_grad_(True) for t in tensors]
+    y = fn(*leaves)
+    dy = torch.randn_like(y).requires_grad_(True)
+    first = torch.autograd.grad(y, leaves, dy, retain_graph=True)
+    again = torch.autograd.grad(y, leaves, dy, create_graph=True)
+    for a, r in zip(again, first):
+        assert a.requires_grad and torch.equal(a, r)
+        with pytest.raises(RuntimeError, match="second derivative|autograd formula"):
+            torch.autograd.grad(a.float().pow(2).sum() + y.float().sum(), leaves, retain_graph=True)
+        with pytest.raises(RuntimeError, match="second derivative|autograd formula"):
+            torch.autograd.grad(a.float().pow(2).sum(), dy, retain_graph=True)

@@ -23,6 +23,7 @@
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/functions/basic_ops.h>
 
 #include <array>
 #include <cctype>
@@ -221,6 +222,22 @@ Tensor swap_pair(const Tensor& t, bool ending) {
   return t.dim() == 5 ? t.transpose(2, 3) : t.transpose(-1, -2);
 }
 
+// The gradients of a backward that ran the kernels.  They have no graph: where the caller asked for
+// one (create_graph turns grad mode on in the backward) they come from a node over the tensors they
+// were made of that raises when it is differentiated: a penalty on a gradient is not silently a constant.
+torch::autograd::variable_list once_differentiable(torch::autograd::variable_list grads, const torch::autograd::variable_list& saved, const Tensor& dout,
+                                                   const char* what) {
+  if (!at::GradMode::is_enabled()) return grads;
+  const size_t n = grads.size();
+  grads.push_back(dout);
+  for (const Tensor& t : saved)
+    if (t.defined() && t.requires_grad()) grads.push_back(t);
+  torch::autograd::DelayedError raises(std::string("trifast: the backward of ") + what + " has no second derivative", static_cast<int>(grads.size()));
+  grads = raises(std::move(grads));
+  grads.resize(n);
+  return grads;
+}
+
 struct Attention : torch::autograd::Function<Attention> {
   static Tensor forward(torch::autograd::AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& b,
                         const Tensor& mask, bool ending) {
@@ -235,11 +252,15 @@ struct Attention : torch::autograd::Function<Attention> {
   static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx, torch::autograd::variable_list grads) {
     const auto saved = ctx->get_saved_variables();
     const bool ending = ctx->saved_data["ending"].toBool();
-    if (!grads[0].defined()) return torch::autograd::variable_list(6);
-    at::AutoDispatchBelowADInplaceOrView below;
-    auto t = [&](int x) { return swap_pair(saved[x], ending); };
-    Grads g = ::backward(swap_pair(grads[0], ending), t(0), t(1), t(2), t(3), t(5), saved[6], t(4), saved[7]);
-    return {swap_pair(g[0], ending), swap_pair(g[1], ending), swap_pair(g[2], ending), swap_pair(g[3], ending), Tensor(), Tensor()};
+    torch::autograd::variable_list out(6);
+    if (!grads[0].defined()) return out;
+    {
+      at::AutoDispatchBelowADInplaceOrView below;
+      auto t = [&](int x) { return swap_pair(saved[x], ending); };
+      const Grads g = ::backward(swap_pair(grads[0], ending), t(0), t(1), t(2), t(3), t(5), saved[6], t(4), saved[7]);
+      for (int i = 0; i < 4; ++i) out[i] = swap_pair(g[i], ending);
+    }
+    return once_differentiable(std::move(out), saved, grads[0], "triangle attention");
   }
 };
 
@@ -436,13 +457,15 @@ struct Block : torch::autograd::Function<Block> {
     if (!grads[0].defined()) return out;
     const auto t = ctx->get_saved_variables();
     const auto s = ctx->saved_data["shape"].toIntVector();
-    at::AutoDispatchBelowADInplaceOrView below;
-    const Params p{t[2], t[3], t[4], t[5], t[6], t[7], t[8], t[9]};
-    const BlockState st{t[10], t[11], t[12], t[13], t[14], t[15], t[16], t[17]};
-    auto [dx, dp] = block_backward(grads[0], t[0], t[1], p, st, s[0], s[1], s[2] != 0, s[3] != 0, s[4] != 0);
-    out[0] = dx;
-    for (int i = 0; i < NPARAMS; ++i) out[2 + i] = dp[i];
-    return out;
+    {
+      at::AutoDispatchBelowADInplaceOrView below;
+      const Params p{t[2], t[3], t[4], t[5], t[6], t[7], t[8], t[9]};
+      const BlockState st{t[10], t[11], t[12], t[13], t[14], t[15], t[16], t[17]};
+      auto [dx, dp] = block_backward(grads[0], t[0], t[1], p, st, s[0], s[1], s[2] != 0, s[3] != 0, s[4] != 0);
+      out[0] = dx;
+      for (int i = 0; i < NPARAMS; ++i) out[2 + i] = dp[i];
+    }
+    return once_differentiable(std::move(out), t, grads[0], "the triangle attention block");
   }
 };
 
@@ -503,9 +526,12 @@ struct Gate : torch::autograd::Function<Gate> {
   }
   static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx, torch::autograd::variable_list grads) {
     const auto t = ctx->get_saved_variables();
-    at::AutoDispatchBelowADInplaceOrView below;
-    auto [dout, dg] = gate_backward(grads[0], t[0], t[1]);
-    return {dout, dg};
+    torch::autograd::variable_list out(2);
+    {
+      at::AutoDispatchBelowADInplaceOrView below;
+      std::tie(out[0], out[1]) = gate_backward(grads[0], t[0], t[1]);
+    }
+    return once_differentiable(std::move(out), t, grads[0], "the output gate");
   }
 };
 
