@@ -332,3 +332,27 @@ def test_second_derivatives_raise(name):
             torch.autograd.grad(a.float().pow(2).sum() + y.float().sum(), leaves, retain_graph=True)
         with pytest.raises(RuntimeError, match="second derivative|autograd formula"):
             torch.autograd.grad(a.float().pow(2).sum(), dy, retain_graph=True)
+
+
+@pytest.mark.parametrize("name", ENTRIES)
+def test_subclasses_with_a_torch_function_keep_it(name):
+    """A tensor subclass that only overrides __torch_function__ sees the registered operators and gets
+    its own type back."""
+    class Seen(torch.Tensor):
+        ops = []
+
+        @classmethod
+        def __torch_function__(cls, func, types, args=(), kwargs=None):
+            cls.ops.append(str(func))
+            return super().__torch_function__(func, types, args, kwargs or {})
+
+    fn, tensors = _entries()[name]
+    want = fn(*tensors)
+    for x in range(len(tensors)):
+        Seen.ops.clear()
+        args = list(tensors)
+        args[x] = args[x].as_subclass(Seen)
+        got = fn(*args)
+        assert type(got) is Seen and any("trifast" in op for op in Seen.ops)
+        tol = 2.0**-7 * want.float().abs().max() if "block" in name else 0
+        assert (got.as_subclass(torch.Tensor).float() - want.float()).abs().max() <= tol

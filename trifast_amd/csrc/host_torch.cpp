@@ -24,6 +24,7 @@
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/functions/basic_ops.h>
+#include <torch/csrc/autograd/python_variable.h>
 
 #include <array>
 #include <cctype>
@@ -37,6 +38,24 @@
 
 namespace py = pybind11;
 using at::Tensor;
+
+// A tensor as Python gives it: `overrides` for a subclass other than Parameter, which may have a
+// __torch_function__ of its own that the registered operators call and the native path would pass by.
+struct PyTensor {
+  Tensor t;
+  bool overrides = false;
+};
+template <>
+struct py::detail::type_caster<PyTensor> {
+  PYBIND11_TYPE_CASTER(PyTensor, const_name("torch.Tensor"));
+  bool load(handle src, bool convert) {
+    make_caster<Tensor> tensor;
+    if (!tensor.load(src, convert)) return false;
+    value.t = cast_op<Tensor&>(tensor);
+    value.overrides = !THPVariable_CheckTypeExact(Py_TYPE(src.ptr()));
+    return true;
+  }
+};
 
 namespace {
 
@@ -287,7 +306,9 @@ bool wants_grad(std::initializer_list<const Tensor*> tensors) {
 }
 
 // The operator on plain tensors; none where the call has to take another path.
-std::optional<Tensor> attention(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& b, const Tensor& mask, bool ending) {
+std::optional<Tensor> attention(const PyTensor& q_, const PyTensor& k_, const PyTensor& v_, const PyTensor& b_, const PyTensor& mask_, bool ending) {
+  if (q_.overrides || k_.overrides || v_.overrides || b_.overrides || mask_.overrides) return std::nullopt;
+  const Tensor &q = q_.t, &k = k_.t, &v = v_.t, &b = b_.t, &mask = mask_.t;
   if (!plain_eager({&q, &k, &v, &b, &mask}) || !inputs_ok(q, k, v, b, mask)) return std::nullopt;
   if (wants_grad({&q, &k, &v, &b})) return Attention::apply(q, k, v, b, mask, ending);
   at::AutoDispatchBelowADInplaceOrView below;
@@ -473,15 +494,19 @@ using OptTensor = std::optional<Tensor>;
 Tensor or_undefined(const OptTensor& t) { return t ? *t : Tensor(); }
 
 // The block on plain tensors; none where the call has to take another path.
-OptTensor block(const Tensor& x, const Tensor& mask, const Tensor& wq, const Tensor& wk, const Tensor& wv, const Tensor& wb, const Tensor& wg,
-                const OptTensor& bg, const Tensor& wo, const OptTensor& bo, int64_t h, int64_t d, bool ending) {
-  const Params p{wq, wk, wv, wb, wg, or_undefined(bg), wo, or_undefined(bo)};
-  if (!plain_eager({&x, &mask, &wq, &wk, &wv, &wb, &wg, &wo}) || !block_ok(x, mask, p, h, d)) return std::nullopt;
+OptTensor block(const PyTensor& x_, const PyTensor& mask_, const PyTensor& wq, const PyTensor& wk, const PyTensor& wv, const PyTensor& wb, const PyTensor& wg,
+                const std::optional<PyTensor>& bg, const PyTensor& wo, const std::optional<PyTensor>& bo, int64_t h, int64_t d, bool ending) {
+  for (const PyTensor* t : {&x_, &mask_, &wq, &wk, &wv, &wb, &wg, &wo})
+    if (t->overrides) return std::nullopt;
+  if ((bg && bg->overrides) || (bo && bo->overrides)) return std::nullopt;
+  const Tensor &x = x_.t, &mask = mask_.t;
+  const Params p{wq.t, wk.t, wv.t, wb.t, wg.t, bg ? bg->t : Tensor(), wo.t, bo ? bo->t : Tensor()};
+  if (!plain_eager({&x, &mask, &p[WQ], &p[WK], &p[WV], &p[WB], &p[WG], &p[WO]}) || !block_ok(x, mask, p, h, d)) return std::nullopt;
   for (int i : {(int)BG, (int)BO})
     if (p[i].defined() && !plain_eager({&p[i]})) return std::nullopt;
-  bool grad = wants_grad({&x, &wq, &wk, &wv, &wb, &wg, &wo});
+  bool grad = wants_grad({&x, &p[WQ], &p[WK], &p[WV], &p[WB], &p[WG], &p[WO]});
   for (int i : {(int)BG, (int)BO}) grad = grad || (p[i].defined() && wants_grad({&p[i]}));
-  if (grad) return Block::apply(x, mask, wq, wk, wv, wb, wg, p[BG], wo, p[BO], h, d, ending);
+  if (grad) return Block::apply(x, mask, p[WQ], p[WK], p[WV], p[WB], p[WG], p[BG], p[WO], p[BO], h, d, ending);
   at::AutoDispatchBelowADInplaceOrView below;
   return block_forward(x, mask, p, h, d, ending).first;
 }
@@ -536,7 +561,9 @@ struct Gate : torch::autograd::Function<Gate> {
 };
 
 // (shapes are the caller's to check)
-OptTensor gate(const Tensor& o, const Tensor& g) {
+OptTensor gate(const PyTensor& o_, const PyTensor& g_) {
+  if (o_.overrides || g_.overrides) return std::nullopt;
+  const Tensor &o = o_.t, &g = g_.t;
   if (!plain_eager({&o, &g})) return std::nullopt;
   if (wants_grad({&o, &g})) return Gate::apply(o, g);
   at::AutoDispatchBelowADInplaceOrView below;
