@@ -356,3 +356,18 @@ def test_subclasses_with_a_torch_function_keep_it(name):
         assert type(got) is Seen and any("trifast" in op for op in Seen.ops)
         tol = 2.0**-7 * want.float().abs().max() if "block" in name else 0
         assert (got.as_subclass(torch.Tensor).float() - want.float()).abs().max() <= tol
+
+
+@pytest.mark.parametrize("name", ENTRIES)
+def test_lazy_upstream_gradients(name):
+    """A lazily negated upstream gradient, and a zero one without memory."""
+    fn, tensors = _entries()[name]
+    leaves = [t.requires_grad_(True) for t in tensors]
+    y = fn(*leaves)
+    dy = torch.randn_like(y)
+    grads = lambda up: torch.autograd.grad(y, leaves, up, retain_graph=True)
+    for a, r in zip(grads(torch._neg_view(dy)), grads(-dy)):
+        assert torch.equal(a, r)
+    zero = torch._efficientzerotensor(y.shape, dtype=y.dtype, device=y.device)
+    for a in grads(zero):
+        assert not a.any()

@@ -264,6 +264,8 @@ def test_tensors_with_a_tangent_do_not_take_the_native_path():
     native = tt._native()
     x = torch.randn(3)
     assert native.plain_eager([x, x.clone().requires_grad_(True)])
+    for lazy in (torch._neg_view(x), torch._efficientzerotensor(3), torch.randn(3, dtype=torch.cfloat).conj()):
+        assert not native.plain_eager([lazy])  # (nor do tensors whose memory does not hold their numbers)
     with fwad.dual_level():
         assert native.plain_eager([x])
         assert not native.plain_eager([x, fwad.make_dual(x, torch.ones_like(x))])

@@ -212,11 +212,19 @@ Forward forward(Tensor q, Tensor k, Tensor v, const Tensor& b, const Tensor& mas
   return f;
 }
 
+// The upstream gradient as numbers in memory: autograd may hand a node a lazily negated view, or a
+// zero tensor without any.
+Tensor materialized(const Tensor& g) {
+  if (g._is_zerotensor()) return at::zeros(g.sizes(), g.options());
+  return g.is_neg() ? g.resolve_neg() : g;
+}
+
 using Grads = std::array<Tensor, 4>;
 
 Grads backward(Tensor dout, Tensor q, Tensor k, Tensor v, const Tensor& b, Tensor o, Tensor lse, const Tensor& mask, const Tensor& saved = Tensor()) {
   const c10::DeviceGuard guard(q.device());
   const Shape s = shape_of(q);
+  dout = materialized(dout);
   if (dout.scalar_type() != q.scalar_type()) dout = dout.to(q.scalar_type());
   dout = vector_ready(broadcast_rows(dout));
   o = o.contiguous();
@@ -293,7 +301,7 @@ bool plain_eager(std::initializer_list<const Tensor*> tensors) {
   if (c10::impl::TorchDispatchModeTLS::stack_len() > 0) return false;
   for (const Tensor* t : tensors)
     if (!t->defined() || t->key_set().has_any(c10::DispatchKeySet({DispatchKey::Python, DispatchKey::FuncTorchGradWrapper, DispatchKey::FuncTorchBatched})) ||
-        t->layout() != at::kStrided || t->is_neg() || t->is_conj() || t->_fw_grad(/*level=*/0).defined())
+        t->layout() != at::kStrided || t->is_neg() || t->is_conj() || t->_is_zerotensor() || t->_fw_grad(/*level=*/0).defined())
       return false;
   return true;
 }
@@ -415,11 +423,11 @@ std::pair<Tensor, BlockState> block_forward(const Tensor& x_in, const Tensor& ma
 }
 
 // dx (undefined unless wanted) and the gradients of the parameters (undefined unless wanted)
-std::pair<Tensor, Params> block_backward(const Tensor& dy_in, const Tensor& x_in, const Tensor& mask, const Params& p, const BlockState& st, int64_t h,
+std::pair<Tensor, Params> block_backward(const Tensor& dy_lazy, const Tensor& x_in, const Tensor& mask, const Params& p, const BlockState& st, int64_t h,
                                          int64_t d, bool ending, bool want_dx, bool want_dw) {
   const c10::DeviceGuard guard(x_in.device());
   const BlockShape s(x_in, h, d, ending);
-  const Tensor x = dense(x_in), dy = dense(dy_in.scalar_type() == x.scalar_type() ? dy_in : dy_in.to(x.scalar_type()));
+  const Tensor dy_in = materialized(dy_lazy), x = dense(x_in), dy = dense(dy_in.scalar_type() == x.scalar_type() ? dy_in : dy_in.to(x.scalar_type()));
   const auto opt = x.options();
   hipStream_t stream = stream_of(x);
   const int64_t rows = s.b * s.n * s.n, hd = h * d;
@@ -533,7 +541,7 @@ Tensor gate_forward(const Tensor& o_in, const Tensor& g_in) {
 
 std::pair<Tensor, Tensor> gate_backward(const Tensor& dy_in, const Tensor& o_in, const Tensor& g_in) {
   const c10::DeviceGuard guard(o_in.device());
-  const Tensor dy = dy_in.contiguous(), o = o_in.contiguous(), g = g_in.contiguous();
+  const Tensor dy = materialized(dy_in).contiguous(), o = o_in.contiguous(), g = g_in.contiguous();
   const GateShape s(o);
   Tensor dout = at::empty_like(o), dg = at::empty_like(g);
   if (dy.numel())
