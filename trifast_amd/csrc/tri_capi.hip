@@ -107,8 +107,22 @@ __device__ __forceinline__ void mask_prep_rows64(const MaskPrepArgs& a, int b, i
   if (wave == 0 && live) a.rowflag[(int64_t)b * a.n + i] = row_kept ? 0 : 1;
 }
 
+// A bias of -inf as the lowest finite number of a 16-bit type.  The kernels that add a bias tile
+// through the matrix pipe multiply it by a selection of zeros and sqrt(d), and 0 * -inf is NaN; a score
+// with the lowest number in it has the probability 0 all the same.  (bf16: times sqrt(d) it is -inf again.)
+template <typename T>
+__device__ __forceinline__ T finite_bias(T x) {
+  if constexpr (sizeof(T) == 2) {
+    constexpr uint16_t kInf = std::is_same_v<T, _Float16> ? 0xfc00 : 0xff80;
+    const uint16_t u = __builtin_bit_cast(uint16_t, x);
+    return __builtin_bit_cast(T, (uint16_t)(u == kInf ? kInf - 1 : u));
+  } else {
+    return x;
+  }
+}
+
 // Bias: re-tile bias[b, h, j, k] (any strides) into the register layouts of the kernels
-// (see BiasPrepArgs), zero-padded to whole tiles.  A wave takes one 32 x 32 tile: it comes in with
+// (see BiasPrepArgs), zero-padded to whole tiles, -inf made finite.  A wave takes one 32 x 32 tile: it comes in with
 // 8-element loads along whichever of j and k is contiguous, and leaves LDS in both layouts.
 template <typename T>
 constexpr int kBiasLd = sizeof(T) == 4 ? 36 : 40;  // (rows of whole 16-byte pieces, off the bank period)
@@ -139,7 +153,7 @@ __device__ __forceinline__ void bias_prep_tile(const BiasPrepArgs& a, int bh, in
         for (int e = 0; e < 8; ++e) v[e] = (row < a.N && col + e < a.N) ? p[e * s_col] : (T)0.f;
       }
 #pragma unroll
-      for (int e = 0; e < 8; ++e) lds[along_j ? (c + e) * LD + r : r * LD + c + e] = v[e];
+      for (int e = 0; e < 8; ++e) lds[along_j ? (c + e) * LD + r : r * LD + c + e] = finite_bias(v[e]);
     }
   }
   __syncthreads();
