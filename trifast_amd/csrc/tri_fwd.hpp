@@ -720,12 +720,12 @@ __global__ __launch_bounds__(NW * 64, (R * ((BKF % kFwdFast) / 32) >= 8 || D * s
 #pragma unroll
             for (int v = 2; v < 16; ++v) mx = fmaxf(mx, sc_cur[v]);
             mx = half_max(mx);
-            // A row that attends to no key of this tile (the same for all its queries): every
-            // score is the mask value alone.  The tile then adds nothing and must not become
+            // A row that attends to no key of this tile (its keep word says so; the same for all its
+            // queries): every score is the mask value.  The tile then adds nothing and must not become
             // the reference: exp2(c * score - reference) would be exp2 of the rounding error of
             // two numbers of the mask value's size.  (With a reference from real scores such a
             // tile's probabilities are exactly zero and it never gets here.)
-            const bool no_key = MASKED && mx < 2.0f * E::kMaskElem;
+            const bool no_key = MASKED && kwc[r] == 0u;
             const float mcn = no_key ? mc[r] : fmaxf(mc[r], mx * c);
             const float alpha = fast_exp2(mc[r] - mcn);
 #pragma unroll
