@@ -24,6 +24,7 @@
 
 #include "tri_args.hpp"
 #include "tri_common.hpp"
+#include "tri_f32_plain.hpp"
 #include "tri_tile.hpp"
 
 namespace tri {
@@ -38,7 +39,7 @@ constexpr int bwd_q_lds_bytes(int D, int es, int NW, int R, int BK) {
 }
 
 template <typename T, int D, int NW, int R, int BK>
-__global__ __launch_bounds__(NW * 64, (R >= 4 || D * sizeof(T) > 256) ? 1 : (sizeof(T) == 2 && R == 1 && BK == 32 && D <= 64) ? 3 : 2) void tri_bwd_q_kernel(const BwdArgs a) {
+__global__ __launch_bounds__(NW * 64, (R >= 4 || D * sizeof(T) > 256) ? 1 : (R == 1 && BK == 32 && D <= (sizeof(T) == 2 ? 64 : 16)) ? 3 : 2) void tri_bwd_q_kernel(const BwdArgs a) {
   using E = Elem<T>;
   using frag = typename E::frag;
   using Tile = typename OperandOffsets<T, D>::Tile;
@@ -407,13 +408,23 @@ __global__ __launch_bounds__(NW * 64, (R >= 4 || D * sizeof(T) > 256) ? 1 : (siz
   else if (!any_flagged) stage_loop(std::integral_constant<int, kMasked>{});
   else stage_loop(std::integral_constant<int, kGeneral>{});
 
-  if (!wave_active) return;
+  float check = 0.f;
+  if (wave_active) {
 #pragma unroll
-  for (int r = 0; r < R; ++r) {
-    const int i = i0 + r;
-    if (i >= N) continue;
-    T* dqrow = reinterpret_cast<T*>(a.dq) + b * a.sdq.b + h * a.sdq.h + i * a.sdq.i + j * a.sdq.j;
-    store_rows_any<T, D, DM>(dqrow, dqacc[r], a.scale, g, j < N);
+    for (int r = 0; r < R; ++r) {
+      const int i = i0 + r;
+      if (i >= N) continue;
+      T* dqrow = reinterpret_cast<T*>(a.dq) + b * a.sdq.b + h * a.sdq.h + i * a.sdq.i + j * a.sdq.j;
+      store_rows_any<T, D, DM>(dqrow, dqacc[r], a.scale, g, j < N);
+      if constexpr (sizeof(T) == 4) {
+#pragma unroll
+        for (int mt = 0; mt < DM; ++mt) check = finite_check(dqacc[r][mt], check);
+      }
+    }
+  }
+  if constexpr (sizeof(T) == 4) {
+    if (workgroup_not_finite<NW>(check, tri_smem, wave, lane))
+      for (int r = 0; r < R && i0 + r < N; ++r) plain_dq_row<D, NW * 32>(a, bh, i0 + r, bx * (NW * 32), tid);
   }
 }
 
