@@ -28,7 +28,8 @@ import time
 import torch
 
 PEAK_BF16_TFLOPS = 2500.0  # MI355X dense bf16/fp16 MFMA
-PEAK_F32_TFLOPS = 157.3
+# fp32 products run as six products of bf16 parts each (csrc/tri_common.hpp: Elem<float>)
+PEAK_F32_TFLOPS = PEAK_BF16_TFLOPS / 6
 PEAK_HBM_GBS = 8000.0
 
 # HBM bytes per launch (fetch + write) of the kernels of workload M with the tiles the

@@ -2,6 +2,7 @@
 validation, stride handling, the tile cache and the tune CLI."""
 
 import json
+from pathlib import Path
 
 import pytest
 import torch
@@ -281,3 +282,13 @@ def test_nothing_takes_the_native_path_while_torch_jit_traces():
 
     torch.jit.trace(fn, (torch.randn(3),), check_trace=False)
     assert seen == [False] and tt._native().plain_eager([torch.randn(3)])
+
+
+def test_bench_prices_fp32_by_the_products_it_runs_as():
+    import re
+
+    import bench
+
+    src = (Path(tt.__file__).parent / "csrc" / "tri_common.hpp").read_text()
+    body = re.search(r"mfma\(const frag& a, const frag& b, f32x16 c\) \{(.*?)\n  \}", src, re.S).group(1)
+    assert bench.PEAK_F32_TFLOPS == bench.PEAK_BF16_TFLOPS / body.count("mfma(a.")
