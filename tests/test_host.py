@@ -292,3 +292,19 @@ def test_bench_prices_fp32_by_the_products_it_runs_as():
     src = (Path(tt.__file__).parent / "csrc" / "tri_common.hpp").read_text()
     body = re.search(r"mfma\(const frag& a, const frag& b, f32x16 c\) \{(.*?)\n  \}", src, re.S).group(1)
     assert bench.PEAK_F32_TFLOPS == bench.PEAK_BF16_TFLOPS / body.count("mfma(a.")
+
+
+@pytest.mark.parametrize("source,flags", [
+    ("tri_bwd_b.hip", ("-DTRI_DB_TIMING",)),
+    ("tri_bwd_b.hip", ("-DTRI_DB_TIMING", "-DTRI_DB_TIMING_LOADS=2")),
+    ("tri_bwd_row_bf16.hip", ("-DTRI_ROW_TIMING",)),
+], ids=["db", "db_loads", "row"])
+def test_probe_builds_of_the_kernels_compile(source, flags):
+    """The builds that time the kernels from inside (benchmark/microbench) keep up with the kernels."""
+    import subprocess
+
+    from trifast_amd import build
+
+    cmd = [build._hipcc(), *build.HIPCC_FLAGS, *flags, "-DTRI_DEV_ONLY_BF16_D32", "--cuda-device-only", "-fsyntax-only", "-I", str(build.CSRC), str(build.CSRC / source)]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    assert res.returncode == 0, res.stderr[-2000:]

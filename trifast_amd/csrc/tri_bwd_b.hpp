@@ -767,7 +767,8 @@ __global__ __launch_bounds__(GJ * GK * 64) void tri_bwd_b_kernel(const BwdArgs a
         const uint64_t t_clk1 = __builtin_amdgcn_s_memtime(), t_real1 = __builtin_amdgcn_s_memrealtime();
         asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
         if (lane == 0) {
-          uint64_t* rec = reinterpret_cast<uint64_t*>(a.db) + ((int64_t)L * NW + wave) * 4;
+          const int64_t L = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
+          uint64_t* rec = reinterpret_cast<uint64_t*>(a.db) + (L * NW + wave) * 4;
           rec[0] = t_clk1 - t_clk0;
           rec[1] = t_wait;
           rec[2] = t_barrier;
