@@ -74,18 +74,6 @@ def _j_stride_ok(t: torch.Tensor, st: list[int]) -> bool:
     return t.dim() != 5 or 0 <= st[3] * t.element_size() < (1 << 24)
 
 
-def _broadcast_rows(t: torch.Tensor) -> torch.Tensor:
-    """An upstream gradient that is one value or one [d] row expanded over b, h, i, j
-    (``o.sum().backward()`` gives such a tensor, all strides 0) becomes a single
-    16-byte-aligned row read through zero strides: nothing of q's size is
-    materialised."""
-    st = _strides(t)
-    if any(st[:-1]) or t.dim() != 5:
-        return t
-    row = t[(0,) * 4].contiguous()  # [d] elements
-    return row.expand(t.shape)
-
-
 def _grad_like(t: torch.Tensor) -> torch.Tensor:
     """Empty gradient buffer for input ``t``: laid out like ``t`` when ``t`` is dense
     and the kernels can write that layout (d contiguous, 16-byte rows), so that a
