@@ -208,6 +208,14 @@ def test_row_resident_tiles_in_the_library_tables():
     assert default(512, 32, _lib.F32) not in fused and default(64, 128, _lib.BF16) not in fused
 
 
+def test_default_forward_tiles_of_128_byte_rows():
+    """The scheduled loop (tile 6) from more than 256 keys on, its general twin below."""
+    pick = lambda n, code, d=64: _lib.load().trifast_default_tile(_lib.KERNEL_FWD, n, 8, d, code)
+    for code in (_lib.BF16, _lib.F16):
+        assert [pick(n, code) for n in (65, 192, 256, 257, 300, 384, 768)] == [4, 4, 4, 6, 6, 6, 6]
+    assert pick(300, _lib.F32, 32) == 4  # (fp32 has no scheduled loop)
+
+
 def test_tune_cli_flags_and_sweep():
     p = tune.build_parser()
     a = p.parse_args([])

@@ -436,14 +436,17 @@ int trifast_default_tile(int kernel, int64_t n, int64_t h, int64_t d, int dtype)
   switch (kernel) {
     case TRIFAST_KERNEL_FWD:
       // pair rows that share a bias tile: one for the smallest and the widest rows; two for
-      // 128-byte rows (16-bit rows of 384 keys and more with the scheduled loop: at
-      // n = 768, h = 8 1.51 against 1.67 ms, at n = 384, b = 2 0.50 against 0.51) and for 64-byte
-      // 16-bit rows of fewer than 768 keys; four above that, with the scheduled loop (n = 1531
-      // 3.4 against 4.0 ms); 32-byte rows: four, or from 256 keys on two with 64 keys per stage
-      // and from 512 on four with the scheduled loop (n = 700 0.32 against 0.37 ms)
+      // 128-byte rows and for 64-byte 16-bit rows of fewer than 768 keys; four above that, with the
+      // scheduled loop (n = 1531 3.4 against 4.0 ms); 32-byte rows: four, or from 256 keys on two
+      // with 64 keys per stage and from 512 on four with the scheduled loop (n = 700 0.32 against
+      // 0.37 ms).  16-bit 128-byte rows take the scheduled loop from more than 256 keys on: with a
+      // random mask it is 3-8 % faster there (n = 320, h = 8 171 against 162 us; 384 239 / 229; 576
+      // 733 / 684), on ragged rows 7-13 % (300 165 / 151; 390 319 / 292) and even without either
+      // (384 219 / 221, 576 664 / 657, scattering by 2-4 %); up to 256 keys rows of whole tiles
+      // lose up to 4 % with it (192 46.6 / 48.3, 256 76.7 / 77.8; masked 50.9 / 51.0, 82.8 / 80.3).
       if (n <= 64 || row_bytes >= 256) pick = 0;
       else if (dtype == TRIFAST_F32) pick = 4;
-      else if (row_bytes == 128) pick = n < 384 ? 4 : 6;
+      else if (row_bytes == 128) pick = n > 256 ? 6 : 4;
       else if (row_bytes == 64) pick = n < 768 ? 4 : 7;
       else pick = n >= 512 ? 7 : n >= 256 ? 1 : 3;
       break;
