@@ -89,6 +89,8 @@ def main():
 
     regular_ms = timed(regular)
     probe_ms = timed(probe)
+    if args.loads == 1 and probe_ms < 0.95 * regular_ms:
+        sys.exit(f"the probe build takes {probe_ms:.3f} ms, the library's kernel {regular_ms:.3f}: it has lost work that the kernel does")
     db.zero_()  # (the library's kernel wrote db; the probe writes its records only)
     run(probe, _lib.KERNEL_BWD_B, args.tile)
     torch.cuda.synchronize()

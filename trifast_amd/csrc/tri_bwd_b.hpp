@@ -766,6 +766,13 @@ __global__ __launch_bounds__(GJ * GK * 64) void tri_bwd_b_kernel(const BwdArgs a
       {
         const uint64_t t_clk1 = __builtin_amdgcn_s_memtime(), t_real1 = __builtin_amdgcn_s_memrealtime();
         asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+        // (the sums are not stored here, and without a use the compiler leaves their arithmetic out)
+#pragma unroll
+        for (int tj = 0; tj < WJ; ++tj)
+#pragma unroll
+          for (int tk = 0; tk < WK; ++tk)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) asm volatile("" : : "v"(dbacc[tj][tk][v]));
         if (lane == 0) {
           const int64_t L = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
           uint64_t* rec = reinterpret_cast<uint64_t*>(a.db) + (L * NW + wave) * 4;
