@@ -1033,7 +1033,7 @@ __global__ __launch_bounds__(GJ * GK * 64) void tri_bwd_b_split_kernel(const Bwd
 #pragma unroll
     for (int tj = 0; tj < WJ; ++tj)
 #pragma unroll
-      for (int tk = 0; tk < WK; ++tk) check = finite_check(dbacc[tj][tk], check);
+      for (int tk = 0; tk < WK; ++tk) check = finite_check<16>(dbacc[tj][tk], check);
   }
   if (workgroup_not_finite<NW>(check, tri_smem, wave, lane)) plain_db_block<D, BJ, BKB, NW * 64>(a, bh, blk.chunk, blk.j, blk.k, i_begin, i_end, tid);
 }

@@ -421,7 +421,7 @@ __global__ __launch_bounds__(NW * 64, (bwd_kv_min_waves<T, D, R, BJ>())) void tr
       store_rows_any<T, D, DM>(dvrow, dvacc[r], 1.0f, g, key < N);
       if constexpr (sizeof(T) == 4) {
 #pragma unroll
-        for (int mt = 0; mt < DM; ++mt) check = finite_check(dvacc[r][mt], finite_check(dkacc[r][mt], check));
+        for (int mt = 0; mt < DM; ++mt) check = finite_check<(D < 32 ? 8 : 16)>(dvacc[r][mt], finite_check<(D < 32 ? 8 : 16)>(dkacc[r][mt], check));
       }
     }
   }

@@ -418,7 +418,7 @@ __global__ __launch_bounds__(NW * 64, (R >= 4 || D * sizeof(T) > 256) ? 1 : (R =
       store_rows_any<T, D, DM>(dqrow, dqacc[r], a.scale, g, j < N);
       if constexpr (sizeof(T) == 4) {
 #pragma unroll
-        for (int mt = 0; mt < DM; ++mt) check = finite_check(dqacc[r][mt], check);
+        for (int mt = 0; mt < DM; ++mt) check = finite_check<(D < 32 ? 8 : 16)>(dqacc[r][mt], check);
       }
     }
   }

@@ -18,10 +18,13 @@
 
 namespace tri {
 
-// 0 as long as everything that went in is finite
+// 0 as long as everything that went in is finite.  VALUES: how many of a lane's 16 values stand for
+// something (8 in the output tile of head dim 16, whose upper rows no operand is defined for and
+// which hold whatever the registers did).
+template <int VALUES>
 TRI_DEV float finite_check(const f32x16& v, float acc) {
 #pragma unroll
-  for (int e = 0; e < 16; ++e) acc = __builtin_fmaf(v[e], 0.f, acc);
+  for (int e = 0; e < VALUES; ++e) acc = __builtin_fmaf(v[e], 0.f, acc);
   return acc;
 }
 

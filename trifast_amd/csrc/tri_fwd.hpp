@@ -859,7 +859,7 @@ __global__ __launch_bounds__(NW * 64, (R * ((BKF % kFwdFast) / 32) >= 8 || D * s
       if constexpr (sizeof(T) == 4) {
         check = __builtin_fmaf(ltot, 0.f, check);
 #pragma unroll
-        for (int mt = 0; mt < DM; ++mt) check = finite_check(oacc[r][mt], check);
+        for (int mt = 0; mt < DM; ++mt) check = finite_check<(D < 32 ? 8 : 16)>(oacc[r][mt], check);
       }
     }
   }
