@@ -1027,15 +1027,14 @@ __global__ __launch_bounds__(GJ * GK * 64) void tri_bwd_b_split_kernel(const Bwd
       __syncthreads();
     }
   }
+  if (!wave_live) return;
+  store_db<T, WJ, WK>(a, dbacc, bh, blk.chunk, j_wave, k_wave, jl, g);
   float check = 0.f;
-  if (wave_live) {
-    store_db<T, WJ, WK>(a, dbacc, bh, blk.chunk, j_wave, k_wave, jl, g);
 #pragma unroll
-    for (int tj = 0; tj < WJ; ++tj)
+  for (int tj = 0; tj < WJ; ++tj)
 #pragma unroll
-      for (int tk = 0; tk < WK; ++tk) check = finite_check<16>(dbacc[tj][tk], check);
-  }
-  if (workgroup_not_finite<NW>(check, tri_smem, wave, lane)) plain_db_block<D, BJ, BKB, NW * 64>(a, bh, blk.chunk, blk.j, blk.k, i_begin, i_end, tid);
+    for (int tk = 0; tk < WK; ++tk) check = finite_check<16>(dbacc[tj][tk], check);
+  if (__any(!(check == 0.f))) plain_db_block<D, WJ * 32, WK * 32>(reloaded_args<BwdArgs>(), bh, blk.chunk, j_wave, k_wave, i_begin, i_end, lane);
 }
 
 // db = sum over chunks of the fp32 partials, in chunk order.  The chunks' loads are in flight

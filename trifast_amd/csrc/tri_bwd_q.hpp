@@ -408,23 +408,24 @@ __global__ __launch_bounds__(NW * 64, (R >= 4 || D * sizeof(T) > 256) ? 1 : (R =
   else if (!any_flagged) stage_loop(std::integral_constant<int, kMasked>{});
   else stage_loop(std::integral_constant<int, kGeneral>{});
 
+  if (!wave_active) return;
   float check = 0.f;
-  if (wave_active) {
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const int i = i0 + r;
-      if (i >= N) continue;
-      T* dqrow = reinterpret_cast<T*>(a.dq) + b * a.sdq.b + h * a.sdq.h + i * a.sdq.i + j * a.sdq.j;
-      store_rows_any<T, D, DM>(dqrow, dqacc[r], a.scale, g, j < N);
-      if constexpr (sizeof(T) == 4) {
+  for (int r = 0; r < R; ++r) {
+    const int i = i0 + r;
+    if (i >= N) continue;
+    T* dqrow = reinterpret_cast<T*>(a.dq) + b * a.sdq.b + h * a.sdq.h + i * a.sdq.i + j * a.sdq.j;
+    store_rows_any<T, D, DM>(dqrow, dqacc[r], a.scale, g, j < N);
+    if constexpr (sizeof(T) == 4) {
 #pragma unroll
-        for (int mt = 0; mt < DM; ++mt) check = finite_check<(D < 32 ? 8 : 16)>(dqacc[r][mt], check);
-      }
+      for (int mt = 0; mt < DM; ++mt) check = finite_check<(D < 32 ? 8 : 16)>(dqacc[r][mt], check);
     }
   }
   if constexpr (sizeof(T) == 4) {
-    if (workgroup_not_finite<NW>(check, tri_smem, wave, lane))
-      for (int r = 0; r < R && i0 + r < N; ++r) plain_dq_row<D, NW * 32>(a, bh, i0 + r, bx * (NW * 32), tid);
+    if (__any(!(check == 0.f))) {
+      const BwdArgs all = reloaded_args<BwdArgs>();
+      for (int r = 0; r < R && i0 + r < all.N; ++r) plain_dq_row<D>(all, bh, i0 + r, j_wave, lane);
+    }
   }
 }
 

@@ -1,14 +1,15 @@
-// fp32 workgroups whose results are not all finite, computed again number by number.
+// Results of an fp32 wave that are not all finite, computed again number by number.
 //
 // The fp32 kernels run on three bf16 parts per number (see Elem<float>).  An infinity has no remainder
 // there, and its products with the parts of another number, zeros and either sign among them, add up
 // to NaN, also in the number that was split beside it; a number that rounds to infinity in bf16 and
 // products past the end of fp32 go the same way.  fp32 itself knows better: an infinite value makes its
-// own column infinite, a score of -inf has the probability zero.  So each kernel looks at what it
-// has computed (a handful of instructions per workgroup), and a workgroup that finds something not
-// finite does its part again here, with fp32 multiply-adds and the same formulas.
+// own column infinite, a score of -inf has the probability zero.  So each wave looks at what it has
+// computed (one instruction per result register), and one that finds something not
+// finite does its part again here, with fp32 multiply-adds and the same formulas.  (Wave by wave: to
+// agree on it the waves of a workgroup would have to meet, which took 1.7 % of a step at n = 110.)
 //
-// Only such workgroups come here, and what bounds these loops is of no interest; they keep few numbers
+// Only such waves come here, and what bounds these loops is of no interest; they keep few numbers
 // alive so that they do not add to the registers of the kernel around them (with the
 // kernels' own code in a second version for the fp32 matrix pipe in their place, the forward at
 // d = 32 went from three waves per SIMD to two).
@@ -28,19 +29,21 @@ TRI_DEV float finite_check(const f32x16& v, float acc) {
   return acc;
 }
 
-// Whether some wave of the workgroup has something that is not finite (`check` is not 0): the same
-// answer for all of them.  Every wave calls it; none uses LDS any more afterwards.
-template <int NW>
-TRI_DEV bool workgroup_not_finite(float check, unsigned char* smem, int wave, int lane) {
-  uint32_t* const words = reinterpret_cast<uint32_t*>(smem);
-  const bool bad = __any(!(check == 0.f));
-  __syncthreads();
-  if (lane == 0) words[wave] = bad;
-  __syncthreads();
-  uint32_t any = 0;
+// The kernel's arguments, read again from where the launch put them: what the loops below need of
+// them is not kept in scalar registers through the kernel's own work (kept, it spilled up to 40 of
+// them, and the fp32 step at n = 110, d = 64 took 1.6 % longer).
+template <typename Args>
+TRI_DEV Args reloaded_args() {
+  static_assert(sizeof(Args) % 4 == 0);
+  typedef const __attribute__((address_space(4))) uint32_t* words;
+  uint64_t at = (uint64_t)(uintptr_t)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(at));  // (opaque: these are not the loads the kernel has made)
+  struct {
+    uint32_t w[sizeof(Args) / 4];
+  } copy;
 #pragma unroll
-  for (int w = 0; w < NW; ++w) any |= words[w];
-  return __builtin_amdgcn_readfirstlane(any) != 0;
+  for (unsigned i = 0; i < sizeof(Args) / 4; ++i) copy.w[i] = ((words)(uintptr_t)at)[i];
+  return __builtin_bit_cast(Args, copy);
 }
 
 // x . y, rows of D numbers (rolled: nothing of a row stays in registers)
@@ -107,12 +110,12 @@ struct PlainRow {
   }
 };
 
-// Queries j_blk .. j_blk + JB - 1 of one pair row by 2 JB threads: thread t takes query t % JB and half of
-// the columns.
-template <int D, int JB>
-TRI_DEV void plain_fwd_row(const FwdArgs& a, int bh, int i, int j_blk, int tid) {
+// Queries j_blk .. j_blk + 31 of one pair row by a wave: lane t takes query t % 32 and half of the
+// columns.
+template <int D>
+TRI_DEV void plain_fwd_row(const FwdArgs& a, int bh, int i, int j_blk, int lane) {
   constexpr int W = D / 2 < 32 ? D / 2 : 32;
-  const int j = j_blk + tid % JB, half = tid / JB;
+  const int j = j_blk + lane % 32, half = lane / 32;
   if (j >= a.N) return;
   const PlainRow<D, FwdArgs> row(a, bh, i);
   float top = kNeg, sum = 0.f;
@@ -145,11 +148,11 @@ TRI_DEV const float* plain_dout(const BwdArgs& a, int bh, int i) {
   return reinterpret_cast<const float*>(a.dout) + bh / a.H * a.sdo.b + bh % a.H * a.sdo.h + i * a.sdo.i;
 }
 
-// dq of queries j_blk .. j_blk + JB - 1, threads as above
-template <int D, int JB>
-TRI_DEV void plain_dq_row(const BwdArgs& a, int bh, int i, int j_blk, int tid) {
+// dq of queries j_blk .. j_blk + 31, lanes as above
+template <int D>
+TRI_DEV void plain_dq_row(const BwdArgs& a, int bh, int i, int j_blk, int lane) {
   constexpr int W = D / 2 < 32 ? D / 2 : 32;
-  const int j = j_blk + tid % JB, half = tid / JB;
+  const int j = j_blk + lane % 32, half = lane / 32;
   if (j >= a.N) return;
   const PlainRow<D, BwdArgs> row(a, bh, i);
   const float* dout = plain_dout(a, bh, i) + j * a.sdo.j;
@@ -168,12 +171,12 @@ TRI_DEV void plain_dq_row(const BwdArgs& a, int bh, int i, int j_blk, int tid) {
   }
 }
 
-// dk and dv of keys k_blk .. k_blk + KB - 1: thread t takes key t % KB, and dk or dv
-template <int D, int KB>
-TRI_DEV void plain_dkv_row(const BwdArgs& a, int bh, int i, int k_blk, int tid) {
+// dk and dv of keys k_blk .. k_blk + 31: lane t takes key t % 32, and dk or dv
+template <int D>
+TRI_DEV void plain_dkv_row(const BwdArgs& a, int bh, int i, int k_blk, int lane) {
   constexpr int W = D < 32 ? D : 32;
-  const int key = k_blk + tid % KB;
-  const bool is_dk = tid < KB;
+  const int key = k_blk + lane % 32;
+  const bool is_dk = lane < 32;
   if (key >= a.N) return;
   const PlainRow<D, BwdArgs> row(a, bh, i);
   const float* dout = plain_dout(a, bh, i);
@@ -194,11 +197,11 @@ TRI_DEV void plain_dkv_row(const BwdArgs& a, int bh, int i, int k_blk, int tid) 
   }
 }
 
-// db of a block of queries and keys, summed over the pair rows of its chunk in order; the threads take
-// the pairs of the block in turn
-template <int D, int BJ, int BKB, int THREADS>
-TRI_DEV void plain_db_block(const BwdArgs& a, int bh, int chunk, int j_blk, int k_blk, int i_begin, int i_end, int tid) {
-  for (int x = tid; x < BJ * BKB; x += THREADS) {
+// db of a block of queries and keys, summed over the pair rows of its chunk in order; the lanes take the
+// pairs of the block in turn
+template <int D, int BJ, int BKB>
+TRI_DEV void plain_db_block(const BwdArgs& a, int bh, int chunk, int j_blk, int k_blk, int i_begin, int i_end, int lane) {
+  for (int x = lane; x < BJ * BKB; x += 64) {
     const int j = j_blk + x % BJ, key = k_blk + x / BJ;
     if (j >= a.N || key >= a.N) continue;
     float acc = 0.f;

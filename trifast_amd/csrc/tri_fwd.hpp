@@ -842,30 +842,31 @@ __global__ __launch_bounds__(NW * 64, (R * ((BKF % kFwdFast) / 32) >= 8 || D * s
     else stage_loop(std::integral_constant<int, kGeneral>{});
   }
 
+  if (!wave_active) return;
   float check = 0.f;
-  if (wave_active) {
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const int i = i0 + r;
-      const float ltot = half_sum(lrun[r]);
-      if (i >= N) continue;  // (wave-uniform; the lanes of queries past the end stay for the exchange inside the store)
-      T* orow = reinterpret_cast<T*>(a.o) + (((int64_t)bh * N + i) * N) * D;
-      store_rows_any<T, D, DM>(orow + (int64_t)j * D, oacc[r], 1.0f / ltot, g, j < N);
-      if (g == 0 && j < N) {
-        float lse = kLn2 * (mc[r] + fast_log2(ltot));
-        if (flagged[r]) lse = a.neg_inf + lse;
-        a.lse[((int64_t)bh * N + i) * N + j] = lse;
-      }
-      if constexpr (sizeof(T) == 4) {
-        check = __builtin_fmaf(ltot, 0.f, check);
+  for (int r = 0; r < R; ++r) {
+    const int i = i0 + r;
+    const float ltot = half_sum(lrun[r]);
+    if (i >= N) continue;  // (wave-uniform; the lanes of queries past the end stay for the exchange inside the store)
+    T* orow = reinterpret_cast<T*>(a.o) + (((int64_t)bh * N + i) * N) * D;
+    store_rows_any<T, D, DM>(orow + (int64_t)j * D, oacc[r], 1.0f / ltot, g, j < N);
+    if (g == 0 && j < N) {
+      float lse = kLn2 * (mc[r] + fast_log2(ltot));
+      if (flagged[r]) lse = a.neg_inf + lse;
+      a.lse[((int64_t)bh * N + i) * N + j] = lse;
+    }
+    if constexpr (sizeof(T) == 4) {
+      check = __builtin_fmaf(ltot, 0.f, check);
 #pragma unroll
-        for (int mt = 0; mt < DM; ++mt) check = finite_check<(D < 32 ? 8 : 16)>(oacc[r][mt], check);
-      }
+      for (int mt = 0; mt < DM; ++mt) check = finite_check<(D < 32 ? 8 : 16)>(oacc[r][mt], check);
     }
   }
   if constexpr (sizeof(T) == 4) {
-    if (workgroup_not_finite<NW>(check, tri_smem, wave, lane))
-      for (int r = 0; r < R && i0 + r < N; ++r) plain_fwd_row<D, NW * 32>(a, bh, i0 + r, bx * (NW * 32), tid);
+    if (__any(!(check == 0.f))) {
+      const FwdArgs all = reloaded_args<FwdArgs>();
+      for (int r = 0; r < R && i0 + r < all.N; ++r) plain_fwd_row<D>(all, bh, i0 + r, j_wave, lane);
+    }
   }
 }
 
