@@ -51,7 +51,7 @@ struct py::detail::type_caster<PyTensor> {
   bool load(handle src, bool convert) {
     make_caster<Tensor> tensor;
     if (!tensor.load(src, convert)) return false;
-    value.t = cast_op<Tensor&>(tensor);
+    value.t = std::move(cast_op<Tensor&>(tensor));
     value.overrides = !THPVariable_CheckTypeExact(Py_TYPE(src.ptr()));
     return true;
   }
@@ -299,10 +299,11 @@ bool plain_eager(std::initializer_list<const Tensor*> tensors) {
   const auto tls = c10::impl::tls_local_dispatch_key_set();
   if (tls.included_.has(DispatchKey::Python) || tls.included_.has(DispatchKey::FuncTorchDynamicLayerFrontMode)) return false;
   if (c10::impl::TorchDispatchModeTLS::stack_len() > 0) return false;
+  // (lazily negated or conjugated tensors and zero tensors: their memory does not hold their numbers)
+  constexpr c10::DispatchKeySet kOther({DispatchKey::Python, DispatchKey::FuncTorchGradWrapper, DispatchKey::FuncTorchBatched, DispatchKey::Negative,
+                                        DispatchKey::Conjugate, DispatchKey::ZeroTensor});
   for (const Tensor* t : tensors)
-    if (!t->defined() || t->key_set().has_any(c10::DispatchKeySet({DispatchKey::Python, DispatchKey::FuncTorchGradWrapper, DispatchKey::FuncTorchBatched})) ||
-        t->layout() != at::kStrided || t->is_neg() || t->is_conj() || t->_is_zerotensor() || t->_fw_grad(/*level=*/0).defined())
-      return false;
+    if (!t->defined() || t->key_set().has_any(kOther) || t->layout() != at::kStrided || t->_fw_grad(/*level=*/0).defined()) return false;
   return true;
 }
 
