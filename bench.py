@@ -38,10 +38,10 @@ PEAK_HBM_GBS = 8000.0
 # as roofline.traffic when the benchmark runs that workload with that tile (keyed by the
 # tile's index in the library's table of the kernel).
 MEASURED_TRAFFIC_MIB = {
-    ("M", "_fwd", 7): 1537.0,
-    ("M", "_bwd_kv", 10): 2563.8,
+    ("M", "_fwd", 7): 1528.7,
+    ("M", "_bwd_kv", 10): 2560.0,
     ("M", "_bwd_b", 4): 1586.0,
-    ("M", "_bwd_b", 3): 1585.0,
+    ("M", "_bwd_b", 3): 1585.2,
 }
 
 # name -> (dtype, b, n, h, d, description)

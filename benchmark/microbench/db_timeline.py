@@ -95,7 +95,7 @@ def main():
     run(probe, _lib.KERNEL_BWD_B, args.tile)
     torch.cuda.synchronize()
     # one record per wave at the workgroup's linear index in the grid, whose last extent is
-    # the (batch*head, row chunk) groups (at most 8 chunks) padded to a multiple of 8; db was
+    # the (batch*head, row chunk) groups (at most 8 chunks beyond 128 keys) padded to a multiple of 8; db was
     # zero before the launch, so every other word still is
     blocks = ((n + info["BLOCK_J"] - 1) // info["BLOCK_J"]) * ((n + info["BLOCK_K"] - 1) // info["BLOCK_K"])
     slots = min(blocks * ((b * h * 8 + 7) // 8 * 8), db.numel() * db.element_size() // (8 * nw * 4))

@@ -16,8 +16,8 @@ struct FwdFamily {
         {4, 4, 32},  // 3: 128 queries x 4 rows, 32 keys per stage
         {4, 2, 32},  // 4: 128 queries x 2 rows, 32 keys per stage (fewer registers: 3 waves per SIMD)
         {8, 4, 32},  // 5: 256 queries x 4 rows, 32 keys per stage
-        {4, 2, 32 + kFwdFast},  // 6: tile 4 with the scheduled loop for workgroups without masked keys (16-bit types)
-        {4, 4, 32 + kFwdFast},  // 7: tile 3 with the scheduled loop for workgroups without masked keys (16-bit types)
+        {4, 2, 32 + kFwdFast},  // 6: tile 4 with the scheduled loop for workgroups without a fully masked row (16-bit types)
+        {4, 4, 32 + kFwdFast},  // 7: tile 3 with the scheduled loop for workgroups without a fully masked row (16-bit types)
     };
     return t[tile][which];
   }
@@ -27,7 +27,7 @@ struct FwdFamily {
     constexpr int BK = BKF0 % kFwdFast;
     constexpr int BKF = (sizeof(T) == 2 && R >= 2 && D <= 64) ? BKF0 : BK;
     // two stages of: K and V rows of the R pair rows + one packed bias tile per wave and key tile
-    // (or the three stages of the scheduled loop)
+    // (or the three or four stages of the scheduled loop)
     constexpr int lds = fwd_main_lds_bytes(D, (int)sizeof(T), NW, R, BKF);
     // R rows of accumulators and Q operands per wave must stay in registers
     constexpr int acc_regs = R * (((D + 31) / 32) * 16 + D / 2 * (int)sizeof(T) / 4);

@@ -45,8 +45,8 @@ namespace tri {
 constexpr float kLazy = 8.0f;
 constexpr float kLazyLimit = 256.0f;  // 2^kLazy
 
-// BKF: keys per stage of the general stage loop, plus kFwdFast when the workgroup may take
-// the scheduled loop below for rows without masked keys.
+// BKF: keys per stage of the general stage loop, plus kFwdFast when a workgroup without a fully
+// masked row takes the scheduled loop below.
 constexpr int kFwdFast = 256;
 // LDS bytes of the two loops (without the key-tile bitmaps that follow them)
 constexpr int fwd_stage_bytes(int D, int es, int NW, int R, int BK) { return 2 * R * BK * lds_row_bytes(D, es) + (es == 4 ? 0 : NW * (BK / 32) * 1024 * es) + 256; }
