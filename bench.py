@@ -254,7 +254,7 @@ def cpu_baseline(name: str, tensors, budget_s: float = 20.0):
     from oracle import triangle_oracle as orc
 
     dtype, b, n, h, d, _ = WORKLOADS[name]
-    # the host share of a one-GPU box is 16 cores, whatever the machine reports
+    # the host share of one GPU is 16 cores, whatever the machine reports
     cores = int(os.environ.get("OMP_NUM_THREADS", 0)) or min(os.cpu_count() or 1, 16)
     torch.set_num_threads(cores)
     q, k, v, bias, mask, do = tensors

@@ -1,6 +1,6 @@
 """CPU oracle for fused triangle self-attention.  TEST INFRASTRUCTURE ONLY.
 
-This module is a checker: it is imported by the tests, by the smoke check and by
+This module is imported by the tests, by the smoke check and by
 the CPU-baseline leg of the benchmark, and by nothing else.  The shipped operator
 never calls into it and has no CPU fallback.
 

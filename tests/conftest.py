@@ -14,7 +14,7 @@ os.environ.setdefault("TRIFAST_AUTOTUNE", "0")
 
 
 def pytest_configure(config):
-    config.addinivalue_line("markers", "gpu: needs a real MI355X (run with -m gpu on the GPU box)")
+    config.addinivalue_line("markers", "gpu: needs a real MI355X (run with -m gpu)")
 
 
 class _ForcedTiles:

@@ -145,7 +145,7 @@ def test_golden_fixtures(name):
             torch.testing.assert_close(got.double(), t[f"{key}_f64"], rtol=1e-4, atol=2e-5, msg=key + "_f64")
 
 
-# ------------------------------------------------- checker helpers, hand-computed
+# ------------------------------------------------- oracle helpers, hand-computed
 def test_cosine_similarity_hand_values():
     # (1,2,2).(2,1,2) = 8, both norms 3: cos = 8/9; orthogonal and opposite vectors
     a, b = torch.tensor([1.0, 2.0, 2.0]), torch.tensor([2.0, 1.0, 2.0])
