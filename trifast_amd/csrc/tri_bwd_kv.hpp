@@ -418,17 +418,18 @@ __global__ __launch_bounds__(NW * 64, (bwd_kv_min_waves<T, D, R, BJ>())) void tr
     T* dkrow = reinterpret_cast<T*>(a.dk) + b * a.sdk.b + h * a.sdk.h + i * a.sdk.i + key * a.sdk.j;
     T* dvrow = reinterpret_cast<T*>(a.dv) + b * a.sdv.b + h * a.sdv.h + i * a.sdv.i + key * a.sdv.j;
     store_rows_any<T, D, DM>(dkrow, dkacc[r], a.scale, g, key < N);
+    if constexpr (sizeof(T) == 4) {
+#pragma unroll
+      for (int mt = 0; mt < DM; ++mt) check = finite_check<(D < 32 ? 8 : 16)>(dkacc[r][mt], check);
+    }
     store_rows_any<T, D, DM>(dvrow, dvacc[r], 1.0f, g, key < N);
     if constexpr (sizeof(T) == 4) {
 #pragma unroll
-      for (int mt = 0; mt < DM; ++mt) check = finite_check<(D < 32 ? 8 : 16)>(dvacc[r][mt], finite_check<(D < 32 ? 8 : 16)>(dkacc[r][mt], check));
+      for (int mt = 0; mt < DM; ++mt) check = finite_check<(D < 32 ? 8 : 16)>(dvacc[r][mt], check);
     }
   }
   if constexpr (sizeof(T) == 4) {
-    if (__any(!(check == 0.f))) {
-      const BwdArgs all = reloaded_args<BwdArgs>();
-      for (int r = 0; r < R && i0 + r < all.N; ++r) plain_dkv_row<D>(all, bh, i0 + r, k_wave, lane);
-    }
+    if (__any(!(check == 0.f))) plain_dkv<D, R>(arg_words(), bh, i0, k_wave, fresh_lane());
   }
 }
 

@@ -422,10 +422,7 @@ __global__ __launch_bounds__(NW * 64, (R >= 4 || D * sizeof(T) > 256) ? 1 : (R =
     }
   }
   if constexpr (sizeof(T) == 4) {
-    if (__any(!(check == 0.f))) {
-      const BwdArgs all = reloaded_args<BwdArgs>();
-      for (int r = 0; r < R && i0 + r < all.N; ++r) plain_dq_row<D>(all, bh, i0 + r, j_wave, lane);
-    }
+    if (__any(!(check == 0.f))) plain_dq<D, R>(arg_words(), bh, i0, j_wave, fresh_lane());
   }
 }
 

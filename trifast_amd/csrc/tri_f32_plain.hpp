@@ -9,10 +9,11 @@
 // finite does its part again here, with fp32 multiply-adds and the same formulas.  (Wave by wave: to
 // agree on it the waves of a workgroup would have to meet, which took 1.7 % of a step at n = 110.)
 //
-// Only such waves come here, and what bounds these loops is of no interest; they keep few numbers
-// alive so that they do not add to the registers of the kernel around them (with the
-// kernels' own code in a second version for the fp32 matrix pipe in their place, the forward at
-// d = 32 went from three waves per SIMD to two).
+// Only such waves come here, and what bounds these loops is of no interest; a sum that has become NaN
+// stays so, and its loop ends there (n = 512: with v NaN throughout a step took 154 ms without that;
+// with q, k and v NaN it takes 2.9 with it, as for finite numbers).  They keep few numbers alive: the
+// kernels' own code in a second version for the fp32 matrix pipe in their place took the forward at
+// d = 32 from three waves per SIMD to two.
 #pragma once
 #include "tri_args.hpp"
 #include "tri_common.hpp"
@@ -29,20 +30,24 @@ TRI_DEV float finite_check(const f32x16& v, float acc) {
   return acc;
 }
 
-// The kernel's arguments, read again from where the launch put them: what the loops below need of
-// them is not kept in scalar registers through the kernel's own work (kept, it spilled up to 40 of
-// them, and the fp32 step at n = 110, d = 64 took 1.6 % longer).
+// What a kernel hands to the functions at the end of this file: where the launch put its arguments,
+// and the lane, neither of which it has to keep through its own work for that (kept, the
+// arguments spilled up to 40 scalar registers, and the fp32 step at n = 110, d = 64 took 1.6 % longer).
+typedef const __attribute__((address_space(4))) uint32_t* ArgWords;
+TRI_DEV ArgWords arg_words() { return (ArgWords)__builtin_amdgcn_kernarg_segment_ptr(); }
+TRI_DEV int fresh_lane() {
+  int lane;
+  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(lane));
+  return lane;
+}
 template <typename Args>
-TRI_DEV Args reloaded_args() {
+TRI_DEV Args read_args(ArgWords at) {
   static_assert(sizeof(Args) % 4 == 0);
-  typedef const __attribute__((address_space(4))) uint32_t* words;
-  uint64_t at = (uint64_t)(uintptr_t)__builtin_amdgcn_kernarg_segment_ptr();
-  asm volatile("" : "+s"(at));  // (opaque: these are not the loads the kernel has made)
   struct {
     uint32_t w[sizeof(Args) / 4];
   } copy;
 #pragma unroll
-  for (unsigned i = 0; i < sizeof(Args) / 4; ++i) copy.w[i] = ((words)(uintptr_t)at)[i];
+  for (unsigned i = 0; i < sizeof(Args) / 4; ++i) copy.w[i] = at[i];
   return __builtin_bit_cast(Args, copy);
 }
 
@@ -119,8 +124,11 @@ TRI_DEV void plain_fwd_row(const FwdArgs& a, int bh, int i, int j_blk, int lane)
   if (j >= a.N) return;
   const PlainRow<D, FwdArgs> row(a, bh, i);
   float top = kNeg, sum = 0.f;
-  for (int key = 0; key < a.N; ++key)
-    if (row.live(key)) top = fmaxf(top, row.score(j, key));
+  for (int key = 0; key < a.N && top == top; ++key)
+    if (row.live(key)) {
+      const float s = row.score(j, key);
+      top = s == s ? fmaxf(top, s) : s;
+    }
   float* o = reinterpret_cast<float*>(a.o) + (((int64_t)bh * a.N + i) * a.N + j) * D;
 #pragma unroll 1
   for (int c0 = half * (D / 2); c0 < (half + 1) * (D / 2); c0 += W) {
@@ -131,6 +139,7 @@ TRI_DEV void plain_fwd_row(const FwdArgs& a, int bh, int i, int j_blk, int lane)
       const float p = fast_exp2((row.score(j, key) - top) * a.c);
       sum += p;
       plain_axpy(acc, p, row.v + key * row.sv + c0);
+      if (sum != sum) break;
     }
     plain_store(o + c0, acc, 1.0f / sum);
   }
@@ -166,6 +175,7 @@ TRI_DEV void plain_dq_row(const BwdArgs& a, int bh, int i, int j_blk, int lane) 
       float p;
       const float ds = plain_dscore<D>(a, row, dout, words, j, key, p);
       plain_axpy(acc, ds, row.k + key * row.sk + c0);
+      if (ds != ds) break;
     }
     plain_store(dq + c0, acc, a.scale);
   }
@@ -191,7 +201,9 @@ TRI_DEV void plain_dkv_row(const BwdArgs& a, int bh, int i, int k_blk, int lane)
         float p;
         const float ds = plain_dscore<D>(a, row, dout + j * a.sdo.j, words, j, key, p);
         const float* from = is_dk ? row.q + j * row.sq : dout + j * a.sdo.j;
-        plain_axpy(acc, is_dk ? ds : p, from + c0);
+        const float w = is_dk ? ds : p;
+        plain_axpy(acc, w, from + c0);
+        if (w != w) break;
       }
     plain_store(out + c0, acc, is_dk ? a.scale : 1.0f);
   }
@@ -205,7 +217,7 @@ TRI_DEV void plain_db_block(const BwdArgs& a, int bh, int chunk, int j_blk, int 
     const int j = j_blk + x % BJ, key = k_blk + x / BJ;
     if (j >= a.N || key >= a.N) continue;
     float acc = 0.f;
-    for (int i = i_begin; i < i_end; ++i) {
+    for (int i = i_begin; i < i_end && acc == acc; ++i) {
       const PlainRow<D, BwdArgs> row(a, bh, i);
       if (!row.live(key)) continue;
       float p;
@@ -214,6 +226,30 @@ TRI_DEV void plain_db_block(const BwdArgs& a, int bh, int chunk, int j_blk, int 
     if (a.nchunks == 1) reinterpret_cast<float*>(a.db)[bh / a.H * a.sdb_b + bh % a.H * a.sdb_h + j * a.sdb_j + key * a.sdb_k] = acc;
     else a.dbpart[(((int64_t)chunk * a.BH + bh) * a.N + j) * a.N + key] = acc;
   }
+}
+
+// The same for a wave that found something not finite.  Called, not inlined: with these loops in their
+// bodies the kernels' own loops got other registers (at d = 64 dk/dv 2 % slower, the step
+// 0.7 %); at d = 128 dk/dv, which spills, is 2 % slower with the look at its results alone.
+#define TRI_CALLED __device__ __attribute__((noinline))
+template <int D, int R>
+TRI_CALLED void plain_fwd(ArgWords at, int bh, int i0, int j_blk, int lane) {
+  const FwdArgs a = read_args<FwdArgs>(at);
+  for (int r = 0; r < R && i0 + r < a.N; ++r) plain_fwd_row<D>(a, bh, i0 + r, j_blk, lane);
+}
+template <int D, int R>
+TRI_CALLED void plain_dq(ArgWords at, int bh, int i0, int j_blk, int lane) {
+  const BwdArgs a = read_args<BwdArgs>(at);
+  for (int r = 0; r < R && i0 + r < a.N; ++r) plain_dq_row<D>(a, bh, i0 + r, j_blk, lane);
+}
+template <int D, int R>
+TRI_CALLED void plain_dkv(ArgWords at, int bh, int i0, int k_blk, int lane) {
+  const BwdArgs a = read_args<BwdArgs>(at);
+  for (int r = 0; r < R && i0 + r < a.N; ++r) plain_dkv_row<D>(a, bh, i0 + r, k_blk, lane);
+}
+template <int D, int BJ, int BKB>
+TRI_CALLED void plain_db(ArgWords at, int bh, int chunk, int j_blk, int k_blk, int i_begin, int i_end, int lane) {
+  plain_db_block<D, BJ, BKB>(read_args<BwdArgs>(at), bh, chunk, j_blk, k_blk, i_begin, i_end, lane);
 }
 
 }  // namespace tri

@@ -863,10 +863,7 @@ __global__ __launch_bounds__(NW * 64, (R * ((BKF % kFwdFast) / 32) >= 8 || D * s
     }
   }
   if constexpr (sizeof(T) == 4) {
-    if (__any(!(check == 0.f))) {
-      const FwdArgs all = reloaded_args<FwdArgs>();
-      for (int r = 0; r < R && i0 + r < all.N; ++r) plain_fwd_row<D>(all, bh, i0 + r, j_wave, lane);
-    }
+    if (__any(!(check == 0.f))) plain_fwd<D, R>(arg_words(), bh, i0, j_wave, fresh_lane());
   }
 }
 
