@@ -64,7 +64,16 @@ struct LdsTile {
   static constexpr int CPR = ROWB / 16;            // 16-byte chunks per row (power of two)
   static constexpr int RPB = SWZ_ROWS > 0 ? SWZ_ROWS : ((256 / ROWB) > 0 ? 256 / ROWB : 1);  // rows per swizzle value
   static constexpr int VEC = 16 / (int)sizeof(T);
-  TRI_DEV static int swz(int r) { return (r / RPB) % CPR; }
+  // Neighbouring swizzle values differ in the high chunk bits: a transposing read takes 4 rows x 64
+  // bytes at once, and the rows that start at the same bank (every second one of 128 bytes, each of 256)
+  // have to lie 64 bytes apart.  (With the plain row number as the value two or four of them met in a
+  // bank, 25 to 30 % of the LDS cycles at d = 64: n = 512, h = 4, d = 128 dk/dv 970 -> 930 us, dq 616 ->
+  // 598; n = 768, h = 8, d = 64 dk/dv 2.52 -> 2.48 ms, the others within 1 %.)
+  TRI_DEV static int swz(int r) {
+    constexpr int B = CPR < 16 ? CPR : 16;  // (16 chunks are all banks)
+    const int x = (r / RPB) % B;
+    return B <= 4 ? x : (x << 2 | x >> (B == 8 ? 1 : 2)) % B;
+  }
   // byte offset, from the tile base, of byte `o` of row r (o must not straddle a chunk)
   TRI_DEV static int off(int r, int o) { return (r * CPR + ((o >> 4) ^ swz(r))) * 16 + (o & 15); }
   template <typename V>
