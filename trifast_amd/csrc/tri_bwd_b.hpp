@@ -152,11 +152,11 @@ __global__ __launch_bounds__(GJ * GK * 64) void tri_bwd_b_kernel(const BwdArgs a
   constexpr int NW = GJ * GK;
   constexpr int BJ = GJ * WJ * 32, BKB = GK * WK * 32;  // queries / keys per workgroup
   constexpr int ROWB = Tile::ROWB;
-  // one stage: lse2[BJ] | 64 spare words | -delta[BJ] | 64 spare words | Q rows | dO rows |
+  // one stage: lse2[BJ] | 64 keep words | -delta[BJ] | 64 spare words | Q rows | dO rows |
   // K rows | V rows.  The small arrays come first so that their offsets in every ring
-  // buffer fit the 16-bit immediate of an LDS read.  (The row's flag and keep words do not
-  // pass through LDS: they are wave-uniform and come by scalar loads.)
-  constexpr int OFF_LSE = 0, OFF_DELTA = OFF_LSE + BJ * 4 + 256;
+  // buffer fit the 16-bit immediate of an LDS read.  (The general loop takes the row's flag and
+  // keep words by scalar loads instead: it branches on them.)
+  constexpr int OFF_LSE = 0, OFF_KW = OFF_LSE + BJ * 4, OFF_DELTA = OFF_KW + 256;
   constexpr int OFF_Q = OFF_DELTA + BJ * 4 + 256, OFF_DO = OFF_Q + BJ * ROWB, OFF_K = OFF_DO + BJ * ROWB, OFF_V = OFF_K + BKB * ROWB;
   constexpr int STAGE = OFF_V + BKB * ROWB;
   static_assert(STAGE == bwd_b_stage_bytes(BJ, BKB, ROWB), "the launcher sizes LDS with bwd_b_stage_bytes");
@@ -175,37 +175,27 @@ __global__ __launch_bounds__(GJ * GK * 64) void tri_bwd_b_kernel(const BwdArgs a
   const int b = bh / a.H, h = bh % a.H;
   const int wj = wave % GJ, wk = wave / GJ;
   const int j_wave = j_blk + wj * (WJ * 32), k_wave = k_blk + wk * (WK * 32);
-  // the plain rows in front (no flag, every key of the block attended) take the loop of their own below
-  constexpr bool kPipelined = WJ == 1 && WK == 2 && NBUF == 4 && D <= 32;
-  // Where the run of fully masked rows at the end of the row range starts (padding), and the first
-  // row of the chunk that is not plain: every thread looks at its share of the rows, the result
-  // goes through words of LDS, which is not yet in use (only where the last row is fully masked: a
-  // scan on every launch cost 2 % at n = 704, 5 rounds of 88 rows).  A chunk is a share of the rows in front
-  // and a share of the run: rows of the run take about half the time of the others.
+  // the rows in front of the first fully masked one take the loop of their own below
+  constexpr bool kPipelined = WJ == 1 && WK == 2 && NBUF >= 2 && D <= 64;
+  // What the rows of the chunk are like: every thread looks at its share of them, the result goes
+  // through words of LDS, which is not yet in use.
+  //   * Where the run of fully masked rows at the end of the row range starts (padding; looked for only where
+  //     the last row is fully masked: a scan on every launch cost 2 % at n = 704, 5 rounds of 88 rows).
+  //     A chunk is a share of the rows in front and a share of the run: rows of the run take about
+  //     half the time of the others.
+  //   * (pipelined walk) The first fully masked row of the chunk; whether any other row masks a key of this
+  //     block; which key tiles of the block have an attended key in any row.
   uint32_t* scan_words = reinterpret_cast<uint32_t*>(tri_smem);
   if (tid == 0) {
     scan_words[0] = 0;
     scan_words[1] = (uint32_t)N;
+    scan_words[2] = 0;  // key tiles with an attended key, then (from bit 16) with a masked one
   }
   __syncthreads();
   const uint32_t* flags = a.rowflag + (int64_t)b * N;
   auto share_of = [&](int rows, int at) { return __builtin_amdgcn_readfirstlane((int)((uint32_t)rows * (uint32_t)at / (uint32_t)a.nchunks)); };
-  auto is_plain = [&](int i) {
-    bool ok = flags[i] == 0;
-    const uint32_t* kw = a.keep + ((int64_t)b * N + i) * a.nwords;
-#pragma unroll
-    for (int w = 0; w < BKB / 32; ++w) ok = ok && (k_blk / 32 + w < a.nwords ? kw[k_blk / 32 + w] : 0u) == 0xffffffffu;
-    return ok;
-  };
-  auto find_first_not_plain = [&](int from, int to) {
-    if constexpr (kPipelined)
-      for (int i = from + tid; i < to; i += NW * 64)
-        if (!is_plain(i)) {
-          atomicMin(scan_words + 1, (uint32_t)i);
-          break;
-        }
-    __syncthreads();
-  };
+  // (keys past the end of the row feed entries that are never stored: they do not count as masked)
+  auto past_end = [&](int word) { return word == a.nwords - 1 && (N & 31) != 0 ? 0xffffffffu << (N & 31) : word >= a.nwords ? 0xffffffffu : 0u; };
   int i_begin = share_of(N, chunk), i_end = share_of(N, chunk + 1), run_begin = N;
   if (uniform_word(a.rowflag, (int64_t)b * N + N - 1) != 0) {
     uint32_t last_other = 0;
@@ -217,13 +207,33 @@ __global__ __launch_bounds__(GJ * GK * 64) void tri_bwd_b_kernel(const BwdArgs a
     i_begin = share_of(run_begin, chunk);
     i_end = share_of(run_begin, chunk + 1);
   }
-  find_first_not_plain(i_begin, i_end);
+  if constexpr (kPipelined) {
+    uint32_t tiles = 0;
+    for (int i = i_begin + tid; i < i_end; i += NW * 64) {
+      if (flags[i] != 0) {
+        atomicMin(scan_words + 1, (uint32_t)i);
+        tiles = 0xffffu | tiles;
+        break;
+      }
+      const uint32_t* kw = a.keep + ((int64_t)b * N + i) * a.nwords;
+#pragma unroll
+      for (int w = 0; w < BKB / 32; ++w) {
+        const uint32_t x = k_blk / 32 + w < a.nwords ? kw[k_blk / 32 + w] : 0u;
+        tiles |= (x != 0 ? 1u << w : 0u) | ((x | past_end(k_blk / 32 + w)) != 0xffffffffu ? 0x10000u << w : 0u);
+      }
+    }
+    if (tiles) atomicOr(scan_words + 2, tiles);
+  }
+  __syncthreads();
   // (pinned to scalar registers: the branches of the walk must be real ones, see compute_row)
   i_begin = __builtin_amdgcn_readfirstlane(i_begin);
   run_begin = __builtin_amdgcn_readfirstlane(run_begin);
-  const int nrows = __builtin_amdgcn_readfirstlane(i_end) - i_begin;
+  int nrows = __builtin_amdgcn_readfirstlane(i_end) - i_begin;
   const int tail_begin = run_begin + share_of(N - run_begin, chunk), tail_end = run_begin + share_of(N - run_begin, chunk + 1);
-  int nplain = __builtin_amdgcn_readfirstlane(min((int)scan_words[1] - i_begin, nrows));
+  // rows that take the pipelined walk, and the block's key tiles (live, and masked from bit 16)
+  int nwalk = kPipelined ? __builtin_amdgcn_readfirstlane(min((int)scan_words[1] - i_begin, nrows)) : 0;
+  const uint32_t block_tiles = kPipelined ? __builtin_amdgcn_readfirstlane(scan_words[2]) : 0xffffu;
+  if ((block_tiles & 0xffffu) == 0) nrows = nwalk = 0;  // no attended key in any row: dS = 0
   __syncthreads();
 
   const T* qbase = reinterpret_cast<const T*>(a.q) + b * a.sq.b + h * a.sq.h;
@@ -234,13 +244,18 @@ __global__ __launch_bounds__(GJ * GK * 64) void tri_bwd_b_kernel(const BwdArgs a
   const float* lse2_bh = reinterpret_cast<const float*>(a.lse2) + (int64_t)bh * N * N;    // 32-bit words, moved as floats
   const float* delta_bh = reinterpret_cast<const float*>(a.delta) + (int64_t)bh * N * N;
 
-  // bias tiles in the raw-score domain: accumulator init of every row's score MFMA
-  f32x16 biasr[WJ][WK];
+  // bias tiles in the raw-score domain: accumulator init of every row's score MFMA.  (Each loop over
+  // the rows fetches its own: tiles that are live across the choice between the loops end up in scratch
+  // memory.  The tag keeps the compiler from making the fetches one again in front of the choice.)
+  auto load_bias = [&](f32x16 (&biasr)[WJ][WK], auto tag) __attribute__((always_inline)) {
+    int lane_now = lane;
+    asm volatile("; bias of loop %1" : "+v"(lane_now) : "n"(decltype(tag)::value));
 #pragma unroll
-  for (int tj = 0; tj < WJ; ++tj)
+    for (int tj = 0; tj < WJ; ++tj)
 #pragma unroll
-    for (int tk = 0; tk < WK; ++tk)
-      biasr[tj][tk] = bias_tile<T>(pack_bh, a.NP, min((j_wave >> 5) + tj, a.NP - 1), min((k_wave >> 5) + tk, a.NP - 1), lane, a.sqrt_d, 0.f);
+      for (int tk = 0; tk < WK; ++tk)
+        biasr[tj][tk] = bias_tile<T>(pack_bh, a.NP, min((j_wave >> 5) + tj, a.NP - 1), min((k_wave >> 5) + tk, a.NP - 1), lane_now, a.sqrt_d, 0.f);
+  };
 
   f32x16 dbacc[WJ][WK];
 #pragma unroll
@@ -257,7 +272,7 @@ __global__ __launch_bounds__(GJ * GK * 64) void tri_bwd_b_kernel(const BwdArgs a
   // the end are clamped (they feed db entries that are never stored).
   constexpr int CPR = Tile::CPR;
   constexpr int GQ = BJ * CPR / 64, GKK = BKB * CPR / 64, GF = BJ / 64;
-  constexpr int TOTW = 2 * GQ + 2 * GKK, TOTF = 2 * GF;
+  constexpr int TOTW = 2 * GQ + 2 * GKK, TOTF = 2 * GF + (kPipelined ? 1 : 0);
   constexpr int XW = (TOTW + NW - 1) / NW, XF = (TOTF + NW - 1) / NW;
   constexpr int XN = XW + XF;
   static_assert(BJ * CPR % 64 == 0 && BKB * CPR % 64 == 0 && BJ % 64 == 0, "whole wave loads only");
@@ -267,9 +282,19 @@ __global__ __launch_bounds__(GJ * GK * 64) void tri_bwd_b_kernel(const BwdArgs a
   };
   // An item's source is a 64-bit base (wave-uniform, scalar registers, stepped from one pair
   // row to the next with scalar adds) plus a 32-bit byte offset per lane that never changes.
-  const char* item_base[XN];
+  // Where every wave takes the same number of items of each tensor, the items of a tensor share
+  // one base, and their places in LDS are the wave's share plus constants.
+  constexpr bool kShared = GQ % NW == 0 && GKK % NW == 0;
+  constexpr int NBASE = kShared ? 4 + XF : XN;
+  auto base_of = [](int x) constexpr {
+    if (!kShared) return x;
+    if (x >= XW) return 4 + x - XW;
+    const int it = x * NW;
+    return it < GQ ? 0 : it < 2 * GQ ? 1 : it < 2 * GQ + GKK ? 2 : 3;
+  };
+  const char* item_base[NBASE];
+  int64_t item_step[NBASE];   // bytes from one pair row to the next (wave-uniform)
   uint32_t item_voff[XN];
-  int64_t item_step[XN];      // bytes from one pair row to the next (wave-uniform)
   int item_lds[XN];           // destination offset inside a stage (wave-uniform)
   // (items 0 .. XW-1 move 16 bytes per lane, items XW .. XN-1 4 bytes)
   {
@@ -277,14 +302,23 @@ __global__ __launch_bounds__(GJ * GK * 64) void tri_bwd_b_kernel(const BwdArgs a
     auto tile_item = [&](int x, int gi, const T* base, int64_t srow, int64_t si, int blk, int off) {
       const int p = gi * 64 + lane;
       const int r = p / CPR, cc = (p % CPR) ^ Tile::swz(r);
-      item_base[x] = reinterpret_cast<const char*>(uniform64((int64_t)(uintptr_t)(base + (int64_t)blk * srow + (int64_t)i_begin * si)));
-      item_voff[x] = (uint32_t)(min(r, N - 1 - blk) * (int)srow + cc * Tile::VEC) * (uint32_t)es;
-      item_step[x] = uniform64(si * es);
+      item_base[base_of(x)] = reinterpret_cast<const char*>(uniform64((int64_t)(uintptr_t)(base + (int64_t)blk * srow + (int64_t)i_begin * si)));
+      // (row strides are below 2^24 bytes)
+      item_voff[x] = __umul24((uint32_t)min(r, N - 1 - blk), (uint32_t)srow * (uint32_t)es) + (uint32_t)(cc * 16);
+      item_step[base_of(x)] = uniform64(si * es);
       item_lds[x] = off + gi * 1024;
     };
 #pragma unroll
     for (int x = 0; x < XN; ++x) {
-      // position in the flat order Q | dO | K | V | lse2 | delta
+      if (kShared && x < XW) {
+        const int first = x * NW;  // (a constant: so is the tensor)
+        if (first < GQ) tile_item(x, first + wave, qbase, a.sq.j, a.sq.i, j_blk, OFF_Q);
+        else if (first < 2 * GQ) tile_item(x, first - GQ + wave, dobase, a.sdo.j, a.sdo.i, j_blk, OFF_DO);
+        else if (first < 2 * GQ + GKK) tile_item(x, first - 2 * GQ + wave, kbase, a.sk.j, a.sk.i, k_blk, OFF_K);
+        else tile_item(x, first - 2 * GQ - GKK + wave, vbase, a.sv.j, a.sv.i, k_blk, OFF_V);
+        continue;
+      }
+      // position in the flat order Q | dO | K | V | lse2 | delta | keep words
       const int it = x < XW ? __builtin_amdgcn_readfirstlane(min(x * NW + wave, TOTW - 1))
                             : TOTW + __builtin_amdgcn_readfirstlane(min((x - XW) * NW + wave, TOTF - 1));
       if (it < GQ) {
@@ -295,14 +329,19 @@ __global__ __launch_bounds__(GJ * GK * 64) void tri_bwd_b_kernel(const BwdArgs a
         tile_item(x, it - 2 * GQ, kbase, a.sk.j, a.sk.i, k_blk, OFF_K);
       } else if (it < 2 * GQ + 2 * GKK) {
         tile_item(x, it - 2 * GQ - GKK, vbase, a.sv.j, a.sv.i, k_blk, OFF_V);
+      } else if (kPipelined && it == TOTW + TOTF - 1) {
+        item_base[base_of(x)] = reinterpret_cast<const char*>(uniform64((int64_t)(uintptr_t)(a.keep + ((int64_t)b * N + i_begin) * a.nwords)));
+        item_voff[x] = (uint32_t)(min(k_blk / 32 + lane, a.nwords - 1) * 4);
+        item_step[base_of(x)] = uniform64((int64_t)a.nwords * 4);
+        item_lds[x] = OFF_KW;
       } else {
         const int f = it - 2 * GQ - 2 * GKK;
         const int gi = f % GF;
         const float* base = (f < GF) ? lse2_bh : delta_bh;
         const int j0 = min(j_blk + gi * 64, N - 1);
-        item_base[x] = reinterpret_cast<const char*>(uniform64((int64_t)(uintptr_t)(base + (int64_t)i_begin * N + j0)));
+        item_base[base_of(x)] = reinterpret_cast<const char*>(uniform64((int64_t)(uintptr_t)(base + (int64_t)i_begin * N + j0)));
         item_voff[x] = (uint32_t)(min(lane, N - 1 - j0) * 4);
-        item_step[x] = uniform64((int64_t)N * 4);
+        item_step[base_of(x)] = uniform64((int64_t)N * 4);
         item_lds[x] = ((f < GF) ? OFF_LSE : OFF_DELTA) + gi * 256;
       }
     }
@@ -324,10 +363,11 @@ __global__ __launch_bounds__(GJ * GK * 64) void tri_bwd_b_kernel(const BwdArgs a
 #pragma unroll
     for (int x = 0; x < XN; ++x) {
       const uint32_t dst = __builtin_amdgcn_readfirstlane(st + (uint32_t)item_lds[x]);
-      if (x < XW) asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(dst), "v"(item_voff[x]), "s"(item_base[x]) : "memory", "m0");
-      else asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" : : "s"(dst), "v"(item_voff[x]), "s"(item_base[x]) : "memory", "m0");
-      item_base[x] += advance & item_step[x];
+      if (x < XW) asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(dst), "v"(item_voff[x]), "s"(item_base[base_of(x)]) : "memory", "m0");
+      else asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" : : "s"(dst), "v"(item_voff[x]), "s"(item_base[base_of(x)]) : "memory", "m0");
     }
+#pragma unroll
+    for (int x = 0; x < NBASE; ++x) item_base[x] += advance & item_step[x];
   };
   // the same, one item at a time (for loops that deal the loads of a row between other work);
   // next_row_advance() once per row, before its items
@@ -340,12 +380,13 @@ __global__ __launch_bounds__(GJ * GK * 64) void tri_bwd_b_kernel(const BwdArgs a
     ++rows_issued;
     return advance;
   };
-  auto issue_item = [&](int buf, auto x_tag, int64_t advance) __attribute__((always_inline)) {
+  auto issue_item = [&](int stage_off, auto x_tag, int64_t advance) __attribute__((always_inline)) {
     constexpr int x = decltype(x_tag)::value;
-    const uint32_t dst = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(TRI_L3 unsigned char*)(tri_smem + buf * STAGE) + (uint32_t)item_lds[x]);
-    if constexpr (x < XW) asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(dst), "v"(item_voff[x]), "s"(item_base[x]) : "memory", "m0");
-    else asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" : : "s"(dst), "v"(item_voff[x]), "s"(item_base[x]) : "memory", "m0");
-    item_base[x] += advance & item_step[x];
+    const uint32_t dst = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(TRI_L3 unsigned char*)(tri_smem + stage_off) + (uint32_t)item_lds[x]);
+    constexpr int bx = base_of(x);
+    if constexpr (x < XW) asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(dst), "v"(item_voff[x]), "s"(item_base[bx]) : "memory", "m0");
+    else asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" : : "s"(dst), "v"(item_voff[x]), "s"(item_base[bx]) : "memory", "m0");
+    if constexpr (x + 1 == XN || base_of(x + 1) != bx) item_base[bx] += advance & item_step[bx];
   };
   // wait until at most the newest `K` rows of this wave's loads are in flight and
   // every LDS read has returned, then meet the other waves
@@ -375,9 +416,12 @@ __global__ __launch_bounds__(GJ * GK * 64) void tri_bwd_b_kernel(const BwdArgs a
   asm volatile("" : "+v"(scalar_off));
   // LDS reads take a 16-bit immediate offset: for ring buffers past the first 64 KiB a
   // second set of lane offsets, moved up by two stages, keeps the buffer's offset an
-  // immediate (the reads of those buffers would otherwise each need an address add)
-  constexpr bool kHighSet = NBUF > 2;
-  constexpr int HIGH = kHighSet ? 2 * STAGE : 0;
+  // immediate (the reads of those buffers would otherwise each need an address add).  The
+  // pipelined walk of 128-byte rows has no registers for a second set: its offsets move from row to row.
+  constexpr int kHighFrom = 2;
+  constexpr bool kMoving = kPipelined && D > 32;
+  constexpr bool kHighSet = NBUF > 2 && !kMoving;
+  constexpr int HIGH = kHighSet ? kHighFrom * STAGE : 0;
   OperandOffsets<T, D> ofk_hi = ofk, ofq_hi = ofq;
   int scalar_off_hi = scalar_off;
   if constexpr (kHighSet) {
@@ -392,10 +436,13 @@ __global__ __launch_bounds__(GJ * GK * 64) void tri_bwd_b_kernel(const BwdArgs a
   // -lse per query and the key mask share one MFMA (see OffsetMask), -delta has its own
   typename OffsetMask<T>::Queries lrank[WJ];
   Rank1<T> drank[WJ];
-#pragma unroll
-  for (int tj = 0; tj < WJ; ++tj) { lrank[tj].init(0u, g); drank[tj].init(); }
   typename OffsetMask<T>::Keys kop;
-  kop.init(perm32(jl), g);
+  // (set up by the loops that use them: the walk has no registers for values that wait for the general loop)
+  auto init_operands = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int tj = 0; tj < WJ; ++tj) { lrank[tj].init(0u, g); drank[tj].init(); }
+    kop.init(perm32(jl), g);
+  };
 
   const float c = a.c;
   // (an integer that the compiler cannot see through: a boolean would be kept as a lane mask
@@ -436,8 +483,8 @@ __global__ __launch_bounds__(GJ * GK * 64) void tri_bwd_b_kernel(const BwdArgs a
     return m;
   };
 
-  auto compute_row = [&](int buf, const RowMeta& meta) __attribute__((always_inline)) {
-    const bool high = kHighSet && buf >= 2;  // (a constant once the ring loop is unrolled)
+  auto compute_row = [&](int buf, const RowMeta& meta, const f32x16 (&biasr)[WJ][WK]) __attribute__((always_inline)) {
+    const bool high = kHighSet && buf >= kHighFrom;  // (a constant once the ring loop is unrolled)
     const int sl = buf * STAGE - (high ? HIGH : 0);  // offset of the buffer for reads through the lane offsets
     const OperandOffsets<T, D>& oq = high ? ofq_hi : ofq;
     const OperandOffsets<T, D>& ok = high ? ofk_hi : ofk;
@@ -527,7 +574,7 @@ __global__ __launch_bounds__(GJ * GK * 64) void tri_bwd_b_kernel(const BwdArgs a
 
   // a row of the trailing run of fully masked ones (see below): dO V^T - delta on top of the accumulator itself
   auto add_uniform_row = [&](int buf) __attribute__((always_inline)) {
-    const bool high = kHighSet && buf >= 2;
+    const bool high = kHighSet && buf >= kHighFrom;
     const int sl = buf * STAGE - (high ? HIGH : 0);
     const OperandOffsets<T, D>& oq = high ? ofq_hi : ofq;
     const OperandOffsets<T, D>& ok = high ? ofk_hi : ofk;
@@ -551,7 +598,7 @@ __global__ __launch_bounds__(GJ * GK * 64) void tri_bwd_b_kernel(const BwdArgs a
     __syncthreads();
     const int last = max(row_end - 1, 0), at = min(rows_issued, last), meta_at = min(meta_rows, last);
 #pragma unroll
-    for (int x = 0; x < XN; ++x) item_base[x] += (int64_t)(row - at) * item_step[x];
+    for (int x = 0; x < NBASE; ++x) item_base[x] += (int64_t)(row - at) * item_step[x];
     flag_word = (const_words)((uintptr_t)flag_word + (uintptr_t)((int64_t)(row - meta_at) * 4));
     keep_word = (const_words)((uintptr_t)keep_word + (uintptr_t)((int64_t)(row - meta_at) * keep_step));
     rows_issued = meta_rows = row;
@@ -561,6 +608,12 @@ __global__ __launch_bounds__(GJ * GK * 64) void tri_bwd_b_kernel(const BwdArgs a
   // the rows from `first_row` to row_end (the loads and the row words stand at the first)
   auto walk_rows = [&](int first_row, auto uniform_tag) __attribute__((always_inline)) {
   constexpr bool UNIFORM = decltype(uniform_tag)::value;
+  init_operands();
+  f32x16 biasr[WJ][WK];
+  if constexpr (!UNIFORM) {
+    load_bias(biasr, std::integral_constant<int, 2>{});
+    wait_dma_known();  // (or the first use in every row would wait for everything in flight)
+  }
   if constexpr (NBUF >= 2) {
     // Ring of NBUF row buffers: the loads run NBUF-1 rows ahead of the compute, which
     // hides the memory latency behind several rows of work.  Row q lives in buffer
@@ -579,7 +632,7 @@ __global__ __launch_bounds__(GJ * GK * 64) void tri_bwd_b_kernel(const BwdArgs a
           const RowMeta next = load_meta();
           if (wave_live != 0) {
             if constexpr (UNIFORM) add_uniform_row(u);
-            else compute_row(u, meta);
+            else compute_row(u, meta, biasr);
           }
           sync_rows(std::integral_constant<int, P - 1>{});  // the next row has landed
           meta = next;
@@ -594,21 +647,29 @@ __global__ __launch_bounds__(GJ * GK * 64) void tri_bwd_b_kernel(const BwdArgs a
       sync_rows(std::integral_constant<int, 0>{});
       if (wave_live != 0) {
         if constexpr (UNIFORM) add_uniform_row(0);
-        else compute_row(0, meta);
+        else compute_row(0, meta, biasr);
       }
       sync_rows(std::integral_constant<int, 0>{});
     }
   }
   };
-  // Waves that own two key tiles (16-bit types, d <= 32) walk the plain rows at the start of
-  // the chunk (not flagged, no masked key in any of the block's key tiles: the common case)
-  // software-pipelined: a wave's matrix instructions of one tile are issued between the
-  // exponentials and multiply-adds of the tile before it (the second tile of a row overlaps
-  // the first, the first tile of the next row overlaps the second), so neither pipe waits
-  // for the other although only one or two waves share a SIMD.  The next row's operands are
-  // read from LDS a whole row ahead.  From the first row that is not plain on (padding: the
-  // rows past the valid length) the loop above takes over.  (The same walk with the masked
-  // form of the score needs about 290 registers per lane: it does not fit 8 waves.)
+  // Waves that own two key tiles (16-bit types, d <= 64) walk the rows in front of the chunk's first
+  // fully masked one software-pipelined: a wave's matrix instructions of one tile are issued
+  // between the exponentials and multiply-adds of the tile before it (the second tile of a row
+  // overlaps the first, the first tile of the next row overlaps the second), so neither pipe
+  // waits for the other although only one or two waves share a SIMD.  The score chain of a tile
+  // runs before its dP chain, and every operand is read from LDS into the register that the
+  // product before it has freed, several products ahead of its use: V where K was, the next tile's K
+  // where V was, the next row's Q and dO where this row's were.  (Two sets of operands took 243 registers
+  // at d = 32 and left none for a mask; d = 64 does not fit two.)  -lse is the addend of the
+  // exponent's fma in every row; where rows have masked keys in this block each tile takes one more
+  // product, which adds the mask element to the scores of the masked keys (keys operand against ones).
+  // Alone, back to back on one card against the walk with two operand sets, which took unmasked rows of up to
+  // 64 bytes only: h = 4, d = 32 n = 1024 0.96 -> 0.91 ms; 2048 with 5 % masked 9.6 (16 waves: 8.9) -> 8.5;
+  // h = 8, d = 64 n = 768 1.80 -> 1.53, half of the keys masked 1.84 -> 1.60, with pair rows 98 KiB apart 1.85 ->
+  // 1.78.  (Within a training step the large ones gain little of it: the chip then lowers its clock, 2.0 GHz at
+  // n = 1024.)  With its loads taken out the d = 64 walk takes 1.10 ms: two row buffers of 64 KiB are
+  // all that fits, and a compute unit takes in 64 bytes per clock.
   // The trailing fully masked rows come first: with P = 1 / n everywhere their part is
   // sum_i (dO_i V_i^T - delta_i) / n, matrix products into the accumulator and one multiply at the
   // end instead of an exponential and two multiply-adds per element and row (n = 1000 with 800 valid
@@ -626,140 +687,221 @@ __global__ __launch_bounds__(GJ * GK * 64) void tri_bwd_b_kernel(const BwdArgs a
     seek(0, nrows);
   }
   if constexpr (kPipelined) {
-    if (nplain < 2 * NBUF) nplain = 0;  // too few to fill the pipeline
-    if (nplain > 0) {
-      struct RowOps {
-        frag q[WJ][DS], dout[WJ][DS], k[WK][DS], v[WK][DS];
-        frag df[WJ];    // -delta of the lane's query as a rank-1 operand
-        float nl2[WJ];  // -lse of the lane's query in the exponent's unit
-        uint32_t lw[WJ], dw[WJ];
+    if (nwalk < 2 * NBUF) nwalk = 0;  // too few to fill the pipeline
+    const uint32_t wave_tiles = __builtin_amdgcn_readfirstlane(block_tiles >> (wk * WK) & ((1u << WK) - 1));
+    auto walk = [&](auto masked_tag, auto busy_tag) __attribute__((always_inline)) {
+      constexpr bool MASKED = decltype(masked_tag)::value;
+      // (a wave without queries or attended keys takes part in the loads and barriers only)
+      constexpr bool BUSY = decltype(busy_tag)::value;
+      typedef uint32_t u32x4v __attribute__((ext_vector_type(4)));
+      f32x16 biasr[WJ][WK];
+      if constexpr (BUSY) {
+        load_bias(biasr, masked_tag);
+        wait_dma_known();
+      }
+      // the tile in flight and the tile being consumed: scores and dP
+      f32x16 sc[2], dpc[2];
+      // Operands of the tile whose matrix instructions run: its K, then, step by step as the score chain has
+      // used them, its V in the same registers; Q and dO of the row; -delta of the lane's query as a
+      // rank-1 operand, -lse in the exponent's unit.
+      frag kv[DS], qf[DS], dof[DS], df;
+      float nl2, nl2_next;
+      uint32_t lw, dw;
+      drank[0].init();
+      // the keep words of the wave's two key tiles (this lane's key is bit perm32(jl))
+      uint32_t kw[WK] = {}, kw_next[WK] = {}, past[WK] = {};
+      const uint32_t key_bit = 1u << perm32(jl);
+      int keep_off = wk * WK * 4 + (int)(uintptr_t)(TRI_L3 const unsigned char*)tri_smem, keep_off_hi = keep_off + HIGH;
+      if constexpr (MASKED) {
+        asm volatile("" : "+v"(keep_off), "+v"(keep_off_hi));
+#pragma unroll
+        for (int tk = 0; tk < WK; ++tk) past[tk] = __builtin_amdgcn_readfirstlane(past_end(k_wave / 32 + tk));
+      }
+      // (kMoving: the lane offsets stand at the buffer that is read)
+      auto step_stages = [&](int bytes) __attribute__((always_inline)) {
+        ofk.shift(bytes);
+        ofq.shift(bytes);
+        ofk.pin();
+        ofq.pin();
+        scalar_off += bytes;
+        keep_off += bytes;
+        asm volatile("" : "+v"(scalar_off), "+v"(keep_off));
       };
-      auto read_ops = [&](int buf, RowOps& o) __attribute__((always_inline)) {
-        const bool high = kHighSet && buf >= 2;
-        const int sl = buf * STAGE - (high ? HIGH : 0);
-        const OperandOffsets<T, D>& oq = high ? ofq_hi : ofq;
-        const OperandOffsets<T, D>& ok = high ? ofk_hi : ofk;
-        const int soff = high ? scalar_off_hi : scalar_off;
+      // operand `sd` of the rows at `off` in row buffer `buf`
+      auto read_keys = [&](int buf, int off, int sd) __attribute__((always_inline)) {
+        const bool high = kHighSet && buf >= kHighFrom;
+        return (high ? ofk_hi : ofk).natural_at((kMoving ? 0 : buf * STAGE) - (high ? HIGH : 0) + off, sd);
+      };
+      auto read_queries = [&](int buf, int off, int sd) __attribute__((always_inline)) {
+        const bool high = kHighSet && buf >= kHighFrom;
+        return (high ? ofq_hi : ofq).natural_at((kMoving ? 0 : buf * STAGE) - (high ? HIGH : 0) + off, sd);
+      };
+      auto read_words = [&](int buf) __attribute__((always_inline)) {
+        const bool high = kHighSet && buf >= kHighFrom;
+        const int at = (kMoving ? 0 : buf * STAGE) - (high ? HIGH : 0);
+        const int words = at + (high ? scalar_off_hi : scalar_off), keeps = at + (high ? keep_off_hi : keep_off) + OFF_KW;
+        lw = *reinterpret_cast<TRI_L3 const uint32_t*>((uintptr_t)(uint32_t)(words + OFF_LSE));
+        dw = *reinterpret_cast<TRI_L3 const uint32_t*>((uintptr_t)(uint32_t)(words + OFF_DELTA));
+        if constexpr (MASKED) {
 #pragma unroll
-        for (int tj = 0; tj < WJ; ++tj) {
-#pragma unroll
-          for (int s = 0; s < DS; ++s) {
-            o.q[tj][s] = oq.natural_at(sl + OFF_Q + tj * 32 * ROWB, s);
-            o.dout[tj][s] = oq.natural_at(sl + OFF_DO + tj * 32 * ROWB, s);
-          }
-          o.lw[tj] = *reinterpret_cast<TRI_L3 const uint32_t*>((uintptr_t)(uint32_t)(sl + OFF_LSE + tj * 128 + soff));
-          o.dw[tj] = *reinterpret_cast<TRI_L3 const uint32_t*>((uintptr_t)(uint32_t)(sl + OFF_DELTA + tj * 128 + soff));
+          for (int tk = 0; tk < WK; ++tk) kw_next[tk] = *reinterpret_cast<TRI_L3 const uint32_t*>((uintptr_t)(uint32_t)(keeps + 4 * tk));
         }
-#pragma unroll
-        for (int tk = 0; tk < WK; ++tk)
-#pragma unroll
-          for (int s = 0; s < DS; ++s) {
-            o.k[tk][s] = ok.natural_at(sl + OFF_K + tk * 32 * ROWB, s);
-            o.v[tk][s] = ok.natural_at(sl + OFF_V + tk * 32 * ROWB, s);
-          }
       };
-      auto finish_ops = [&](RowOps& o) __attribute__((always_inline)) {
-#pragma unroll
-        for (int tj = 0; tj < WJ; ++tj) {
-          o.nl2[tj] = split_value<T>(o.lw[tj]) * c;
-          o.df[tj] = drank[tj].set(g ? 0u : o.dw[tj]);
-        }
+      auto mask_operand = [&](uint32_t keepw, int tk) __attribute__((always_inline)) {
+        u32x4v t = {0u, ((keepw | past[tk]) & key_bit) ? 0u : OffsetMask<T>::mask_dword(), 0u, 0u};
+        return __builtin_bit_cast(frag, t);
       };
-      // The tiles of a wave in the order they are walked: tile t is (t / WK, t % WK).  The
-      // matrix instructions of tile TN of row `on` (scores from the bias tile, dP from
-      // -delta) go into sn / dpn, dealt between the elementwise work of tile TC of row
-      // `oc`, whose scores s and dP are complete: db += exp2(c s - lse) dP.
-      constexpr int NT = WJ * WK;
-      constexpr int NM = 2 * DS + 1;  // matrix instructions of a tile
-      static_assert(NT % 2 == 0, "the two accumulator sets swap once per tile");
-      auto phase = [&](const RowOps& on, auto tn_tag, f32x16& sn, f32x16& dpn, const RowOps& oc, auto tc_tag, const f32x16& s,
-                       const f32x16& dp, auto&& between) __attribute__((always_inline)) {
-        constexpr int TN = decltype(tn_tag)::value, TC = decltype(tc_tag)::value;
-        constexpr int nj = TN / WK, nk = TN % WK, cj = TC / WK, ck = TC % WK;
+      constexpr int M = MASKED ? 1 : 0;
+      constexpr int NM = 2 * DS + 1 + M;  // matrix instructions of a tile
+      // the elements of the tile before that are dealt to slot X: [dealt(X), dealt(X + 1))
+      auto dealt = [](int X) constexpr { return 16 * X / NM; };
+      // The matrix instructions of key tile TN (scores from the bias tile, dP from -delta) go into sn / dpn, dealt
+      // between the elementwise work of the tile before it, whose scores s and dP are complete: db +=
+      // exp2(c s - lse) dP.  `cur`, `next`: row buffers of the tile and of the tile after it; `turn` comes
+      // between the two chains.
+      auto phase = [&](auto tn_tag, int cur, int next, uint32_t keepw, f32x16& sn, f32x16& dpn, const f32x16& s, const f32x16& dp, float addend,
+                       auto&& turn, auto&& between) __attribute__((always_inline)) {
+        constexpr int TN = decltype(tn_tag)::value, TC = 1 - TN;
+        frag mk;
+        if constexpr (MASKED) mk = mask_operand(keepw, TN);
         static_for<NM>([&](auto xc) __attribute__((always_inline)) {
           constexpr int X = decltype(xc)::value;
-          // the two chains alternate, so that an instruction seldom waits for the one before it
-          constexpr bool IS_S = X == 0 || (X >= 2 && X % 2 == 0 && X / 2 < DS);
-          constexpr int before = (X - 1) / 2 < DS - 1 ? (X - 1) / 2 : DS - 1;  // score steps among slots 1 .. X-1
-          constexpr int DI = X - 2 - before;                                    // dP steps among them, less the -delta one
-          if constexpr (X == 0) sn = E::mfma(on.k[nk][0], on.q[nj][0], biasr[nj][nk]);
-          else if constexpr (X == 1) dpn = E::mfma(ones, on.df[nj], zero16());
-          else if constexpr (IS_S) sn = E::mfma(on.k[nk][X / 2], on.q[nj][X / 2], sn);
-          else dpn = E::mfma(on.v[nk][DI], on.dout[nj][DI], dpn);
-          between(std::integral_constant<int, TC * NM + X>{});
+          if constexpr (X < M) {
+            sn = E::mfma(mk, ones, biasr[0][TN]);
+          } else if constexpr (X < M + DS) {
+            constexpr int sd = X - M;
+            sn = E::mfma(kv[sd], qf[sd], X == 0 ? biasr[0][TN] : sn);
+            kv[sd] = read_keys(cur, OFF_V + TN * 32 * ROWB, sd);
+            if constexpr (TN == 0) dof[sd] = read_queries(cur, OFF_DO, sd);
+          } else if constexpr (X == M + DS) {
+            dpn = E::mfma(ones, df, zero16());
+          } else {
+            constexpr int sd = X - M - DS - 1;
+            dpn = E::mfma(kv[sd], dof[sd], dpn);
+            kv[sd] = read_keys(next, OFF_K + TC * 32 * ROWB, sd);
+            if constexpr (TN == 1) {
+              qf[sd] = read_queries(next, OFF_Q, sd);
+              if constexpr (sd == 0) read_words(next);
+            }
+          }
+          between(std::integral_constant<int, X>{});
 #pragma unroll
-          for (int v = 16 * X / NM; v < 16 * (X + 1) / NM; ++v) {
-            const float p = fast_exp2(__builtin_fmaf(s[v], c, oc.nl2[cj]));
-            dbacc[cj][ck][v] = __builtin_fmaf(p, dp[v], dbacc[cj][ck][v]);
+          for (int v = dealt(X); v < dealt(X + 1); ++v) {
+            const float p = fast_exp2(__builtin_fmaf(s[v], c, addend));
+            dbacc[0][TC][v] = __builtin_fmaf(p, dp[v], dbacc[0][TC][v]);
           }
           __builtin_amdgcn_sched_barrier(0);
+          if constexpr (X == M + DS) {
+            turn();
+            __builtin_amdgcn_sched_barrier(0);
+          }
         });
       };
-      constexpr int AHEAD = NBUF;  // rows between the loads and the compute
+      auto take_words = [&]() __attribute__((always_inline)) {
+        nl2_next = split_value<T>(lw) * c;
+        df = drank[0].set(g ? 0u : dw);
+      };
 #pragma unroll
-      for (int u = 0; u < AHEAD; ++u) issue_row(u);
-      sync_rows(std::integral_constant<int, AHEAD - 2>{});  // rows 0 and 1 have landed
-      // (two sets of operand registers that swap roles from row to row: no copies)
-      RowOps ops[2];
-      f32x16 sc[2], dpc[2];  // scores and dP of the tile in flight and the tile being consumed
-      read_ops(0, ops[0]);
-      finish_ops(ops[0]);
-      // (the first tile of the first row has nothing to overlap with)
-      sc[0] = E::mfma(ops[0].k[0][0], ops[0].q[0][0], biasr[0][0]);
+      for (int u = 0; u < NBUF; ++u) issue_row(u);
+      sync_rows(std::integral_constant<int, NBUF - 1>{});  // row 0 has landed
+      if constexpr (BUSY) {
+        // the first tile of the first row has nothing to overlap with
+        read_words(0);
 #pragma unroll
-      for (int sd = 1; sd < DS; ++sd) sc[0] = E::mfma(ops[0].k[0][sd], ops[0].q[0][sd], sc[0]);
-      dpc[0] = E::mfma(ones, ops[0].df[0], zero16());
+        for (int sd = 0; sd < DS; ++sd) {
+          qf[sd] = read_queries(0, OFF_Q, sd);
+          dof[sd] = read_queries(0, OFF_DO, sd);
+          kv[sd] = read_keys(0, OFF_K, sd);
+        }
+        take_words();
+        nl2 = nl2_next;
 #pragma unroll
-      for (int sd = 0; sd < DS; ++sd) dpc[0] = E::mfma(ops[0].v[0][sd], ops[0].dout[0][sd], dpc[0]);
-      sc[1] = zero16();
-      dpc[1] = zero16();
-      sync_rows(std::integral_constant<int, AHEAD - 2>{});  // every wave has read row 0: its buffer is free
+        for (int tk = 0; tk < WK; ++tk) kw[tk] = kw_next[tk];
+        sc[0] = biasr[0][0];
+        if constexpr (MASKED) sc[0] = E::mfma(mask_operand(kw[0], 0), ones, sc[0]);
+#pragma unroll
+        for (int sd = 0; sd < DS; ++sd) {
+          sc[0] = E::mfma(kv[sd], qf[sd], sc[0]);
+          kv[sd] = read_keys(0, OFF_V, sd);
+        }
+        dpc[0] = E::mfma(ones, df, zero16());
+#pragma unroll
+        for (int sd = 0; sd < DS; ++sd) {
+          dpc[0] = E::mfma(kv[sd], dof[sd], dpc[0]);
+          kv[sd] = read_keys(0, OFF_K + 32 * ROWB, sd);
+        }
+      }
 #ifdef TRI_DB_TIMING
       uint64_t t_wait = 0, t_barrier = 0;
       const uint64_t t_clk0 = __builtin_amdgcn_s_memtime(), t_real0 = __builtin_amdgcn_s_memrealtime();
 #endif
-      for (int r = 0; r < nplain; r += NBUF) {
-#pragma unroll
-        for (int u = 0; u < NBUF; ++u) {
-          if (r + u < nplain) {
-            RowOps& cur = ops[u & 1];
-            RowOps& next = ops[(u + 1) & 1];
-            // row r + u + NBUF goes into the buffer whose row is in registers already; its
-            // loads are dealt over the row (a burst of them would hold up the wave's other
-            // instructions until the memory pipeline has taken them all)
-            const int64_t advance = next_row_advance();
-            auto deal_loads = [&](auto slot_tag) __attribute__((always_inline)) {
-              constexpr int slot = decltype(slot_tag)::value;
-              static_for<XN>([&](auto xt) __attribute__((always_inline)) {
-                constexpr int x = decltype(xt)::value;
+      // Row r, in buffer `cur` (offset stage_off): its second tile beside the elementwise work of its first, and the
+      // first tile of the next row beside that of its second.  Between the two chains of the second
+      // tile every wave is done with the row's buffer (V of that tile was the last it had to read): the
+      // next row's rows have landed there, and the loads of row r + NBUF go into the buffer, dealt
+      // over the slots up to the end of the row (a burst of them would hold up the wave's other
+      // instructions until the memory pipeline has taken them all).
+      constexpr int kEarly = 2;
+      auto row = [&](int stage_off, int cur, int next, int step) __attribute__((always_inline)) {
+        const int64_t advance = next_row_advance();
+        auto deal_loads = [&](auto slot_tag) __attribute__((always_inline)) {
+          constexpr int slot = decltype(slot_tag)::value;  // 0 .. DS - 1: rest of the second tile; then the first tile
+          static_for<XN>([&](auto xt) __attribute__((always_inline)) {
+            constexpr int x = decltype(xt)::value;
 #if !defined(TRI_DB_TIMING) || TRI_DB_TIMING_LOADS != 0
-                if constexpr (slot == (x * NT * NM) / XN) issue_item(u, xt, advance);
+            if constexpr (slot == (x * (NBUF == 2 ? kEarly : DS + NM)) / XN) issue_item(stage_off, xt, advance);
 #endif
-              });
-            };
-            read_ops((u + 1) % NBUF, next);
-            __builtin_amdgcn_sched_barrier(0);
-            static_for<NT - 1>([&](auto tc) __attribute__((always_inline)) {
-              constexpr int t = decltype(tc)::value;
-              phase(cur, std::integral_constant<int, t + 1>{}, sc[(t + 1) & 1], dpc[(t + 1) & 1], cur, tc, sc[t & 1], dpc[t & 1], deal_loads);
-            });
-            finish_ops(next);
-            phase(next, std::integral_constant<int, 0>{}, sc[0], dpc[0], cur, std::integral_constant<int, NT - 1>{}, sc[(NT - 1) & 1], dpc[(NT - 1) & 1], deal_loads);
+          });
+        };
+        auto turn = [&]() __attribute__((always_inline)) {
 #ifdef TRI_DB_TIMING
-            {
-              const uint64_t m0 = __builtin_amdgcn_s_memtime();
-              asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" : : "n"((AHEAD - 2) * XN) : "memory");
-              const uint64_t m1 = __builtin_amdgcn_s_memtime();
-              asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-              const uint64_t m2 = __builtin_amdgcn_s_memtime();
-              asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-              t_wait += m1 - m0;
-              t_barrier += m2 - m1;
-            }
+          const uint64_t m0 = __builtin_amdgcn_s_memtime();
+          asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" : : "n"((NBUF - 2) * XN) : "memory");
+          const uint64_t m1 = __builtin_amdgcn_s_memtime();
+          asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+          const uint64_t m2 = __builtin_amdgcn_s_memtime();
+          asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+          t_wait += m1 - m0;
+          t_barrier += m2 - m1;
 #else
-            sync_rows(std::integral_constant<int, AHEAD - 2>{});  // rows up to r + u + 2 have landed
+          sync_rows(std::integral_constant<int, NBUF - 2>{});
 #endif
-          }
+          if constexpr (kMoving && BUSY) step_stages(step);
+        };
+        if constexpr (BUSY) {
+          // (used and defined in every row: the compiler's allocator otherwise parks what the loop only reads in
+          // scratch memory, with registers to spare, and a reload from there waits for every load in flight)
+          asm volatile("" : "+v"(biasr[0][0]), "+v"(biasr[0][1]));
+          phase(std::integral_constant<int, 1>{}, cur, next, kw[1], sc[1], dpc[1], sc[0], dpc[0], nl2, turn, [&](auto slot) __attribute__((always_inline)) {
+            constexpr int after = decltype(slot)::value - (M + DS + 1);
+            if constexpr (after >= 0) deal_loads(std::integral_constant<int, after>{});
+          });
+          take_words();
+          phase(std::integral_constant<int, 0>{}, next, next, kw_next[0], sc[0], dpc[0], sc[1], dpc[1], nl2, [] {}, [&](auto slot) __attribute__((always_inline)) {
+            deal_loads(std::integral_constant<int, DS + decltype(slot)::value>{});
+          });
+          nl2 = nl2_next;
+          kw[1] = kw_next[1];
+        } else {
+          turn();
+          static_for<DS + NM>(deal_loads);
+        }
+      };
+      if constexpr (kMoving) {
+        int at = 0;  // offset of row r's buffer
+#pragma unroll 1
+        for (int r = 0; r < nwalk; ++r) {
+          const int step = at == (NBUF - 1) * STAGE ? -(NBUF - 1) * STAGE : STAGE;
+          row(at, 0, 0, step);
+          at += step;
+        }
+        if constexpr (BUSY) step_stages(-at);  // (back to the first buffer)
+      } else {
+        for (int r = 0; r < nwalk; r += NBUF) {
+          static_for<NBUF>([&](auto uc) __attribute__((always_inline)) {
+            constexpr int u = decltype(uc)::value;
+            if (r + u < nwalk) row(u * STAGE, u, (u + 1) % NBUF, 0);
+          });
         }
       }
 #ifdef TRI_DB_TIMING
@@ -768,11 +910,9 @@ __global__ __launch_bounds__(GJ * GK * 64) void tri_bwd_b_kernel(const BwdArgs a
         asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
         // (the sums are not stored here, and without a use the compiler leaves their arithmetic out)
 #pragma unroll
-        for (int tj = 0; tj < WJ; ++tj)
+        for (int tk = 0; tk < WK; ++tk)
 #pragma unroll
-          for (int tk = 0; tk < WK; ++tk)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) asm volatile("" : : "v"(dbacc[tj][tk][v]));
+          for (int v = 0; v < 16; ++v) asm volatile("" : : "v"(dbacc[0][tk][v]));
         if (lane == 0) {
           const int64_t L = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
           uint64_t* rec = reinterpret_cast<uint64_t*>(a.db) + (L * NW + wave) * 4;
@@ -784,12 +924,21 @@ __global__ __launch_bounds__(GJ * GK * 64) void tri_bwd_b_kernel(const BwdArgs a
         return;
       }
 #endif
-      if (nplain < row_end) {
-        // hand over: nothing in flight, the loads and the row words moved to row nplain
-        seek(nplain, row_end);
+    };
+    if (nwalk > 0) {
+      const bool busy = wave_live != 0 && wave_tiles != 0, masked = block_tiles >> 16 != 0;
+      if (!busy) walk(std::false_type{}, std::false_type{});
+      else if (masked) walk(std::true_type{}, std::true_type{});
+      else walk(std::false_type{}, std::true_type{});
+#ifdef TRI_DB_TIMING
+      return;
+#endif
+      if (nwalk < row_end) {
+        // hand over: nothing in flight, the loads and the row words moved to row nwalk
+        seek(nwalk, row_end);
       }
     }
-    if (nplain < row_end) walk_rows(nplain, std::false_type{});
+    if (nwalk < row_end) walk_rows(nwalk, std::false_type{});
   } else if (row_end > 0) {
     walk_rows(0, std::false_type{});
   }

@@ -465,9 +465,9 @@ int trifast_default_tile(int kernel, int64_t n, int64_t h, int64_t d, int dtype)
       break;
     case TRIFAST_KERNEL_BWD_B:
       // 64 x 64 block of 4 waves up to 256 keys (more workgroups than a larger block gives
-      // there), for 32-byte rows and for the widest ones; else 128 x 128 of 16 waves, of 8 waves
-      // for 128-byte rows
-      pick = (n <= 256 || row_bytes <= 32 || row_bytes >= 256) ? 2 : (row_bytes == 128 ? 3 : 4);
+      // there), for 32-byte rows and for the widest ones; else 128 x 128 of 8 waves with the
+      // pipelined walk
+      pick = (n <= 256 || row_bytes <= 32 || row_bytes >= 256) ? 2 : 3;
       // fp32 splits a row's numbers once per block: 64 x 128 (two buffers) for short rows, the
       // largest block that fits for long ones
       if (dtype == TRIFAST_F32 && d <= 32) pick = n <= 256 ? (d == 32 ? 5 : 2) : 3;
