@@ -160,22 +160,31 @@ struct RowSchedOf {
 // (one tile more in LDS when the row takes several passes: the words of the queries then leave
 // LDS the room, and the dq carried between the passes takes registers)
 constexpr int bwd_row_v_lds_tiles(int D, int KT, bool multi = false) { return KT * (D / 16) < 16 ? 0 : D <= 32 ? KT - (multi ? 2 : 3) : 1; }
+// Two waves per SIMD (256 registers each, the accumulators among the ordinary ones) where a wave holds at
+// most two key tiles of rows of up to 64 bytes.  Two workgroups of four waves per compute unit for up to
+// 256 keys: one row's loads and stores, and the waits inside its query tiles, go on beside the other
+// row's arithmetic (h = 4, d = 32: n = 256 71.8 -> 52.1 us, 200 59.7 -> 41.7, 128 23.4 -> 17.8, 77
+// 20.3 -> 15.9; with the accumulators in AGPRs the kernel had 279 registers and one workgroup).  One
+// workgroup of eight waves (KTB > 0, see the kernel) for up to 512.
+constexpr bool bwd_row_two_waves(int D, int KT) { return D <= 32 && KT <= 2; }
+constexpr int bwd_row_waves(int KTB) { return KTB > 0 ? 2 * kRowWaves : kRowWaves; }
 // LDS bytes of the kernel below.  dq partials: two buffers (one barrier per query tile) of
-// three quarters of a tile per wave (the quarter a wave sums itself waits in its dS tile)
-constexpr int bwd_row_red_bytes(int D) { return kRowWaves * 3 * ((D + 31) / 32) * 1024; }
-constexpr int bwd_row_base_lds_bytes(int D, int es, int KT, bool multi) {  // (without the per-query words)
-  const int rowb = D * es, keys = kRowWaves * KT * 32;
-  return keys * rowb + 3 * (2 * 32 * rowb) + kRowWaves * 2048 + 2 * bwd_row_red_bytes(D) +
+// three quarters of a tile per wave (the quarter a wave sums itself waits in its dS tile); with eight
+// waves all of every tile
+constexpr int bwd_row_red_bytes(int D, int KTB = 0) { return kRowWaves * (KTB > 0 ? 8 : 3) * ((D + 31) / 32) * 1024; }
+constexpr int bwd_row_base_lds_bytes(int D, int es, int KT, bool multi, int KTB) {  // (without the per-query words)
+  const int rowb = D * es, keys = kRowWaves * (KT + KTB) * 32;
+  return keys * rowb + 3 * (2 * 32 * rowb) + bwd_row_waves(KTB) * 2048 + 2 * bwd_row_red_bytes(D, KTB) +
          kRowWaves * bwd_row_v_lds_tiles(D, KT, multi) * (D / 16) * 1024;
 }
 // The per-query operand words of the row (two planes of 4 bytes per query) live in LDS where
 // there is room and the row takes one pass; else they come from the global planes that the
 // prologue writes, one query tile ahead.
-constexpr bool bwd_row_words_in_lds(int D, int es, int KT, bool multi) {
-  return !multi && bwd_row_base_lds_bytes(D, es, KT, multi) + 2 * kRowWaves * KT * 32 * 4 <= 160 * 1024;
+constexpr bool bwd_row_words_in_lds(int D, int es, int KT, bool multi, int KTB = 0) {
+  return !multi && bwd_row_base_lds_bytes(D, es, KT, multi, KTB) + 2 * kRowWaves * (KT + KTB) * 32 * 4 <= 160 * 1024;
 }
-constexpr int bwd_row_lds_bytes(int D, int es, int KT, bool multi = false) {
-  return bwd_row_base_lds_bytes(D, es, KT, multi) + (bwd_row_words_in_lds(D, es, KT, multi) ? 2 * kRowWaves * KT * 32 * 4 : 0);
+constexpr int bwd_row_lds_bytes(int D, int es, int KT, bool multi = false, int KTB = 0) {
+  return bwd_row_base_lds_bytes(D, es, KT, multi, KTB) + (bwd_row_words_in_lds(D, es, KT, multi, KTB) ? 2 * kRowWaves * (KT + KTB) * 32 * 4 : 0);
 }
 
 // XCDs that work on a head together: the smallest power of two whose heads side by side (8 / share of
@@ -191,8 +200,8 @@ constexpr int64_t bwd_row_blocks(int bh, int n) {
 
 // LDS bytes of bwd_uniform_row: each wave's four 32-row tiles and 64 floats of delta, then the
 // sums of the row (two D x D products, three vectors)
-constexpr int bwd_uniform_lds_bytes(int D, int es) {
-  const int tiles = kRowWaves * (4 * 32 * D * es + 256), sums = (2 * D * D + 3 * D) * 4;
+constexpr int bwd_uniform_lds_bytes(int D, int es, int NW) {
+  const int tiles = NW * (4 * 32 * D * es + 256), sums = (2 * D * D + 3 * D) * 4;
   return tiles + sums;
 }
 
@@ -209,7 +218,7 @@ constexpr int bwd_uniform_lds_bytes(int D, int es) {
 // 397 valid positions (bf16, h = 4, d = 32), with the same rule in db and the rows dealt evenly:
 // 605 -> 543 us.
 // (Several passes over a long row: the first one does all of it.)
-template <typename T, int D>
+template <typename T, int D, int NW>
 TRI_DEV void bwd_uniform_row(const BwdArgs& a, int bh, int i, unsigned char* smem, int wave, int lane) {
   using E = Elem<T>;
   using frag = typename E::frag;
@@ -230,7 +239,7 @@ TRI_DEV void bwd_uniform_row(const BwdArgs& a, int bh, int i, unsigned char* sme
   constexpr int TILE = 32 * Tile::ROWB;
   unsigned char* const mine = smem + wave * (4 * TILE + 256);
   float* const delta = reinterpret_cast<float*>(mine + 4 * TILE);  // [32]
-  float* const m1 = reinterpret_cast<float*>(smem + kRowWaves * (4 * TILE + 256));  // [D][D]
+  float* const m1 = reinterpret_cast<float*>(smem + NW * (4 * TILE + 256));  // [D][D]
   float* const m2 = m1 + D * D;
   float* const sk = m2 + D * D;  // sK, sQ, sO
   float* const sq = sk + D;
@@ -260,7 +269,7 @@ TRI_DEV void bwd_uniform_row(const BwdArgs& a, int bh, int i, unsigned char* sme
     }
   };
   if constexpr (AHEAD) load_tile(wave);
-  for (int t = wave; t < a.nwords; t += kRowWaves) {
+  for (int t = wave; t < a.nwords; t += NW) {
     if constexpr (!AHEAD) load_tile(t);
     vec x[4][NV], ov[NV];
 #pragma unroll
@@ -269,7 +278,7 @@ TRI_DEV void bwd_uniform_row(const BwdArgs& a, int bh, int i, unsigned char* sme
       for (int w = 0; w < 4; ++w) x[w][u] = xn[w][u];
       ov[u] = on[u];
     }
-    if constexpr (AHEAD) load_tile(t + kRowWaves);
+    if constexpr (AHEAD) load_tile(t + NW);
     // rows past the end count as zeros
 #pragma unroll
     for (int u = 0; u < NV; ++u) {
@@ -328,7 +337,7 @@ TRI_DEV void bwd_uniform_row(const BwdArgs& a, int bh, int i, unsigned char* sme
     __builtin_amdgcn_wave_barrier();
   }
   // the waves' parts, in wave order
-  for (int w = 0; w < kRowWaves; ++w) {
+  for (int w = 0; w < NW; ++w) {
     if (wave == w) {
 #pragma unroll
       for (int mt = 0; mt < DM; ++mt)
@@ -416,7 +425,7 @@ TRI_DEV void bwd_uniform_row(const BwdArgs& a, int bh, int i, unsigned char* sme
     }
   };
   if constexpr (AHEAD) load_ops(wave);
-  for (int t = wave; t < a.nwords; t += kRowWaves) {
+  for (int t = wave; t < a.nwords; t += NW) {
     if constexpr (!AHEAD) load_ops(t);
     const int j = 32 * t + jl;
     frag df[DS], vf[DS];
@@ -429,7 +438,7 @@ TRI_DEV void bwd_uniform_row(const BwdArgs& a, int bh, int i, unsigned char* sme
       for (int e = 0; e < 8; ++e) d += (float)pn[s][e] * (float)dn[s][e];
     }
     d = half_sum(d);
-    if constexpr (AHEAD) load_ops(t + kRowWaves);
+    if constexpr (AHEAD) load_ops(t + NW);
     f32x16 q[DM], k[DM];
 #pragma unroll
     for (int mt = 0; mt < DM; ++mt) {
@@ -450,37 +459,49 @@ TRI_DEV void bwd_uniform_row(const BwdArgs& a, int bh, int i, unsigned char* sme
   }
 }
 
-template <typename T, int D, int KT, bool MULTI = false>
-__global__ __launch_bounds__(kRowWaves * 64, 1) void tri_bwd_row_kernel(const BwdArgs a) {
+// KTB > 0: eight waves, two per SIMD.  Waves 0..3 hold KTA key tiles, waves 4..7 (which also add up
+// dq) KTB <= KTA.  One wave per SIMD leaves the SIMD idle wherever its own chain waits: at the start of a
+// query tile, behind its barrier, in front of the first scores (with four key tiles 1.8 of 4.7 thousand
+// clocks of a query tile).  Against four waves of KTA + KTB key tiles on one card, h = 4: d = 16 n = 384
+// 150 -> 136 us, 512 326 -> 284; d = 32 n = 300 121 -> 117, 384 176 -> 171, 449 334 -> 329, 512 344 / 344, with
+// padding from 397 on 320 -> 311 (eight waves write twice the dq partials, and they still meet at one
+// barrier per query tile).  Wider rows and more key tiles do not fit 256 registers.
+template <typename T, int D, int KTA, bool MULTI = false, int KTB = 0>
+__global__ __launch_bounds__(bwd_row_waves(KTB) * 64, bwd_row_two_waves(D, KTA) ? 2 : 1) void tri_bwd_row_kernel(const BwdArgs a) {
+  constexpr int KT = KTA;
+  // (two waves per SIMD: the accumulators are ordinary registers)
+  constexpr bool TWO = bwd_row_two_waves(D, KT);
+  static_assert(KTB == 0 || (TWO && !MULTI && KTB <= KT), "eight waves: two per SIMD, one pass");
   static_assert(sizeof(T) == 2, "16-bit inputs only (the transposing LDS reads)");
   using E = Elem<T>;
   using frag = typename E::frag;
   using Tile = LdsTile<T, D>;
   using DsTile = LdsTile<T, 32, 2>;  // the wave's dS tile: 16-byte stores of whole rows, transposed reads
-  constexpr int NWV = kRowWaves;
+  constexpr int NWV = bwd_row_waves(KTB);  // waves
+  constexpr int NWT = kRowWaves;           // key tiles from one of a wave's tiles to its next
   constexpr int KP = E::KP;
   constexpr int DS = D / (2 * KP);
   constexpr int DM = (D + 31) / 32;
   constexpr int PS = 2;
   constexpr int ROWB = Tile::ROWB;
-  constexpr int KEYS = NWV * KT * 32;         // keys (and queries) the workgroup can hold
-  constexpr bool WORDS_LDS = bwd_row_words_in_lds(D, (int)sizeof(T), KT, MULTI);  // per-query words of the row in LDS (else from the global planes)
+  constexpr int KEYS = NWT * (KT + KTB) * 32;         // keys (and queries) the workgroup can hold
+  constexpr bool WORDS_LDS = bwd_row_words_in_lds(D, (int)sizeof(T), KT, MULTI, KTB);  // per-query words of the row in LDS (else from the global planes)
   constexpr int STAGE = 2 * 32 * ROWB;        // Q tile | dO tile
   constexpr int OFF_K = 0;
   constexpr int OFF_ST = KEYS * ROWB;
   constexpr int OFF_DS = OFF_ST + 3 * STAGE;  // three stages: in use, ready, in flight
   constexpr int OFF_RED = OFF_DS + NWV * 2048;
-  constexpr int OFF_NL = OFF_RED + 2 * bwd_row_red_bytes(D);
+  constexpr int OFF_NL = OFF_RED + 2 * bwd_row_red_bytes(D, KTB);
   constexpr int PLANE = WORDS_LDS ? KEYS * 4 : 0;  // per-query words of the row
   constexpr int OFF_ND = OFF_NL + PLANE;
   constexpr int G2W = (2 * 32 * (ROWB / 16) / 64 + NWV - 1) / NWV;  // global->LDS loads per wave and stage
   constexpr int VL = bwd_row_v_lds_tiles(D, KT, MULTI);  // this wave's last VL key tiles keep V in LDS
   constexpr int VR = KT - VL;
   constexpr int OFF_V = OFF_ND + PLANE;
-  static_assert(OFF_V + NWV * VL * DS * 1024 == bwd_row_lds_bytes(D, (int)sizeof(T), KT, MULTI), "the launcher sizes LDS with bwd_row_lds_bytes");
-  static_assert(bwd_row_lds_bytes(D, (int)sizeof(T), KT, MULTI) <= 160 * 1024, "LDS of one compute unit");
-  static_assert(bwd_uniform_lds_bytes(D, (int)sizeof(T)) <= bwd_row_lds_bytes(D, (int)sizeof(T), KT, MULTI), "LDS of a fully masked row");
-  static_assert((KT - 1) * NWV * 32 * ROWB + 32 * ROWB <= 65536, "key tile offsets are LDS immediates");
+  static_assert(OFF_V + NWV * VL * DS * 1024 == bwd_row_lds_bytes(D, (int)sizeof(T), KT, MULTI, KTB), "the launcher sizes LDS with bwd_row_lds_bytes");
+  static_assert(bwd_row_lds_bytes(D, (int)sizeof(T), KT, MULTI, KTB) <= 160 * 1024, "LDS of one compute unit");
+  static_assert(bwd_uniform_lds_bytes(D, (int)sizeof(T), NWV) <= bwd_row_lds_bytes(D, (int)sizeof(T), KT, MULTI, KTB), "LDS of a fully masked row");
+  static_assert((KT - 1) * NWT * 32 * ROWB + 32 * ROWB <= 65536, "key tile offsets are LDS immediates");
   extern __shared__ __attribute__((aligned(16))) unsigned char tri_smem[];
 
   TRI_ROW_MARK(t_entry);
@@ -488,6 +509,8 @@ __global__ __launch_bounds__(kRowWaves * 64, 1) void tri_bwd_row_kernel(const Bw
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int kl = lane & 31, g = lane >> 5;
+  // this wave's key tiles: first_tile, first_tile + 4, ... of the pass
+  const int first_tile = KTB > 0 && wave >= kRowWaves ? kRowWaves * KT + wave - kRowWaves : wave;
   const int N = a.N;
   const int NJ = a.nwords;  // 32-tiles of the row (queries and keys)
   // this pass: key tiles KT0 .. KT0 + 4 KT - 1 of the row (tiles past the row's end are empty)
@@ -538,6 +561,7 @@ __global__ __launch_bounds__(kRowWaves * 64, 1) void tri_bwd_row_kernel(const Bw
     const int jrow = 32 * jt;
 #pragma unroll
     for (int x = 0; x < (G2 + NWV - 1) / NWV; ++x) {
+      if (G2 < NWV && wave >= G2) break;  // (more waves than loads: what these waves have in flight is bias tiles alone)
       const int gi = (x * NWV + wave) % G2;
       const bool is_q = gi < G2 / 2;  // wave-uniform
       const T* rows = is_q ? qrow : dorow;
@@ -560,19 +584,19 @@ __global__ __launch_bounds__(kRowWaves * 64, 1) void tri_bwd_row_kernel(const Bw
   if (uniform_word(a.rowflag, b * N + i) != 0) {
     wait_dma();  // (the loads on their way into the LDS it uses)
     __syncthreads();
-    if (first_pass) bwd_uniform_row<T, D>(a, bh, i, tri_smem, wave, lane);
+    if (first_pass) bwd_uniform_row<T, D, NWV>(a, bh, i, tri_smem, wave, lane);
     return;
   }
   // keep words of this wave's key tiles (bit k set = key k of the tile is attended)
   uint32_t kw[KT];
 #pragma unroll
   for (int t = 0; t < KT; ++t) {
-    const int kt = KT0 + NWV * t + wave;
+    const int kt = KT0 + NWT * t + first_tile;
     kw[t] = uniform_word(a.keep, (b * N + i) * a.nwords + min(kt, NJ - 1));
   }
 #pragma unroll
   for (int t = 0; t < KT; ++t)
-    if (KT0 + NWV * t + wave >= NJ) kw[t] = 0u;
+    if (KT0 + NWT * t + first_tile >= NJ) kw[t] = 0u;
   TRI_ROW_MARK(t_p1);
   const uint32_t lanebit = 1u << kl;
 
@@ -586,7 +610,7 @@ __global__ __launch_bounds__(kRowWaves * 64, 1) void tri_bwd_row_kernel(const Bw
   frag vx[KT][DS];
 #pragma unroll
   for (int t = 0; t < KT; ++t) {
-    const int key = min(32 * (KT0 + NWV * t + wave) + kl, N - 1);
+    const int key = min(32 * (KT0 + NWT * t + first_tile) + kl, N - 1);
 #pragma unroll
     for (int s = 0; s < DS; ++s) vx[t][s] = *reinterpret_cast<const frag*>(vrow + (int64_t)key * a.sv.j + 2 * KP * s + KP * g);
   }
@@ -682,7 +706,7 @@ __global__ __launch_bounds__(kRowWaves * 64, 1) void tri_bwd_row_kernel(const Bw
   OperandOffsets<T, D> ofq, ofk;
   ofq.init(perm32(kl), lane);
   ofk.init(kl, lane);
-  ofk.shift(wave * 32 * ROWB);  // key tile t of this wave starts (4 t + wave) * 32 rows into K
+  ofk.shift(first_tile * 32 * ROWB);  // key tile t of this wave starts (4 t + first_tile) * 32 rows into K
   OperandOffsets<T, 32, 2> ofd;
   ofd.init(0, lane);
   // (one tile: the wave reads dS of a key tile back before it writes the next one)
@@ -698,7 +722,7 @@ __global__ __launch_bounds__(kRowWaves * 64, 1) void tri_bwd_row_kernel(const Bw
   uint32_t bias_lane = (uint32_t)((perm32(kl) + 32 * g) * 8 * sizeof(T));
   asm volatile("" : "+v"(bias_lane));
   auto bias_load = [&](int jt, int t, u32x4v* dst) {
-    const int kt = min(KT0 + NWV * t + wave, a.NP - 1);
+    const int kt = min(KT0 + NWT * t + first_tile, a.NP - 1);
     const char* tile = reinterpret_cast<const char*>(pack_bh + ((int64_t)min(jt, a.NP - 1) * a.NP + kt) * 1024);
     uint32_t vo = bias_lane;
     asm volatile("" : "+v"(vo));  // (opaque here: the sum of the lane offset and the head's base is not hoisted as a 64-bit vector)
@@ -751,17 +775,19 @@ __global__ __launch_bounds__(kRowWaves * 64, 1) void tri_bwd_row_kernel(const Bw
   // key-tile steps they would be spilled, and a reload from scratch waits for every load
   // in flight.
   static_assert(DM * 1024 <= 2048, "the own quarter of a dq tile fits the wave's dS tile");
-  constexpr int RED_BYTES = bwd_row_red_bytes(D);
+  constexpr int RED_BYTES = bwd_row_red_bytes(D, KTB);
   // byte offsets in LDS, all wave-uniform and the same for every query tile: where this wave
   // leaves quarter q of its tile (per buffer), where its own quarter waits, and where the other
   // waves leave their parts of its quarter (three slots side by side)
-  int part_wr[2][NWV];
+  // (Eight waves: all parts of a quarter side by side, in wave order, and wave 4 + q sums quarter q.)
+  const int quarter = KTB > 0 ? wave & (kRowWaves - 1) : wave;
+  int part_wr[2][kRowWaves];
 #pragma unroll
-  for (int q = 0; q < NWV; ++q)
+  for (int q = 0; q < kRowWaves; ++q)
 #pragma unroll
     for (int bf = 0; bf < 2; ++bf)
-      part_wr[bf][q] = q == wave ? OFF_DS + wave * 2048 : OFF_RED + bf * RED_BYTES + (q * 3 + (wave < q ? wave : wave - 1)) * DM * 1024;
-  const int part_own = OFF_DS + wave * 2048, part_rd = OFF_RED + wave * 3 * DM * 1024;
+      part_wr[bf][q] = KTB > 0 ? OFF_RED + bf * RED_BYTES + (q * NWV + wave) * DM * 1024 : q == wave ? OFF_DS + wave * 2048 : OFF_RED + bf * RED_BYTES + (q * 3 + (wave < q ? wave : wave - 1)) * DM * 1024;
+  const int part_own = OFF_DS + wave * 2048, part_rd = OFF_RED + quarter * (KTB > 0 ? NWV : 3) * DM * 1024;
   T* dqrow = reinterpret_cast<T*>(a.dq) + b * a.sdq.b + h * a.sdq.h + i * a.sdq.i;
   T* lorow = reinterpret_cast<T*>(a.dq_lo) + ((int64_t)bh * N + i) * N * D;  // (several passes only)
   typedef uint32_t u32x2v __attribute__((ext_vector_type(2)));
@@ -786,7 +812,7 @@ __global__ __launch_bounds__(kRowWaves * 64, 1) void tri_bwd_row_kernel(const Bw
     int ln = lane;
     asm volatile("" : "+v"(ln));
 #pragma unroll
-    for (int q = 0; q < NWV; ++q)
+    for (int q = 0; q < kRowWaves; ++q)
 #pragma unroll
       for (int mt = 0; mt < DM; ++mt) {
         f32x4 x;
@@ -796,12 +822,21 @@ __global__ __launch_bounds__(kRowWaves * 64, 1) void tri_bwd_row_kernel(const Bw
       }
   };
   // the four parts of this wave's quarter: its own, then the other waves' in wave order
+  // (eight waves: four parts at a time)
   struct DqParts {
-    f32x4 v[NWV][DM];
+    f32x4 v[4][DM];
   };
-  auto load_partials = [&](int buf, DqParts& pp) {
+  auto load_partials = [&](int buf, DqParts& pp, int half = 0) {
     int ln = lane;
     asm volatile("" : "+v"(ln));
+    if constexpr (KTB > 0) {
+      const f32x4* parts = reinterpret_cast<const f32x4*>(tri_smem + part_rd + (buf ? RED_BYTES : 0)) + ln;
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+#pragma unroll
+        for (int mt = 0; mt < DM; ++mt) pp.v[k][mt] = parts[((4 * half + k) * DM + mt) * 64];
+      return;
+    }
     const f32x4* own = reinterpret_cast<const f32x4*>(tri_smem + part_own) + ln;
     const f32x4* others = reinterpret_cast<const f32x4*>(tri_smem + part_rd + (buf ? RED_BYTES : 0)) + ln;
 #pragma unroll
@@ -821,8 +856,19 @@ __global__ __launch_bounds__(kRowWaves * 64, 1) void tri_bwd_row_kernel(const Bw
     u32x2v hi[DM], lo[DM];
     uint32_t off;
   };
-  constexpr int kSumPieces = 6;
-  auto sum_dq_piece = [&](int piece, int jt, const DqParts& pp, const DqCarry& cy, DqOut& o) {
+  constexpr int kSumPieces = KTB > 0 ? 8 : 6;
+  auto sum_dq_piece = [&](int piece, int jt, DqParts& pp, const DqCarry& cy, DqOut& o) {
+    if constexpr (KTB > 0) {
+      if (piece == 3 || piece == 4) {
+#pragma unroll
+        for (int mt = 0; mt < DM; ++mt) {
+          if (piece == 3) o.sum[mt] = (o.sum[mt] + pp.v[0][mt]) + pp.v[1][mt];
+          else o.sum[mt] = (o.sum[mt] + pp.v[2][mt]) + pp.v[3][mt];
+        }
+        return;
+      }
+      if (piece > 4) piece -= 2;
+    }
     if (piece == 0) {
 #pragma unroll
       for (int mt = 0; mt < DM; ++mt) o.sum[mt] = pp.v[0][mt] + pp.v[1][mt];
@@ -857,7 +903,7 @@ __global__ __launch_bounds__(kRowWaves * 64, 1) void tri_bwd_row_kernel(const Bw
     } else {
       int ln = lane;
       asm volatile("" : "+v"(ln));
-      const int jl = ln & 31, d0 = 8 * wave + 4 * (ln >> 5);
+      const int jl = ln & 31, d0 = 8 * quarter + 4 * (ln >> 5);
       const bool live = jt >= 0 && jl < N - 32 * jt && d0 < D;
       // (row strides of the gradients are below 2^24 elements, like those of the inputs)
       o.off = live ? (__umul24((uint32_t)jl, (uint32_t)a.sdq.j) + (uint32_t)d0) * (uint32_t)sizeof(T) : ~0u;
@@ -869,7 +915,7 @@ __global__ __launch_bounds__(kRowWaves * 64, 1) void tri_bwd_row_kernel(const Bw
     if (o.off != ~0u) {
 #pragma unroll
       for (int mt = 0; mt < DM; ++mt) {
-        if (32 * mt + 8 * wave >= D) continue;  // (wave-uniform; head dims that are no multiple of 32)
+        if (32 * mt + 8 * quarter >= D) continue;  // (wave-uniform; head dims that are no multiple of 32)
         asm volatile("global_store_dwordx2 %0, %1, %2 offset:%3" : : "v"(o.off), "v"(o.hi[mt]), "s"(base), "n"(64 * mt) : "memory");
         if constexpr (MULTI) {
           if (!last_pass) {
@@ -892,8 +938,10 @@ __global__ __launch_bounds__(kRowWaves * 64, 1) void tri_bwd_row_kernel(const Bw
   // tiles attended (no mask work) and some keys masked out.  Inside a query tile the key tiles run as a software pipeline: the score
   // and dP MFMAs of tile t+1 are issued before the exponentials of tile t, and the dq
   // MFMAs of tile t-1 (whose dS has been through LDS by then) after them.
-  auto query_tiles = [&](auto masked_tag) __attribute__((always_inline)) {
-    constexpr bool MASKED = decltype(masked_tag)::value;
+  // (eight waves: in two versions each, for the waves that sum dq and for the others)
+  auto query_tiles = [&](auto masked_tag, auto tiles_tag, auto sums_tag) __attribute__((always_inline)) {
+    constexpr bool MASKED = decltype(masked_tag)::value, SUMS = decltype(sums_tag)::value;
+    constexpr int KT = decltype(tiles_tag)::value;  // this wave's key tiles
     // (each version has its own accumulators, from zeroing to the final stores: merging
     // the versions' accumulators where they meet would copy all of them)
     f32x16 dkacc[KT][DM], dvacc[KT][DM];
@@ -901,8 +949,12 @@ __global__ __launch_bounds__(kRowWaves * 64, 1) void tri_bwd_row_kernel(const Bw
     for (int t = 0; t < KT; ++t)
 #pragma unroll
       for (int mt = 0; mt < DM; ++mt) {
-        E::mfma_acc_zero(dkacc[t][mt]);
-        E::mfma_acc_zero(dvacc[t][mt]);
+        if constexpr (TWO) {
+          dkacc[t][mt] = dvacc[t][mt] = zero16();
+        } else {
+          E::mfma_acc_zero(dkacc[t][mt]);
+          E::mfma_acc_zero(dvacc[t][mt]);
+        }
       }
     // The wave is alone on its SIMD, so nothing but its own instruction order hides a
     // latency: the code below is laid out as the schedule it should run in, and scheduling
@@ -919,7 +971,7 @@ __global__ __launch_bounds__(kRowWaves * 64, 1) void tri_bwd_row_kernel(const Bw
       bias_load(jt + t / KT, t % KT, bias_ring[(t % KT) % 2]);
     };
     fetch_bias(0, 0);
-    fetch_bias(0, 1);
+    if constexpr (KT > 1) fetch_bias(0, 1);  // (a wave of one key tile fetches its next one behind its first step's last use)
     uint32_t lw_next = 0u, dw_next = 0u;  // words from the global planes: those of the next query tile
     if constexpr (!WORDS_LDS) fetch_words(0, lw_next, dw_next);
     DqCarry carry;
@@ -983,7 +1035,7 @@ __global__ __launch_bounds__(kRowWaves * 64, 1) void tri_bwd_row_kernel(const Bw
       frag dst_prev[PS], ktr_prev[DM][PS];
       frag vn[DS];           // V operands of the next tile when they live in LDS
       auto load_kn = [&](int t) {
-        const unsigned char* ktile = lds_k + NWV * t * 32 * ROWB;
+        const unsigned char* ktile = lds_k + NWT * t * 32 * ROWB;
 #pragma unroll
         for (int s = 0; s < DS; ++s) kn[s] = ofk.natural(ktile, s);
       };
@@ -1010,10 +1062,27 @@ __global__ __launch_bounds__(kRowWaves * 64, 1) void tri_bwd_row_kernel(const Bw
         // (words from the global planes: those of the next query tile, fetched before the last
         // bias tile of this one so that no wait for them is a wait for everything in flight)
         if constexpr (!WORDS_LDS && t == KT - 1) fetch_words(jt + 1, lw_next, dw_next);
-        if constexpr (valu && !refill) fetch_bias(jt, t + 2);
+        if constexpr (KT > 1 && valu && !refill) fetch_bias(jt, t + 2);
         frag kb = keys_op.plain();
         if constexpr (has_next && MASKED) kb = keys_op.masked(kw[tn]);
         SB();
+        auto unit = [&](int u) __attribute__((always_inline)) {
+          if (u < 8) {
+#pragma unroll
+            for (int e = 0; e < 2; ++e) p[2 * u + e] = fast_exp2(s_cur[2 * u + e] * c);
+          } else if (u < 12) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) ds[4 * (u - 8) + e] = p[4 * (u - 8) + e] * p_cur[4 * (u - 8) + e];
+          } else if (u < 14) {
+            pf[u - 12] = E::pack(&p[KP * (u - 12)]);
+          } else {
+            dsf[u - 14] = E::pack(&ds[KP * (u - 14)]);
+          }
+        };
+        if constexpr (NM == 0) {  // (the one key tile of the wave: nothing beside it)
+#pragma unroll
+          for (int u = 0; u < NU; ++u) unit(u);
+        }
         static_for<NM>([&](auto xc) __attribute__((always_inline)) {
           constexpr int x = decltype(xc)::value;
           constexpr int kind = Sch::value.kind[x], idx = Sch::value.idx[x];
@@ -1030,7 +1099,9 @@ __global__ __launch_bounds__(kRowWaves * 64, 1) void tri_bwd_row_kernel(const Bw
             else p_nxt = E::mfma(don[idx], vn[idx], p_nxt);
           } else if constexpr (kind == R_ACC) {
             constexpr int s2 = (idx / 2) / DM, mt = (idx / 2) % DM;
-            if constexpr (idx % 2 == 0) E::mfma_acc(dotr[mt][s2], pf[s2], dvacc[tp][mt]);
+            if constexpr (TWO && idx % 2 == 0) dvacc[tp][mt] = E::mfma(dotr[mt][s2], pf[s2], dvacc[tp][mt]);
+            else if constexpr (TWO) dkacc[tp][mt] = E::mfma(qtr[mt][s2], dsf[s2], dkacc[tp][mt]);
+            else if constexpr (idx % 2 == 0) E::mfma_acc(dotr[mt][s2], pf[s2], dvacc[tp][mt]);
             else E::mfma_acc(qtr[mt][s2], dsf[s2], dkacc[tp][mt]);
           } else {
             if constexpr (tp == 0 && idx / DM == 0) dqacc[idx % DM] = E::mfma(ktr_prev[idx % DM][idx / DM], dst_prev[idx / DM], zero16());
@@ -1046,11 +1117,14 @@ __global__ __launch_bounds__(kRowWaves * 64, 1) void tri_bwd_row_kernel(const Bw
           // not stored).  No wait for a load that could follow within the time a store takes
           // allows fewer than two operations in flight, so none of them waits for this store
           // (a wait for loads issued after a store is a wait for the store as well).
-          if constexpr (t == -1) {
+          if constexpr (t == -1 && SUMS) {
             if constexpr (x == 0) load_partials((jt + 1) & 1, parts);
 #pragma unroll
             for (int piece = 0; piece < kSumPieces; ++piece)
-              if ((piece + 3 < NM ? piece + 3 : NM - 1) == x) sum_dq_piece(piece, jt - 1, parts, carry, dq_words);
+              if ((piece + 3 < NM ? piece + 3 : NM - 1) == x) {
+                sum_dq_piece(piece, jt - 1, parts, carry, dq_words);
+                if (KTB > 0 && piece == 2) load_partials((jt + 1) & 1, parts, 1);
+              }
             if constexpr (x == NM - 1) {
               store_dq(jt - 1, dq_base, dq_words);
               if (jt > 0) dq_base += 32 * a.sdq.j;
@@ -1062,7 +1136,7 @@ __global__ __launch_bounds__(kRowWaves * 64, 1) void tri_bwd_row_kernel(const Bw
           if constexpr (has_prev && x == Sch::value.dq_reads_at) {
             // dS of tile t-1 comes back from LDS with the key index in-lane, with the K
             // rows of that tile transposed beside it
-            const unsigned char* ktile = lds_k + NWV * tp * 32 * ROWB;
+            const unsigned char* ktile = lds_k + NWT * tp * 32 * ROWB;
 #pragma unroll
             for (int s2 = 0; s2 < PS; ++s2) {
               dst_prev[s2] = ofd.transposed(ds_tile, s2, 0);
@@ -1081,19 +1155,7 @@ __global__ __launch_bounds__(kRowWaves * 64, 1) void tri_bwd_row_kernel(const Bw
             for (int s = 0; s < DS; ++s) vn[s] = v_lds[((tn - VR) * DS + s) * 64];
           }
 #pragma unroll
-          for (int u = x * NU / NM; u < (x + 1) * NU / NM; ++u) {
-            if (u < 8) {
-#pragma unroll
-              for (int e = 0; e < 2; ++e) p[2 * u + e] = fast_exp2(s_cur[2 * u + e] * c);
-            } else if (u < 12) {
-#pragma unroll
-              for (int e = 0; e < 4; ++e) ds[4 * (u - 8) + e] = p[4 * (u - 8) + e] * p_cur[4 * (u - 8) + e];
-            } else if (u < 14) {
-              pf[u - 12] = E::pack(&p[KP * (u - 12)]);
-            } else {
-              dsf[u - 14] = E::pack(&ds[KP * (u - 14)]);
-            }
-          }
+          for (int u = x * NU / NM; u < (x + 1) * NU / NM; ++u) unit(u);
           SB();
         });
         if constexpr (valu) {
@@ -1119,12 +1181,15 @@ __global__ __launch_bounds__(kRowWaves * 64, 1) void tri_bwd_row_kernel(const Bw
       TRI_ROW_TICK(KT + 4);
       buf = buf == 2 ? 0 : buf + 1;
     }
-    {
+    if constexpr (SUMS) {
       DqParts parts;
       DqOut dq_words;
       load_partials((NJ - 1) & 1, parts);
 #pragma unroll
-      for (int piece = 0; piece < kSumPieces; ++piece) sum_dq_piece(piece, NJ - 1, parts, carry, dq_words);
+      for (int piece = 0; piece < kSumPieces; ++piece) {
+        sum_dq_piece(piece, NJ - 1, parts, carry, dq_words);
+        if (KTB > 0 && piece == 2) load_partials((NJ - 1) & 1, parts, 1);
+      }
       store_dq(NJ - 1, dq_base, dq_words);
     }
 #ifdef TRI_ROW_TIMING
@@ -1138,12 +1203,14 @@ __global__ __launch_bounds__(kRowWaves * 64, 1) void tri_bwd_row_kernel(const Bw
     T* dvrow = reinterpret_cast<T*>(a.dv) + b * a.sdv.b + h * a.sdv.h + i * a.sdv.i;
   #pragma unroll
     for (int t = 0; t < KT; ++t) {
-      const int key = 32 * (KT0 + NWV * t + wave) + kl;
+      const int key = 32 * (KT0 + NWT * t + first_tile) + kl;
   #pragma unroll
       for (int mt = 0; mt < DM; ++mt) {
 #ifndef TRI_MFMA_ACC_BUILTIN
-        asm volatile("s_nop 15" : "+a"(dkacc[t][mt]));
-        asm volatile("s_nop 15" : "+a"(dvacc[t][mt]));
+        if constexpr (!TWO) {
+          asm volatile("s_nop 15" : "+a"(dkacc[t][mt]));
+          asm volatile("s_nop 15" : "+a"(dvacc[t][mt]));
+        }
 #endif
       }
       store_rows_wide<T, D, DM>(dkrow + (int64_t)key * a.sdk.j, dkacc[t], a.scale, g, key < N);
@@ -1165,9 +1232,17 @@ __global__ __launch_bounds__(kRowWaves * 64, 1) void tri_bwd_row_kernel(const Bw
   };
   bool plain = true;
 #pragma unroll
-  for (int t = 0; t < KT; ++t) plain = plain && kw[t] == 0xffffffffu;
-  if (plain) query_tiles(std::false_type{});
-  else query_tiles(std::true_type{});
+  for (int t = 0; t < KT; ++t) plain = plain && (kw[t] == 0xffffffffu || (KTB > 0 && wave >= kRowWaves && t >= KTB));
+  auto version = [&](auto tiles_tag, auto sums_tag) __attribute__((always_inline)) {
+    if (plain) query_tiles(std::false_type{}, tiles_tag, sums_tag);
+    else query_tiles(std::true_type{}, tiles_tag, sums_tag);
+  };
+  if constexpr (KTB > 0) {
+    if (wave < kRowWaves) version(std::integral_constant<int, KT>{}, std::false_type{});
+    else version(std::integral_constant<int, KTB>{}, std::true_type{});
+  } else {
+    version(std::integral_constant<int, KT>{}, std::true_type{});
+  }
 
 }
 

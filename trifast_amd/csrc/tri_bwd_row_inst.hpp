@@ -12,13 +12,15 @@ constexpr int kRowKT[kBwdRowTiles] = {2, 3, 4, 5, 6, 7, 8, 8};  // (the last one
 template <typename T, int D, int KT>
 hipError_t bwd_row_run(const BwdArgs& a, int bh, hipStream_t st, bool dry) {
   constexpr int DM = (D + 31) / 32;
-  constexpr int lds = bwd_row_lds_bytes(D, (int)sizeof(T), KT);
-  // the dk, dv accumulators of KT key tiles stay in registers (half of the file at most)
+  if (a.N > kRowWaves * KT * 32) return hipErrorInvalidConfiguration;
+  // rows of three and four key tiles for four waves, up to 64 bytes: eight waves of two and of one or two
+  constexpr int KTB = D <= 32 && (KT == 3 || KT == 4) ? KT - 2 : 0, KTA = KT - KTB;
+  constexpr int lds = bwd_row_lds_bytes(D, (int)sizeof(T), KTA, false, KTB);
+  // the dk, dv accumulators of a wave's key tiles stay in registers (half of the file at most)
   if constexpr (2 * KT * DM * 16 <= 256 && lds <= kMaxLds) {
-    if (a.N > kRowWaves * KT * 32) return hipErrorInvalidConfiguration;
     if (dry) return hipSuccess;
     const dim3 grid((unsigned)bwd_row_blocks(bh, a.N));
-    return launch_dyn(tri_bwd_row_kernel<T, D, KT>, grid, dim3(kRowWaves * 64), lds, st, a);
+    return launch_dyn(tri_bwd_row_kernel<T, D, KTA, false, KTB>, grid, dim3(bwd_row_waves(KTB) * 64), lds, st, a);
   } else {
     return hipErrorInvalidConfiguration;
   }
