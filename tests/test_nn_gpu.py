@@ -160,6 +160,50 @@ def test_weight_gradient_against_float64(dtype, rows, k, n):
     assert bool(((db.double() - want_b).abs() <= bound_b).all())
 
 
+@pytest.mark.parametrize("dtype,k,ns,n,hd,swap", [
+    (torch.bfloat16, 128, [128, 128, 128, 4, 128], 17, 32, False),  # 289 rows: 33 in the second chunk, one in its second half-stage
+    (torch.float16, 64, [64, 32, 2], 16, 32, True),                 # one chunk, rows a whole number of stages; layers share a group
+    (torch.bfloat16, 32, [32, 96, 30], 33, 16, False),              # 65 rows in the last chunk; no full 1 KiB share per wave
+    (torch.float16, 128, [128, 3], 40, 0, True),                    # an odd number of outputs does not ride
+    (torch.bfloat16, 128, [36, 92, 8], 65, 0, True),                # blocks that end in the middle, rows of dy not on 16 bytes
+    (torch.bfloat16, 256, [128, 32], 33, 64, False),                # the widest input: nothing rides
+])
+def test_weight_gradients_of_several_layers(dtype, k, ns, n, hd, swap):
+    """All layers in one launch against float64: which blocks of outputs share a workgroup, the layer
+    that rides with the first group, ends of chunks, of stages and of their halves, both row orders.
+    The last row's first channel is infinite: it must not reach any other column."""
+    import ctypes
+
+    from trifast_amd import _lib
+
+    rows = n * n
+    gen = torch.Generator().manual_seed(rows + k)
+    x = torch.randn(n, n, k, generator=gen).to(DEV, dtype)
+    x[-1, -1, 0] = float("inf")
+    hds = [hd if hd and m % hd == 0 else 0 for m in ns]
+    dys = [torch.randn(rows, m, generator=gen).to(DEV, dtype) for m in ns]
+    outer = [d.view(rows, m // c, c).transpose(0, 1).contiguous() if c else d for d, m, c in zip(dys, ns, hds)]
+    dw = [torch.full((m, k), 7.0, device=DEV, dtype=dtype) for m in ns]
+    db = [torch.full((m,), 7.0, device=DEV, dtype=dtype) if i % 2 else None for i, m in enumerate(ns)]
+    lib, i64, ptrs = _lib.load(), _lib.i64_array, lambda ts: (ctypes.c_void_p * len(ts))(*[None if t is None else t.data_ptr() for t in ts])
+    ws = torch.empty(lib.trifast_block_dw_workspace_bytes(rows, k, len(ns), i64(ns)), dtype=torch.uint8, device=DEV)
+    _lib.check(lib.trifast_block_in_bwd(None, ptrs(dw), ptrs(db), x.data_ptr(), 1, n, k, len(ns), ptrs(outer), ptrs(dys), i64(ns), i64(hds), swap,
+                                        _lib.BF16 if dtype == torch.bfloat16 else _lib.F16, ws.data_ptr(), ws.numel(),
+                                        torch.cuda.current_stream().cuda_stream), "trifast_block_in_bwd")
+    xr = (x.transpose(0, 1) if swap else x).reshape(rows, k)[:, 1:].double()
+    eps, tiny = torch.finfo(dtype).eps, torch.finfo(dtype).smallest_normal
+    for p, dy in enumerate(dys):
+        dy = dy.double()
+        assert not torch.isfinite(dw[p][:, 0]).any()
+        want, size = dy.t() @ xr, dy.abs().t() @ xr.abs()
+        # fp32 accumulation of exact products in a fixed order, one rounding to the dtype
+        bound = 0.5 * eps * want.abs() + rows**0.5 * 2.0**-22 * size + tiny
+        assert bool(((dw[p][:, 1:].double() - want).abs() <= bound).all()), f"layer {p}"
+        if db[p] is not None:
+            want, size = dy.sum(0), dy.abs().sum(0)
+            assert bool(((db[p].double() - want).abs() <= 0.5 * eps * want.abs() + rows**0.5 * 2.0**-22 * size + tiny).all()), f"layer {p} bias"
+
+
 def test_linear_gradients_are_those_of_the_layer():
     torch.manual_seed(5)
     dtype = torch.bfloat16

@@ -777,12 +777,24 @@ static void dw_layer(tri::LinearDwArgs& a, const void* dy, int64_t n, int64_t he
   a.total += n * a.K;
   a.off_b[p] = db ? a.total : -1;
   if (db) a.total += n;
-  a.groups += (int)((n + 127) / 128);
+}
+// how a launch whose layers are complete is split
+static void dw_split(tri::LinearDwArgs& a) {
+  const tri::LinearDwGroups s = tri::linear_dw_groups(a.n, a.nlayers, a.K);
+  a.groups = s.groups;
+  a.rider = s.rider;
+  a.rows_per_chunk = tri::linear_dw_rows_per_chunk(a.rows, a.groups, a.K);
+  a.chunks = (int)((a.rows + a.rows_per_chunk - 1) / a.rows_per_chunk);
+}
+static int64_t dw_chunks(int64_t rows, int64_t k, int nlayers, const int64_t* n) {
+  const int64_t per = tri::linear_dw_rows_per_chunk(rows, tri::linear_dw_groups(n, nlayers, k).groups, k);
+  return (rows + per - 1) / per;
 }
 
 int64_t trifast_linear_dw_workspace_bytes(int64_t rows, int64_t k, int64_t n) {
   if (rows < 1 || k < 1 || n < 1) return fail(TRIFAST_EINVAL, "sizes must be positive");
-  return align256(tri::linear_dw_chunks(rows) * n * k * 4) + align256(tri::linear_dw_chunks(rows) * n * 4);
+  const int64_t chunks = dw_chunks(rows, k, 1, &n);
+  return align256(chunks * n * k * 4) + align256(chunks * n * 4);
 }
 
 int trifast_linear_dw(void* dw, void* db, const void* dy, const void* x, int64_t rows, int64_t k, int64_t n, int64_t head_dim, int dtype,
@@ -799,9 +811,9 @@ int trifast_linear_dw(void* dw, void* db, const void* dy, const void* x, int64_t
     return fail(TRIFAST_EWORKSPACE, "linear_dw: workspace missing, misaligned or smaller than trifast_linear_dw_workspace_bytes");
   tri::LinearDwArgs a{};
   a.x = x; a.part = static_cast<float*>(workspace);
-  a.rows = rows; a.rows_per_chunk = tri::linear_dw_rows_per_chunk(rows); a.chunks = (int)tri::linear_dw_chunks(rows);
-  a.K = (int)k;
+  a.rows = rows; a.K = (int)k;
   dw_layer(a, dy, n, head_dim, dw, db);
+  dw_split(a);
   const hipError_t e = tri::linear_dw_launch(a, dtype, static_cast<hipStream_t>(stream));
   if (e != hipSuccess) return hip_fail(e, "linear_dw launch");
   return 0;
@@ -818,7 +830,7 @@ static int linear_fwd_impl(const void* x, int64_t rows, int64_t k, int nlayers, 
   if ((reinterpret_cast<uintptr_t>(x) & 15) != 0) return fail(TRIFAST_EALIGN, "linear_fwd: x is not 16-byte aligned");
   tri::LinearFwdArgs a{};
   a.x = x; a.rows = rows; a.K = (int)k; a.nlayers = nlayers;
-  a.xmap.n = swap_n;
+  a.xmap = tri::row_map(swap_n);
   for (int p = 0; p < nlayers; ++p) {
     if (!w[p] || !y[p]) return fail(TRIFAST_EINVAL, "linear_fwd: layer %d: null pointer", p);
     if (n[p] < 1 || n[p] > (1 << 20)) return fail(TRIFAST_EINVAL, "linear_fwd: layer %d: %lld outputs", p, (long long)n[p]);
@@ -848,7 +860,7 @@ static int linear_dx_impl(void* dx, int64_t rows, int64_t k, int nlayers, const 
   if ((reinterpret_cast<uintptr_t>(dx) & 15) != 0) return fail(TRIFAST_EALIGN, "linear_dx: dx is not 16-byte aligned");
   tri::LinearDxArgs a{};
   a.dx = dx; a.rows = rows; a.K = (int)k; a.nlayers = nlayers;
-  a.map.n = swap_n;
+  a.map = tri::row_map(swap_n);
   for (int p = 0; p < nlayers; ++p) {
     if (!dy[p] || !w[p]) return fail(TRIFAST_EINVAL, "linear_dx: layer %d: null pointer", p);
     if (n[p] < 1 || n[p] > (1 << 20)) return fail(TRIFAST_EINVAL, "linear_dx: layer %d: %lld outputs", p, (long long)n[p]);
@@ -876,19 +888,14 @@ static int check_block(int64_t b, int64_t n, int dtype) {
 
 int64_t trifast_block_dw_workspace_bytes(int64_t rows, int64_t k, int nlayers, const int64_t* n) {
   if (rows < 1 || k < 1 || nlayers < 1 || !n) return fail(TRIFAST_EINVAL, "sizes must be positive");
-  int64_t total = 0, groups = 0;
-  for (int p = 0; p < nlayers; ++p) {
-    total += n[p] * k + n[p];
-    groups += (n[p] + 127) / 128;
-  }
-  const int64_t per = tri::linear_dw_rows_per_chunk(rows, (int)groups);
-  return align256((rows + per - 1) / per * total * 4);
+  int64_t total = 0;
+  for (int p = 0; p < nlayers; ++p) total += n[p] * k + n[p];
+  return align256(dw_chunks(rows, k, nlayers, n) * total * 4);
 }
 
 // the weight-gradient launch of layers whose arguments are complete but for the split of the rows
 static int block_dw(tri::LinearDwArgs& a, int dtype, void* workspace, int64_t workspace_bytes, void* stream) {
-  a.rows_per_chunk = tri::linear_dw_rows_per_chunk(a.rows, a.groups);
-  a.chunks = (int)((a.rows + a.rows_per_chunk - 1) / a.rows_per_chunk);
+  dw_split(a);
   if (!workspace || (reinterpret_cast<uintptr_t>(workspace) & 255) != 0 || workspace_bytes < (int64_t)a.chunks * a.total * 4)
     return fail(TRIFAST_EWORKSPACE, "block: workspace missing, misaligned or smaller than trifast_block_dw_workspace_bytes");
   a.part = static_cast<float*>(workspace);
@@ -919,7 +926,7 @@ int trifast_block_in_bwd(void* dx, void* const* dw, void* const* db, const void*
   if (!tri::linear_dw_k_ok(k)) return fail(TRIFAST_EUNSUPPORTED, "block_in_bwd: %lld input channels (32, 64, 128 or 256 are compiled)", (long long)k);
   if (!x || (reinterpret_cast<uintptr_t>(x) & 15) != 0) return fail(TRIFAST_EALIGN, "block_in_bwd: x is null or not 16-byte aligned");
   tri::LinearDwArgs a{};
-  a.x = x; a.rows = rows; a.K = (int)k; a.xmap.n = swap_n;
+  a.x = x; a.rows = rows; a.K = (int)k; a.xmap = tri::row_map(swap_n);
   for (int p = 0; p < nlayers; ++p) {
     if (!dy[p] || !dw[p]) return fail(TRIFAST_EINVAL, "block_in_bwd: layer %d: null pointer", p);
     if (nout[p] < 1 || nout[p] > (1 << 20)) return fail(TRIFAST_EINVAL, "block_in_bwd: layer %d: %lld outputs", p, (long long)nout[p]);
@@ -948,8 +955,8 @@ int trifast_block_out_fwd(void* out, const void* o, const void* g, const void* w
   if (!out || (reinterpret_cast<uintptr_t>(out) & 15) != 0) return fail(TRIFAST_EALIGN, "block_out_fwd: out is null or not 16-byte aligned");
   tri::LinearFwdArgs a{};
   a.w[0] = w; a.bias[0] = bias; a.y[0] = out; a.n[0] = (int)c; a.nlayers = 1;
-  a.rows = b * n * n; a.K = (int)(h * d); a.ymap.n = swap ? (uint32_t)n : 0;
-  a.o = o; a.g = g; a.plane = (uint32_t)(n * n); a.H = (int)h; a.D = (int)d; a.lgD = __builtin_ctzll((unsigned long long)d);
+  a.rows = b * n * n; a.K = (int)(h * d); a.ymap = tri::row_map(swap ? (uint32_t)n : 0);
+  a.o = o; a.g = g; a.plane = tri::make_divisor((uint32_t)(n * n)); a.H = (int)h; a.D = (int)d; a.lgD = __builtin_ctzll((unsigned long long)d);
   const hipError_t e = tri::linear_fwd_launch(a, dtype, static_cast<hipStream_t>(stream));
   if (e != hipSuccess) return hip_fail(e, "block_out_fwd launch");
   return 0;
@@ -966,15 +973,15 @@ int trifast_block_out_bwd(void* dout_o, void* dg, void* dw, void* db, const void
     if (!dg || ((reinterpret_cast<uintptr_t>(dout_o) | reinterpret_cast<uintptr_t>(dg)) & 15) != 0) return fail(TRIFAST_EALIGN, "block_out_bwd: do and dg must be 16-byte aligned");
     tri::LinearGateBwdArgs a{};
     a.dout = dout; a.w = w; a.o = o; a.g = g; a.dox = dout_o; a.dg = dg;
-    a.rows = b * n * n; a.plane = (uint32_t)(n * n); a.K = (int)c; a.C = (int)(h * d); a.H = (int)h; a.D = (int)d; a.lgD = lgd;
-    a.map.n = swap ? (uint32_t)n : 0;
+    a.rows = b * n * n; a.plane = tri::make_divisor((uint32_t)(n * n)); a.K = (int)c; a.C = (int)(h * d); a.H = (int)h; a.D = (int)d; a.lgD = lgd;
+    a.map = tri::row_map(swap ? (uint32_t)n : 0);
     const hipError_t e = tri::linear_gate_bwd_launch(a, dtype, static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return hip_fail(e, "block_out_bwd launch");
   }
   if (!dw) return 0;
   tri::LinearDwArgs a{};
-  a.x = o; a.g = g; a.rows = b * n * n; a.K = (int)(h * d); a.ymap.n = swap ? (uint32_t)n : 0;
-  a.plane = (uint32_t)(n * n); a.H = (int)h; a.D = (int)d; a.lgD = lgd;
+  a.x = o; a.g = g; a.rows = b * n * n; a.K = (int)(h * d); a.ymap = tri::row_map(swap ? (uint32_t)n : 0);
+  a.plane = tri::make_divisor((uint32_t)(n * n)); a.H = (int)h; a.D = (int)d; a.lgD = lgd;
   dw_layer(a, dout, c, 0, dw, db);
   return block_dw(a, dtype, workspace, workspace_bytes, stream);
 }

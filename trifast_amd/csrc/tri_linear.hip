@@ -89,12 +89,11 @@ hipError_t dx_k(const LinearDxArgs& a, hipStream_t st) {
 
 template <typename T, int KD>
 hipError_t dw_run(const LinearDwArgs& a, hipStream_t st) {
-  const dim3 grid((unsigned)((a.chunks + 7) / 8 * 8 * a.groups)), block(256);
-  if (a.g) hipLaunchKernelGGL((linear_dw_kernel<T, KD, true>), grid, block, 0, st, a);
-  else hipLaunchKernelGGL((linear_dw_kernel<T, KD, false>), grid, block, 0, st, a);
-  hipError_t e = hipGetLastError();
+  const dim3 grid((unsigned)((a.chunks + 7) / 8 * 8 * a.groups));
+  const hipError_t e = a.g ? launch_dyn(linear_dw_kernel<T, KD, true>, grid, dim3(512), LinearDwShape<T, KD, true>::LDS, st, a)
+                           : launch_dyn(linear_dw_kernel<T, KD, false>, grid, dim3(512), LinearDwShape<T, KD, false>::LDS, st, a);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL((linear_dw_reduce_kernel<T>), dim3((unsigned)((a.total + 31) / 32)), block, 0, st, a);
+  hipLaunchKernelGGL((linear_dw_reduce_kernel<T>), dim3((unsigned)((a.total + 31) / 32)), dim3(256), 0, st, a);
   return hipGetLastError();
 }
 

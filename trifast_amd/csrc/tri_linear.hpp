@@ -53,17 +53,21 @@ struct ChunkColumns {
   }
 };
 
+// x / v.d for x < 2^31
+TRI_DEV uint32_t quotient(uint32_t x, const Divisor& v) { return v.mul == 0 ? x : __umulhi(x, v.mul) >> v.shift; }
+
 // row of a tensor in pair order (b, i, j) for row `r` of the order the operator works in
 TRI_DEV int64_t mapped_row(const RowMap& m, int64_t r) {
-  if (m.n == 0) return r;
-  const uint32_t q = (uint32_t)r / m.n, j = (uint32_t)r % m.n;  // q = b n + i
-  const uint32_t b = q / m.n, i = q % m.n;
-  return ((int64_t)b * m.n + j) * m.n + i;
+  if (m.by.d == 0) return r;
+  const uint32_t n = m.by.d, q = quotient((uint32_t)r, m.by), j = (uint32_t)r - q * n;  // q = b n + i
+  const uint32_t b = quotient(q, m.by), i = q - b * n;
+  return (b * n + j) * n + i;
 }
 
 // Element offset of head row 0 of row r in the operator's layout [b, H, n, n, D] (head h: + h * plane * D)
-TRI_DEV int64_t outer_row(int64_t r, uint32_t plane, int H, int D) {
-  return ((int64_t)((uint32_t)r / plane) * H * plane + (uint32_t)r % plane) * D;
+TRI_DEV int64_t outer_row(int64_t r, const Divisor& plane, int H, int D) {
+  const uint32_t b = quotient((uint32_t)r, plane);
+  return ((int64_t)b * H * plane.d + ((uint32_t)r - b * plane.d)) * D;
 }
 // ... and of channel k (of H * D) from there; D is a power of two
 TRI_DEV int64_t outer_channel(int k, uint32_t plane, int lgD) { return ((int64_t)(k >> lgD) * plane << lgD) + (k & ((1 << lgD) - 1)); }
@@ -156,7 +160,7 @@ __global__ __launch_bounds__(256) void linear_fwd_kernel(const LinearFwdArgs a) 
 #pragma unroll
       for (int s = 0; s < KS; ++s) {
         const int k = 16 * s + 8 * g;
-        xf[t][s] = gated_piece<T>(*reinterpret_cast<const vec*>(o + outer_channel(k, a.plane, a.lgD)), *reinterpret_cast<const vec*>(gt + k));
+        xf[t][s] = gated_piece<T>(*reinterpret_cast<const vec*>(o + outer_channel(k, a.plane.d, a.lgD)), *reinterpret_cast<const vec*>(gt + k));
       }
     } else {
       const T* x = reinterpret_cast<const T*>(a.x) + mapped_row(a.xmap, rr) * KD;
@@ -289,7 +293,7 @@ __global__ __launch_bounds__(256) void linear_gate_bwd_kernel(const LinearGateBw
 #pragma unroll
     for (int half = 0; half < 2; ++half) {
       const int k = 32 * min(q0 + q, a.C / 32 - 1) + 16 * half + 8 * g;
-      oofs[q][half] = outer + outer_channel(k, a.plane, a.lgD);
+      oofs[q][half] = outer + outer_channel(k, a.plane.d, a.lgD);
       gv[q][half] = *reinterpret_cast<const vec*>(reinterpret_cast<const T*>(a.g) + rr * a.C + k);
       ov[q][half] = *reinterpret_cast<const vec*>(reinterpret_cast<const T*>(a.o) + oofs[q][half]);
     }
@@ -451,151 +455,332 @@ __global__ __launch_bounds__(256) void linear_dx_kernel(const LinearDxArgs a) {
 // The contraction runs over the long dimension and the result is tiny, which is the one shape of
 // the block's linear layers that a BLAS library serves badly (one or two workgroups walk all the
 // rows: 1.7 ms per layer at rows = 2^20, K = N = 128).  Here the rows are split into chunks,
-// one workgroup per (chunk, group of 128 output rows of one layer): it streams its rows of dy and
-// x through LDS 32 at a time (both operands have the contraction index as their memory row, so
-// both are read back transposed, ds_read_tr), keeps its part of dW in fp32 accumulators (wave w:
-// rows n of its 32-block, all K columns), and writes it as an fp32 partial; a second kernel adds
-// the partials of all layers in a fixed order (deterministic, no atomics) and rounds once.
-// The groups of all layers run in one launch (the x rows of a chunk come from L2 for all but
-// the first), because the layers one by one leave most of the GPU idle below a million rows.
-// GATED: x is o * sigmoid(g) (see linear_fwd).
+// one workgroup per (chunk, group of four 32-output blocks of the layers): it streams its rows of
+// dy and x through a ring of LDS stages of 64 rows (both operands have the contraction index as
+// their memory row, so both are read back transposed, ds_read_tr), keeps its part of dW in fp32
+// accumulators, and writes it as an fp32 partial; a second kernel adds the partials of all layers
+// in a fixed order (deterministic, no atomics) and rounds once.
+//
+// Eight waves: waves 0-3 take the first 32 rows of a stage, 4-7 the other 32, wave w the outputs of
+// block w % 4 and all K columns; the halves are added through LDS at the end.  One workgroup fills
+// a CU (two at K <= 64), so a launch writes a third of the partials that three workgroups of four
+// waves would.  A wave loads its own dy tile and a quarter of its half's x tile, straight into LDS:
+// nothing that is in flight is in registers.  The ring is as deep as the blocks of the group leave room.
+//
+// A layer of up to 16 outputs that would open a group for itself (the four biases next to four
+// layers of 128 outputs) rides in the first group, each of its waves taking one K block of it in
+// four: as a group of its own it read all of x for 3 % of the work.
+//
+// Bound by HBM.  rows = 147456, K = 128, four layers of 128 outputs and one of 4: 80 -> 51 us, 3.9
+// TB/s of dy, x and partials (three workgroups of four waves per CU with padded tiles filled through
+// registers, the four outputs a group: 61 % of its LDS cycles were bank conflicts); gated, one layer: 42
+// -> 33 us; the sum of the partials 10.5 -> 6.3 us, each.  One layer alone, 2^20 rows: K = 256, 128
+// outputs 215 -> 160 us, K = 128 131 -> 107, 8 outputs 66 -> 69 (an odd number of outputs, loaded one at a
+// time: 102 -> 140 at K = 128, faster below 10^5 rows and at the other K).
+//
+// GATED: x is o * sigmoid(g) (see linear_fwd); o and g land in LDS and each wave gates the pieces
+// it loaded before the stage is handed over.
 // ---------------------------------------------------------------------------------------
 template <typename T, int KD, bool GATED>
-__global__ __launch_bounds__(256) void linear_dw_kernel(const LinearDwArgs a) {
+struct LinearDwShape {
+  static constexpr int XB = 32 * KD * (int)sizeof(T), YB = 32 * 32 * (int)sizeof(T);  // x tile of a half, dy tile of a wave
+  static constexpr int XP = XB / 1024;           // 1 KiB loads of an x tile, shared by the four waves of the half
+  static constexpr int XN = (XP + 3) / 4;        // ... per wave (a wave without one loads into `DUMP`)
+  static constexpr int OFF_G = 2 * XB, OFF_Y = (GATED ? 4 : 2) * XB;
+  static constexpr bool RIDER = !GATED && KD <= 128;  // (the gated layer comes alone)
+  static constexpr int RB = 32 * kLinearDwRider * (int)sizeof(T);  // dy tile of a riding layer, of a half
+  static constexpr int LDS = 160 * 1024 / kLinearDwPerCu<KD>, DUMP = XP % 4 ? LDS - 1024 : LDS;
+  // loads per wave and stage: of x, of dy (16 or, where its rows keep only 4-byte alignment, 4 bytes per lane)
+  static constexpr int X_LOADS = (GATED ? 2 : 1) * XN, Y_LOADS = 2, Y4_LOADS = 8;
+  static constexpr int MOST = 6;  // stages of a ring
+};
+
+// 16 (or 4) bytes per lane into LDS at dst + the lane's piece; unseen by the compiler (see StageRing)
+TRI_DEV void dma16(uint32_t dst, const void* src) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(dst), "v"(src) : "memory", "m0");
+}
+TRI_DEV void dma4(uint32_t dst, const void* src) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" : : "s"(dst), "v"(src) : "memory", "m0");
+}
+// wait until at most n (wave-uniform) loads are in flight; the count is part of the instruction
+template <int LO, int HI>
+TRI_DEV void wait_loads(int n) {
+  if constexpr (LO == HI) {
+    asm volatile("s_waitcnt vmcnt(%0)" : : "n"(LO) : "memory");
+  } else {
+    constexpr int mid = (LO + HI + 1) / 2;
+    if (n >= mid) wait_loads<mid, HI>(n);
+    else wait_loads<LO, mid - 1>(n);
+  }
+}
+
+// the two halves of a transposing operand read
+template <typename T>
+TRI_DEV typename Elem<T>::frag tr_pair(const unsigned char* p_lo, const unsigned char* p_hi) {
+  const auto lo = lds_tr4(reinterpret_cast<const T*>(p_lo));
+  const auto hi = lds_tr4(reinterpret_cast<const T*>(p_hi));
+  typename Elem<T>::frag f;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) { f[e] = lo[e]; f[4 + e] = hi[e]; }
+  return f;
+}
+
+template <typename T, int KD, bool GATED>
+__global__ __launch_bounds__(512, 2 * kLinearDwPerCu<KD>) void linear_dw_kernel(const LinearDwArgs a) {
   using E = Elem<T>;
   using frag = typename E::frag;
   using vec = typename E::vec;
-  constexpr int ND = 128;
-  constexpr int KB = KD / 32;                // 32-column blocks of x
-  constexpr int LDX = KD + 8, LDY = ND + 8;  // padded rows (16-byte multiples)
-  constexpr int XCH = 32 * KD / 8, YCH = 32 * ND / 8;      // 16-byte chunks of a step's tiles
-  constexpr int XC = (XCH + 255) / 256, YC = YCH / 256;  // ... per lane
-  __shared__ __attribute__((aligned(16))) T xs[2][32][LDX];
-  __shared__ __attribute__((aligned(16))) T ys[2][32][LDY];
+  using S = LinearDwShape<T, KD, GATED>;
+  using XTile = LdsTile<T, KD>;
+  using YTile = LdsTile<T, 32>;
+  using RTile = LdsTile<T, kLinearDwRider>;
+  constexpr int XN = S::XN;
+  constexpr int KB = KD / 32, KE = (KB + 4) / 4;  // K blocks; ... and the bias sums of a riding layer, per wave
+  extern __shared__ __attribute__((aligned(16))) unsigned char lin_smem[];
 
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int half = wave >> 2, wc = wave & 3;
   const int g = lane >> 5;
   int chunk, grp;
   rows_remap(a.groups, chunk, grp);
   if (chunk >= a.chunks) return;
-  int p = 0;
-  while (p + 1 < a.nlayers && grp >= (a.n[p] + ND - 1) / ND) grp -= (a.n[p++] + ND - 1) / ND;
-  const int N = a.n[p], hd = a.hd[p];
-  const int n_grp = grp * ND;  // first output row of this workgroup
+  // this wave's block: layer p, outputs col0 .. (not live: there is none)
+  int p = 0, col0 = 0, blocks_here = -4 * grp;  // (blocks_here: of this group)
+  bool live = true;
+  {
+    int at = -1, left = 4 * grp + wc;
+    for (int l = 0; l < a.nlayers; ++l) {
+      if (l == a.rider) continue;
+      const int blocks = (a.n[l] + 31) / 32;
+      if (at < 0) { p = l; col0 = 32 * min(left, blocks - 1); }
+      if (at < 0 && left < blocks) at = l;
+      left -= blocks;
+      blocks_here += blocks;
+    }
+    live = at >= 0;
+  }
+  blocks_here = min(blocks_here, 4);
+  const int N = a.n[p];
+  const bool rides = S::RIDER && a.rider >= 0 && grp == 0;
   const int64_t r_begin = (int64_t)chunk * a.rows_per_chunk;
   const int64_t r_end = min(a.rows, r_begin + a.rows_per_chunk);
-  const int steps = (int)((r_end - r_begin + 31) / 32);
-  const T* xg = reinterpret_cast<const T*>(a.x);
+  const int steps = (int)((r_end - r_begin + 63) / 64);
+  const bool even = (N % 8) != 0 && (N % 2) == 0, odd = (N % 2) != 0;  // rows of dy keep 4- or 2-byte alignment
+
+  // where this lane's pieces of the tiles lie: tile row and address in row 0
   const T* yg = reinterpret_cast<const T*>(a.dy[p]);
-  const bool y_vec = (N % 8) == 0;  // rows of dY keep 16-byte alignment
-  // this lane's column piece of the tiles is the same in every step: where it starts in row 0, and
-  // the distance between rows
-  const int xcol = 8 * (tid % (KD / 8)), ycol = n_grp + 8 * (tid % (ND / 8));
-  const T* x_lane = xg + (GATED ? outer_channel(xcol, a.plane, a.lgD) : xcol);
-  const T* g_lane = reinterpret_cast<const T*>(a.g) + xcol;
-  const T* y_lane = yg + linear_offset(0, ycol, N, hd, a.rows);
-  const int y_pitch = hd ? hd : N;
+  const int y_pitch = a.hd[p] ? a.hd[p] : N;
+  int xr[XN], rr = 0;
+  const T *xp[XN], *gp[XN], *rp = nullptr;
+  bool own[XN];  // (wave-uniform)
+#pragma unroll
+  for (int x = 0; x < XN; ++x) {
+    own[x] = 4 * x + wc < S::XP;
+    const int piece = min(4 * x + wc, S::XP - 1) * 64 + lane;
+    xr[x] = piece / XTile::CPR;
+    const int col = 8 * ((piece % XTile::CPR) ^ XTile::swz(xr[x]));
+    xp[x] = reinterpret_cast<const T*>(a.x) + (GATED ? outer_channel(col, a.plane.d, a.lgD) : col);
+    gp[x] = GATED ? reinterpret_cast<const T*>(a.g) + col : nullptr;
+  }
+  // (the second 16 rows of a dy tile have the swizzle of the first)
+  const int yr = lane / 4, ycol = col0 + 8 * ((lane % 4) ^ YTile::swz(yr));
+  // (columns past the layer's last: the block's first again, their outputs are not stored)
+  const T* yp = yg + linear_offset(0, ycol < N ? ycol : col0, N, a.hd[p], a.rows);
+  const int rN = rides ? a.n[a.rider] : 0;
+  const int r_pitch = rides && a.hd[a.rider] ? a.hd[a.rider] : rN;
+  if (rides) {
+    const int piece = wc * 64 + lane;  // of 4 bytes
+    rr = piece / (kLinearDwRider / 2);
+    const int in = piece % (kLinearDwRider / 2), col = 8 * ((in / 4) ^ RTile::swz(rr)) + 2 * (in % 4);
+    rp = reinterpret_cast<const T*>(a.dy[a.rider]) + linear_offset(0, col < rN ? col : 0, rN, a.hd[a.rider], a.rows);
+  }
+  // a stage: the x tiles of the two halves (o, then g), the dy tiles of their blocks, those of a riding layer
+  const int off_y = S::OFF_Y + (half * blocks_here + wc) * S::YB;
+  const int off_r = S::OFF_Y + 2 * blocks_here * S::YB + half * S::RB;
+  const int stage = S::OFF_Y + 2 * blocks_here * S::YB + (rides ? 2 * S::RB : 0);
+  const int depth = min(S::DUMP / stage, S::MOST), end = depth * stage;
+  const int in_flight = (depth - 2) * (S::X_LOADS + (!live ? 0 : even ? S::Y4_LOADS : S::Y_LOADS) + (rides ? 1 : 0));
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(TRI_L3 const unsigned char*)lin_smem;
+  auto uni = [](uint32_t x) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)x); };
 
-  // this lane's chunks of a step's tiles (tile row, first column), fetched two steps ahead of
-  // their use: one set of registers per step in flight
-  vec xr2[2][XC], yr2[2][YC], gr2[2][GATED ? XC : 1];
-  auto load_step = [&](int s, vec* xr, vec* yr, vec* gr) {
-    const int64_t r0 = r_begin + 32 * (int64_t)s;
+  // ask for stage s (rows past the end: the last one again) into the ring buffer at `boff`
+  auto issue = [&](int s, uint32_t boff) __attribute__((always_inline)) {
+    const int64_t first = r_begin + 64 * (int64_t)s + 32 * half, last = r_end - 1;
 #pragma unroll
-    for (int c = 0; c < XC; ++c) {
-      const int q = c * 256 + tid, r = q / (KD / 8);
-      vec v = {}, gv = {};
-      if (q < XCH && r0 + r < r_end) {
-        if constexpr (GATED) {
-          v = *reinterpret_cast<const vec*>(x_lane + outer_row(r0 + r, a.plane, a.H, a.D));
-          gv = *reinterpret_cast<const vec*>(g_lane + (r0 + r) * KD);
-        } else {
-          v = *reinterpret_cast<const vec*>(x_lane + mapped_row(a.xmap, r0 + r) * KD);
-        }
+    for (int x = 0; x < XN; ++x) {
+      const int64_t r = min(first + xr[x], last);
+      const uint32_t at = own[x] ? boff + half * S::XB + (4 * x + wc) * 1024 : S::DUMP;
+      if constexpr (GATED) {
+        dma16(uni(lds0 + at), xp[x] + outer_row(r, a.plane, a.H, a.D));
+        dma16(uni(lds0 + (own[x] ? at + S::OFF_G : at)), gp[x] + r * KD);
+      } else {
+        dma16(uni(lds0 + at), xp[x] + mapped_row(a.xmap, r) * KD);
       }
-      xr[c] = v;
-      if constexpr (GATED) gr[c] = gv;
     }
+    const uint32_t ybuf = boff + off_y;
+    if (!live) {
+      // (nobody reads its tile)
+    } else if (even) {
+      int ln = lane;
+      asm volatile("" : "+v"(ln));  // (what follows from the lane is worked out here, not kept in registers)
 #pragma unroll
-    for (int c = 0; c < YC; ++c) {
-      const int r = (c * 256 + tid) / (ND / 8);
-      vec v = {};
-      if (r0 + r < r_end && ycol < N) {
-        const T* src = y_lane + mapped_row(a.ymap, r0 + r) * y_pitch;
-        if (y_vec) {
-          v = *reinterpret_cast<const vec*>(src);
-        } else {
-#pragma unroll
-          for (int e = 0; e < 8; ++e)
-            if (ycol + e < N) v[e] = src[e];
-        }
+      for (int t = 0; t < 8; ++t) {
+        const int row = 4 * t + ln / 16, col = col0 + 8 * ((ln % 16 / 4) ^ YTile::swz(row)) + 2 * (ln % 4);
+        dma4(uni(lds0 + ybuf + t * 256), yg + mapped_row(a.ymap, min(first + row, last)) * N + (col < N ? col : col0));
       }
-      yr[c] = v;
+    } else if (!odd) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t) dma16(uni(lds0 + ybuf + t * 1024), yp + mapped_row(a.ymap, min(first + 16 * t + yr, last)) * y_pitch);
+    } else {
+      int ln = lane;
+      asm volatile("" : "+v"(ln));
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        const int row = 16 * t + ln / 4, col = col0 + 8 * ((ln % 4) ^ YTile::swz(row));
+        const T* src = yg + mapped_row(a.ymap, min(first + row, last)) * N;
+        vec v = {};
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          if (col + e < N) v[e] = src[col + e];
+        *reinterpret_cast<vec*>(lin_smem + ybuf + t * 1024 + lane * 16) = v;
+      }
     }
+    if (rides) dma4(uni(lds0 + boff + off_r + wc * 256), rp + mapped_row(a.ymap, min(first + rr, last)) * r_pitch);
   };
-  auto store_step = [&](int buf, const vec* xr, const vec* yr, const vec* gr) {
+  // what this wave loaded of stage s has landed: gate it, and clear rows past the end
+  auto finish = [&](int s, uint32_t boff) __attribute__((always_inline)) {
+    unsigned char* xbuf = lin_smem + boff + half * S::XB + lane * 16;
+    if constexpr (GATED) {
 #pragma unroll
-    for (int c = 0; c < XC; ++c) {
-      const int q = c * 256 + tid, r = q / (KD / 8), col = 8 * (q % (KD / 8));
-      // (rows past the end: o = 0, so the gated value is 0 too)
-      if (q < XCH) *reinterpret_cast<vec*>(&xs[buf][r][col]) = GATED ? gated_piece<T>(xr[c], gr[GATED ? c : 0]) : xr[c];
+      for (int x = 0; x < XN; ++x) {
+        if (!own[x]) continue;
+        vec* o = reinterpret_cast<vec*>(xbuf + (4 * x + wc) * 1024);
+        *o = gated_piece<T>(*o, *reinterpret_cast<const vec*>(xbuf + S::OFF_G + (4 * x + wc) * 1024));
+      }
     }
+    const int64_t first = r_begin + 64 * (int64_t)s + 32 * half;
+    if (first + 32 <= r_end) return;
+    const vec none = {};
 #pragma unroll
-    for (int c = 0; c < YC; ++c) {
-      const int q = c * 256 + tid, r = q / (ND / 8), col = 8 * (q % (ND / 8));
-      *reinterpret_cast<vec*>(&ys[buf][r][col]) = yr[c];
+    for (int x = 0; x < XN; ++x)
+      if (own[x] && first + xr[x] >= r_end) *reinterpret_cast<vec*>(xbuf + (4 * x + wc) * 1024) = none;
+    if (live) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+        if (first + 16 * t + yr >= r_end) *reinterpret_cast<vec*>(lin_smem + boff + off_y + t * 1024 + lane * 16) = none;
     }
+    if (rides && first + rr >= r_end) *reinterpret_cast<uint32_t*>(lin_smem + boff + off_r + wc * 256 + lane * 4) = 0u;
   };
 
-  f32x16 acc[KB];
+  f32x16 acc[KB], racc[KE];
 #pragma unroll
   for (int i = 0; i < KB; ++i) acc[i] = zero16();
-  // (a wave whose output rows lie past N only stages)
-  const bool wave_live = __builtin_amdgcn_readfirstlane((int)(n_grp + 32 * wave < N)) != 0;
+#pragma unroll
+  for (int i = 0; i < KE; ++i) racc[i] = zero16();
   // the bias gradient, the column sums of dy, rides along as one more product: dy^T times ones
-  const bool sums = a.off_b[p] >= 0;
+  const bool sums = a.off_b[p] >= 0, rsums = rides && a.off_b[a.rider < 0 ? 0 : a.rider] >= 0;
   const frag ones = E::osplat(1.0f);
   f32x16 bacc = zero16();
 
-  load_step(0, xr2[0], yr2[0], gr2[0]);
-  if (steps > 1) load_step(1, xr2[1], yr2[1], gr2[1]);
-  store_step(0, xr2[0], yr2[0], gr2[0]);
-  lds_sync();
-  auto one_step = [&](int s, auto parity) __attribute__((always_inline)) {
-    constexpr int buf = decltype(parity)::value;  // s % 2: the LDS buffer of step s, the register set of step s + 2
-    if (s + 2 < steps) load_step(s + 2, xr2[buf], yr2[buf], gr2[buf]);
-    if (wave_live) {
+  OperandOffsets<T, KD> xo;
+  OperandOffsets<T, 32> yo;
+  xo.init(0, lane);
+  yo.init(0, lane);
+  // a riding layer: its own tile, and the K blocks of this wave: wc, wc + 4, .. (block KB: its column sums)
+  const int r16lo = RTile::off(8 * g + ((lane & 15) >> 2), 8 * (lane & 3)), r16hi = RTile::off(8 * g + 4 + ((lane & 15) >> 2), 8 * (lane & 3));
+  int rlo[KE], rhi[KE];
 #pragma unroll
-      for (int s2 = 0; s2 < 2; ++s2) {
-        // A: dY^T (output row n in the lane, 8 memory rows as contraction slots); B: x^T
-        const frag af = lds_tr_frag<T, LDY>(ys[buf], 16 * s2 + 8 * g, 32 * wave, lane);
+  for (int i = 0; i < KE; ++i) {
+    const int row = 8 * g + ((lane & 15) >> 2), col = 32 * min(wc + 4 * i, KB - 1) + 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+    rlo[i] = XTile::off(row, col * 2);
+    rhi[i] = XTile::off(row + 4, col * 2);
+  }
+  auto compute = [&](uint32_t boff) __attribute__((always_inline)) {
+    const unsigned char *xt = lin_smem + boff + half * S::XB, *yt = lin_smem + boff + off_y;
+#pragma unroll
+    for (int s2 = 0; s2 < 2; ++s2) {
+      if (live) {
+        // A: dy^T (output row n in the lane, 8 memory rows as contraction slots); B: x^T
+        const frag af = yo.transposed(yt, s2, 0);
         if (sums) bacc = E::mfma(af, ones, bacc);
 #pragma unroll
-        for (int i = 0; i < KB; ++i) acc[i] = E::mfma(af, lds_tr_frag<T, LDX>(xs[buf], 16 * s2 + 8 * g, 32 * i, lane), acc[i]);
+        for (int i = 0; i < KB; ++i) acc[i] = E::mfma(af, xo.transposed(xt, s2, i), acc[i]);
+      }
+      if (rides) {
+        // (16 outputs: lanes 16-31 hold them again and are not stored)
+        const unsigned char* rt = lin_smem + boff + off_r + 16 * s2 * RTile::ROWB;
+        const frag rf = tr_pair<T>(rt + r16lo, rt + r16hi);
+#pragma unroll
+        for (int i = 0; i < KE; ++i) {
+          const unsigned char* xs = xt + 16 * s2 * XTile::ROWB;
+          if (wc + 4 * i < KB) racc[i] = E::mfma(rf, tr_pair<T>(xs + rlo[i], xs + rhi[i]), racc[i]);
+          else if (wc + 4 * i == KB && rsums) racc[i] = E::mfma(rf, ones, racc[i]);
+        }
       }
     }
-    // the other buffer was last read in step s - 1, which every wave left before the
-    // barrier that ended it
-    if (s + 1 < steps) store_step(buf ^ 1, xr2[buf ^ 1], yr2[buf ^ 1], gr2[buf ^ 1]);
-    lds_sync();
   };
-  for (int s = 0; s < steps; s += 2) {
-    one_step(s, std::integral_constant<int, 0>{});
-    if (s + 1 < steps) one_step(s + 1, std::integral_constant<int, 1>{});
+
+  for (int s = 0; s < min(depth - 1, steps); ++s) issue(s, s * stage);
+  int now = 0, next = end - stage;  // ring buffers of stages s and s + depth - 1
+  for (int s = 0; s < steps; ++s) {
+    // stage s of this wave has landed once at most the stages s + 1 .. s + depth - 2 are in flight
+    // (rows of dy that are loaded one number at a time have to arrive anyway)
+    wait_loads<0, 40>(odd || s + depth - 1 > steps ? 0 : in_flight);
+    finish(s, now);
+    lds_sync();
+    // (buffer `next` held stage s - 1, which every wave has read)
+    if (s + depth - 1 < steps) issue(s + depth - 1, next);
+    compute(now);
+    now = now + stage == end ? 0 : now + stage;
+    next = next + stage == end ? 0 : next + stage;
   }
-  if (!wave_live) return;
+
+  // the second half's sums -> LDS -> added to the first half's
+  auto fold = [&](f32x16* set, int count, int slot) __attribute__((always_inline)) {
+    float* at = reinterpret_cast<float*>(lin_smem) + ((slot * 4 + wc) * 16) * 64 + lane;
+#pragma unroll
+    for (int i = 0; i < count; ++i)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        float* f = at + (i * 4 * 16 + v) * 64;
+        if (half) *f = set[i][v];
+        else set[i][v] += *f;
+      }
+  };
+  lds_sync();
+  if (half) fold(acc, KB, 0);
+  lds_sync();
+  if (!half) fold(acc, KB, 0);
+  lds_sync();
+  if (half) {
+    fold(&bacc, 1, 0);
+    if (S::RIDER) fold(racc, KE, 1);
+  }
+  lds_sync();
+  if (half) return;
+  fold(&bacc, 1, 0);
+  if (S::RIDER) fold(racc, KE, 1);
+
   // partial [chunk][layer's n][k]: the lane holds column k = 32 kb + lane % 32 and rows
-  // n = 32 wave + 8 q + 4 g + e of the group
+  // n = 8 q + 4 g + e of the block
   float* part = a.part + (int64_t)chunk * a.total;
 #pragma unroll
   for (int v = 0; v < 16; ++v) {
-    const int n = n_grp + 32 * wave + 8 * (v / 4) + 4 * g + (v % 4);
-    if (n >= N) continue;
-    // (every column of the sums' product holds the same values: lanes 0 and 32 store theirs)
-    if (sums && (lane & 31) == 0) part[a.off_b[p] + n] = bacc[v];
+    const int in = 8 * (v / 4) + 4 * g + (v % 4), n = col0 + in;
+    if (live && n < N) {
+      // (every column of the sums' product holds the same values: lanes 0 and 32 store theirs)
+      if (sums && (lane & 31) == 0) part[a.off_b[p] + n] = bacc[v];
 #pragma unroll
-    for (int i = 0; i < KB; ++i) part[a.off_w[p] + (int64_t)n * KD + 32 * i + (lane & 31)] = acc[i][v];
+      for (int i = 0; i < KB; ++i) part[a.off_w[p] + (int64_t)n * KD + 32 * i + (lane & 31)] = acc[i][v];
+    }
+    if (rides && in < rN) {
+#pragma unroll
+      for (int i = 0; i < KE; ++i) {
+        if (wc + 4 * i == KB && rsums && (lane & 31) == 0) part[a.off_b[a.rider] + in] = racc[i][v];
+        if (wc + 4 * i < KB) part[a.off_w[a.rider] + (int64_t)in * KD + 32 * (wc + 4 * i) + (lane & 31)] = racc[i][v];
+      }
+    }
   }
 }
 

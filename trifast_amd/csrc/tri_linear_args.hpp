@@ -8,12 +8,26 @@ namespace tri {
 
 constexpr int kLinearLayers = 6;
 
-// Row order: n = 0, rows are taken as they lie; otherwise the tensor is in pair order (b, i, j)
+// Division of x < 2^31 by a launch's constant d as a product: with 2^s the next power of two at or above d and
+// mul = ceil(2^(31+s) / d) < 2^32, x / d = x mul >> 31 + s (the excess x (mul d - 2^(31+s)) / d stays below
+// 2^(31+s) / d).  mul = 0: d = 1.
+struct Divisor {
+  uint32_t d, mul, shift;
+};
+inline Divisor make_divisor(uint32_t d) {
+  if (d <= 1) return Divisor{d, 0, 0};
+  uint32_t s = 1;
+  while ((uint64_t(1) << s) < d) ++s;
+  return Divisor{d, (uint32_t)(((uint64_t(1) << (31 + s)) + d - 1) / d), s - 1};
+}
+
+// Row order: d = 0, rows are taken as they lie; otherwise the tensor is in pair order (b, i, j), i, j < d,
 // while the work runs over the pair-transposed order (ending node): row (b, i, j) of the work is
 // row (b, j, i) of the tensor.  (rows < 2^31)
 struct RowMap {
-  uint32_t n;
+  Divisor by;
 };
+inline RowMap row_map(uint32_t n) { return RowMap{make_divisor(n)}; }
 
 struct LinearFwdArgs {
   const void* x;                    // [rows, K] in the order of xmap
@@ -28,7 +42,7 @@ struct LinearFwdArgs {
   RowMap xmap, ymap;
   // gated source in place of x: o [b, H, n, n, D] (K = H D, plane = n^2) and g [rows, K]
   const void *o, *g;
-  uint32_t plane;
+  Divisor plane;
   int H, D, lgD;
   // filled by the launcher: 32-column chunks of all layers, chunks per workgroup, workgroups per row block
   int total_chunks, chunks, groups;
@@ -42,7 +56,7 @@ struct LinearGateBwdArgs {
   void* dox;         // like o
   void* dg;          // like g
   int64_t rows;
-  uint32_t plane;
+  Divisor plane;
   int K, C, H, D, lgD;
   RowMap map;
   int chunks, groups;  // filled by the launcher
@@ -71,31 +85,47 @@ struct LinearDwArgs {
   float* part;                      // [chunks][total] partial sums
   int64_t off_w[kLinearLayers], off_b[kLinearLayers];  // of a layer's parts in a chunk's row; off_b < 0: no bias gradient
   int64_t total;
-  int64_t rows, rows_per_chunk;     // (a multiple of 32)
-  int chunks, groups;
+  int64_t rows, rows_per_chunk;     // (a multiple of 64)
+  int chunks, groups, rider;        // (see linear_dw_groups)
   int K;
   RowMap xmap, ymap;
   const void* g;                    // gated source: g [rows, K]
-  uint32_t plane;
+  Divisor plane;
   int H, D, lgD;
 };
 
-// Rows of one chunk of the weight-gradient kernel: at least 1024 (the partials of a chunk cost as
-// much traffic as 128 rows), and at most 768 chunks: three workgroups per CU are resident at once,
-// and a grid that is not a whole number of such rounds leaves CUs idle in the last one.
-inline int64_t linear_dw_rows_per_chunk(int64_t rows) {
-  const int64_t per = ((rows + 767) / 768 + 31) / 32 * 32;
-  return per < 1024 ? 1024 : per;
+constexpr int kLinearDwRider = 16;  // outputs of a riding layer at most (see linear_dw_groups)
+
+// How the weight-gradient kernel's outputs are split over workgroups: groups of four 32-output blocks,
+// the layers' blocks one after the other.  A layer of one block that would be a group for itself
+// rides in the first group instead (an even number of outputs: it is loaded 4 bytes at a time; up
+// to 128 channels: the accumulators of one block and a part of another fill the registers at 256).
+struct LinearDwGroups {
+  int groups, rider;  // rider: layer, or -1
+};
+template <typename Int>
+inline LinearDwGroups linear_dw_groups(const Int* n, int nlayers, int64_t k) {
+  int64_t blocks = 0;
+  int small = -1;
+  for (int p = 0; p < nlayers; ++p) {
+    blocks += (n[p] + 31) / 32;
+    if (n[p] <= kLinearDwRider && n[p] % 2 == 0) small = p;
+  }
+  const bool rides = k <= 128 && small >= 0 && blocks > 1 && blocks % 4 == 1;
+  return LinearDwGroups{(int)((blocks - (rides ? 1 : 0) + 3) / 4), rides ? small : -1};
 }
-inline int64_t linear_dw_chunks(int64_t rows) {
-  const int64_t per = linear_dw_rows_per_chunk(rows);
-  return (rows + per - 1) / per;
-}
-// The same for several layers in one launch of `groups` workgroups per chunk.  (Down to 256 rows
-// per chunk: below 10^5 rows the GPU is not full, and the chunks' partials stay in the caches.)
-inline int64_t linear_dw_rows_per_chunk(int64_t rows, int groups) {
-  const int64_t most = 768 / groups < 1 ? 1 : 768 / groups;
-  const int64_t per = ((rows + most - 1) / most + 31) / 32 * 32;
+// Workgroups of eight waves per CU: two for narrow rows, where one step's latency shows next to the few
+// bytes of a stage (2^20 rows, 8 or 64 outputs: K = 32 59 us with one, 41 to 46 with two, K = 64 61 to 63
+// and 44 to 59).  At 128 and 256 the accumulators take more than a fourth of a SIMD's registers.
+template <int64_t K>
+constexpr int kLinearDwPerCu = K <= 64 ? 2 : 1;
+// Rows of one chunk: the groups of a chunk run on one XCD of 32 CUs, so 8 * (resident workgroups of an
+// XCD / groups) chunks are one full round; at least 256 rows (the partials of a chunk cost as much
+// traffic as 128 rows).
+inline int64_t linear_dw_rows_per_chunk(int64_t rows, int groups, int64_t k) {
+  const int64_t slots = 32 * (k <= 64 ? kLinearDwPerCu<64> : kLinearDwPerCu<128>);
+  const int64_t most = 8 * (slots / groups < 1 ? 1 : slots / groups);
+  const int64_t per = ((rows + most - 1) / most + 63) / 64 * 64;
   return per < 256 ? 256 : per;
 }
 
