@@ -282,6 +282,57 @@ def test_linear_outputs_against_float64(dtype, rows, k, ns, with_bias):
         assert bool((err <= bound).all()), f"N={w.shape[0]}: max excess {(err - bound).max().item():.3e}"
 
 
+@pytest.mark.parametrize("dtype,k,ns,hd,n,swap", [
+    (torch.bfloat16, 128, [128, 128, 128, 4, 128], 32, 211, True),  # 44521 rows: a part of a tile, a round in which some waves have none
+    (torch.float16, 128, [64, 2, 64], 64, 203, False),              # four chunks, one quad per tile
+    (torch.bfloat16, 128, [16, 128], 0, 257, True),                 # the widest narrow layer, first in the list
+    (torch.bfloat16, 64, [256, 256, 256, 8, 256], 32, 513, True),   # 32 chunks: the weights fill LDS
+    (torch.float16, 32, [96, 32], 32, 3, False),                    # one tile for all waves
+    (torch.bfloat16, 64, [128, 6], 0, 1, False),                    # one row
+])
+def test_layers_whose_weights_stay_in_lds(dtype, k, ns, hd, n, swap):
+    """Outputs and input gradient of several layers against float64 at the sizes where whole chunks,
+    a narrow layer and tiles of rows end, in both row orders.  One infinite output gradient of the
+    narrow layer reaches its own row only."""
+    import ctypes
+
+    from trifast_amd import _lib
+
+    rows = n * n
+    gen = torch.Generator().manual_seed(rows + k)
+    hds = [hd if hd and m % hd == 0 and m > 16 else 0 for m in ns]
+    x = torch.randn(n, n, k, generator=gen).to(DEV, dtype)
+    ws = [(torch.randn(m, k, generator=gen) * k**-0.5).to(DEV, dtype) for m in ns]
+    bs = [torch.randn(m, generator=gen).to(DEV, dtype) if i % 2 else None for i, m in enumerate(ns)]
+    dys = [torch.randn(rows, m, generator=gen).to(DEV, dtype) for m in ns]
+    hurt = rows // 2
+    for dy, m in zip(dys, ns):
+        if m <= 16 and rows > 1:
+            dy[hurt, 0] = float("inf")
+    outer = [d.view(rows, m // c, c).transpose(0, 1).contiguous() if c else d for d, m, c in zip(dys, ns, hds)]
+    ys = [torch.full_like(d, 7.0) for d in outer]
+    dx = torch.full_like(x, 7.0)
+    lib, i64, ptrs = _lib.load(), _lib.i64_array, lambda ts: (ctypes.c_void_p * len(ts))(*[None if t is None else t.data_ptr() for t in ts])
+    code, st = _lib.BF16 if dtype == torch.bfloat16 else _lib.F16, torch.cuda.current_stream().cuda_stream
+    _lib.check(lib.trifast_block_in_fwd(x.data_ptr(), 1, n, k, len(ns), ptrs(ws), ptrs(bs), ptrs(ys), i64(ns), i64(hds), swap, code, st), "block_in_fwd")
+    _lib.check(lib.trifast_block_in_bwd(dx.data_ptr(), None, None, None, 1, n, k, len(ns), ptrs(outer), ptrs(ws), i64(ns), i64(hds), swap, code, None, 0, st), "block_in_bwd")
+    eps, tiny = torch.finfo(dtype).eps, torch.finfo(dtype).smallest_normal
+    xr = (x.transpose(0, 1) if swap else x).reshape(rows, k).double()
+    for w, b, y, c in zip(ws, bs, ys, hds):
+        y = y.transpose(0, 1).reshape(rows, -1) if c else y
+        b64 = None if b is None else b.double()
+        want, size = torch.nn.functional.linear(xr, w.double(), b64), torch.nn.functional.linear(xr.abs(), w.double().abs(), None if b is None else b64.abs())
+        # fp32 accumulation of exact products, one rounding to the dtype
+        assert bool(((y.double() - want).abs() <= 0.5 * eps * want.abs() + k * 2.0**-23 * size + tiny).all()), f"outputs of the layer of {w.shape[0]}"
+    got = (dx.transpose(0, 1) if swap else dx).reshape(rows, k).double()
+    want, size = sum(d.double() @ w.double() for d, w in zip(dys, ws)), sum(d.double().abs() @ w.double().abs() for d, w in zip(dys, ws))
+    ok = (got - want).abs() <= 0.5 * eps * want.abs() + sum(ns) * 2.0**-23 * size + tiny
+    if any(m <= 16 for m in ns) and rows > 1:
+        assert not torch.isfinite(got[hurt]).any()
+        ok[hurt] = True
+    assert bool(ok.all())
+
+
 def test_projection_gradients_are_those_of_the_layers():
     """project(x, layers) against the layers themselves: outputs, input and parameter gradients
     within bf16 rounding, also when one output is unused."""

@@ -82,13 +82,13 @@ inline hipError_t raise_lds_limit(const void* kernel, int lds) {
 }
 
 // Launch with `lds` bytes of dynamic LDS.
-template <typename Kernel, typename Args>
-hipError_t launch_dyn(Kernel kernel, dim3 grid, dim3 block, int lds, hipStream_t st, const Args& a) {
+template <typename Kernel, typename... Args>
+hipError_t launch_dyn(Kernel kernel, dim3 grid, dim3 block, int lds, hipStream_t st, const Args&... a) {
   if (lds > kMaxStaticLds) {
     const hipError_t e = raise_lds_limit(reinterpret_cast<const void*>(kernel), lds);
     if (e != hipSuccess) return e;
   }
-  hipLaunchKernelGGL(kernel, grid, block, lds, st, a);
+  hipLaunchKernelGGL(kernel, grid, block, lds, st, a...);
   return hipGetLastError();
 }
 

@@ -36,7 +36,17 @@ hipError_t fwd_run(LinearFwdArgs a, hipStream_t st) {
 template <typename T, int KD>
 hipError_t fwd_rows(const LinearFwdArgs& a, hipStream_t st) {
   if (a.o) return fwd_run<T, KD, 1, true>(a, st);
-  if constexpr (KD <= 128) return two_row_tiles(a.rows) ? fwd_run<T, KD, 2, false>(a, st) : fwd_run<T, KD, 1, false>(a, st);
+  if constexpr (KD <= 128) {
+    // Five tiles of 32 rows per CU and more (K = 128, 17 chunks: 65536 rows 32 -> 28 us, 16384 14 -> 18).  Narrower
+    // rows are as fast through the other kernel until the layers are many (K = 64, 33 chunks: 2^20
+    // rows 584 -> 522 us, 65536 44 -> 46; 17 chunks: 2^20 rows 304 -> 295).
+    const ResidentPlan plan = resident_plan(a);
+    const int lds = linear_fwd_resident_lds(KD, plan.chunks);
+    const bool gains = KD == 128 ? a.rows >= kResidentWgs * 32 * 5 : plan.chunks >= 32 && a.rows >= kResidentWgs * 32 * 32;
+    if (plan.chunks && gains && a.rows < (int64_t(1) << 31) && lds <= kResidentLds)
+      return launch_dyn(linear_fwd_resident_kernel<T, KD>, dim3(kResidentWgs), dim3(64 * kResidentWaves), lds, st, a, plan);
+    return two_row_tiles(a.rows) ? fwd_run<T, KD, 2, false>(a, st) : fwd_run<T, KD, 1, false>(a, st);
+  }
   else return hipErrorInvalidConfiguration;
 }
 
@@ -71,6 +81,12 @@ hipError_t gate_bwd_k(const LinearGateBwdArgs& a, hipStream_t st) {
 
 template <typename T, int KD>
 hipError_t dx_run(const LinearDxArgs& a, hipStream_t st) {
+  // (wherever the weights fit, from the smallest sizes on: K = 128, 17 chunks, 500 rows 15.6 -> 11.0 us, 2^20
+  // 320 -> 276; K = 64 13.5 -> 8.6 and 253 -> 243; K = 32 12.6 -> 7.6 and 221 -> 225)
+  const ResidentPlan plan = resident_plan(a);
+  const int lds = linear_dx_lds(KD, plan.chunks);
+  if (plan.chunks && a.rows < (int64_t(1) << 31) && lds <= kResidentLds)
+    return launch_dyn(linear_dx_resident_kernel<T, KD>, dim3(kResidentWgs), dim3(64 * kResidentWaves), lds, st, a, plan);
   const dim3 block(256);
   if (two_row_tiles(a.rows)) hipLaunchKernelGGL((linear_dx_kernel<T, KD, 2>), dim3((unsigned)((a.rows + 255) / 256)), block, 0, st, a);
   else hipLaunchKernelGGL((linear_dx_kernel<T, KD, 1>), dim3((unsigned)((a.rows + 127) / 128)), block, 0, st, a);

@@ -232,6 +232,135 @@ __global__ __launch_bounds__(256) void linear_fwd_kernel(const LinearFwdArgs a) 
   }
 }
 
+// The resident kernels (below, and for dx): one workgroup of eight waves per CU fills LDS with every
+// layer's weights once, then each wave walks row tiles of its own without another barrier.  The layers are
+// whole 32-column chunks in rows of one pitch (chunk q's address in row 0 and pitch stand in an
+// LDS table), in multiples of four chunks, but for one layer of an even number of outputs up to 16, whose
+// columns move 4 bytes at a time.
+struct ResidentPlan {
+  int chunks, narrow;  // whole chunks; the narrow layer, or -1; chunks = 0: not for these kernels
+};
+template <typename Args>
+inline ResidentPlan resident_plan(const Args& a) {
+  ResidentPlan plan{0, -1};
+  for (int p = 0; p < a.nlayers; ++p) {
+    if (a.n[p] % 32 == 0 && a.hd[p] % 32 == 0) plan.chunks += a.n[p] / 32;
+    else if (a.n[p] <= 16 && a.n[p] % 2 == 0 && a.hd[p] == 0 && plan.narrow < 0) plan.narrow = p;
+    else return ResidentPlan{0, -1};
+  }
+  return plan.chunks % 4 ? ResidentPlan{0, -1} : plan;
+}
+constexpr int kResidentWgs = 256, kResidentWaves = 8, kResidentLds = 160 * 1024;
+struct ChunkRow {
+  uint64_t base;   // byte address of the chunk in row 0
+  uint32_t pitch;  // bytes from row to row
+  uint32_t pad;
+};
+// Tiles of 32 rows: number k of a wave.  The rounds of all workgroups interleave, so that a last
+// round that is not full occupies a part of every CU.
+TRI_DEV int resident_tile(int k, int wave) { return (kResidentWaves * k + wave) * kResidentWgs + (int)blockIdx.x; }
+
+// The same for many rows: bound by HBM, and by how long a workgroup that loads, multiplies and stores once
+// has nothing in flight.  A wave stores a tile while the next one's rows arrive.  No store of whole
+// chunks stands behind a branch, and at least four chunks follow the loads: where the paths of a loop
+// differ, the compiler's waits go by the path with the fewest operations, and would wait for the
+// stores.  (Lanes past the last row repeat it, values and all.)  rows = 147456, K = 128, four layers of
+// 128 outputs and one of 4, launched back to back: 56 -> 45 us, 4.2 TB/s.  (The gated layer stays with the
+// kernel above: 32 us with it, 33 with gated fragments here.)
+constexpr int linear_fwd_resident_lds(int kd, int chunks) { return (chunks + 1) * (32 * kd * 2 + 32 * 2 + (int)sizeof(ChunkRow)); }
+template <typename T, int KD>
+__global__ __launch_bounds__(512, 2) void linear_fwd_resident_kernel(const LinearFwdArgs a, const ResidentPlan plan) {
+  using E = Elem<T>;
+  using frag = typename E::frag;
+  using vec = typename E::vec;
+  using Tile = LdsTile<T, KD>;
+  constexpr int KS = KD / 16, CHUNK_B = 32 * Tile::ROWB;
+  extern __shared__ __attribute__((aligned(16))) unsigned char lin_smem[];
+  T* const biases = reinterpret_cast<T*>(lin_smem + (plan.chunks + 1) * CHUNK_B);
+  ChunkRow* const table = reinterpret_cast<ChunkRow*>(biases + (plan.chunks + 1) * 32);
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int cl = lane & 31, g = lane >> 5;
+  const int tiles = (int)((a.rows + 31) / 32);
+  auto row_at = [&](int k) { return min((int64_t)min(resident_tile(k, wave), tiles - 1) * 32 + cl, a.rows - 1); };
+  frag xn[KS];  // the next tile's rows
+  auto load = [&](int k) __attribute__((always_inline)) {
+    const T* x = reinterpret_cast<const T*>(a.x) + mapped_row(a.xmap, row_at(k)) * KD;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) xn[s] = *reinterpret_cast<const frag*>(x + 16 * s + 8 * g);
+  };
+  load(0);
+
+  int q0 = 0;
+  for (int p = 0; p < a.nlayers; ++p) {
+    const int N = a.n[p], hd = a.hd[p];
+    const T* bias = reinterpret_cast<const T*>(a.bias[p]);
+    for (int c0 = 0; c0 < N; c0 += 32) {
+      const int q = p == plan.narrow ? plan.chunks : q0++;
+      // (weight rows past a narrow layer's last repeat it: their outputs are not stored)
+      const T* w = reinterpret_cast<const T*>(a.w[p]);
+      Tile::template fill<32, kResidentWaves>(lin_smem + q * CHUNK_B, [&](int r) { return w + (int64_t)min(c0 + r, N - 1) * KD; }, wave, lane);
+      if (threadIdx.x < 32) biases[32 * q + threadIdx.x] = bias && c0 + (int)threadIdx.x < N ? bias[c0 + threadIdx.x] : (T)0.0f;
+      if (threadIdx.x == 0)
+        table[q] = ChunkRow{(uint64_t)(reinterpret_cast<const T*>(a.y[p]) + linear_offset(0, c0, N, hd, a.rows)), (uint32_t)((hd ? hd : N) * sizeof(T)), 0u};
+    }
+  }
+  wait_dma_known();
+  __syncthreads();
+
+  OperandOffsets<T, KD> ofs;
+  ofs.init(perm32(cl), lane);
+  const int nn = plan.narrow >= 0 ? a.n[plan.narrow] : 0;
+  for (int k = 0; resident_tile(k, wave) < tiles; ++k) {
+    frag xf[KS];
+#pragma unroll
+    for (int s = 0; s < KS; ++s) xf[s] = xn[s];
+    load(k + 1);  // (past the last tile: its rows again, which nobody uses)
+    const uint64_t orow = (uint64_t)mapped_row(a.ymap, row_at(k));
+    // this lane's 16 columns of chunk q: 16 half + 8 g + 0..7
+    auto product = [&](int q, vec (&v)[2]) __attribute__((always_inline)) {
+      f32x16 acc;
+#pragma unroll
+      for (int half = 0; half < 2; ++half) {
+        const vec bv = *reinterpret_cast<const vec*>(biases + 32 * q + 16 * half + 8 * g);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[8 * half + e] = (float)bv[e];
+      }
+#pragma unroll
+      for (int s = 0; s < KS; ++s) acc = E::mfma(ofs.natural(lin_smem + q * CHUNK_B, s), xf[s], acc);
+#pragma unroll
+      for (int half = 0; half < 2; ++half)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[half][e] = (T)acc[8 * half + e];
+    };
+    int q = 0;
+    do {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        vec v[2];
+        product(q + u, v);
+        const ChunkRow at = table[q + u];
+        auto* dst = reinterpret_cast<TRI_G1 vec*>(at.base + orow * at.pitch + 16 * g);
+        dst[0] = v[0];
+        dst[2] = v[1];
+      }
+      q += 4;
+    } while (q < plan.chunks);
+    if (nn) {
+      typedef uint32_t u32x4s __attribute__((ext_vector_type(4)));
+      vec v[2];
+      product(plan.chunks, v);
+      const ChunkRow at = table[plan.chunks];
+      auto* dst = reinterpret_cast<TRI_G1 uint32_t*>(at.base + orow * at.pitch + 16 * g);
+      const u32x4s w = __builtin_bit_cast(u32x4s, v[0]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (8 * g + 2 * e < nn) dst[e] = w[e];
+    }
+  }
+}
+
 // ---------------------------------------------------------------------------------------
 // Backward of the gated output layer up to the gate's inputs:
 //   dy = dout W (dout [rows, K], W [K, C]),  do = dy * s,  dg = dy * o * s (1 - s),  s = sigmoid(g)
@@ -331,7 +460,8 @@ __global__ __launch_bounds__(256) void linear_gate_bwd_kernel(const LinearGateBw
 // through memory nine times for five layers).  A workgroup owns 128 * RT rows and all KD
 // columns, accumulated in fp32 over the layers.  The layers' contraction columns pass in chunks
 // of 32, two chunks ahead in registers: the rows' fragments, and the same 32 rows of W_p, which go
-// to LDS one step before their use (32-column tiles, read back transposed).
+// to LDS one step before their use (32-column tiles, read back transposed).  For layers whose weights do
+// not fit LDS together, or whose columns are no whole chunks; the others take linear_dx_resident_kernel.
 // ---------------------------------------------------------------------------------------
 template <typename T, int KD, int RT>
 __global__ __launch_bounds__(256) void linear_dx_kernel(const LinearDxArgs a) {
@@ -384,9 +514,12 @@ __global__ __launch_bounds__(256) void linear_dx_kernel(const LinearDxArgs a) {
           if ((N % 8) == 0) {
             v = *reinterpret_cast<const vec*>(src);
           } else {
+            // (all loads, then the columns past the layer's last cleared: a load behind a condition of its own
+            // is waited for before the next)
 #pragma unroll
-            for (int e = 0; e < 8; ++e)
-              if (lc + in + e < N) v[e] = src[e];
+            for (int e = 0; e < 8; ++e) v[e] = src[lc + in + e < N ? e : 0];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] = lc + in + e < N ? v[e] : (T)0.0f;
           }
         }
         f[t][s] = v;
@@ -447,6 +580,125 @@ __global__ __launch_bounds__(256) void linear_dx_kernel(const LinearDxArgs a) {
         for (int e = 0; e < 8; ++e) v[e] = (T)acc[t][kb][8 * half + e];
         *reinterpret_cast<vec*>(dst + 32 * kb + 16 * half + 8 * g) = v;
       }
+  }
+}
+
+// The same with every layer's weights resident in LDS (see ResidentPlan): the row fragments of four
+// chunks at a time go straight to registers, the next four in flight under the products.  No load
+// stands behind a branch that some rounds do not take, but for the narrow layer's (see
+// linear_fwd_resident_kernel).  Bound by HBM.  rows = 147456, K = 128, four layers of 128 outputs and one
+// of 4, launched back to back: 56 -> 38 us, 5.0 TB/s (in the kernel above each of a narrow layer's columns was a
+// load of its own that was waited for, and 577 workgroups shared 512 places).
+constexpr int linear_dx_lds(int kd, int chunks) { return (chunks + 1) * (32 * kd * 2 + (int)sizeof(ChunkRow)); }
+
+template <typename T, int KD>
+__global__ __launch_bounds__(512, 2) void linear_dx_resident_kernel(const LinearDxArgs a, const ResidentPlan plan) {
+  using E = Elem<T>;
+  using frag = typename E::frag;
+  using vec = typename E::vec;
+  using Tile = LdsTile<T, 32>;
+  typedef uint32_t u32x4s __attribute__((ext_vector_type(4)));
+  constexpr int KB = KD / 32, U = 4;
+  constexpr int BLOCK_B = 32 * Tile::ROWB, CHUNK_B = KB * BLOCK_B;
+  extern __shared__ __attribute__((aligned(16))) unsigned char lin_smem[];
+  ChunkRow* const table = reinterpret_cast<ChunkRow*>(lin_smem + (plan.chunks + 1) * CHUNK_B);
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int cl = lane & 31, g = lane >> 5;
+  int q0 = 0;
+  for (int p = 0; p < a.nlayers; ++p) {
+    const int N = a.n[p], hd = a.hd[p];
+    for (int c0 = 0; c0 < N; c0 += 32) {
+      const int q = p == plan.narrow ? plan.chunks : q0++;
+      // (weight rows past a narrow layer's last repeat it: the row fragments are zero there)
+      const T* w = reinterpret_cast<const T*>(a.w[p]);
+      for (int gi = wave; gi < 2 * KB; gi += 8) {
+        const int r = 16 * (gi & 1) + lane / 4, c = (lane % 4) ^ Tile::swz(r);
+        const T* src = w + (int64_t)min(c0 + r, N - 1) * KD + 32 * (gi >> 1) + 8 * c;
+        __builtin_amdgcn_global_load_lds((const TRI_G1 void*)src, (TRI_L3 void*)(lin_smem + q * CHUNK_B + gi * 1024), 16, 0, 0);
+      }
+      if (threadIdx.x == 0)
+        table[q] = ChunkRow{(uint64_t)(reinterpret_cast<const T*>(a.dy[p]) + linear_offset(0, c0, N, hd, a.rows)), (uint32_t)((hd ? hd : N) * sizeof(T)), 0u};
+    }
+  }
+  wait_dma_known();
+  __syncthreads();
+
+  const int tiles = (int)((a.rows + 31) / 32), quads = plan.chunks / U;
+  auto row_at = [&](int k) { return min((int64_t)min(resident_tile(k, wave), tiles - 1) * 32 + cl, a.rows - 1); };
+  const int nn = plan.narrow >= 0 ? a.n[plan.narrow] : 0;
+  vec yf[2][U][2];
+  u32x4s nf[2];
+  // the quad the next load takes (past the last tile: its rows again, which nobody uses)
+  int lk = 0, lq = 0;
+  auto load = [&](vec (&f)[U][2], u32x4s& narrow) __attribute__((always_inline)) {
+    const uint64_t row = (uint64_t)row_at(lk);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const ChunkRow at = table[U * lq + u];
+      const auto* src = reinterpret_cast<TRI_G1 const vec*>(at.base + (row & 0xffffffffu) * at.pitch + 16 * g);
+      f[u][0] = src[0];
+      f[u][1] = src[2];
+    }
+    if (++lq < quads) return;
+    lq = 0;
+    ++lk;
+    if (nn) {
+      const ChunkRow at = table[plan.chunks];
+      const auto* src = reinterpret_cast<TRI_G1 const uint32_t*>(at.base + (row & 0xffffffffu) * at.pitch);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) narrow[e] = src[8 * g + 2 * e < nn ? 4 * g + e : 0];
+    }
+  };
+  load(yf[0], nf[0]);
+
+  f32x16 acc[KB];
+#pragma unroll
+  for (int kb = 0; kb < KB; ++kb) acc[kb] = zero16();
+  int k = 0, q = 0;  // the quad the next products take
+  T* dx = reinterpret_cast<T*>(a.dx);
+  auto step = [&](auto which) __attribute__((always_inline)) {
+    constexpr int set = decltype(which)::value;
+    load(yf[set ^ 1], nf[set ^ 1]);
+    const unsigned char* tile = lin_smem + U * q * CHUNK_B;
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int s = 0; s < 2; ++s)
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb)
+          acc[kb] = E::mfma(tr_perm_operand<T>(tile + u * CHUNK_B + kb * BLOCK_B, 16 * s + 8 * g, lane), __builtin_bit_cast(frag, yf[set][u][s]), acc[kb]);
+    if (++q < quads) return;
+    if (nn) {
+      u32x4s v;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = 8 * g + 2 * e < nn ? nf[set][e] : 0u;
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb)
+        acc[kb] = E::mfma(tr_perm_operand<T>(lin_smem + plan.chunks * CHUNK_B + kb * BLOCK_B, 8 * g, lane), __builtin_bit_cast(frag, v), acc[kb]);
+    }
+    const int64_t row = (int64_t)resident_tile(k, wave) * 32 + cl;
+    if (resident_tile(k, wave) < tiles && row < a.rows) {
+      T* dst = dx + mapped_row(a.map, row) * KD;
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+          vec v;
+#pragma unroll
+          for (int e = 0; e < 8; ++e) v[e] = (T)acc[kb][8 * half + e];
+          *reinterpret_cast<vec*>(dst + 32 * kb + 16 * half + 8 * g) = v;
+        }
+    }
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) acc[kb] = zero16();
+    q = 0;
+    ++k;
+  };
+  while (resident_tile(k, wave) < tiles) {
+    step(std::integral_constant<int, 0>{});
+    step(std::integral_constant<int, 1>{});
   }
 }
 
