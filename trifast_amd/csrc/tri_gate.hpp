@@ -34,9 +34,20 @@ struct GateVec {
 
 // sigmoid(x) and its derivative s (1 - s) from e = exp(-|x|) <= 1: no overflow, and no
 // cancellation in 1 - s for large |x|.
+// 1 / (1 + e), 1 <= 1 + e <= 2: for 16-bit results the reciprocal with one Newton step in place of the
+// division's eleven instructions (they were half of the gated layer's).  Its error is at most
+// 2^-24 (1 + 2^-22) of the result, the division's 2^-24; those of e are larger, and the result is rounded to
+// 16 bits.
+template <typename T>
 TRI_DEV void gate_sigmoid(float x, float& s, float& ds) {
   const float e = __expf(-fabsf(x));
-  const float r = 1.0f / (1.0f + e);
+  float r;
+  if constexpr (sizeof(T) == 2) {
+    const float d = 1.0f + e, r0 = __builtin_amdgcn_rcpf(d);
+    r = __builtin_fmaf(r0, __builtin_fmaf(-d, r0, 1.0f), r0);
+  } else {
+    r = 1.0f / (1.0f + e);
+  }
   s = x >= 0.0f ? r : e * r;
   ds = e * r * r;
 }
@@ -62,7 +73,7 @@ __global__ __launch_bounds__(256) void gate_kernel(const GateArgs a) {
 #pragma unroll
       for (int e = 0; e < VEC; ++e) {
         float s, ds;
-        gate_sigmoid((float)gv[e], s, ds);
+        gate_sigmoid<T>((float)gv[e], s, ds);
         yv[e] = (T)((float)ov[e] * s);
       }
       *reinterpret_cast<vec*>(reinterpret_cast<T*>(a.y) + inter) = yv;
@@ -72,7 +83,7 @@ __global__ __launch_bounds__(256) void gate_kernel(const GateArgs a) {
 #pragma unroll
       for (int e = 0; e < VEC; ++e) {
         float s, ds;
-        gate_sigmoid((float)gv[e], s, ds);
+        gate_sigmoid<T>((float)gv[e], s, ds);
         const float d = (float)dyv[e];
         dov[e] = (T)(d * s);
         dgv[e] = (T)(d * (float)ov[e] * ds);

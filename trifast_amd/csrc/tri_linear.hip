@@ -5,9 +5,12 @@ namespace tri {
 namespace {
 
 // How the outputs of a row block are split over workgroups: `most` 32-column chunks per workgroup
-// at most (their weights share LDS), fewer while the launch has less than four workgroups per CU.
-void split_chunks(int64_t row_blocks, int total, int most, int& chunks, int& groups) {
-  int64_t per = row_blocks * total / 1024;
+// at most (their weights share LDS), fewer while the launch has less than `wgs` workgroups: four per
+// CU for the projections; one where the rows are gated first, which every workgroup of a row block
+// does for itself (K = 128, 128 outputs, 25600 rows: 16.7 us with four, 11.4 with one; the gate's
+// backward 15.2 and 11.3; the projections of 10000 rows 9.1 to 11.0 and 11.9).
+void split_chunks(int64_t row_blocks, int total, int most, int wgs, int& chunks, int& groups) {
+  int64_t per = row_blocks * total / wgs;
   per = per < 1 ? 1 : (per > most ? most : per);
   groups = (int)((total + per - 1) / per);
   chunks = (total + groups - 1) / groups;
@@ -29,7 +32,7 @@ hipError_t fwd_run(LinearFwdArgs a, hipStream_t st) {
   for (int p = 0; p < a.nlayers; ++p) a.total_chunks += (a.n[p] + 31) / 32;
   constexpr int chunk_bytes = 32 * KD * (int)sizeof(T);
   const int64_t blocks = (a.rows + 128 * RT - 1) / (128 * RT);
-  split_chunks(blocks, a.total_chunks, 40 * 1024 / chunk_bytes, a.chunks, a.groups);
+  split_chunks(blocks, a.total_chunks, 40 * 1024 / chunk_bytes, GATED ? 256 : 1024, a.chunks, a.groups);
   return launch_dyn(linear_fwd_kernel<T, KD, RT, GATED>, row_grid(a.rows, 128 * RT, a.groups), dim3(256), a.chunks * chunk_bytes, st, a);
 }
 
@@ -65,7 +68,7 @@ template <typename T, int KD>
 hipError_t gate_bwd_run(LinearGateBwdArgs a, hipStream_t st) {
   constexpr int chunk_bytes = KD * 32 * (int)sizeof(T), kMost = 4;
   const int64_t blocks = (a.rows + 127) / 128;
-  split_chunks(blocks, a.C / 32, kMost, a.chunks, a.groups);
+  split_chunks(blocks, a.C / 32, kMost, 256, a.chunks, a.groups);
   return launch_dyn(linear_gate_bwd_kernel<T, KD, kMost>, row_grid(a.rows, 128, a.groups), dim3(256), a.chunks * chunk_bytes, st, a);
 }
 
