@@ -2,6 +2,7 @@
 // argument checking, workspace carving, the mask pre-pass and the fixed launch
 // order of the backward kernels.  Nothing here allocates device memory.
 #include <hip/hip_runtime.h>
+#include <algorithm>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -779,11 +780,12 @@ static void dw_layer(tri::LinearDwArgs& a, const void* dy, int64_t n, int64_t he
   if (db) a.total += n;
 }
 // how a launch whose layers are complete is split
-static void dw_split(tri::LinearDwArgs& a) {
+static void dw_split(tri::LinearDwArgs& a, int64_t most_chunks) {
   const tri::LinearDwGroups s = tri::linear_dw_groups(a.n, a.nlayers, a.K);
   a.groups = s.groups;
   a.rider = s.rider;
-  a.rows_per_chunk = tri::linear_dw_rows_per_chunk(a.rows, a.groups, a.K);
+  const int64_t fewest_rows = (a.rows + most_chunks - 1) / most_chunks;
+  a.rows_per_chunk = std::max(tri::linear_dw_rows_per_chunk(a.rows, a.groups, a.K), (fewest_rows + 63) / 64 * 64);
   a.chunks = (int)((a.rows + a.rows_per_chunk - 1) / a.rows_per_chunk);
 }
 static int64_t dw_chunks(int64_t rows, int64_t k, int nlayers, const int64_t* n) {
@@ -793,8 +795,7 @@ static int64_t dw_chunks(int64_t rows, int64_t k, int nlayers, const int64_t* n)
 
 int64_t trifast_linear_dw_workspace_bytes(int64_t rows, int64_t k, int64_t n) {
   if (rows < 1 || k < 1 || n < 1) return fail(TRIFAST_EINVAL, "sizes must be positive");
-  const int64_t chunks = dw_chunks(rows, k, 1, &n);
-  return align256(chunks * n * k * 4) + align256(chunks * n * 4);
+  return align256(tri::linear_dw_chunks(rows) * n * k * 4) + align256(tri::linear_dw_chunks(rows) * n * 4);
 }
 
 int trifast_linear_dw(void* dw, void* db, const void* dy, const void* x, int64_t rows, int64_t k, int64_t n, int64_t head_dim, int dtype,
@@ -813,7 +814,7 @@ int trifast_linear_dw(void* dw, void* db, const void* dy, const void* x, int64_t
   a.x = x; a.part = static_cast<float*>(workspace);
   a.rows = rows; a.K = (int)k;
   dw_layer(a, dy, n, head_dim, dw, db);
-  dw_split(a);
+  dw_split(a, tri::linear_dw_chunks(rows));
   const hipError_t e = tri::linear_dw_launch(a, dtype, static_cast<hipStream_t>(stream));
   if (e != hipSuccess) return hip_fail(e, "linear_dw launch");
   return 0;
@@ -895,7 +896,7 @@ int64_t trifast_block_dw_workspace_bytes(int64_t rows, int64_t k, int nlayers, c
 
 // the weight-gradient launch of layers whose arguments are complete but for the split of the rows
 static int block_dw(tri::LinearDwArgs& a, int dtype, void* workspace, int64_t workspace_bytes, void* stream) {
-  dw_split(a);
+  dw_split(a, a.rows);
   if (!workspace || (reinterpret_cast<uintptr_t>(workspace) & 255) != 0 || workspace_bytes < (int64_t)a.chunks * a.total * 4)
     return fail(TRIFAST_EWORKSPACE, "block: workspace missing, misaligned or smaller than trifast_block_dw_workspace_bytes");
   a.part = static_cast<float*>(workspace);

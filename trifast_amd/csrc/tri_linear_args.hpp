@@ -129,6 +129,12 @@ inline int64_t linear_dw_rows_per_chunk(int64_t rows, int groups, int64_t k) {
   return per < 256 ? 256 : per;
 }
 
+// One layer by itself is given room for the partials of chunks of at least 1024 rows, at most 768 of them.
+inline int64_t linear_dw_chunks(int64_t rows) {
+  const int64_t even = ((rows + 767) / 768 + 31) / 32 * 32, per = even < 1024 ? 1024 : even;
+  return (rows + per - 1) / per;
+}
+
 inline bool linear_fwd_k_ok(int64_t k) { return k == 32 || k == 64 || k == 128; }
 inline bool linear_gated_k_ok(int64_t k) { return k == 32 || k == 64 || k == 128 || k == 256; }
 // (the accumulators of 64 rows x K columns per wave stay in registers: K up to 128)
