@@ -45,7 +45,7 @@ def main():
 
     q, k, v, bias, mask, do = bench.make_workload(args.workload, "cuda")
     if mask.any():
-        sys.exit("the pipelined walk covers plain rows: pick a workload without a mask")
+        sys.exit("the probe times the walk of rows without masked keys: pick a workload without a mask")
     b, h, n, _, d = q.shape
     code = tt._DTYPE_CODE[q.dtype]
     with torch.no_grad():

@@ -15,13 +15,13 @@
 // the bias tiles (register-resident, fp32, raw-score domain) are the accumulator
 // init of every row's score MFMA; -delta (per query) enters through one extra MFMA
 // (see rank1_operand); -lse is one number per lane and is the addend of the fma that
-// scales the score for exp2.  That leaves two fmas and one exp2 per element.  In a tile
-// with masked keys -lse moves to an extra MFMA that it shares with the key mask (see
+// scales the score for exp2.  That leaves two fmas and one exp2 per element.  In the general
+// loop a tile with masked keys takes -lse in an extra MFMA that it shares with the key mask (see
 // OffsetMask): masked keys get a large negative score there.
 //
-// Waves that own two key tiles walk the plain rows at the start of a chunk as a hand-made
-// software pipeline (matrix instructions of one tile between the vector instructions of the
-// tile before it, operands a row ahead); see kPipelined below.
+// Waves that own two key tiles of rows of up to 128 bytes walk the rows, masked or not, as a
+// hand-made software pipeline (matrix instructions of one tile between the vector instructions of
+// the tile before it, operands a row ahead); see kPipelined below.
 //
 // All workgroups of one (batch*head, chunk) read the same rows at about the same
 // time; the block index is remapped so that they run on one XCD and share its L2.

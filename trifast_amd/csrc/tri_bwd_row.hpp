@@ -2,7 +2,8 @@
 // scores and of dP (the dq kernel and the dk/dv kernel each recompute both).
 //
 // Work unit: (batch*head, pair row i), one workgroup of four waves, one wave per
-// SIMD with the whole register file.  The keys of the row are dealt to the waves
+// SIMD with the whole register file (rows of up to 64 bytes and 512 keys: two per SIMD, of two
+// workgroups or of one of eight waves, see bwd_row_two_waves).  The keys of the row are dealt to the waves
 // in tiles of 32 (wave w owns key tiles w, w+4, ...; at most KT of them): their
 // dk, dv accumulators stay in registers for the whole row, their V rows too (B
 // operands; in a private piece of LDS where the registers do not hold them all), and
