@@ -282,6 +282,45 @@ def test_linear_outputs_against_float64(dtype, rows, k, ns, with_bias):
         assert bool((err <= bound).all()), f"N={w.shape[0]}: max excess {(err - bound).max().item():.3e}"
 
 
+@pytest.mark.parametrize("dtype,c,h,d,n,swap", [
+    (torch.bfloat16, 128, 4, 32, 16, False),  # one chunk of whole stages
+    (torch.float16, 64, 2, 32, 17, True),     # 33 rows in the second chunk, one in the second half of its stage
+    (torch.bfloat16, 32, 1, 64, 33, True),    # one block of outputs: most waves load and gate only
+    (torch.float16, 128, 8, 16, 65, False),   # heads narrower than a block, 65 rows in the last chunk
+    (torch.bfloat16, 128, 1, 64, 1, False),   # one row
+])
+def test_gate_backward_with_the_weight_gradient(dtype, c, h, d, n, swap):
+    """The output layer's gradients in one call (one kernel: gate backward and weight gradient) against
+    the same call asked for do and dg, and for dW and db, alone."""
+    from trifast_amd import _lib
+
+    rows, hd = n * n, h * d
+    gen = torch.Generator().manual_seed(rows + c)
+    o, g, dout, w = (torch.randn(*shape, generator=gen).to(DEV, dtype) for shape in ((h, rows, d), (rows, hd), (rows, c), (c, hd)))
+    lib = _lib.load()
+    ws = torch.empty(lib.trifast_block_dw_workspace_bytes(rows, hd, 1, _lib.i64_array([c])), dtype=torch.uint8, device=DEV)
+
+    def grads(gate, weight):
+        out = [torch.full_like(o, 7.0), torch.full_like(g, 7.0), torch.full_like(w, 7.0), torch.full((c,), 7.0, device=DEV, dtype=dtype)]
+        p = [t.data_ptr() if want else None for t, want in zip(out, (gate, gate, weight, weight))]
+        _lib.check(lib.trifast_block_out_bwd(*p, dout.data_ptr(), o.data_ptr(), g.data_ptr(), w.data_ptr(), 1, h, n, d, c, swap,
+                                             _lib.BF16 if dtype == torch.bfloat16 else _lib.F16, ws.data_ptr(), ws.numel(),
+                                             torch.cuda.current_stream().cuda_stream), "trifast_block_out_bwd")
+        return out
+
+    both, gate, weight = grads(True, True), grads(True, False), grads(False, True)
+    assert torch.equal(both[0], gate[0]) and torch.equal(both[1], gate[1])  # the same products in the same order
+    y = (o.float() * torch.sigmoid(g.view(rows, h, d).transpose(0, 1).float())).to(dtype).transpose(0, 1).reshape(rows, hd)
+    d64 = (dout.view(n, n, c).transpose(0, 1).reshape(rows, c) if swap else dout).double()
+    eps, tiny = torch.finfo(dtype).eps, torch.finfo(dtype).smallest_normal
+    for got, alone, right in ((both[2], weight[2], y.double()), (both[3], weight[3], torch.ones(rows, 1, device=DEV, dtype=torch.float64))):
+        want, size = (d64.t() @ right).view(got.shape), (d64.abs().t() @ right.abs()).view(got.shape)
+        # fp32 accumulation in a fixed order, one rounding; a gated value may round to either neighbour (half an ulp of it)
+        bound = 0.5 * eps * want.abs() + rows**0.5 * 2.0**-22 * size + 0.02 * eps * size + tiny
+        for x in (got, alone):
+            assert bool(((x.double() - want).abs() <= bound).all())
+
+
 @pytest.mark.parametrize("dtype,k,ns,hd,n,swap", [
     (torch.bfloat16, 128, [128, 128, 128, 4, 128], 32, 211, True),  # 44521 rows: a part of a tile, a round in which some waves have none
     (torch.float16, 128, [64, 2, 64], 64, 203, False),              # four chunks, one quad per tile

@@ -785,7 +785,8 @@ static void dw_split(tri::LinearDwArgs& a, int64_t most_chunks) {
   a.groups = s.groups;
   a.rider = s.rider;
   const int64_t fewest_rows = (a.rows + most_chunks - 1) / most_chunks;
-  a.rows_per_chunk = std::max(tri::linear_dw_rows_per_chunk(a.rows, a.groups, a.K), (fewest_rows + 63) / 64 * 64);
+  const int64_t k = a.gw ? std::max(a.K, 128) : a.K;  // (with the gate's backward one workgroup is resident per CU)
+  a.rows_per_chunk = std::max(tri::linear_dw_rows_per_chunk(a.rows, a.groups, k), (fewest_rows + 63) / 64 * 64);
   a.chunks = (int)((a.rows + a.rows_per_chunk - 1) / a.rows_per_chunk);
 }
 static int64_t dw_chunks(int64_t rows, int64_t k, int nlayers, const int64_t* n) {
@@ -970,8 +971,9 @@ int trifast_block_out_bwd(void* dout_o, void* dg, void* dw, void* db, const void
   if (int rc = check_block_out(o, g, w, b, h, n, d, c, dtype)) return rc;
   if (!dout || (reinterpret_cast<uintptr_t>(dout) & 15) != 0) return fail(TRIFAST_EALIGN, "block_out_bwd: dout is null or not 16-byte aligned");
   const int lgd = __builtin_ctzll((unsigned long long)d);
-  if (dout_o) {
-    if (!dg || ((reinterpret_cast<uintptr_t>(dout_o) | reinterpret_cast<uintptr_t>(dg)) & 15) != 0) return fail(TRIFAST_EALIGN, "block_out_bwd: do and dg must be 16-byte aligned");
+  if (dout_o && (!dg || ((reinterpret_cast<uintptr_t>(dout_o) | reinterpret_cast<uintptr_t>(dg)) & 15) != 0)) return fail(TRIFAST_EALIGN, "block_out_bwd: do and dg must be 16-byte aligned");
+  const bool fused = dout_o && dw && tri::linear_dw_with_gate_bwd(h * d);
+  if (dout_o && !fused) {
     tri::LinearGateBwdArgs a{};
     a.dout = dout; a.w = w; a.o = o; a.g = g; a.dox = dout_o; a.dg = dg;
     a.rows = b * n * n; a.plane = tri::make_divisor((uint32_t)(n * n)); a.K = (int)c; a.C = (int)(h * d); a.H = (int)h; a.D = (int)d; a.lgD = lgd;
@@ -983,6 +985,7 @@ int trifast_block_out_bwd(void* dout_o, void* dg, void* dw, void* db, const void
   tri::LinearDwArgs a{};
   a.x = o; a.g = g; a.rows = b * n * n; a.K = (int)(h * d); a.ymap = tri::row_map(swap ? (uint32_t)n : 0);
   a.plane = tri::make_divisor((uint32_t)(n * n)); a.H = (int)h; a.D = (int)d; a.lgD = lgd;
+  if (fused) { a.gw = w; a.dox = dout_o; a.dg = dg; }
   dw_layer(a, dout, c, 0, dw, db);
   return block_dw(a, dtype, workspace, workspace_bytes, stream);
 }

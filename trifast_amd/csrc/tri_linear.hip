@@ -109,8 +109,15 @@ hipError_t dx_k(const LinearDxArgs& a, hipStream_t st) {
 template <typename T, int KD>
 hipError_t dw_run(const LinearDwArgs& a, hipStream_t st) {
   const dim3 grid((unsigned)((a.chunks + 7) / 8 * 8 * a.groups));
-  const hipError_t e = a.g ? launch_dyn(linear_dw_kernel<T, KD, true>, grid, dim3(512), LinearDwShape<T, KD, true>::LDS, st, a)
-                           : launch_dyn(linear_dw_kernel<T, KD, false>, grid, dim3(512), LinearDwShape<T, KD, false>::LDS, st, a);
+  hipError_t e;
+  if (!a.g) {
+    e = launch_dyn(linear_dw_kernel<T, KD, kDwPlain>, grid, dim3(512), LinearDwShape<T, KD, kDwPlain>::LDS, st, a);
+  } else if (!a.gw) {
+    e = launch_dyn(linear_dw_kernel<T, KD, kDwGated>, grid, dim3(512), LinearDwShape<T, KD, kDwGated>::LDS, st, a);
+  } else {
+    if constexpr (KD == 64 || KD == 128) e = launch_dyn(linear_dw_kernel<T, KD, kDwGateBwd>, grid, dim3(512), LinearDwShape<T, KD, kDwGateBwd>::LDS, st, a);
+    else return hipErrorInvalidConfiguration;
+  }
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL((linear_dw_reduce_kernel<T>), dim3((unsigned)((a.total + 31) / 32)), dim3(256), 0, st, a);
   return hipGetLastError();

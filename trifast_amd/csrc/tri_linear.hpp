@@ -3,7 +3,7 @@
 // with the output gate folded into the layer that reads it:
 //   linear_fwd        y_p = x W_p^T + bias_p for several layers in one pass
 //   gated out layer   out = (o * sigmoid(g)) W^T + bias             (linear_fwd with a gated source)
-//   gate backward     do, dg from dout W                            (linear_gate_bwd)
+//   gate backward     do, dg from dout W                            (linear_gate_bwd, or with dW: linear_dw)
 //   linear_dx         dx = sum_p dy_p W_p
 //   linear_dw         dW_p = dy_p^T x, db_p = column sums of dy_p, several layers in one pass
 // All of them are bound by HBM: a row is a few hundred bytes per tensor and 10^5 multiply-adds.
@@ -743,18 +743,24 @@ __global__ __launch_bounds__(512, 2) void linear_dx_resident_kernel(const Linear
 // outputs 215 -> 160 us, K = 128 131 -> 107, 8 outputs 66 -> 69 (an odd number of outputs, loaded one at a
 // time: 102 -> 140 at K = 128, faster below 10^5 rows and at the other K).
 //
-// GATED: x is o * sigmoid(g) (see linear_fwd); o and g land in LDS and each wave gates the pieces
-// it loaded before the stage is handed over.
+// kDwGated: x is o * sigmoid(g) (see linear_fwd); o and g land in LDS and each wave gates the pieces
+// it loaded before the stage is handed over.  kDwGateBwd: the gate's backward (linear_gate_bwd) from the
+// same stages, which hold all it reads: dy = dout W for the rows of the stage, W resident, do and dg
+// stored, and the gated rows written over o for the weight gradient.  rows = 147456, K = 128, 128
+// outputs, with the sum of the partials: 44 us, 65 as two launches.
 // ---------------------------------------------------------------------------------------
-template <typename T, int KD, bool GATED>
+constexpr int kDwPlain = 0, kDwGated = 1, kDwGateBwd = 2;
+template <typename T, int KD, int MODE>
 struct LinearDwShape {
+  static constexpr bool GATED = MODE != kDwPlain, FUSED = MODE == kDwGateBwd;
+  static constexpr int PER_CU = FUSED ? 1 : kLinearDwPerCu<KD>;
   static constexpr int XB = 32 * KD * (int)sizeof(T), YB = 32 * 32 * (int)sizeof(T);  // x tile of a half, dy tile of a wave
   static constexpr int XP = XB / 1024;           // 1 KiB loads of an x tile, shared by the four waves of the half
   static constexpr int XN = (XP + 3) / 4;        // ... per wave (a wave without one loads into `DUMP`)
   static constexpr int OFF_G = 2 * XB, OFF_Y = (GATED ? 4 : 2) * XB;
   static constexpr bool RIDER = !GATED && KD <= 128;  // (the gated layer comes alone)
   static constexpr int RB = 32 * kLinearDwRider * (int)sizeof(T);  // dy tile of a riding layer, of a half
-  static constexpr int LDS = 160 * 1024 / kLinearDwPerCu<KD>, DUMP = XP % 4 ? LDS - 1024 : LDS;
+  static constexpr int LDS = 160 * 1024 / PER_CU, DUMP = XP % 4 ? LDS - 1024 : LDS;
   // loads per wave and stage: of x, of dy (16 or, where its rows keep only 4-byte alignment, 4 bytes per lane)
   static constexpr int X_LOADS = (GATED ? 2 : 1) * XN, Y_LOADS = 2, Y4_LOADS = 8;
   static constexpr int MOST = 6;  // stages of a ring
@@ -790,12 +796,13 @@ TRI_DEV typename Elem<T>::frag tr_pair(const unsigned char* p_lo, const unsigned
   return f;
 }
 
-template <typename T, int KD, bool GATED>
-__global__ __launch_bounds__(512, 2 * kLinearDwPerCu<KD>) void linear_dw_kernel(const LinearDwArgs a) {
+template <typename T, int KD, int MODE>
+__global__ __launch_bounds__(512, (2 * LinearDwShape<T, KD, MODE>::PER_CU)) void linear_dw_kernel(const LinearDwArgs a) {
   using E = Elem<T>;
   using frag = typename E::frag;
   using vec = typename E::vec;
-  using S = LinearDwShape<T, KD, GATED>;
+  using S = LinearDwShape<T, KD, MODE>;
+  constexpr bool GATED = S::GATED, FUSED = S::FUSED;
   using XTile = LdsTile<T, KD>;
   using YTile = LdsTile<T, 32>;
   using RTile = LdsTile<T, kLinearDwRider>;
@@ -864,7 +871,9 @@ __global__ __launch_bounds__(512, 2 * kLinearDwPerCu<KD>) void linear_dw_kernel(
   const int off_y = S::OFF_Y + (half * blocks_here + wc) * S::YB;
   const int off_r = S::OFF_Y + 2 * blocks_here * S::YB + half * S::RB;
   const int stage = S::OFF_Y + 2 * blocks_here * S::YB + (rides ? 2 * S::RB : 0);
-  const int depth = min(S::DUMP / stage, S::MOST), end = depth * stage;
+  // (the gate's backward: W, [N][32] tiles of the K blocks, in front of the ring)
+  const int ring = FUSED ? N * KD * (int)sizeof(T) : 0;
+  const int depth = min((S::DUMP - ring) / stage, S::MOST), end = ring + depth * stage;
   const int in_flight = (depth - 2) * (S::X_LOADS + (!live ? 0 : even ? S::Y4_LOADS : S::Y_LOADS) + (rides ? 1 : 0));
   const uint32_t lds0 = (uint32_t)(uintptr_t)(TRI_L3 const unsigned char*)lin_smem;
   auto uni = [](uint32_t x) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)x); };
@@ -916,7 +925,7 @@ __global__ __launch_bounds__(512, 2 * kLinearDwPerCu<KD>) void linear_dw_kernel(
   // what this wave loaded of stage s has landed: gate it, and clear rows past the end
   auto finish = [&](int s, uint32_t boff) __attribute__((always_inline)) {
     unsigned char* xbuf = lin_smem + boff + half * S::XB + lane * 16;
-    if constexpr (GATED) {
+    if constexpr (GATED && !FUSED) {
 #pragma unroll
       for (int x = 0; x < XN; ++x) {
         if (!own[x]) continue;
@@ -929,7 +938,10 @@ __global__ __launch_bounds__(512, 2 * kLinearDwPerCu<KD>) void linear_dw_kernel(
     const vec none = {};
 #pragma unroll
     for (int x = 0; x < XN; ++x)
-      if (own[x] && first + xr[x] >= r_end) *reinterpret_cast<vec*>(xbuf + (4 * x + wc) * 1024) = none;
+      if (own[x] && first + xr[x] >= r_end) {
+        *reinterpret_cast<vec*>(xbuf + (4 * x + wc) * 1024) = none;
+        if constexpr (FUSED) *reinterpret_cast<vec*>(xbuf + S::OFF_G + (4 * x + wc) * 1024) = none;
+      }
     if (live) {
 #pragma unroll
       for (int t = 0; t < 2; ++t)
@@ -951,7 +963,7 @@ __global__ __launch_bounds__(512, 2 * kLinearDwPerCu<KD>) void linear_dw_kernel(
   OperandOffsets<T, KD> xo;
   OperandOffsets<T, 32> yo;
   xo.init(0, lane);
-  yo.init(0, lane);
+  yo.init(lane & 31, lane);
   // a riding layer: its own tile, and the K blocks of this wave: wc, wc + 4, .. (block KB: its column sums)
   const int r16lo = RTile::off(8 * g + ((lane & 15) >> 2), 8 * (lane & 3)), r16hi = RTile::off(8 * g + 4 + ((lane & 15) >> 2), 8 * (lane & 3));
   int rlo[KE], rhi[KE];
@@ -986,19 +998,68 @@ __global__ __launch_bounds__(512, 2 * kLinearDwPerCu<KD>) void linear_dw_kernel(
     }
   };
 
-  for (int s = 0; s < min(depth - 1, steps); ++s) issue(s, s * stage);
-  int now = 0, next = end - stage;  // ring buffers of stages s and s + depth - 1
+  // the gate's backward of stage s: dy = dout W for this half's rows and K block wc, and with it do, dg and,
+  // in place of o, the gated row
+  auto gate_bwd = [&](int s, uint32_t boff) __attribute__((always_inline)) {
+    if (wc >= KB) return;
+    f32x16 dy = zero16();
+    const unsigned char* wt = lin_smem + wc * N * YTile::ROWB;
+    for (int q = 0; q < blocks_here; ++q) {
+      const unsigned char* tile = lin_smem + boff + S::OFF_Y + (half * blocks_here + q) * S::YB;
+#pragma unroll
+      for (int s2 = 0; s2 < 2; ++s2) dy = E::mfma(tr_perm_operand<T>(wt, 32 * q + 16 * s2 + 8 * g, lane), yo.natural(tile, s2), dy);
+    }
+    const int64_t row = r_begin + 64 * (int64_t)s + 32 * half + (lane & 31);
+    T* dox = reinterpret_cast<T*>(a.dox) + outer_row(row, a.plane, a.H, a.D) + 8 * g;
+    T* dg = reinterpret_cast<T*>(a.dg) + row * KD + 32 * wc + 8 * g;
+    unsigned char* xt = lin_smem + boff + half * S::XB;
+#pragma unroll
+    for (int h2 = 0; h2 < 2; ++h2) {
+      vec* const o = reinterpret_cast<vec*>(xt + XTile::off(lane & 31, 2 * (32 * wc + 16 * h2 + 8 * g)));
+      const vec ov = *o, gv = *reinterpret_cast<const vec*>(reinterpret_cast<unsigned char*>(o) + S::OFF_G);
+      vec yv, dov, dgv;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        float sg, ds;
+        gate_sigmoid<T>((float)gv[e], sg, ds);
+        yv[e] = (T)((float)ov[e] * sg);
+        dov[e] = (T)(dy[8 * h2 + e] * sg);
+        dgv[e] = (T)(dy[8 * h2 + e] * (float)ov[e] * ds);
+      }
+      *o = yv;
+      if (row < r_end) {
+        *reinterpret_cast<vec*>(dox + outer_channel(32 * wc + 16 * h2, a.plane.d, a.lgD)) = dov;
+        *reinterpret_cast<vec*>(dg + 16 * h2) = dgv;
+      }
+    }
+  };
+  if constexpr (FUSED) {
+    const T* w = reinterpret_cast<const T*>(a.gw);
+    for (int gi = wave; gi < KB * (N / 16); gi += 8) {
+      const int kb = gi / (N / 16), part = gi % (N / 16), r = 16 * part + lane / 4;
+      dma16(uni(lds0 + gi * 1024), w + (int64_t)r * KD + 32 * kb + 8 * ((lane % 4) ^ YTile::swz(r)));
+    }
+  }
+
+  for (int s = 0; s < min(depth - 1, steps); ++s) issue(s, ring + s * stage);
+  int now = ring, next = end - stage;  // ring buffers of stages s and s + depth - 1
   for (int s = 0; s < steps; ++s) {
     // stage s of this wave has landed once at most the stages s + 1 .. s + depth - 2 are in flight
     // (rows of dy that are loaded one number at a time have to arrive anyway)
-    wait_loads<0, 40>(odd || s + depth - 1 > steps ? 0 : in_flight);
+    // (and the four stores of each of the depth - 1 stages before this one)
+    const int stores = FUSED && wc < KB ? 4 * min(s, depth - 1) : 0;
+    wait_loads<0, 40>(odd || s + depth - 1 > steps ? 0 : in_flight + stores);
     finish(s, now);
     lds_sync();
     // (buffer `next` held stage s - 1, which every wave has read)
     if (s + depth - 1 < steps) issue(s + depth - 1, next);
+    if constexpr (FUSED) {
+      gate_bwd(s, now);
+      lds_sync();
+    }
     compute(now);
-    now = now + stage == end ? 0 : now + stage;
-    next = next + stage == end ? 0 : next + stage;
+    now = now + stage == end ? ring : now + stage;
+    next = next + stage == end ? ring : next + stage;
   }
 
   // the second half's sums -> LDS -> added to the first half's
