@@ -68,11 +68,13 @@ struct LdsTile {
   // bytes at once, and the rows that start at the same bank (every second one of 128 bytes, each of 256)
   // have to lie 64 bytes apart.  (With the plain row number as the value two or four of them met in a
   // bank, 25 to 30 % of the LDS cycles at d = 64: n = 512, h = 4, d = 128 dk/dv 970 -> 930 us, dq 616 ->
-  // 598; n = 768, h = 8, d = 64 dk/dv 2.52 -> 2.48 ms, the others within 1 %.)
+  // 598; n = 768, h = 8, d = 64 dk/dv 2.52 -> 2.48 ms, the others within 1 %.  As 5 x the value is one
+  // instruction away from the row number; with the chunk bits rotated, which is as free of conflicts, a
+  // step at n = 242, h = 8, d = 64 took 410 us, with 5 x 399, with the row number 399.)
   TRI_DEV static int swz(int r) {
     constexpr int B = CPR < 16 ? CPR : 16;  // (16 chunks are all banks)
     const int x = (r / RPB) % B;
-    return B <= 4 ? x : (x << 2 | x >> (B == 8 ? 1 : 2)) % B;
+    return B <= 4 ? x : (x + (x << 2)) % B;  // (5 x: bits 2 and 3 take what bits 0 and 1 are)
   }
   // byte offset, from the tile base, of byte `o` of row r (o must not straddle a chunk)
   TRI_DEV static int off(int r, int o) { return (r * CPR + ((o >> 4) ^ swz(r))) * 16 + (o & 15); }
