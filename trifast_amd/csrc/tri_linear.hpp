@@ -12,7 +12,7 @@
 //     global memory straight into registers: the MFMA's "columns" are rows of the tensor, so a
 //     lane owns a row, and the eight loads of a 256-byte row hit the same cache lines.
 //   * Weights pass through LDS (direct global->LDS loads, swizzled tiles, see LdsTile), shared by
-//     the four waves of a workgroup.
+//     the four waves of a workgroup, or stay there for all layers (eight waves, see ResidentPlan).
 //   * Products are computed transposed (W x^T) with the weight rows in the order perm32, so that
 //     a lane ends up with two runs of 8 consecutive channels of its own row: 16-byte stores.
 //   * Workgroups that share rows (different output columns of the same rows) run on one XCD, next
