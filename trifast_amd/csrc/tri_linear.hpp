@@ -147,6 +147,16 @@ __global__ __launch_bounds__(256) void linear_fwd_kernel(const LinearFwdArgs a) 
     const int last = a.n[at.p] - 1;
     Tile::template fill<32, 4>(lin_smem + q * CHUNK_B, [&](int r) { return w + (int64_t)min(at.col0 + r, last) * KD; }, wave, lane);
   }
+  // ... and their biases (a bias loaded in front of a chunk's products waits for the stores of the chunk before:
+  // gated, K = 128, 128 outputs with bias, 40000 rows 12.0 -> 11.7 us, 147456 25.4 -> 24.0; K = 64 20.1 -> 19.7)
+  T* const biases = reinterpret_cast<T*>(lin_smem + nq * CHUNK_B);
+  for (int q = wave; q < nq; q += 4) {
+    const ChunkAt at = chunk_at(a, q0 + q);
+    const T* bias = reinterpret_cast<const T*>(a.bias[at.p]);
+    T value = (T)0.0f;
+    if (bias && at.col0 + cl < a.n[at.p]) value = bias[at.col0 + cl];
+    biases[32 * q + cl] = value;
+  }
   // the rows' fragments (rows past the end repeat the last one and are not stored)
   int64_t row[RT];
   frag xf[RT][KS];
@@ -191,25 +201,14 @@ __global__ __launch_bounds__(256) void linear_fwd_kernel(const LinearFwdArgs a) 
   for (int q = 0; q < nq; ++q) {
     const ChunkAt at = chunk_at(a, q0 + q);
     const int N = a.n[at.p], hd = a.hd[at.p];
-    const T* bias = reinterpret_cast<const T*>(a.bias[at.p]);
     T* y = reinterpret_cast<T*>(a.y[at.p]);
-    const bool wide = (N % 8) == 0, wide_bias = wide && (reinterpret_cast<uintptr_t>(bias) & 15) == 0;
+    const bool wide = (N % 8) == 0;
     const ChunkColumns cols(at.col0, N, hd, a.rows);
     // this lane's 16 columns: col0 + 16 half + 8 g + 0..7
     f32x16 acc[RT];
 #pragma unroll
     for (int half = 0; half < 2; ++half) {
-      const int col = at.col0 + 16 * half + 8 * g;
-      vec bv = {};
-      if (bias) {
-        if (wide_bias) {
-          if (col < N) bv = *reinterpret_cast<const vec*>(bias + col);
-        } else {
-#pragma unroll
-          for (int e = 0; e < 8; ++e)
-            if (col + e < N) bv[e] = bias[col + e];
-        }
-      }
+      const vec bv = *reinterpret_cast<const vec*>(biases + 32 * q + 16 * half + 8 * g);
 #pragma unroll
       for (int e = 0; e < 8; ++e)
 #pragma unroll
