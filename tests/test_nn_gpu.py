@@ -160,6 +160,17 @@ def test_weight_gradient_against_float64(dtype, rows, k, n):
     assert bool(((db.double() - want_b).abs() <= bound_b).all())
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("rows", [1, 97, 300001])
+@pytest.mark.parametrize("k,n", [(128, 1), (128, 3), (64, 7), (32, 15), (128, 31), (128, 33), (64, 63), (256, 5), (256, 97),  # odd
+                                 (128, 44), (64, 20), (256, 6), (64, 50),                                              # even, not of 8
+                                 (128, 8), (128, 16), (128, 6), (64, 2), (32, 10)])                                    # alone in a group without blocks
+def test_weight_gradient_of_narrow_and_unaligned_layers(dtype, rows, k, n):
+    """One layer whose rows of dy keep 2- or 4-byte alignment only, or of a few outputs: each width of a
+    row of words, last blocks of a few outputs, rings that wrap (19 stages and more per chunk)."""
+    test_weight_gradient_against_float64(dtype, rows, k, n)
+
+
 @pytest.mark.parametrize("dtype,k,ns,n,hd,swap", [
     (torch.bfloat16, 128, [128, 128, 128, 4, 128], 17, 32, False),  # 289 rows: 33 in the second chunk, one in its second half-stage
     (torch.float16, 64, [64, 32, 2], 16, 32, True),                 # one chunk, rows a whole number of stages; layers share a group
@@ -202,6 +213,21 @@ def test_weight_gradients_of_several_layers(dtype, k, ns, n, hd, swap):
         if db[p] is not None:
             want, size = dy.sum(0), dy.abs().sum(0)
             assert bool(((db[p].double() - want).abs() <= 0.5 * eps * want.abs() + rows**0.5 * 2.0**-22 * size + tiny).all()), f"layer {p} bias"
+
+
+@pytest.mark.parametrize("dtype,k,ns,n,hd,swap", [
+    (torch.bfloat16, 128, [128, 128, 128, 4, 128], 211, 32, True),  # 11 stages per chunk through a ring of four, a riding layer
+    (torch.bfloat16, 128, [96, 96, 96, 3, 96], 211, 32, True),      # an odd layer, in a group of its own
+    (torch.float16, 64, [96, 96, 96, 3, 96], 301, 32, False),
+    (torch.float16, 128, [32, 33, 5, 20], 257, 32, False),          # one group: whole pieces, wide words, narrow words, 4 bytes
+    (torch.bfloat16, 32, [32, 7, 64], 300, 0, True),
+    (torch.float16, 64, [97, 4], 257, 0, False),                    # wide words: the narrow layer does not ride
+    (torch.bfloat16, 64, [128, 128, 128, 64, 33], 151, 32, True),   # wide words next to whole pieces, two groups of them
+    (torch.bfloat16, 256, [5, 160, 4], 150, 32, False),             # words first, the last block of its group
+])
+def test_weight_gradients_of_several_layers_over_many_stages(dtype, k, ns, n, hd, swap):
+    """The same over chunks that are longer than the ring, with layers whose rows of dy are no whole 16-byte pieces."""
+    test_weight_gradients_of_several_layers(dtype, k, ns, n, hd, swap)
 
 
 def test_linear_gradients_are_those_of_the_layer():

@@ -784,6 +784,7 @@ static void dw_split(tri::LinearDwArgs& a, int64_t most_chunks) {
   const tri::LinearDwGroups s = tri::linear_dw_groups(a.n, a.nlayers, a.K);
   a.groups = s.groups;
   a.rider = s.rider;
+  a.y_tile = tri::linear_dw_y_tile(a.n, a.nlayers);
   const int64_t fewest_rows = (a.rows + most_chunks - 1) / most_chunks;
   const int64_t k = a.gw ? std::max(a.K, 128) : a.K;  // (with the gate's backward one workgroup is resident per CU)
   a.rows_per_chunk = std::max(tri::linear_dw_rows_per_chunk(a.rows, a.groups, k), (fewest_rows + 63) / 64 * 64);

@@ -110,7 +110,9 @@ template <typename T, int KD>
 hipError_t dw_run(const LinearDwArgs& a, hipStream_t st) {
   const dim3 grid((unsigned)((a.chunks + 7) / 8 * 8 * a.groups));
   hipError_t e;
-  if (!a.g) {
+  if (!a.g && linear_dw_words(a.n, a.nlayers, a.rider)) {
+    e = launch_dyn(linear_dw_kernel<T, KD, kDwWords>, grid, dim3(512), LinearDwShape<T, KD, kDwWords>::LDS, st, a);
+  } else if (!a.g) {
     e = launch_dyn(linear_dw_kernel<T, KD, kDwPlain>, grid, dim3(512), LinearDwShape<T, KD, kDwPlain>::LDS, st, a);
   } else if (!a.gw) {
     e = launch_dyn(linear_dw_kernel<T, KD, kDwGated>, grid, dim3(512), LinearDwShape<T, KD, kDwGated>::LDS, st, a);

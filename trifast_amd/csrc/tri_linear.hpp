@@ -739,19 +739,24 @@ __global__ __launch_bounds__(512, 2) void linear_dx_resident_kernel(const Linear
 // TB/s of dy, x and partials (three workgroups of four waves per CU with padded tiles filled through
 // registers, the four outputs a group: 61 % of its LDS cycles were bank conflicts); gated, one layer: 42
 // -> 33 us; the sum of the partials 10.5 -> 6.3 us, each.  One layer alone, 2^20 rows: K = 256, 128
-// outputs 215 -> 160 us, K = 128 131 -> 107, 8 outputs 66 -> 69 (an odd number of outputs, loaded one at a
-// time: 102 -> 140 at K = 128, faster below 10^5 rows and at the other K).
+// outputs 215 -> 160 us, K = 128 123 -> 104, 8 outputs 64 -> 55, 3 outputs 101 -> 82 (see kDwWords).
 //
 // kDwGated: x is o * sigmoid(g) (see linear_fwd); o and g land in LDS and each wave gates the pieces
 // it loaded before the stage is handed over.  kDwGateBwd: the gate's backward (linear_gate_bwd) from the
 // same stages, which hold all it reads: dy = dout W for the rows of the stage, W resident, do and dg
 // stored, and the gated rows written over o for the weight gradient.  rows = 147456, K = 128, 128
 // outputs, with the sum of the partials: 44 us, 65 as two launches.
+//
+// kDwWords: launches with a layer (but a riding one) whose rows of dy are no whole 16-byte pieces, see
+// words_log2.  A kernel of its own: with the choice in the plain one every launch paid for it (K = 64, 4096
+// rows, 128 outputs 19.9 us alone, 21.6 with it).  Loaded through registers instead, with a wait for
+// everything in flight in every stage, 3 outputs at K = 128 and 2^20 rows took 141 us in place of 82, and four layers
+// of 96 outputs and one of 3, 147456 rows, 84 in place of 56.
 // ---------------------------------------------------------------------------------------
-constexpr int kDwPlain = 0, kDwGated = 1, kDwGateBwd = 2;
+constexpr int kDwPlain = 0, kDwGated = 1, kDwGateBwd = 2, kDwWords = 3;
 template <typename T, int KD, int MODE>
 struct LinearDwShape {
-  static constexpr bool GATED = MODE != kDwPlain, FUSED = MODE == kDwGateBwd;
+  static constexpr bool GATED = MODE == kDwGated || MODE == kDwGateBwd, FUSED = MODE == kDwGateBwd;
   static constexpr int PER_CU = FUSED ? 1 : kLinearDwPerCu<KD>;
   static constexpr int XB = 32 * KD * (int)sizeof(T), YB = 32 * 32 * (int)sizeof(T);  // x tile of a half, dy tile of a wave
   static constexpr int XP = XB / 1024;           // 1 KiB loads of an x tile, shared by the four waves of the half
@@ -762,7 +767,9 @@ struct LinearDwShape {
   static constexpr int LDS = 160 * 1024 / PER_CU, DUMP = XP % 4 ? LDS - 1024 : LDS;
   // loads per wave and stage: of x, of dy (16 or, where its rows keep only 4-byte alignment, 4 bytes per lane)
   static constexpr int X_LOADS = (GATED ? 2 : 1) * XN, Y_LOADS = 2, Y4_LOADS = 8;
-  static constexpr int MOST = 6;  // stages of a ring
+  static constexpr int MOST = 6;  // stages of a ring, at least two: four blocks with a riding layer, or of wide tiles
+  static_assert(YB == kLinearDwTile && 2 * (OFF_Y + 8 * YB + (RIDER ? 2 * RB : 0)) + (FUSED ? 128 * KD * (int)sizeof(T) : 0) <= DUMP, "two stages");
+  static_assert(MODE != kDwWords || 2 * (OFF_Y + 8 * kLinearDwWideTile) <= DUMP, "two stages of wide tiles");
 };
 
 // 16 (or 4) bytes per lane into LDS at dst + the lane's piece; unseen by the compiler (see StageRing)
@@ -771,6 +778,10 @@ TRI_DEV void dma16(uint32_t dst, const void* src) {
 }
 TRI_DEV void dma4(uint32_t dst, const void* src) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" : : "s"(dst), "v"(src) : "memory", "m0");
+}
+// 2 bytes per lane, 4 bytes apart in LDS, the upper two of them zero
+TRI_DEV void dma2(uint32_t dst, const void* src) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_ushort %1, off" : : "s"(dst), "v"(src) : "memory", "m0");
 }
 // wait until at most n (wave-uniform) loads are in flight; the count is part of the instruction
 template <int LO, int HI>
@@ -794,6 +805,12 @@ TRI_DEV typename Elem<T>::frag tr_pair(const unsigned char* p_lo, const unsigned
   for (int e = 0; e < 4; ++e) { f[e] = lo[e]; f[4 + e] = hi[e]; }
   return f;
 }
+
+// Rows of dy of an odd number of outputs start at any 2 bytes: they are loaded one output per lane and lie in LDS as
+// one word per output, the block's outputs rounded up to a power of two per row (the words past the
+// layer's last hold its last again).  Blocks of a few outputs of any number that is not a multiple of 8 take the same way:
+// fewer loads than 4 bytes at a time for all 32 columns.
+TRI_DEV int words_log2(int outputs) { return 32 - __builtin_clz((uint32_t)max(min(outputs, 32), 2) - 1u); }
 
 template <typename T, int KD, int MODE>
 __global__ __launch_bounds__(512, (2 * LinearDwShape<T, KD, MODE>::PER_CU)) void linear_dw_kernel(const LinearDwArgs a) {
@@ -837,7 +854,9 @@ __global__ __launch_bounds__(512, (2 * LinearDwShape<T, KD, MODE>::PER_CU)) void
   const int64_t r_begin = (int64_t)chunk * a.rows_per_chunk;
   const int64_t r_end = min(a.rows, r_begin + a.rows_per_chunk);
   const int steps = (int)((r_end - r_begin + 63) / 64);
-  const bool even = (N % 8) != 0 && (N % 2) == 0, odd = (N % 2) != 0;  // rows of dy keep 4- or 2-byte alignment
+  // rows of dy that keep 4- or 2-byte alignment only: loaded 4 bytes at a time, or one output per lane (see words_log2)
+  const bool words = MODE == kDwWords && N % 8 != 0 && (N % 2 != 0 || N - col0 <= kLinearDwRider);
+  const bool even = MODE == kDwWords && N % 8 != 0 && !words;
 
   // where this lane's pieces of the tiles lie: tile row and address in row 0
   const T* yg = reinterpret_cast<const T*>(a.dy[p]);
@@ -867,18 +886,21 @@ __global__ __launch_bounds__(512, (2 * LinearDwShape<T, KD, MODE>::PER_CU)) void
     rp = reinterpret_cast<const T*>(a.dy[a.rider]) + linear_offset(0, col < rN ? col : 0, rN, a.hd[a.rider], a.rows);
   }
   // a stage: the x tiles of the two halves (o, then g), the dy tiles of their blocks, those of a riding layer
-  const int off_y = S::OFF_Y + (half * blocks_here + wc) * S::YB;
-  const int off_r = S::OFF_Y + 2 * blocks_here * S::YB + half * S::RB;
-  const int stage = S::OFF_Y + 2 * blocks_here * S::YB + (rides ? 2 * S::RB : 0);
+  const int yb = MODE == kDwWords ? a.y_tile : S::YB;
+  const int off_y = S::OFF_Y + (half * blocks_here + wc) * yb;
+  const int off_r = S::OFF_Y + 2 * blocks_here * yb + half * S::RB;
+  const int stage = S::OFF_Y + 2 * blocks_here * yb + (rides ? 2 * S::RB : 0);
+  const int lw = words ? words_log2(N - col0) : 0;
   // (the gate's backward: W, [N][32] tiles of the K blocks, in front of the ring)
   const int ring = FUSED ? N * KD * (int)sizeof(T) : 0;
   const int depth = min((S::DUMP - ring) / stage, S::MOST), end = ring + depth * stage;
-  const int in_flight = (depth - 2) * (S::X_LOADS + (!live ? 0 : even ? S::Y4_LOADS : S::Y_LOADS) + (rides ? 1 : 0));
+  const int in_flight = (depth - 2) * (S::X_LOADS + (!live ? 0 : words ? 1 << (lw - 1) : even ? S::Y4_LOADS : S::Y_LOADS) + (rides ? 1 : 0));
   const uint32_t lds0 = (uint32_t)(uintptr_t)(TRI_L3 const unsigned char*)lin_smem;
   auto uni = [](uint32_t x) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)x); };
 
   // ask for stage s (rows past the end: the last one again) into the ring buffer at `boff`
-  auto issue = [&](int s, uint32_t boff) __attribute__((always_inline)) {
+  auto issue = [&](int s, uint32_t boff, auto words_tag) __attribute__((always_inline)) {
+    constexpr bool WORDS = decltype(words_tag)::value;
     const int64_t first = r_begin + 64 * (int64_t)s + 32 * half, last = r_end - 1;
 #pragma unroll
     for (int x = 0; x < XN; ++x) {
@@ -894,7 +916,7 @@ __global__ __launch_bounds__(512, (2 * LinearDwShape<T, KD, MODE>::PER_CU)) void
     const uint32_t ybuf = boff + off_y;
     if (!live) {
       // (nobody reads its tile)
-    } else if (even) {
+    } else if (!WORDS && even) {
       int ln = lane;
       asm volatile("" : "+v"(ln));  // (what follows from the lane is worked out here, not kept in registers)
 #pragma unroll
@@ -902,27 +924,21 @@ __global__ __launch_bounds__(512, (2 * LinearDwShape<T, KD, MODE>::PER_CU)) void
         const int row = 4 * t + ln / 16, col = col0 + 8 * ((ln % 16 / 4) ^ YTile::swz(row)) + 2 * (ln % 4);
         dma4(uni(lds0 + ybuf + t * 256), yg + mapped_row(a.ymap, min(first + row, last)) * N + (col < N ? col : col0));
       }
-    } else if (!odd) {
+    } else if (!WORDS) {
 #pragma unroll
       for (int t = 0; t < 2; ++t) dma16(uni(lds0 + ybuf + t * 1024), yp + mapped_row(a.ymap, min(first + 16 * t + yr, last)) * y_pitch);
     } else {
       int ln = lane;
       asm volatile("" : "+v"(ln));
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        const int row = 16 * t + ln / 4, col = col0 + 8 * ((ln % 4) ^ YTile::swz(row));
-        const T* src = yg + mapped_row(a.ymap, min(first + row, last)) * N;
-        vec v = {};
-#pragma unroll
-        for (int e = 0; e < 8; ++e)
-          if (col + e < N) v[e] = src[col + e];
-        *reinterpret_cast<vec*>(lin_smem + ybuf + t * 1024 + lane * 16) = v;
-      }
+      const int col = min(col0 + (ln & ((1 << lw) - 1)), N - 1);
+#pragma unroll 1
+      for (int t = 0; t < 32; t += 64 >> lw) dma2(uni(lds0 + ybuf + (t << lw) * 4), yg + mapped_row(a.ymap, min(first + t + (ln >> lw), last)) * N + col);
     }
     if (rides) dma4(uni(lds0 + boff + off_r + wc * 256), rp + mapped_row(a.ymap, min(first + rr, last)) * r_pitch);
   };
   // what this wave loaded of stage s has landed: gate it, and clear rows past the end
-  auto finish = [&](int s, uint32_t boff) __attribute__((always_inline)) {
+  auto finish = [&](int s, uint32_t boff, auto words_tag) __attribute__((always_inline)) {
+    constexpr bool WORDS = decltype(words_tag)::value;
     unsigned char* xbuf = lin_smem + boff + half * S::XB + lane * 16;
     if constexpr (GATED && !FUSED) {
 #pragma unroll
@@ -941,7 +957,11 @@ __global__ __launch_bounds__(512, (2 * LinearDwShape<T, KD, MODE>::PER_CU)) void
         *reinterpret_cast<vec*>(xbuf + (4 * x + wc) * 1024) = none;
         if constexpr (FUSED) *reinterpret_cast<vec*>(xbuf + S::OFF_G + (4 * x + wc) * 1024) = none;
       }
-    if (live) {
+    if (live && WORDS) {
+#pragma unroll 1
+      for (int t = 0; t < 32; t += 64 >> lw)
+        if (first + t + (lane >> lw) >= r_end) *reinterpret_cast<uint32_t*>(lin_smem + boff + off_y + ((t << lw) + lane) * 4) = 0u;
+    } else if (live) {
 #pragma unroll
       for (int t = 0; t < 2; ++t)
         if (first + 16 * t + yr >= r_end) *reinterpret_cast<vec*>(lin_smem + boff + off_y + t * 1024 + lane * 16) = none;
@@ -972,13 +992,25 @@ __global__ __launch_bounds__(512, (2 * LinearDwShape<T, KD, MODE>::PER_CU)) void
     rlo[i] = XTile::off(row, col * 2);
     rhi[i] = XTile::off(row + 4, col * 2);
   }
-  auto compute = [&](uint32_t boff) __attribute__((always_inline)) {
+  auto words_frag = [&](const unsigned char* yt, int s2) __attribute__((always_inline)) {
+    typedef uint32_t u32x4s __attribute__((ext_vector_type(4)));
+    int ln = lane;
+    asm volatile("" : "+v"(ln));
+    const uint32_t* w = reinterpret_cast<const uint32_t*>(yt) + ((16 * s2 + 8 * (ln >> 5)) << lw) + (ln & 31 & ((1 << lw) - 1));
+    u32x4s v;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = w[(2 * e) << lw] | w[(2 * e + 1) << lw] << 16;
+    return __builtin_bit_cast(frag, v);
+  };
+  auto compute = [&](uint32_t boff, auto words_tag) __attribute__((always_inline)) {
     const unsigned char *xt = lin_smem + boff + half * S::XB, *yt = lin_smem + boff + off_y;
 #pragma unroll
     for (int s2 = 0; s2 < 2; ++s2) {
       if (live) {
         // A: dy^T (output row n in the lane, 8 memory rows as contraction slots); B: x^T
-        const frag af = yo.transposed(yt, s2, 0);
+        frag af;
+        if constexpr (decltype(words_tag)::value) af = words_frag(yt, s2);
+        else af = yo.transposed(yt, s2, 0);
         if (sums) bacc = E::mfma(af, ones, bacc);
 #pragma unroll
         for (int i = 0; i < KB; ++i) acc[i] = E::mfma(af, xo.transposed(xt, s2, i), acc[i]);
@@ -1004,7 +1036,7 @@ __global__ __launch_bounds__(512, (2 * LinearDwShape<T, KD, MODE>::PER_CU)) void
     f32x16 dy = zero16();
     const unsigned char* wt = lin_smem + wc * N * YTile::ROWB;
     for (int q = 0; q < blocks_here; ++q) {
-      const unsigned char* tile = lin_smem + boff + S::OFF_Y + (half * blocks_here + q) * S::YB;
+      const unsigned char* tile = lin_smem + boff + S::OFF_Y + (half * blocks_here + q) * yb;
 #pragma unroll
       for (int s2 = 0; s2 < 2; ++s2) dy = E::mfma(tr_perm_operand<T>(wt, 32 * q + 16 * s2 + 8 * g, lane), yo.natural(tile, s2), dy);
     }
@@ -1040,26 +1072,31 @@ __global__ __launch_bounds__(512, (2 * LinearDwShape<T, KD, MODE>::PER_CU)) void
     }
   }
 
-  for (int s = 0; s < min(depth - 1, steps); ++s) issue(s, ring + s * stage);
-  int now = ring, next = end - stage;  // ring buffers of stages s and s + depth - 1
-  for (int s = 0; s < steps; ++s) {
-    // stage s of this wave has landed once at most the stages s + 1 .. s + depth - 2 are in flight
-    // (rows of dy that are loaded one number at a time have to arrive anyway)
-    // (and the four stores of each of the depth - 1 stages before this one)
-    const int stores = FUSED && wc < KB ? 4 * min(s, depth - 1) : 0;
-    wait_loads<0, 40>(odd || s + depth - 1 > steps ? 0 : in_flight + stores);
-    finish(s, now);
-    lds_sync();
-    // (buffer `next` held stage s - 1, which every wave has read)
-    if (s + depth - 1 < steps) issue(s + depth - 1, next);
-    if constexpr (FUSED) {
-      gate_bwd(s, now);
+  auto walk = [&](auto words_tag) __attribute__((always_inline)) {
+    for (int s = 0; s < min(depth - 1, steps); ++s) issue(s, ring + s * stage, words_tag);
+    int now = ring, next = end - stage;  // ring buffers of stages s and s + depth - 1
+    for (int s = 0; s < steps; ++s) {
+      // stage s of this wave has landed once at most the stages s + 1 .. s + depth - 2 are in flight
+      // (and the four stores of each of the depth - 1 stages before this one)
+      const int stores = FUSED && wc < KB ? 4 * min(s, depth - 1) : 0;
+      wait_loads<0, 40>(s + depth - 1 > steps ? 0 : in_flight + stores);
+      finish(s, now, words_tag);
       lds_sync();
+      // (buffer `next` held stage s - 1, which every wave has read)
+      if (s + depth - 1 < steps) issue(s + depth - 1, next, words_tag);
+      if constexpr (FUSED) {
+        gate_bwd(s, now);
+        lds_sync();
+      }
+      compute(now, words_tag);
+      now = now + stage == end ? ring : now + stage;
+      next = next + stage == end ? ring : next + stage;
     }
-    compute(now);
-    now = now + stage == end ? ring : now + stage;
-    next = next + stage == end ? ring : next + stage;
-  }
+  };
+  // (a loop of its own for the waves whose dy lies in words: with the choice inside the loop 2^20 rows, K = 128, 3 outputs
+  // take 92 us in place of 85)
+  if (words) walk(std::integral_constant<bool, MODE == kDwWords>{});
+  else walk(std::false_type{});
 
   // the second half's sums -> LDS -> added to the first half's
   auto fold = [&](f32x16* set, int count, int slot) __attribute__((always_inline)) {

@@ -87,6 +87,7 @@ struct LinearDwArgs {
   int64_t total;
   int64_t rows, rows_per_chunk;     // (a multiple of 64)
   int chunks, groups, rider;        // (see linear_dw_groups)
+  int y_tile;                       // (see linear_dw_y_tile)
   int K;
   RowMap xmap, ymap;
   const void* g;                    // gated source: g [rows, K]
@@ -97,11 +98,25 @@ struct LinearDwArgs {
 };
 
 constexpr int kLinearDwRider = 16;  // outputs of a riding layer at most (see linear_dw_groups)
+constexpr int kLinearDwTile = 2048, kLinearDwWideTile = 4096;
+
+// LDS bytes of a block's tile of 32 rows of dy: 64 per row; those of an odd number of outputs lie there as one word
+// per output, which beyond 16 of them is twice as much.
+template <typename Int>
+inline int linear_dw_y_tile(const Int* n, int nlayers) {
+  for (int p = 0; p < nlayers; ++p)
+    if (n[p] % 2 != 0 && n[p] > 16) return kLinearDwWideTile;
+  return kLinearDwTile;
+}
 
 // How the weight-gradient kernel's outputs are split over workgroups: groups of four 32-output blocks,
 // the layers' blocks one after the other.  A layer of one block that would be a group for itself
 // rides in the first group instead (an even number of outputs: it is loaded 4 bytes at a time; up
-// to 128 channels: the accumulators of one block and a part of another fill the registers at 256).
+// to 128 channels: the accumulators of one block and a part of another fill the registers at 256; next to
+// tiles of the ordinary size: with wide ones two stages and its own would not fit LDS at 64 channels).
+// Alone it rides in a group without blocks, so that four waves share the work of a stage in place of
+// one (2^20 rows, K = 128, 8 outputs: 71 -> 55 us); of 8 or 16 outputs of up to 64 channels one wave
+// keeps up (K = 64 39.9 us and 44.4, K = 32 36.8 and 42.2; of 4, which are loaded in words then, 49.9 and 44.3).
 struct LinearDwGroups {
   int groups, rider;  // rider: layer, or -1
 };
@@ -113,8 +128,15 @@ inline LinearDwGroups linear_dw_groups(const Int* n, int nlayers, int64_t k) {
     blocks += (n[p] + 31) / 32;
     if (n[p] <= kLinearDwRider && n[p] % 2 == 0) small = p;
   }
-  const bool rides = k <= 128 && small >= 0 && blocks > 1 && blocks % 4 == 1;
-  return LinearDwGroups{(int)((blocks - (rides ? 1 : 0) + 3) / 4), rides ? small : -1};
+  const bool rides = k <= 128 && linear_dw_y_tile(n, nlayers) == kLinearDwTile && small >= 0 && blocks % 4 == 1 && (blocks > 1 || k == 128 || n[small] % 8 != 0);
+  return LinearDwGroups{blocks == 1 ? 1 : (int)((blocks - (rides ? 1 : 0) + 3) / 4), rides ? small : -1};
+}
+// Whether rows of dy of some layer (but the riding one) are not whole 16-byte pieces.
+template <typename Int>
+inline bool linear_dw_words(const Int* n, int nlayers, int rider) {
+  for (int p = 0; p < nlayers; ++p)
+    if (p != rider && n[p] % 8 != 0) return true;
+  return false;
 }
 // Workgroups of eight waves per CU: two for narrow rows, where one step's latency shows next to the few
 // bytes of a stage (2^20 rows, 8 or 64 outputs: K = 32 59 us with one, 41 to 46 with two, K = 64 61 to 63
