@@ -427,6 +427,13 @@ def test_row_resident_backward_size_classes(n, h, d, dtype, forced_tiles):
     assert kern_out[2][:, :, 5, : n - 7].abs().max() == 0 and kern_out[3][:, :, 5, : n - 7].abs().max() == 0
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("n", [450, 520, 700, 800, 1000])
+def test_row_resident_backward_of_narrow_heads(n, dtype, forced_tiles):
+    """The size classes of head dim 16 beyond 384 keys (where not every wave has a share in a stage's loads)."""
+    test_row_resident_backward_size_classes(n, 1, 16, dtype, forced_tiles)
+
+
 # ---------------------------------------------------------------------------
 # golden fixtures (inputs and answers fixed on disk)
 # ---------------------------------------------------------------------------

@@ -70,16 +70,7 @@ bool bwd_kv_supports(int tile, int64_t n, int d, int dtype) {
 }
 
 hipError_t bwd_kv_launch(const BwdArgs& a, int bh, int d, int dtype, int tile, hipStream_t st) {
-  if (bwd_kv_tile_writes_dq(tile)) {
-    // The smallest row-resident tile that holds the row: a pick is kept for a range of lengths (one of n = 449
-    // serves n = 384, one of 300 serves 200), and the larger tile runs the shorter row with key tiles that are
-    // not there (h = 4, tile that holds it and the next: d = 32 n = 384 172 and 193 us, 256 55 and 82, 128 19 and
-    // 28, 700 793 and 870; d = 16 n = 384 133 and 157; d = 64 n = 256 119 and 139).
-    int row = tile - BwdKVFamily::kNumTiles;
-    if (row < kBwdRowTiles - 1)
-      while (row > 0 && a.N <= 128 * kRowKeyTiles[row - 1]) --row;
-    return row_launch(a, bh, d, dtype, row, st, false);
-  }
+  if (bwd_kv_tile_writes_dq(tile)) return row_launch(a, bh, d, dtype, tile - BwdKVFamily::kNumTiles, st, false);
   return dispatch<BwdKVFamily>(a, bh, d, dtype, tile, st, false);
 }
 
