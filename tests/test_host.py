@@ -173,6 +173,30 @@ def test_pick_charges_a_tile_what_it_leaves_to_other_kernels(tmp_path, monkeypat
     tuner.reset()
 
 
+def test_pick_times_what_can_win(tmp_path, monkeypatch):
+    """On a miss every tile is timed once, and a second time unless it is far behind; of the row-resident
+    tiles only the one that fits the length, which is what a later hit takes too."""
+    monkeypatch.setenv("TRIFAST_CONFIG_DIR", str(tmp_path))
+    monkeypatch.setenv("TRIFAST_AUTOTUNE", "1")
+    monkeypatch.delenv("TRIFAST_FORCE_TUNE", raising=False)
+    monkeypatch.setattr(tuner, "_device_tag", lambda device=None: "Test-GPU_9-5")
+    lib = _lib.load()
+    for n in (31, 256, 300, 700, 1024):
+        timed = []
+        fits = lib.trifast_default_tile(_lib.KERNEL_BWD_KV, n, 4, 32, _lib.BF16)
+        slow = {0: 9.0, fits: 2.0}  # (the first time of the tile that fits is a cold one)
+        monkeypatch.setattr(tuner, "_time_launch", lambda launch, t, **kw: timed.append(t) or (1.0 if timed.count(t) > 1 and t == fits else slow.get(t, 1.6)))
+        tuner.reset()
+        assert tuner.pick(_lib.KERNEL_BWD_KV, n, 4, 32, torch.bfloat16, lambda t: None) == fits
+        rows = [t for t in timed if lib.trifast_bwd_kv_tile_writes_dq(t)]
+        streaming = [t for t in tuner.supported_tiles(_lib.KERNEL_BWD_KV, n, 4, 32, torch.bfloat16) if not lib.trifast_bwd_kv_tile_writes_dq(t)]
+        assert rows == [fits, fits] and timed.count(0) == 1
+        assert [timed.count(t) for t in streaming[1:]] == [2] * len(streaming[1:])
+        for f in tmp_path.glob("*.json"):
+            f.unlink()
+    tuner.reset()
+
+
 def test_row_resident_tiles_in_the_library_tables():
     """The row-resident kernel appears as the last eight tiles of the dk/dv family: seven for rows
     of up to 256, 384, ..., 1024 keys, for 16-bit inputs, and one that runs longer rows (up to
