@@ -663,10 +663,8 @@ __global__ __launch_bounds__(GJ * GK * 64) void tri_bwd_b_kernel(const BwdArgs a
   // where V was, the next row's Q and dO where this row's were.  (Two sets of operands took 243 registers
   // at d = 32 and left none for a mask; d = 64 does not fit two.)  -lse is the addend of the
   // exponent's fma in every row; where rows have masked keys in this block each tile takes one more
-  // product, which adds the mask element to the scores of the masked keys (keys operand against ones), and
-  // skips the vector work of tiles without an attended key, a branch per step (n = 512 with 397 valid positions,
-  // training step 557 us with it and 557 without; h = 8, d = 64 n = 768 with half of the keys masked 7.84 and 7.92 ms: the
-  // branches leave the compiler fewer values to hold at once, and the loop no spilled ones).
+  // product, which adds the mask element to the scores of the masked keys (keys operand against ones), and leaves
+  // out tiles without an attended key (see phase).
   // Alone, back to back on one card against the walk with two operand sets, which took unmasked rows of up to
   // 64 bytes only: h = 4, d = 32 n = 1024 0.96 -> 0.91 ms; 2048 with 5 % masked 9.6 (16 waves: 8.9) -> 8.5;
   // h = 8, d = 64 n = 768 1.80 -> 1.53, half of the keys masked 1.84 -> 1.60, with pair rows 98 KiB apart 1.85 ->
@@ -762,13 +760,24 @@ __global__ __launch_bounds__(GJ * GK * 64) void tri_bwd_b_kernel(const BwdArgs a
       // between the elementwise work of the tile before it, whose scores s and dP are complete: db +=
       // exp2(c s - lse) dP.  `cur`, `next`: row buffers of the tile and of the tile after it; `turn` comes
       // between the two chains.
-      auto phase = [&](auto tn_tag, int cur, int next, uint32_t keepw, uint32_t attended, f32x16& sn, f32x16& dpn, const f32x16& s, const f32x16& dp,
+      auto phase = [&](auto tn_tag, int cur, int next, uint32_t keepw, uint32_t attended, f32x16& sn, f32x16& dpn, f32x16& s, f32x16& dp,
                        float addend, auto&& turn, auto&& between) __attribute__((always_inline)) {
         constexpr int TN = decltype(tn_tag)::value, TC = 1 - TN;
         // A tile without an attended key (`attended`: the keep word of the tile before) adds nothing: dS = 0 whatever its K and V
         // rows and its bias hold.  Where they are infinite or NaN, as padding may be, zero probabilities
-        // times their dP are not zero.
-        const uint32_t adds = MASKED ? __builtin_amdgcn_readfirstlane(attended) : 1u;
+        // times their dP are not zero.  Its elementwise work is skipped, a branch per step, or, in rows of 128 bytes, done on
+        // zeros, one branch per tile (n = 768, h = 8 with half of the keys masked: 1.62 ms, 1.69 with a branch per step; n = 1024,
+        // d = 32, four blocks of keys that attend to themselves: 0.82 ms with a branch per step, 1.19 on zeros).
+        uint32_t adds = 1u;
+        if constexpr (MASKED) adds = __builtin_amdgcn_readfirstlane(attended);
+        if constexpr (MASKED && kMoving) {
+          if (adds == 0) {
+            asm volatile("" ::);
+#pragma unroll
+            for (int v = 0; v < 16; ++v) s[v] = dp[v] = 0.f;
+            addend = 0.f;
+          }
+        }
         frag mk;
         if constexpr (MASKED) mk = mask_operand(keepw, TN);
         static_for<NM>([&](auto xc) __attribute__((always_inline)) {
@@ -799,7 +808,7 @@ __global__ __launch_bounds__(GJ * GK * 64) void tri_bwd_b_kernel(const BwdArgs a
               dbacc[0][TC][v] = __builtin_fmaf(p, dp[v], dbacc[0][TC][v]);
             }
           };
-          if constexpr (!MASKED) add();
+          if constexpr (!MASKED || kMoving) add();
           else if (adds != 0) add();
           __builtin_amdgcn_sched_barrier(0);
           if constexpr (X == M + DS) {
