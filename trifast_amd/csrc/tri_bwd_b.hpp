@@ -184,12 +184,13 @@ __global__ __launch_bounds__(GJ * GK * 64) void tri_bwd_b_kernel(const BwdArgs a
   //     A chunk is a share of the rows in front and a share of the run: rows of the run take about
   //     half the time of the others.
   //   * (pipelined walk) The first fully masked row of the chunk; whether any other row masks a key of this
-  //     block; which key tiles of the block have an attended key in any row.
+  //     block; which key tiles of the block have an attended key in any row, and which have none in some row.
   uint32_t* scan_words = reinterpret_cast<uint32_t*>(tri_smem);
   if (tid == 0) {
     scan_words[0] = 0;
     scan_words[1] = (uint32_t)N;
-    scan_words[2] = 0;  // key tiles with an attended key, then (from bit 16) with a masked one
+    scan_words[2] = 0;  // key tiles with an attended key in some row; from bit 8 on those with a masked one; from bit 16 on
+                        // those without an attended one in some row
   }
   __syncthreads();
   const uint32_t* flags = a.rowflag + (int64_t)b * N;
@@ -212,14 +213,15 @@ __global__ __launch_bounds__(GJ * GK * 64) void tri_bwd_b_kernel(const BwdArgs a
     for (int i = i_begin + tid; i < i_end; i += NW * 64) {
       if (flags[i] != 0) {
         atomicMin(scan_words + 1, (uint32_t)i);
-        tiles = 0xffffu | tiles;
+        tiles |= 0xffu;
         break;
       }
       const uint32_t* kw = a.keep + ((int64_t)b * N + i) * a.nwords;
 #pragma unroll
       for (int w = 0; w < BKB / 32; ++w) {
         const uint32_t x = k_blk / 32 + w < a.nwords ? kw[k_blk / 32 + w] : 0u;
-        tiles |= (x != 0 ? 1u << w : 0u) | ((x | past_end(k_blk / 32 + w)) != 0xffffffffu ? 0x10000u << w : 0u);
+        const uint32_t past = past_end(k_blk / 32 + w);
+        tiles |= (x != 0 ? 1u << w : past != 0xffffffffu ? 0x10000u << w : 0u) | ((x | past) != 0xffffffffu ? 0x100u << w : 0u);
       }
     }
     if (tiles) atomicOr(scan_words + 2, tiles);
@@ -230,10 +232,10 @@ __global__ __launch_bounds__(GJ * GK * 64) void tri_bwd_b_kernel(const BwdArgs a
   run_begin = __builtin_amdgcn_readfirstlane(run_begin);
   int nrows = __builtin_amdgcn_readfirstlane(i_end) - i_begin;
   const int tail_begin = run_begin + share_of(N - run_begin, chunk), tail_end = run_begin + share_of(N - run_begin, chunk + 1);
-  // rows that take the pipelined walk, and the block's key tiles (live, and masked from bit 16)
+  // rows that take the pipelined walk, and the block's key tiles (see scan_words)
   int nwalk = kPipelined ? __builtin_amdgcn_readfirstlane(min((int)scan_words[1] - i_begin, nrows)) : 0;
-  const uint32_t block_tiles = kPipelined ? __builtin_amdgcn_readfirstlane(scan_words[2]) : 0xffffu;
-  if ((block_tiles & 0xffffu) == 0) nrows = nwalk = 0;  // no attended key in any row: dS = 0
+  const uint32_t block_tiles = kPipelined ? __builtin_amdgcn_readfirstlane(scan_words[2]) : 0xffu;
+  if ((block_tiles & 0xffu) == 0) nrows = nwalk = 0;  // no attended key in any row: dS = 0
   __syncthreads();
 
   const T* qbase = reinterpret_cast<const T*>(a.q) + b * a.sq.b + h * a.sq.h;
@@ -689,9 +691,11 @@ __global__ __launch_bounds__(GJ * GK * 64) void tri_bwd_b_kernel(const BwdArgs a
   }
   if constexpr (kPipelined) {
     if (nwalk < 2 * NBUF) nwalk = 0;  // too few to fill the pipeline
-    const uint32_t wave_tiles = __builtin_amdgcn_readfirstlane(block_tiles >> (wk * WK) & ((1u << WK) - 1));
+    static_assert(BKB / 32 <= 8, "eight key tiles per field of the block's words");
+    const uint32_t wave_tiles = __builtin_amdgcn_readfirstlane(block_tiles >> (wk * WK));
+    // masked_tag: 0 every key is attended, 1 some are masked, 2 some tile of the wave has no attended key in some row
     auto walk = [&](auto masked_tag, auto busy_tag) __attribute__((always_inline)) {
-      constexpr bool MASKED = decltype(masked_tag)::value;
+      constexpr bool MASKED = decltype(masked_tag)::value != 0, DEAD = decltype(masked_tag)::value == 2;
       // (a wave without queries or attended keys takes part in the loads and barriers only)
       constexpr bool BUSY = decltype(busy_tag)::value;
       typedef uint32_t u32x4v __attribute__((ext_vector_type(4)));
@@ -765,12 +769,14 @@ __global__ __launch_bounds__(GJ * GK * 64) void tri_bwd_b_kernel(const BwdArgs a
         constexpr int TN = decltype(tn_tag)::value, TC = 1 - TN;
         // A tile without an attended key (`attended`: the keep word of the tile before) adds nothing: dS = 0 whatever its K and V
         // rows and its bias hold.  Where they are infinite or NaN, as padding may be, zero probabilities
-        // times their dP are not zero.  Its elementwise work is skipped, a branch per step, or, in rows of 128 bytes, done on
-        // zeros, one branch per tile (n = 768, h = 8 with half of the keys masked: 1.62 ms, 1.69 with a branch per step; n = 1024,
-        // d = 32, four blocks of keys that attend to themselves: 0.82 ms with a branch per step, 1.19 on zeros).
+        // times their dP are not zero.  Its elementwise work is skipped, a branch per step, in a loop of its own for waves
+        // with such a tile (n = 1024, d = 32, four blocks of keys that attend to themselves: 0.81 ms, 1.19 done on zeros;
+        // with the branches in every masked loop n = 2048 with 5 % masked 8.24 -> 8.5 ms from a cool chip).  In rows of
+        // 128 bytes a second masked loop leaves the compiler spilling in the first: there the work is done on zeros, one
+        // branch per tile in the one loop (n = 768, h = 8 with half of the keys masked: 1.61 ms, as without it).
         uint32_t adds = 1u;
-        if constexpr (MASKED) adds = __builtin_amdgcn_readfirstlane(attended);
-        if constexpr (MASKED && kMoving) {
+        if constexpr (DEAD) adds = __builtin_amdgcn_readfirstlane(attended);
+        if constexpr (DEAD && kMoving) {
           if (adds == 0) {
             asm volatile("" ::);
 #pragma unroll
@@ -808,7 +814,7 @@ __global__ __launch_bounds__(GJ * GK * 64) void tri_bwd_b_kernel(const BwdArgs a
               dbacc[0][TC][v] = __builtin_fmaf(p, dp[v], dbacc[0][TC][v]);
             }
           };
-          if constexpr (!MASKED || kMoving) add();
+          if constexpr (!DEAD || kMoving) add();
           else if (adds != 0) add();
           __builtin_amdgcn_sched_barrier(0);
           if constexpr (X == M + DS) {
@@ -947,10 +953,13 @@ __global__ __launch_bounds__(GJ * GK * 64) void tri_bwd_b_kernel(const BwdArgs a
 #endif
     };
     if (nwalk > 0) {
-      const bool busy = wave_live != 0 && wave_tiles != 0, masked = block_tiles >> 16 != 0;
-      if (!busy) walk(std::false_type{}, std::false_type{});
-      else if (masked) walk(std::true_type{}, std::true_type{});
-      else walk(std::false_type{}, std::true_type{});
+      constexpr uint32_t kMine = (1u << WK) - 1;
+      const bool busy = wave_live != 0 && (wave_tiles & kMine) != 0, masked = (block_tiles & 0xff00u) != 0;
+      const bool dead = kMoving || (wave_tiles >> 16 & kMine) != 0;
+      if (!busy) walk(std::integral_constant<int, 0>{}, std::false_type{});
+      else if (!masked) walk(std::integral_constant<int, 0>{}, std::true_type{});
+      else if (dead) walk(std::integral_constant<int, 2>{}, std::true_type{});
+      else if constexpr (!kMoving) walk(std::integral_constant<int, 1>{}, std::true_type{});
 #ifdef TRI_DB_TIMING
       return;
 #endif
