@@ -347,6 +347,19 @@ def test_gate_backward_with_the_weight_gradient(dtype, c, h, d, n, swap):
             assert bool(((x.double() - want).abs() <= bound).all())
 
 
+@pytest.mark.parametrize("dtype,c,h,d,swap", [
+    (torch.bfloat16, 32, 4, 32, True),   # a ring of four stages
+    (torch.float16, 64, 4, 32, False),   # of three
+    (torch.bfloat16, 128, 4, 32, True),  # of two
+    (torch.float16, 128, 2, 32, True),   # four, two K blocks: half of the waves do not gate
+    (torch.bfloat16, 64, 4, 16, False),  # five
+    (torch.float16, 32, 1, 64, True),    # six
+])
+def test_gate_backward_with_the_weight_gradient_over_many_stages(dtype, c, h, d, swap):
+    """The same over chunks of ten stages: every ring wraps, beside the stores of do and dg."""
+    test_gate_backward_with_the_weight_gradient(dtype, c, h, d, 401, swap)
+
+
 @pytest.mark.parametrize("dtype,k,ns,hd,n,swap", [
     (torch.bfloat16, 128, [128, 128, 128, 4, 128], 32, 211, True),  # 44521 rows: a part of a tile, a round in which some waves have none
     (torch.float16, 128, [64, 2, 64], 64, 203, False),              # four chunks, one quad per tile

@@ -212,7 +212,7 @@ constexpr int bwd_uniform_lds_bytes(int D, int es, int NW) {
 //   dq_j = s / n (M1 dO_j - delta_j sK),   M1 = sum_k K_k V_k^T,  sK = sum_k K_k
 //   dk_k = s / n (M2 V_k - sQ),            M2 = sum_j Q_j dO_j^T, sQ = sum_j delta_j Q_j
 //   dv_k = sO / n,                          sO = sum_j dO_j
-// The sums run on the matrix pipe over 32-row tiles (wave w takes tiles w, w + 4, ...; every
+// The sums run on the matrix pipe over 32-row tiles (wave w takes tiles w, w + NW, ...; every
 // wave's part is added in wave order), in fp32; M1 and M2 go into the second products as hi + lo parts
 // (scaled for fp16, see there).
 // What is left is the memory traffic of the row and its latency.  A training step over n = 512 with
@@ -556,13 +556,13 @@ __global__ __launch_bounds__(bwd_row_waves(KTB) * 64, bwd_row_two_waves(D, KTA) 
     unsigned char* st = tri_smem + OFF_ST + buf * STAGE;
     int lane_now = lane;
     asm volatile("" : "+v"(lane_now));  // (opaque: nothing derived from it is hoisted out of the loop)
-    // the stage is one 64-row tile (Q rows, then dO rows) of G2 wave loads of 1 KiB; every
-    // wave issues the same number of them (with fewer loads than waves some are issued twice)
+    // the stage is one 64-row tile (Q rows, then dO rows) of G2 wave loads of 1 KiB: the same number for
+    // every wave, or, with fewer loads than waves (head dim 16; eight waves), one each for the first G2
     constexpr int G2 = 2 * 32 * Tile::CPR / 64;
     const int jrow = 32 * jt;
 #pragma unroll
     for (int x = 0; x < (G2 + NWV - 1) / NWV; ++x) {
-      if (G2 < NWV && wave >= G2) break;  // (more waves than loads: what these waves have in flight is bias tiles alone)
+      if (G2 < NWV && wave >= G2) break;  // (their counted wait is for nothing of theirs: the barrier behind it stands for the others')
       const int gi = (x * NWV + wave) % G2;
       const bool is_q = gi < G2 / 2;  // wave-uniform
       const T* rows = is_q ? qrow : dorow;
@@ -770,8 +770,7 @@ __global__ __launch_bounds__(bwd_row_waves(KTB) * 64, bwd_row_two_waves(D, KTA) 
   // those three; the wave's own part waits in its dS tile, which is idle between the last key
   // tile of a query tile and the first of the next.  A wave adds its own part first, then the
   // others' in wave order (deterministic, no atomics).
-  // The store is written as asm: a store the compiler knows of makes its waits for loads
-  // waits for everything in flight (stores and loads retire out of order with each other).
+  // The store is written as asm, as one instruction with its base in scalar registers.
   // Addresses are rebuilt from the lane id at every use: kept in registers across the
   // key-tile steps they would be spilled, and a reload from scratch waits for every load
   // in flight.
@@ -957,8 +956,8 @@ __global__ __launch_bounds__(bwd_row_waves(KTB) * 64, bwd_row_two_waves(D, KTA) 
           E::mfma_acc_zero(dvacc[t][mt]);
         }
       }
-    // The wave is alone on its SIMD, so nothing but its own instruction order hides a
-    // latency: the code below is laid out as the schedule it should run in, and scheduling
+    // One wave per SIMD, or two, leave most of hiding a latency to a wave's own instruction
+    // order: the code below is laid out as the schedule it should run in, and scheduling
     // barriers between the pieces keep the compiler from re-ordering it.
     auto SB = [] { __builtin_amdgcn_sched_barrier(0); };
     constexpr int NACC = 2 * PS * DM;  // dv, dk MFMAs of a tile

@@ -1077,7 +1077,9 @@ __global__ __launch_bounds__(512, (2 * LinearDwShape<T, KD, MODE>::PER_CU)) void
     int now = ring, next = end - stage;  // ring buffers of stages s and s + depth - 1
     for (int s = 0; s < steps; ++s) {
       // stage s of this wave has landed once at most the stages s + 1 .. s + depth - 2 are in flight
-      // (and the four stores of each of the depth - 1 stages before this one)
+      // (and the four stores of each of the depth - 1 stages before this one, which are younger than stage s: loads and
+      // stores leave the counter in one order, see ring_sync; gate_bwd's pieces of a row are four stores of the widest kind, no
+      // fewer instructions can make them)
       const int stores = FUSED && wc < KB ? 4 * min(s, depth - 1) : 0;
       wait_loads<0, 40>(s + depth - 1 > steps ? 0 : in_flight + stores);
       finish(s, now, words_tag);

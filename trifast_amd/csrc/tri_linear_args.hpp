@@ -161,7 +161,7 @@ inline int64_t linear_dw_chunks(int64_t rows) {
 
 // The gated output layer's weight gradient and the gate's backward in one launch: o, g and dout are read once
 // for both.  K = 128, 128 outputs: 16384 rows 25.7 -> 23.8 us, 147456 65 -> 44, 2^20 452 -> 281; K = 64, 64 outputs:
-// 16384 rows 18.2 -> 18.8 (and one launch less), 147456 45.6 -> 36.9, 2^20 251 -> 173.  At K = 32 the weight gradient runs
+// 16384 rows 20.2 -> 19.0, 147456 45.6 -> 36.9, 2^20 251 -> 173.  At K = 32 the weight gradient runs
 // two workgroups per CU, which the gate's backward has no registers for (2^20 rows 125 -> 147); at K = 256 two
 // stages and W do not fit LDS.
 inline bool linear_dw_with_gate_bwd(int64_t k) { return k == 64 || k == 128; }

@@ -39,9 +39,13 @@ TRI_DEV void wait_dma_known() {
   asm volatile("" ::: "memory");
 }
 
+// The order every counted wait here relies on: vmcnt counts a wave's vector loads (direct loads into LDS
+// among them) and its stores together, and both leave it in the order of issue, so that "at most n outstanding"
+// means that everything but the newest n has completed.  (The compiler places its own waits on gfx950 by the
+// same rule: a load, two stores, a use of the load give vmcnt(2).)
 // Stage hand-over for a ring of LDS buffers: wait until at most the newest
-// IN_FLIGHT loads of this wave are outstanding (loads complete in issue order, so
-// everything issued before them has landed in LDS) and every LDS read of the wave
+// IN_FLIGHT loads of this wave are outstanding (everything issued before them
+// has landed in LDS) and every LDS read of the wave
 // has returned, then meet the other waves.  A plain barrier instruction: the
 // fence of __syncthreads() would wait for every load in flight.
 template <int IN_FLIGHT>
