@@ -178,19 +178,24 @@ __global__ __launch_bounds__(GJ * GK * 64) void tri_bwd_b_kernel(const BwdArgs a
   // the rows in front of the first fully masked one take the loop of their own below
   constexpr bool kPipelined = WJ == 1 && WK == 2 && NBUF >= 2 && D <= 64;
   // What the rows of the chunk are like: every thread looks at its share of them, the result goes
-  // through words of LDS, which is not yet in use.
+  // through words of LDS, which is not yet in use (scan_words).
   //   * Where the run of fully masked rows at the end of the row range starts (padding; looked for only where
   //     the last row is fully masked: a scan on every launch cost 2 % at n = 704, 5 rounds of 88 rows).
   //     A chunk is a share of the rows in front and a share of the run: rows of the run take about
   //     half the time of the others.
-  //   * (pipelined walk) The first fully masked row of the chunk; whether any other row masks a key of this
-  //     block; which key tiles of the block have an attended key in any row, and which have none in some row.
+  //   * (pipelined walk) The rows from the first to the last with an attended key of this block: the others add
+  //     nothing and are left out (n = 1024, h = 4, d = 32, four parts that attend to themselves: 0.81 -> 0.26 ms; before
+  //     the walk took masked rows 0.75, in the 16-wave block 0.69).
+  //     Of those rows, the first fully masked one; whether any other masks a key of the block; which key tiles of the
+  //     block have an attended key in any of them, and which have none in some.
   uint32_t* scan_words = reinterpret_cast<uint32_t*>(tri_smem);
   if (tid == 0) {
     scan_words[0] = 0;
     scan_words[1] = (uint32_t)N;
-    scan_words[2] = 0;  // key tiles with an attended key in some row; from bit 8 on those with a masked one; from bit 16 on
-                        // those without an attended one in some row
+    scan_words[2] = 0;            // key tiles with an attended key in some row; from bit 8 on those with a masked one; from bit 16
+                                  // on those without an attended one in some row
+    scan_words[3] = (uint32_t)N;  // the first row with an attended key of the block, the row past the last, how many there are
+    scan_words[4] = scan_words[5] = 0;
   }
   __syncthreads();
   const uint32_t* flags = a.rowflag + (int64_t)b * N;
@@ -209,32 +214,65 @@ __global__ __launch_bounds__(GJ * GK * 64) void tri_bwd_b_kernel(const BwdArgs a
     i_end = share_of(run_begin, chunk + 1);
   }
   if constexpr (kPipelined) {
+    // (a wave takes 64 rows side by side: what they are like together is a few scalar instructions)
     uint32_t tiles = 0;
-    for (int i = i_begin + tid; i < i_end; i += NW * 64) {
-      if (flags[i] != 0) {
-        atomicMin(scan_words + 1, (uint32_t)i);
-        tiles |= 0xffu;
-        break;
-      }
-      const uint32_t* kw = a.keep + ((int64_t)b * N + i) * a.nwords;
+    int first = N, last = 0, count = 0, first_flagged = N;
+    for (int i0 = i_begin + wave * 64; i0 < i_end; i0 += NW * 64) {
+      const int i = i0 + lane;
+      const bool flagged = i < i_end && flags[i] != 0;
+      uint32_t live = 0, rest = 0;
+      if (i < i_end && !flagged) {
+        const uint32_t* kw = a.keep + ((int64_t)b * N + i) * a.nwords;
 #pragma unroll
-      for (int w = 0; w < BKB / 32; ++w) {
-        const uint32_t x = k_blk / 32 + w < a.nwords ? kw[k_blk / 32 + w] : 0u;
-        const uint32_t past = past_end(k_blk / 32 + w);
-        tiles |= (x != 0 ? 1u << w : past != 0xffffffffu ? 0x10000u << w : 0u) | ((x | past) != 0xffffffffu ? 0x100u << w : 0u);
+        for (int w = 0; w < BKB / 32; ++w) {
+          const uint32_t x = k_blk / 32 + w < a.nwords ? kw[k_blk / 32 + w] : 0u;
+          const uint32_t past = past_end(k_blk / 32 + w);
+          live |= x != 0 ? 1u << w : 0u;
+          rest |= (x == 0 && past != 0xffffffffu ? 0x10000u << w : 0u) | ((x | past) != 0xffffffffu ? 0x100u << w : 0u);
+        }
       }
+      const uint64_t fl = __ballot(flagged), lv = __ballot(flagged || live != 0);
+      if (fl != 0) {
+        first_flagged = min(first_flagged, i0 + __builtin_ctzll(fl));
+        tiles |= 0xffu;
+      }
+      if (lv != 0) {
+        first = min(first, i0 + __builtin_ctzll(lv));
+        last = i0 + 64 - __builtin_clzll(lv);
+        count += __builtin_popcountll(lv);
+      }
+      const uint32_t t = live != 0 ? live | rest : 0u;
+#pragma unroll
+      for (int w = 0; w < BKB / 32; ++w)
+#pragma unroll
+        for (int f = 0; f < 3; ++f) tiles |= __ballot((t >> (8 * f + w) & 1u) != 0) != 0 ? 1u << (8 * f + w) : 0u;
     }
-    if (tiles) atomicOr(scan_words + 2, tiles);
+    if (lane == 0 && count != 0) {
+      atomicMin(scan_words + 1, (uint32_t)first_flagged);
+      atomicOr(scan_words + 2, tiles);
+      atomicMin(scan_words + 3, (uint32_t)first);
+      atomicMax(scan_words + 4, (uint32_t)last);
+      atomicAdd(scan_words + 5, (uint32_t)count);
+    }
   }
   __syncthreads();
   // (pinned to scalar registers: the branches of the walk must be real ones, see compute_row)
   i_begin = __builtin_amdgcn_readfirstlane(i_begin);
   run_begin = __builtin_amdgcn_readfirstlane(run_begin);
+  uint32_t block_tiles = 0xffu;
+  if constexpr (kPipelined) {
+    block_tiles = __builtin_amdgcn_readfirstlane(scan_words[2]);
+    const int count = __builtin_amdgcn_readfirstlane((int)scan_words[5]);
+    if (count != 0) {
+      i_begin = __builtin_amdgcn_readfirstlane((int)scan_words[3]);
+      i_end = __builtin_amdgcn_readfirstlane((int)scan_words[4]);
+      if (count != i_end - i_begin) block_tiles |= 0xffff00u;  // rows without an attended key among them
+    }
+  }
   int nrows = __builtin_amdgcn_readfirstlane(i_end) - i_begin;
   const int tail_begin = run_begin + share_of(N - run_begin, chunk), tail_end = run_begin + share_of(N - run_begin, chunk + 1);
   // rows that take the pipelined walk, and the block's key tiles (see scan_words)
   int nwalk = kPipelined ? __builtin_amdgcn_readfirstlane(min((int)scan_words[1] - i_begin, nrows)) : 0;
-  const uint32_t block_tiles = kPipelined ? __builtin_amdgcn_readfirstlane(scan_words[2]) : 0xffu;
   if ((block_tiles & 0xffu) == 0) nrows = nwalk = 0;  // no attended key in any row: dS = 0
   __syncthreads();
 
@@ -770,8 +808,8 @@ __global__ __launch_bounds__(GJ * GK * 64) void tri_bwd_b_kernel(const BwdArgs a
         // A tile without an attended key (`attended`: the keep word of the tile before) adds nothing: dS = 0 whatever its K and V
         // rows and its bias hold.  Where they are infinite or NaN, as padding may be, zero probabilities
         // times their dP are not zero.  Its elementwise work is skipped, a branch per step, in a loop of its own for waves
-        // with such a tile (n = 1024, d = 32, four blocks of keys that attend to themselves: 0.81 ms, 1.19 done on zeros;
-        // with the branches in every masked loop n = 2048 with 5 % masked 8.24 -> 8.5 ms from a cool chip).  In rows of
+        // with such a tile (n = 1024, d = 32, four parts that attend to themselves with all rows walked: 0.81 ms, 1.19 done on
+        // zeros; with the branches in every masked loop n = 2048 with 5 % masked 8.24 -> 8.5 ms from a cool chip).  In rows of
         // 128 bytes a second masked loop leaves the compiler spilling in the first: there the work is done on zeros, one
         // branch per tile in the one loop (n = 768, h = 8 with half of the keys masked: 1.61 ms, as without it).
         uint32_t adds = 1u;
