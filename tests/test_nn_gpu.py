@@ -222,6 +222,9 @@ def test_weight_gradients_of_several_layers(dtype, k, ns, n, hd, swap):
     (torch.float16, 128, [32, 33, 5, 20], 257, 32, False),          # one group: whole pieces, wide words, narrow words, 4 bytes
     (torch.bfloat16, 32, [32, 7, 64], 300, 0, True),
     (torch.float16, 64, [97, 4], 257, 0, False),                    # wide words: the narrow layer does not ride
+    (torch.bfloat16, 128, [7, 96, 4], 211, 32, True),               # words next to whole pieces, and a riding layer
+    (torch.float16, 64, [100, 4], 257, 0, True),                    # 4 bytes at a time, a last block in words, a riding layer
+    (torch.bfloat16, 32, [13, 96, 10], 300, 32, False),
     (torch.bfloat16, 64, [128, 128, 128, 64, 33], 151, 32, True),   # wide words next to whole pieces, two groups of them
     (torch.bfloat16, 256, [5, 160, 4], 150, 32, False),             # words first, the last block of its group
 ])
