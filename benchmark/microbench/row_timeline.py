@@ -9,7 +9,8 @@ the benchmark's workload and prints, per workgroup and per compute unit:
 
 * prologue / loop / epilogue / gap to the next workgroup on the same compute unit (us),
 * when the prologue's loads were issued, when V had arrived, when delta was done,
-* shader clocks per step of a query tile (step -1 starts tile 0, step KT finishes tile KT-1),
+* shader clocks per step of a query tile (step -1 starts tile 0, step KT finishes tile KT-1; short rows have
+  steps 0 .. KT-1 alone, each starting the next pair and finishing the one before),
   per partial-tile store and per barrier, and the shader clock rate inside the loop.
 
     python3 benchmark/microbench/row_timeline.py [--workload M] [--lib PATH]
@@ -82,6 +83,9 @@ def main():
     e.synchronize()
     info = _lib.tile_info(_lib.KERNEL_BWD_KV, tile)
     KT = info["BLOCK_K"] // 128
+    short = d <= 32 and n <= 512  # (tri_bwd_row_short.hpp: one wave, or two)
+    if short:
+        KT = (n + 31) // 32 if n <= 256 else ((n + 31) // 32 + 1) // 2
     print(f"workload {args.workload}: row-resident tile {tile} of {kt} ({KT} key tiles per wave), timing build: {s.elapsed_time(e):.3f} ms per launch")
 
     rec = rec_buf[: rows * 32].view(rows, 32).cpu()
@@ -115,7 +119,11 @@ def main():
     loop_us = us(5, 6)
     print(f"shader clock inside the loop: {float((clocks / loop_us).mean()):.0f} MHz")
     nj = (n + 31) // 32
-    names = ["before step -1"] + [f"step {t}" for t in range(-1, KT + 1)] + ["partial-tile store", "barrier"]
+    if short:
+        # (step 0's end has slots of its own)
+        names = [f"step {KT - 1}", "behind the barrier"] + [f"step {t}" for t in range(1, KT - 1)] + ["step 0", "partial-tile store", "barrier"]
+    else:
+        names = ["before step -1"] + [f"step {t}" for t in range(-1, KT + 1)] + ["partial-tile store", "barrier"]
     print("shader clocks per query tile (mean over the workgroups):")
     total = 0.0
     for idx, name in enumerate(names):

@@ -2,8 +2,8 @@
 // scores and of dP (the dq kernel and the dk/dv kernel each recompute both).
 //
 // Work unit: (batch*head, pair row i), one workgroup of four waves, one wave per
-// SIMD with the whole register file (rows of up to 64 bytes and 512 keys: two per SIMD, of two
-// workgroups or of one of eight waves, see bwd_row_two_waves).  The keys of the row are dealt to the waves
+// SIMD with the whole register file.  (Rows of up to 64 bytes and 512 keys have a kernel of their own, of one or two
+// waves: tri_bwd_row_short.hpp.)  The keys of the row are dealt to the waves
 // in tiles of 32 (wave w owns key tiles w, w+4, ...; at most KT of them): their
 // dk, dv accumulators stay in registers for the whole row, their V rows too (B
 // operands; in a private piece of LDS where the registers do not hold them all), and
@@ -90,17 +90,20 @@ struct RowSched {
   int last_sqk;      // the last MFMA that reads the K rows of the next tile
   int v_reads_at;    // V operands kept in LDS are read after this MFMA
   int last_sb;       // the last MFMA that reads bias words (0 without any)
+  int last_acc;      // the last dv/dk MFMA (-1 without any)
 };
 // Two dependent chains start a tile (scores: per-query offset and key mask, bias parts,
 // q.k; dP: -delta, dO.v) and three finish the one before (dv/dk, dq).  Dependent MFMAs are
 // kept apart: first the head of the score chain alternates with the dv/dk MFMAs, then dq,
-// the q.k part and the dP chain take turns.
-constexpr RowSched make_row_sched(bool has_prev, bool has_next, int nsb, int ds, int nacc, int ndq) {
+// the q.k part and the dP chain take turns.  (delta_early: -delta stands behind the bias parts instead, three MFMAs in front of the
+// first that adds to it.)
+constexpr RowSched make_row_sched(bool has_prev, bool has_next, int nsb, int ds, int nacc, int ndq, bool delta_early) {
   RowSched s{};
   s.dq_reads_at = -1;
   s.last_sqk = -1;
   s.v_reads_at = -1;
   s.last_sb = 0;
+  s.last_acc = -1;
   int lk[16] = {}, li[16] = {}, ns = 0;
   if (has_next) {
     lk[ns] = R_SOFF;
@@ -108,6 +111,10 @@ constexpr RowSched make_row_sched(bool has_prev, bool has_next, int nsb, int ds,
     for (int i = 0; i < nsb; ++i) {
       lk[ns] = R_SB;
       li[ns++] = i;
+    }
+    if (delta_early) {
+      lk[ns] = R_DOFF;
+      li[ns++] = 0;
     }
   }
   const int na = has_prev ? nacc : 0;
@@ -124,12 +131,13 @@ constexpr RowSched make_row_sched(bool has_prev, bool has_next, int nsb, int ds,
       s.idx[s.n++] = li[is++];
     }
     if (ia < na) {
+      s.last_acc = s.n;
       s.kind[s.n] = R_ACC;
       s.idx[s.n++] = ia++;
     }
   }
   const int nq = has_prev ? ndq : 0, nk = has_next ? ds : 0, np = has_next ? 1 + ds : 0;
-  int iq = 0, ik = 0, ip = 0, first_dq = -1;
+  int iq = 0, ik = 0, ip = delta_early ? 1 : 0, first_dq = -1;
   while (iq < nq || ik < nk || ip < np) {
     if (iq < nq) {
       if (first_dq < 0) first_dq = s.n;
@@ -151,9 +159,9 @@ constexpr RowSched make_row_sched(bool has_prev, bool has_next, int nsb, int ds,
   if (first_dq >= 0) s.dq_reads_at = first_dq >= 3 ? first_dq - 3 : 0;
   return s;
 }
-template <bool HAS_PREV, bool HAS_NEXT, int NSB, int DS, int NACC, int NDQ>
+template <bool HAS_PREV, bool HAS_NEXT, int NSB, int DS, int NACC, int NDQ, bool DELTA_EARLY = false>
 struct RowSchedOf {
-  static constexpr RowSched value = make_row_sched(HAS_PREV, HAS_NEXT, NSB, DS, NACC, NDQ);
+  static constexpr RowSched value = make_row_sched(HAS_PREV, HAS_NEXT, NSB, DS, NACC, NDQ, DELTA_EARLY);
 };
 
 // Key tiles per wave whose V operands live in LDS instead of registers: the longest rows
@@ -161,31 +169,25 @@ struct RowSchedOf {
 // (one tile more in LDS when the row takes several passes: the words of the queries then leave
 // LDS the room, and the dq carried between the passes takes registers)
 constexpr int bwd_row_v_lds_tiles(int D, int KT, bool multi = false) { return KT * (D / 16) < 16 ? 0 : D <= 32 ? KT - (multi ? 2 : 3) : 1; }
-// Two waves per SIMD (256 registers each, the accumulators among the ordinary ones) where a wave holds at
-// most two key tiles of rows of up to 64 bytes.  Two workgroups of four waves per compute unit for up to
-// 256 keys: one row's loads and stores, and the waits inside its query tiles, go on beside the other
-// row's arithmetic (h = 4, d = 32: n = 256 71.8 -> 52.1 us, 200 59.7 -> 41.7, 128 23.4 -> 17.8, 77
-// 20.3 -> 15.9; with the accumulators in AGPRs the kernel had 279 registers and one workgroup).  One
-// workgroup of eight waves (KTB > 0, see the kernel) for up to 512.
+// Two waves per SIMD (256 registers each, the accumulators among the ordinary ones), of two workgroups, where a wave holds two key
+// tiles of 64-byte rows (the last pass over a long row).
 constexpr bool bwd_row_two_waves(int D, int KT) { return D <= 32 && KT <= 2; }
-constexpr int bwd_row_waves(int KTB) { return KTB > 0 ? 2 * kRowWaves : kRowWaves; }
 // LDS bytes of the kernel below.  dq partials: two buffers (one barrier per query tile) of
-// three quarters of a tile per wave (the quarter a wave sums itself waits in its dS tile); with eight
-// waves all of every tile
-constexpr int bwd_row_red_bytes(int D, int KTB = 0) { return kRowWaves * (KTB > 0 ? 8 : 3) * ((D + 31) / 32) * 1024; }
-constexpr int bwd_row_base_lds_bytes(int D, int es, int KT, bool multi, int KTB) {  // (without the per-query words)
-  const int rowb = D * es, keys = kRowWaves * (KT + KTB) * 32;
-  return keys * rowb + 3 * (2 * 32 * rowb) + bwd_row_waves(KTB) * 2048 + 2 * bwd_row_red_bytes(D, KTB) +
+// three quarters of a tile per wave (the quarter a wave sums itself waits in its dS tile)
+constexpr int bwd_row_red_bytes(int D) { return kRowWaves * 3 * ((D + 31) / 32) * 1024; }
+constexpr int bwd_row_base_lds_bytes(int D, int es, int KT, bool multi) {  // (without the per-query words)
+  const int rowb = D * es, keys = kRowWaves * KT * 32;
+  return keys * rowb + 3 * (2 * 32 * rowb) + kRowWaves * 2048 + 2 * bwd_row_red_bytes(D) +
          kRowWaves * bwd_row_v_lds_tiles(D, KT, multi) * (D / 16) * 1024;
 }
 // The per-query operand words of the row (two planes of 4 bytes per query) live in LDS where
 // there is room and the row takes one pass; else they come from the global planes that the
 // prologue writes, one query tile ahead.
-constexpr bool bwd_row_words_in_lds(int D, int es, int KT, bool multi, int KTB = 0) {
-  return !multi && bwd_row_base_lds_bytes(D, es, KT, multi, KTB) + 2 * kRowWaves * (KT + KTB) * 32 * 4 <= 160 * 1024;
+constexpr bool bwd_row_words_in_lds(int D, int es, int KT, bool multi) {
+  return !multi && bwd_row_base_lds_bytes(D, es, KT, multi) + 2 * kRowWaves * KT * 32 * 4 <= 160 * 1024;
 }
-constexpr int bwd_row_lds_bytes(int D, int es, int KT, bool multi = false, int KTB = 0) {
-  return bwd_row_base_lds_bytes(D, es, KT, multi, KTB) + (bwd_row_words_in_lds(D, es, KT, multi, KTB) ? 2 * kRowWaves * (KT + KTB) * 32 * 4 : 0);
+constexpr int bwd_row_lds_bytes(int D, int es, int KT, bool multi = false) {
+  return bwd_row_base_lds_bytes(D, es, KT, multi) + (bwd_row_words_in_lds(D, es, KT, multi) ? 2 * kRowWaves * KT * 32 * 4 : 0);
 }
 
 // XCDs that work on a head together: the smallest power of two whose heads side by side (8 / share of
@@ -460,49 +462,39 @@ TRI_DEV void bwd_uniform_row(const BwdArgs& a, int bh, int i, unsigned char* sme
   }
 }
 
-// KTB > 0: eight waves, two per SIMD.  Waves 0..3 hold KTA key tiles, waves 4..7 (which also add up
-// dq) KTB <= KTA.  One wave per SIMD leaves the SIMD idle wherever its own chain waits: at the start of a
-// query tile, behind its barrier, in front of the first scores (with four key tiles 1.8 of 4.7 thousand
-// clocks of a query tile).  Against four waves of KTA + KTB key tiles on one card, h = 4: d = 16 n = 384
-// 150 -> 136 us, 512 326 -> 284; d = 32 n = 300 121 -> 117, 384 176 -> 171, 449 334 -> 329, 512 344 / 344, with
-// padding from 397 on 320 -> 311 (eight waves write twice the dq partials, and they still meet at one
-// barrier per query tile).  Wider rows and more key tiles do not fit 256 registers.
-template <typename T, int D, int KTA, bool MULTI = false, int KTB = 0>
-__global__ __launch_bounds__(bwd_row_waves(KTB) * 64, bwd_row_two_waves(D, KTA) ? 2 : 1) void tri_bwd_row_kernel(const BwdArgs a) {
-  constexpr int KT = KTA;
+template <typename T, int D, int KT, bool MULTI = false>
+__global__ __launch_bounds__(kRowWaves * 64, bwd_row_two_waves(D, KT) ? 2 : 1) void tri_bwd_row_kernel(const BwdArgs a) {
   // (two waves per SIMD: the accumulators are ordinary registers)
   constexpr bool TWO = bwd_row_two_waves(D, KT);
-  static_assert(KTB == 0 || (TWO && !MULTI && KTB <= KT), "eight waves: two per SIMD, one pass");
   static_assert(sizeof(T) == 2, "16-bit inputs only (the transposing LDS reads)");
   using E = Elem<T>;
   using frag = typename E::frag;
   using Tile = LdsTile<T, D>;
   using DsTile = LdsTile<T, 32, 2>;  // the wave's dS tile: 16-byte stores of whole rows, transposed reads
-  constexpr int NWV = bwd_row_waves(KTB);  // waves
-  constexpr int NWT = kRowWaves;           // key tiles from one of a wave's tiles to its next
+  constexpr int NW = kRowWaves;
   constexpr int KP = E::KP;
   constexpr int DS = D / (2 * KP);
   constexpr int DM = (D + 31) / 32;
   constexpr int PS = 2;
   constexpr int ROWB = Tile::ROWB;
-  constexpr int KEYS = NWT * (KT + KTB) * 32;         // keys (and queries) the workgroup can hold
-  constexpr bool WORDS_LDS = bwd_row_words_in_lds(D, (int)sizeof(T), KT, MULTI, KTB);  // per-query words of the row in LDS (else from the global planes)
+  constexpr int KEYS = NW * KT * 32;         // keys (and queries) the workgroup can hold
+  constexpr bool WORDS_LDS = bwd_row_words_in_lds(D, (int)sizeof(T), KT, MULTI);  // per-query words of the row in LDS (else from the global planes)
   constexpr int STAGE = 2 * 32 * ROWB;        // Q tile | dO tile
   constexpr int OFF_K = 0;
   constexpr int OFF_ST = KEYS * ROWB;
   constexpr int OFF_DS = OFF_ST + 3 * STAGE;  // three stages: in use, ready, in flight
-  constexpr int OFF_RED = OFF_DS + NWV * 2048;
-  constexpr int OFF_NL = OFF_RED + 2 * bwd_row_red_bytes(D, KTB);
+  constexpr int OFF_RED = OFF_DS + NW * 2048;
+  constexpr int OFF_NL = OFF_RED + 2 * bwd_row_red_bytes(D);
   constexpr int PLANE = WORDS_LDS ? KEYS * 4 : 0;  // per-query words of the row
   constexpr int OFF_ND = OFF_NL + PLANE;
-  constexpr int G2W = (2 * 32 * (ROWB / 16) / 64 + NWV - 1) / NWV;  // global->LDS loads per wave and stage
+  constexpr int G2W = (2 * 32 * (ROWB / 16) / 64 + NW - 1) / NW;  // global->LDS loads per wave and stage
   constexpr int VL = bwd_row_v_lds_tiles(D, KT, MULTI);  // this wave's last VL key tiles keep V in LDS
   constexpr int VR = KT - VL;
   constexpr int OFF_V = OFF_ND + PLANE;
-  static_assert(OFF_V + NWV * VL * DS * 1024 == bwd_row_lds_bytes(D, (int)sizeof(T), KT, MULTI, KTB), "the launcher sizes LDS with bwd_row_lds_bytes");
-  static_assert(bwd_row_lds_bytes(D, (int)sizeof(T), KT, MULTI, KTB) <= 160 * 1024, "LDS of one compute unit");
-  static_assert(bwd_uniform_lds_bytes(D, (int)sizeof(T), NWV) <= bwd_row_lds_bytes(D, (int)sizeof(T), KT, MULTI, KTB), "LDS of a fully masked row");
-  static_assert((KT - 1) * NWT * 32 * ROWB + 32 * ROWB <= 65536, "key tile offsets are LDS immediates");
+  static_assert(OFF_V + NW * VL * DS * 1024 == bwd_row_lds_bytes(D, (int)sizeof(T), KT, MULTI), "the launcher sizes LDS with bwd_row_lds_bytes");
+  static_assert(bwd_row_lds_bytes(D, (int)sizeof(T), KT, MULTI) <= 160 * 1024, "LDS of one compute unit");
+  static_assert(bwd_uniform_lds_bytes(D, (int)sizeof(T), NW) <= bwd_row_lds_bytes(D, (int)sizeof(T), KT, MULTI), "LDS of a fully masked row");
+  static_assert((KT - 1) * NW * 32 * ROWB + 32 * ROWB <= 65536, "key tile offsets are LDS immediates");
   extern __shared__ __attribute__((aligned(16))) unsigned char tri_smem[];
 
   TRI_ROW_MARK(t_entry);
@@ -510,8 +502,6 @@ __global__ __launch_bounds__(bwd_row_waves(KTB) * 64, bwd_row_two_waves(D, KTA) 
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int kl = lane & 31, g = lane >> 5;
-  // this wave's key tiles: first_tile, first_tile + 4, ... of the pass
-  const int first_tile = KTB > 0 && wave >= kRowWaves ? kRowWaves * KT + wave - kRowWaves : wave;
   const int N = a.N;
   const int NJ = a.nwords;  // 32-tiles of the row (queries and keys)
   // this pass: key tiles KT0 .. KT0 + 4 KT - 1 of the row (tiles past the row's end are empty)
@@ -540,7 +530,7 @@ __global__ __launch_bounds__(bwd_row_waves(KTB) * 64, bwd_row_two_waves(D, KTA) 
 
   // ---- prologue -----------------------------------------------------------------
   // K row -> LDS (rows past the end repeat the last key; their keep bits are clear)
-  Tile::template fill<KEYS, NWV>(lds_k, [&](int r) { return krow + (int64_t)min(32 * KT0 + r, N - 1) * a.sk.j; }, wave, lane);
+  Tile::template fill<KEYS, NW>(lds_k, [&](int r) { return krow + (int64_t)min(32 * KT0 + r, N - 1) * a.sk.j; }, wave, lane);
   // query tiles 0 (and 1) -> the two stage buffers
   // (per-lane source pointers for query tile 0, computed once; a tile inside the row adds
   // one uniform offset, the ragged last one clamps the query index)
@@ -557,13 +547,13 @@ __global__ __launch_bounds__(bwd_row_waves(KTB) * 64, bwd_row_two_waves(D, KTA) 
     int lane_now = lane;
     asm volatile("" : "+v"(lane_now));  // (opaque: nothing derived from it is hoisted out of the loop)
     // the stage is one 64-row tile (Q rows, then dO rows) of G2 wave loads of 1 KiB: the same number for
-    // every wave, or, with fewer loads than waves (head dim 16; eight waves), one each for the first G2
+    // every wave, or, with fewer loads than waves (head dim 16), one each for the first G2
     constexpr int G2 = 2 * 32 * Tile::CPR / 64;
     const int jrow = 32 * jt;
 #pragma unroll
-    for (int x = 0; x < (G2 + NWV - 1) / NWV; ++x) {
-      if (G2 < NWV && wave >= G2) break;  // (their counted wait is for nothing of theirs: the barrier behind it stands for the others')
-      const int gi = (x * NWV + wave) % G2;
+    for (int x = 0; x < (G2 + NW - 1) / NW; ++x) {
+      if (G2 < NW && wave >= G2) break;  // (their counted wait is for nothing of theirs: the barrier behind it stands for the others')
+      const int gi = (x * NW + wave) % G2;
       const bool is_q = gi < G2 / 2;  // wave-uniform
       const T* rows = is_q ? qrow : dorow;
       const int64_t stride = is_q ? a.sq.j : a.sdo.j;
@@ -585,19 +575,19 @@ __global__ __launch_bounds__(bwd_row_waves(KTB) * 64, bwd_row_two_waves(D, KTA) 
   if (uniform_word(a.rowflag, b * N + i) != 0) {
     wait_dma();  // (the loads on their way into the LDS it uses)
     __syncthreads();
-    if (first_pass) bwd_uniform_row<T, D, NWV>(a, bh, i, tri_smem, wave, lane);
+    if (first_pass) bwd_uniform_row<T, D, NW>(a, bh, i, tri_smem, wave, lane);
     return;
   }
   // keep words of this wave's key tiles (bit k set = key k of the tile is attended)
   uint32_t kw[KT];
 #pragma unroll
   for (int t = 0; t < KT; ++t) {
-    const int kt = KT0 + NWT * t + first_tile;
+    const int kt = KT0 + NW * t + wave;
     kw[t] = uniform_word(a.keep, (b * N + i) * a.nwords + min(kt, NJ - 1));
   }
 #pragma unroll
   for (int t = 0; t < KT; ++t)
-    if (KT0 + NWT * t + first_tile >= NJ) kw[t] = 0u;
+    if (KT0 + NW * t + wave >= NJ) kw[t] = 0u;
   TRI_ROW_MARK(t_p1);
   const uint32_t lanebit = 1u << kl;
 
@@ -611,19 +601,19 @@ __global__ __launch_bounds__(bwd_row_waves(KTB) * 64, bwd_row_two_waves(D, KTA) 
   frag vx[KT][DS];
 #pragma unroll
   for (int t = 0; t < KT; ++t) {
-    const int key = min(32 * (KT0 + NWT * t + first_tile) + kl, N - 1);
+    const int key = min(32 * (KT0 + NW * t + wave) + kl, N - 1);
 #pragma unroll
     for (int s = 0; s < DS; ++s) vx[t][s] = *reinterpret_cast<const frag*>(vrow + (int64_t)key * a.sv.j + 2 * KP * s + KP * g);
   }
   const T* const orow = reinterpret_cast<const T*>(a.o) + ((int64_t)bh * N + i) * N * D;
   const float* const lserow = a.lse + ((int64_t)bh * N + i) * N;
-  constexpr int NIT = WORDS_LDS ? (KEYS + NWV * 64 - 1) / (NWV * 64) : 1;  // queries per thread (single pass)
+  constexpr int NIT = WORDS_LDS ? (KEYS + NW * 64 - 1) / (NW * 64) : 1;  // queries per thread (single pass)
   typename E::vec ov[NIT][D / 8], dv[NIT][D / 8];
   float lv[NIT];
   if constexpr (WORDS_LDS) {
 #pragma unroll
     for (int it = 0; it < NIT; ++it) {
-      const int jc = min(tid + it * NWV * 64, N - 1);
+      const int jc = min(tid + it * NW * 64, N - 1);
 #pragma unroll
       for (int s = 0; s < D / 8; ++s) {
         ov[it][s] = *reinterpret_cast<const typename E::vec*>(orow + (int64_t)jc * D + 8 * s);
@@ -665,16 +655,16 @@ __global__ __launch_bounds__(bwd_row_waves(KTB) * 64, bwd_row_two_waves(D, KTA) 
     if constexpr (WORDS_LDS) {
 #pragma unroll
       for (int it = 0; it < NIT; ++it) {
-        const int j = tid + it * NWV * 64;
+        const int j = tid + it * NW * 64;
         float dsum = 0.f;
 #pragma unroll
         for (int s = 0; s < D / 8; ++s)
 #pragma unroll
           for (int e = 0; e < 8; ++e) dsum += (float)ov[it][s][e] * (float)dv[it][s][e];
-        if (KEYS % (NWV * 64) == 0 || j < KEYS) query_words(j, dsum, lv[it]);
+        if (KEYS % (NW * 64) == 0 || j < KEYS) query_words(j, dsum, lv[it]);
       }
     } else {
-      for (int j = tid; j < N; j += NWV * 64) {
+      for (int j = tid; j < N; j += NW * 64) {
         float dsum = 0.f;
 #pragma unroll
         for (int s = 0; s < D / 8; ++s) {
@@ -707,7 +697,7 @@ __global__ __launch_bounds__(bwd_row_waves(KTB) * 64, bwd_row_two_waves(D, KTA) 
   OperandOffsets<T, D> ofq, ofk;
   ofq.init(perm32(kl), lane);
   ofk.init(kl, lane);
-  ofk.shift(first_tile * 32 * ROWB);  // key tile t of this wave starts (4 t + first_tile) * 32 rows into K
+  ofk.shift(wave * 32 * ROWB);  // key tile t of this wave starts (4 t + wave) * 32 rows into K
   OperandOffsets<T, 32, 2> ofd;
   ofd.init(0, lane);
   // (one tile: the wave reads dS of a key tile back before it writes the next one)
@@ -723,7 +713,7 @@ __global__ __launch_bounds__(bwd_row_waves(KTB) * 64, bwd_row_two_waves(D, KTA) 
   uint32_t bias_lane = (uint32_t)((perm32(kl) + 32 * g) * 8 * sizeof(T));
   asm volatile("" : "+v"(bias_lane));
   auto bias_load = [&](int jt, int t, u32x4v* dst) {
-    const int kt = min(KT0 + NWT * t + first_tile, a.NP - 1);
+    const int kt = min(KT0 + NW * t + wave, a.NP - 1);
     const char* tile = reinterpret_cast<const char*>(pack_bh + ((int64_t)min(jt, a.NP - 1) * a.NP + kt) * 1024);
     uint32_t vo = bias_lane;
     asm volatile("" : "+v"(vo));  // (opaque here: the sum of the lane offset and the head's base is not hoisted as a 64-bit vector)
@@ -775,19 +765,17 @@ __global__ __launch_bounds__(bwd_row_waves(KTB) * 64, bwd_row_two_waves(D, KTA) 
   // key-tile steps they would be spilled, and a reload from scratch waits for every load
   // in flight.
   static_assert(DM * 1024 <= 2048, "the own quarter of a dq tile fits the wave's dS tile");
-  constexpr int RED_BYTES = bwd_row_red_bytes(D, KTB);
+  constexpr int RED_BYTES = bwd_row_red_bytes(D);
   // byte offsets in LDS, all wave-uniform and the same for every query tile: where this wave
   // leaves quarter q of its tile (per buffer), where its own quarter waits, and where the other
   // waves leave their parts of its quarter (three slots side by side)
-  // (Eight waves: all parts of a quarter side by side, in wave order, and wave 4 + q sums quarter q.)
-  const int quarter = KTB > 0 ? wave & (kRowWaves - 1) : wave;
   int part_wr[2][kRowWaves];
 #pragma unroll
   for (int q = 0; q < kRowWaves; ++q)
 #pragma unroll
     for (int bf = 0; bf < 2; ++bf)
-      part_wr[bf][q] = KTB > 0 ? OFF_RED + bf * RED_BYTES + (q * NWV + wave) * DM * 1024 : q == wave ? OFF_DS + wave * 2048 : OFF_RED + bf * RED_BYTES + (q * 3 + (wave < q ? wave : wave - 1)) * DM * 1024;
-  const int part_own = OFF_DS + wave * 2048, part_rd = OFF_RED + quarter * (KTB > 0 ? NWV : 3) * DM * 1024;
+      part_wr[bf][q] = q == wave ? OFF_DS + wave * 2048 : OFF_RED + bf * RED_BYTES + (q * 3 + (wave < q ? wave : wave - 1)) * DM * 1024;
+  const int part_own = OFF_DS + wave * 2048, part_rd = OFF_RED + wave * 3 * DM * 1024;
   T* dqrow = reinterpret_cast<T*>(a.dq) + b * a.sdq.b + h * a.sdq.h + i * a.sdq.i;
   T* lorow = reinterpret_cast<T*>(a.dq_lo) + ((int64_t)bh * N + i) * N * D;  // (several passes only)
   typedef uint32_t u32x2v __attribute__((ext_vector_type(2)));
@@ -822,21 +810,12 @@ __global__ __launch_bounds__(bwd_row_waves(KTB) * 64, bwd_row_two_waves(D, KTA) 
       }
   };
   // the four parts of this wave's quarter: its own, then the other waves' in wave order
-  // (eight waves: four parts at a time)
   struct DqParts {
     f32x4 v[4][DM];
   };
-  auto load_partials = [&](int buf, DqParts& pp, int half = 0) {
+  auto load_partials = [&](int buf, DqParts& pp) {
     int ln = lane;
     asm volatile("" : "+v"(ln));
-    if constexpr (KTB > 0) {
-      const f32x4* parts = reinterpret_cast<const f32x4*>(tri_smem + part_rd + (buf ? RED_BYTES : 0)) + ln;
-#pragma unroll
-      for (int k = 0; k < 4; ++k)
-#pragma unroll
-        for (int mt = 0; mt < DM; ++mt) pp.v[k][mt] = parts[((4 * half + k) * DM + mt) * 64];
-      return;
-    }
     const f32x4* own = reinterpret_cast<const f32x4*>(tri_smem + part_own) + ln;
     const f32x4* others = reinterpret_cast<const f32x4*>(tri_smem + part_rd + (buf ? RED_BYTES : 0)) + ln;
 #pragma unroll
@@ -856,19 +835,8 @@ __global__ __launch_bounds__(bwd_row_waves(KTB) * 64, bwd_row_two_waves(D, KTA) 
     u32x2v hi[DM], lo[DM];
     uint32_t off;
   };
-  constexpr int kSumPieces = KTB > 0 ? 8 : 6;
+  constexpr int kSumPieces = 6;
   auto sum_dq_piece = [&](int piece, int jt, DqParts& pp, const DqCarry& cy, DqOut& o) {
-    if constexpr (KTB > 0) {
-      if (piece == 3 || piece == 4) {
-#pragma unroll
-        for (int mt = 0; mt < DM; ++mt) {
-          if (piece == 3) o.sum[mt] = (o.sum[mt] + pp.v[0][mt]) + pp.v[1][mt];
-          else o.sum[mt] = (o.sum[mt] + pp.v[2][mt]) + pp.v[3][mt];
-        }
-        return;
-      }
-      if (piece > 4) piece -= 2;
-    }
     if (piece == 0) {
 #pragma unroll
       for (int mt = 0; mt < DM; ++mt) o.sum[mt] = pp.v[0][mt] + pp.v[1][mt];
@@ -903,7 +871,7 @@ __global__ __launch_bounds__(bwd_row_waves(KTB) * 64, bwd_row_two_waves(D, KTA) 
     } else {
       int ln = lane;
       asm volatile("" : "+v"(ln));
-      const int jl = ln & 31, d0 = 8 * quarter + 4 * (ln >> 5);
+      const int jl = ln & 31, d0 = 8 * wave + 4 * (ln >> 5);
       const bool live = jt >= 0 && jl < N - 32 * jt && d0 < D;
       // (row strides of the gradients are below 2^24 elements, like those of the inputs)
       o.off = live ? (__umul24((uint32_t)jl, (uint32_t)a.sdq.j) + (uint32_t)d0) * (uint32_t)sizeof(T) : ~0u;
@@ -915,7 +883,7 @@ __global__ __launch_bounds__(bwd_row_waves(KTB) * 64, bwd_row_two_waves(D, KTA) 
     if (o.off != ~0u) {
 #pragma unroll
       for (int mt = 0; mt < DM; ++mt) {
-        if (32 * mt + 8 * quarter >= D) continue;  // (wave-uniform; head dims that are no multiple of 32)
+        if (32 * mt + 8 * wave >= D) continue;  // (wave-uniform; head dims that are no multiple of 32)
         asm volatile("global_store_dwordx2 %0, %1, %2 offset:%3" : : "v"(o.off), "v"(o.hi[mt]), "s"(base), "n"(64 * mt) : "memory");
         if constexpr (MULTI) {
           if (!last_pass) {
@@ -938,10 +906,8 @@ __global__ __launch_bounds__(bwd_row_waves(KTB) * 64, bwd_row_two_waves(D, KTA) 
   // tiles attended (no mask work) and some keys masked out.  Inside a query tile the key tiles run as a software pipeline: the score
   // and dP MFMAs of tile t+1 are issued before the exponentials of tile t, and the dq
   // MFMAs of tile t-1 (whose dS has been through LDS by then) after them.
-  // (eight waves: in two versions each, for the waves that sum dq and for the others)
-  auto query_tiles = [&](auto masked_tag, auto tiles_tag, auto sums_tag) __attribute__((always_inline)) {
-    constexpr bool MASKED = decltype(masked_tag)::value, SUMS = decltype(sums_tag)::value;
-    constexpr int KT = decltype(tiles_tag)::value;  // this wave's key tiles
+  auto query_tiles = [&](auto masked_tag) __attribute__((always_inline)) {
+    constexpr bool MASKED = decltype(masked_tag)::value;
     // (each version has its own accumulators, from zeroing to the final stores: merging
     // the versions' accumulators where they meet would copy all of them)
     f32x16 dkacc[KT][DM], dvacc[KT][DM];
@@ -971,7 +937,7 @@ __global__ __launch_bounds__(bwd_row_waves(KTB) * 64, bwd_row_two_waves(D, KTA) 
       bias_load(jt + t / KT, t % KT, bias_ring[(t % KT) % 2]);
     };
     fetch_bias(0, 0);
-    if constexpr (KT > 1) fetch_bias(0, 1);  // (a wave of one key tile fetches its next one behind its first step's last use)
+    fetch_bias(0, 1);
     uint32_t lw_next = 0u, dw_next = 0u;  // words from the global planes: those of the next query tile
     if constexpr (!WORDS_LDS) fetch_words(0, lw_next, dw_next);
     DqCarry carry;
@@ -1035,7 +1001,7 @@ __global__ __launch_bounds__(bwd_row_waves(KTB) * 64, bwd_row_two_waves(D, KTA) 
       frag dst_prev[PS], ktr_prev[DM][PS];
       frag vn[DS];           // V operands of the next tile when they live in LDS
       auto load_kn = [&](int t) {
-        const unsigned char* ktile = lds_k + NWT * t * 32 * ROWB;
+        const unsigned char* ktile = lds_k + NW * t * 32 * ROWB;
 #pragma unroll
         for (int s = 0; s < DS; ++s) kn[s] = ofk.natural(ktile, s);
       };
@@ -1062,7 +1028,7 @@ __global__ __launch_bounds__(bwd_row_waves(KTB) * 64, bwd_row_two_waves(D, KTA) 
         // (words from the global planes: those of the next query tile, fetched before the last
         // bias tile of this one so that no wait for them is a wait for everything in flight)
         if constexpr (!WORDS_LDS && t == KT - 1) fetch_words(jt + 1, lw_next, dw_next);
-        if constexpr (KT > 1 && valu && !refill) fetch_bias(jt, t + 2);
+        if constexpr (valu && !refill) fetch_bias(jt, t + 2);
         frag kb = keys_op.plain();
         if constexpr (has_next && MASKED) kb = keys_op.masked(kw[tn]);
         SB();
@@ -1079,10 +1045,6 @@ __global__ __launch_bounds__(bwd_row_waves(KTB) * 64, bwd_row_two_waves(D, KTA) 
             dsf[u - 14] = E::pack(&ds[KP * (u - 14)]);
           }
         };
-        if constexpr (NM == 0) {  // (the one key tile of the wave: nothing beside it)
-#pragma unroll
-          for (int u = 0; u < NU; ++u) unit(u);
-        }
         static_for<NM>([&](auto xc) __attribute__((always_inline)) {
           constexpr int x = decltype(xc)::value;
           constexpr int kind = Sch::value.kind[x], idx = Sch::value.idx[x];
@@ -1117,14 +1079,11 @@ __global__ __launch_bounds__(bwd_row_waves(KTB) * 64, bwd_row_two_waves(D, KTA) 
           // not stored).  No wait for a load that could follow within the time a store takes
           // allows fewer than two operations in flight, so none of them waits for this store
           // (a wait for loads issued after a store is a wait for the store as well).
-          if constexpr (t == -1 && SUMS) {
+          if constexpr (t == -1) {
             if constexpr (x == 0) load_partials((jt + 1) & 1, parts);
 #pragma unroll
             for (int piece = 0; piece < kSumPieces; ++piece)
-              if ((piece + 3 < NM ? piece + 3 : NM - 1) == x) {
-                sum_dq_piece(piece, jt - 1, parts, carry, dq_words);
-                if (KTB > 0 && piece == 2) load_partials((jt + 1) & 1, parts, 1);
-              }
+              if ((piece + 3 < NM ? piece + 3 : NM - 1) == x) sum_dq_piece(piece, jt - 1, parts, carry, dq_words);
             if constexpr (x == NM - 1) {
               store_dq(jt - 1, dq_base, dq_words);
               if (jt > 0) dq_base += 32 * a.sdq.j;
@@ -1136,7 +1095,7 @@ __global__ __launch_bounds__(bwd_row_waves(KTB) * 64, bwd_row_two_waves(D, KTA) 
           if constexpr (has_prev && x == Sch::value.dq_reads_at) {
             // dS of tile t-1 comes back from LDS with the key index in-lane, with the K
             // rows of that tile transposed beside it
-            const unsigned char* ktile = lds_k + NWT * tp * 32 * ROWB;
+            const unsigned char* ktile = lds_k + NW * tp * 32 * ROWB;
 #pragma unroll
             for (int s2 = 0; s2 < PS; ++s2) {
               dst_prev[s2] = ofd.transposed(ds_tile, s2, 0);
@@ -1181,15 +1140,12 @@ __global__ __launch_bounds__(bwd_row_waves(KTB) * 64, bwd_row_two_waves(D, KTA) 
       TRI_ROW_TICK(KT + 4);
       buf = buf == 2 ? 0 : buf + 1;
     }
-    if constexpr (SUMS) {
+    {
       DqParts parts;
       DqOut dq_words;
       load_partials((NJ - 1) & 1, parts);
 #pragma unroll
-      for (int piece = 0; piece < kSumPieces; ++piece) {
-        sum_dq_piece(piece, NJ - 1, parts, carry, dq_words);
-        if (KTB > 0 && piece == 2) load_partials((NJ - 1) & 1, parts, 1);
-      }
+      for (int piece = 0; piece < kSumPieces; ++piece) sum_dq_piece(piece, NJ - 1, parts, carry, dq_words);
       store_dq(NJ - 1, dq_base, dq_words);
     }
 #ifdef TRI_ROW_TIMING
@@ -1203,7 +1159,7 @@ __global__ __launch_bounds__(bwd_row_waves(KTB) * 64, bwd_row_two_waves(D, KTA) 
     T* dvrow = reinterpret_cast<T*>(a.dv) + b * a.sdv.b + h * a.sdv.h + i * a.sdv.i;
   #pragma unroll
     for (int t = 0; t < KT; ++t) {
-      const int key = 32 * (KT0 + NWT * t + first_tile) + kl;
+      const int key = 32 * (KT0 + NW * t + wave) + kl;
   #pragma unroll
       for (int mt = 0; mt < DM; ++mt) {
 #ifndef TRI_MFMA_ACC_BUILTIN
@@ -1232,17 +1188,9 @@ __global__ __launch_bounds__(bwd_row_waves(KTB) * 64, bwd_row_two_waves(D, KTA) 
   };
   bool plain = true;
 #pragma unroll
-  for (int t = 0; t < KT; ++t) plain = plain && (kw[t] == 0xffffffffu || (KTB > 0 && wave >= kRowWaves && t >= KTB));
-  auto version = [&](auto tiles_tag, auto sums_tag) __attribute__((always_inline)) {
-    if (plain) query_tiles(std::false_type{}, tiles_tag, sums_tag);
-    else query_tiles(std::true_type{}, tiles_tag, sums_tag);
-  };
-  if constexpr (KTB > 0) {
-    if (wave < kRowWaves) version(std::integral_constant<int, KT>{}, std::false_type{});
-    else version(std::integral_constant<int, KTB>{}, std::true_type{});
-  } else {
-    version(std::integral_constant<int, KT>{}, std::true_type{});
-  }
+  for (int t = 0; t < KT; ++t) plain = plain && kw[t] == 0xffffffffu;
+  if (plain) query_tiles(std::false_type{});
+  else query_tiles(std::true_type{});
 
 }
 

@@ -2,6 +2,7 @@
 // (one translation unit per type, so that they compile in parallel).
 #pragma once
 #include "tri_bwd_row.hpp"
+#include "tri_bwd_row_short.hpp"
 #include "tri_dispatch.hpp"
 
 namespace tri {
@@ -9,20 +10,57 @@ namespace tri {
 // tile index -> key tiles per wave; a workgroup holds rows of up to 128 * KT keys
 constexpr int kRowKT[kBwdRowTiles] = {2, 3, 4, 5, 6, 7, 8, 8};  // (the last one: several passes of 8)
 
+// One launch of the kernel of short rows: NW waves of KT key tiles per row.
+template <typename T, int D, int KT, int NW>
+hipError_t bwd_row_run_short(const BwdArgs& a, int bh, hipStream_t st, bool dry) {
+  if (dry) return hipSuccess;
+  const dim3 grid((unsigned)bwd_row_blocks(bh, a.N));
+  return launch_dyn(tri_bwd_row_short_kernel<T, D, KT, NW>, grid, dim3(NW * 64), bwd_short_lds_bytes(D, (int)sizeof(T), KT, NW), st, a);
+}
+
+// ... and of the one with four waves of KT key tiles.
 template <typename T, int D, int KT>
-hipError_t bwd_row_run(const BwdArgs& a, int bh, hipStream_t st, bool dry) {
-  constexpr int DM = (D + 31) / 32;
-  if (a.N > kRowWaves * KT * 32) return hipErrorInvalidConfiguration;
-  // rows of three and four key tiles for four waves, up to 64 bytes: eight waves of two and of one or two
-  constexpr int KTB = D <= 32 && (KT == 3 || KT == 4) ? KT - 2 : 0, KTA = KT - KTB;
-  constexpr int lds = bwd_row_lds_bytes(D, (int)sizeof(T), KTA, false, KTB);
+hipError_t bwd_row_run_four(const BwdArgs& a, int bh, hipStream_t st, bool dry) {
+  constexpr int DM = (D + 31) / 32, lds = bwd_row_lds_bytes(D, (int)sizeof(T), KT, false);
   // the dk, dv accumulators of a wave's key tiles stay in registers (half of the file at most)
   if constexpr (2 * KT * DM * 16 <= 256 && lds <= kMaxLds) {
     if (dry) return hipSuccess;
     const dim3 grid((unsigned)bwd_row_blocks(bh, a.N));
-    return launch_dyn(tri_bwd_row_kernel<T, D, KTA, false, KTB>, grid, dim3(bwd_row_waves(KTB) * 64), lds, st, a);
+    return launch_dyn(tri_bwd_row_kernel<T, D, KT>, grid, dim3(kRowWaves * 64), lds, st, a);
   } else {
     return hipErrorInvalidConfiguration;
+  }
+}
+
+template <typename T, int D, int KT>
+hipError_t bwd_row_run(const BwdArgs& a, int bh, hipStream_t st, bool dry) {
+  if (a.N > kRowWaves * KT * 32) return hipErrorInvalidConfiguration;
+  if constexpr (D <= 32 && KT == 2) {
+    // Up to 256 keys: one wave with as many key tiles as the row has.  Few rows leave SIMDs without one (256 compute units of four): up
+    // to 512 of them take two waves each where the row has three or four key tiles, and the four waves of the other kernel where it has more
+    // (d = 32, us, one or two waves / four: h = 4, n = 128 17.2 / 18.4; h = 2, n = 200 26.4 / 24.1, 256 30.7 / 30.2; h = 1, n = 256 25.5 / 20.8;
+    // with more rows h = 8, n = 128 23.5 / 29.8; h = 4, n = 200 36.4 / 41.4).
+    if (a.nwords > 2 && (int64_t)bh * a.N <= 512) {
+      if (a.nwords <= 4) return bwd_row_run_short<T, D, 2, 2>(a, bh, st, dry);
+      return bwd_row_run_four<T, D, 2>(a, bh, st, dry);
+    }
+    switch (a.nwords) {
+      case 1:
+      case 2: return bwd_row_run_short<T, D, 2, 1>(a, bh, st, dry);
+      case 3: return bwd_row_run_short<T, D, 3, 1>(a, bh, st, dry);
+      case 4: return bwd_row_run_short<T, D, 4, 1>(a, bh, st, dry);
+      case 5: return bwd_row_run_short<T, D, 5, 1>(a, bh, st, dry);
+      case 6: return bwd_row_run_short<T, D, 6, 1>(a, bh, st, dry);
+      case 7: return bwd_row_run_short<T, D, 7, 1>(a, bh, st, dry);
+      default: return bwd_row_run_short<T, D, 8, 1>(a, bh, st, dry);
+    }
+  } else if constexpr (D <= 32 && KT <= 4) {
+    // up to 384 and 512 keys: two waves, in two sizes each
+    static_assert(kRowWaves * 4 * 32 == kShortRowKeys);
+    if (a.nwords <= 4 * KT - 2) return bwd_row_run_short<T, D, 2 * KT - 1, 2>(a, bh, st, dry);
+    return bwd_row_run_short<T, D, 2 * KT, 2>(a, bh, st, dry);
+  } else {
+    return bwd_row_run_four<T, D, KT>(a, bh, st, dry);
   }
 }
 

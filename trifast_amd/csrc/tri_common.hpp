@@ -460,6 +460,10 @@ TRI_DEV uint32_t uniform_word(const uint32_t* p, int idx) {
 TRI_DEV float pair_sum(bf16x2 w, bf16x2 ones, float acc) { return __builtin_amdgcn_fdot2_f32_bf16(w, ones, acc, false); }
 TRI_DEV float pair_sum(f16x2 w, f16x2 ones, float acc) { return __builtin_amdgcn_fdot2(w, ones, acc, false); }
 
+// acc + the products of two pairs (fp16 by mixed fmas, which keep the type's denormals; bf16's are those of fp32)
+TRI_DEV float pair_dot(bf16x2 x, bf16x2 y, float acc) { return __builtin_amdgcn_fdot2_f32_bf16(x, y, acc, false); }
+TRI_DEV float pair_dot(f16x2 x, f16x2 y, float acc) { return __builtin_fmaf((float)x[1], (float)y[1], __builtin_fmaf((float)x[0], (float)y[0], acc)); }
+
 TRI_DEV f32x16 zero16() {
   f32x16 z;
 #pragma unroll

@@ -171,6 +171,11 @@ struct OperandOffsets {
   // transposed operand (row index in-lane): rows cidx(KP*step.., g), column 32*mt + lane%32
   TRI_DEV frag transposed(const unsigned char* tile, int step, int mt) const {
     if (D % 32 != 0 && 32 * mt + (lane & 31) >= D) return Elem<T>::zero();
+    return transposed_all(tile, step, mt);
+  }
+  // The same without the branch: lanes whose column lies past the end of a row get bytes of the LDS behind it.  For operand rows whose
+  // results nobody uses.
+  TRI_DEV frag transposed_all(const unsigned char* tile, int step, int mt) const {
     return parts([&](int o) {
       const unsigned char* p = tile + 16 * step * Tile::ROWB + o;
       const auto lo = lds_tr4(reinterpret_cast<const P*>(p + tlo[mt]));
