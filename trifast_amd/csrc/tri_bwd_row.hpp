@@ -39,6 +39,13 @@
 // The prologue also computes delta = rowsum(o * do) of the row and leaves it, with
 // the row's log-sum-exp, in the per-query planes the db kernel reads.
 //
+// The loop over the query tiles has no branch: the compiler sinks what stands in front of one behind it, out of the schedule.  Lanes
+// and waves without a share are masked with exec inside asm statements, pointers advance by masked steps, transposing reads past the
+// columns of a short row return bytes nobody uses; nothing of the loop lies in scratch (a reload waits for every load in flight), which
+// is why masked key operands are made in the step and not kept.  Before that, on one card, this kernel alone, h = 4: d = 16, n = 700
+// 786 -> 652 us, n = 1024 1964 -> 1607; d = 32, n = 600 546 -> 530, n = 768 951 -> 939, n = 1024 1995 -> 1980 (bound by issue and clock);
+// d = 64, n = 300 219 -> 195, h = 8, n = 256 240 -> 228, fp16, two of n = 384 with half of the keys masked 1172 -> 1140.
+//
 // Rows up to 128*KT keys fit (1024 keys at head dim 32).  Longer rows run the kernel in
 // several passes (MULTI), one launch per 128*KT keys: dk and dv of a pass's keys are complete
 // after it, dq is the sum over the passes and travels from one to the next as two numbers of
@@ -501,6 +508,9 @@ __global__ __launch_bounds__(kRowWaves * 64, bwd_row_two_waves(D, KT) ? 2 : 1) v
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // the lane id for addresses inside the loop: opaque wherever it is used, so that nothing derived from it is hoisted out of the loop
+  // and kept in registers (it would be spilled, and a reload from scratch waits for every load in flight)
+  int lane_o = lane;
   const int kl = lane & 31, g = lane >> 5;
   const int N = a.N;
   const int NJ = a.nwords;  // 32-tiles of the row (queries and keys)
@@ -542,33 +552,51 @@ __global__ __launch_bounds__(kRowWaves * 64, bwd_row_two_waves(D, KT) ? 2 : 1) v
   // a load it does not know of only makes the counter it waits on larger.  (The source
   // addresses are rebuilt from the lane id every time: kept in registers from one query tile
   // to the next they would be spilled, and a reload from scratch waits for every load in flight.)
-  auto issue_stage = [&](int jt, int buf) {
-    unsigned char* st = tri_smem + OFF_ST + buf * STAGE;
-    int lane_now = lane;
-    asm volatile("" : "+v"(lane_now));  // (opaque: nothing derived from it is hoisted out of the loop)
-    // the stage is one 64-row tile (Q rows, then dO rows) of G2 wave loads of 1 KiB: the same number for
-    // every wave, or, with fewer loads than waves (head dim 16), one each for the first G2
-    constexpr int G2 = 2 * 32 * Tile::CPR / 64;
-    const int jrow = 32 * jt;
+  // (No branch: what stands in front of one is sunk behind it by the compiler, out of the schedule of the loop below.)
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(TRI_L3 unsigned char*)tri_smem;
+  // the stage is two tiles (Q rows, dO rows) of LT wave loads of 1 KiB, dealt to the waves in turn: GX loads for each, or, with fewer
+  // loads than waves (head dim 16), one each for the first; fill[] are the first rows of the next stage to request, per load
+  constexpr int LT = 32 * Tile::CPR / 64, GX = (2 * LT + NW - 1) / NW;
+  const T* fill[GX];
+  int64_t fill_step[GX];
+  uint32_t fill_row[GX];  // bytes between rows (below 2^24: a limit of the entry points)
 #pragma unroll
-    for (int x = 0; x < (G2 + NW - 1) / NW; ++x) {
-      if (G2 < NW && wave >= G2) break;  // (their counted wait is for nothing of theirs: the barrier behind it stands for the others')
-      const int gi = (x * NW + wave) % G2;
-      const bool is_q = gi < G2 / 2;  // wave-uniform
-      const T* rows = is_q ? qrow : dorow;
-      const int64_t stride = is_q ? a.sq.j : a.sdo.j;
-      const int p = gi * 64 + lane_now;
-      const int r = p / Tile::CPR, cc = (p % Tile::CPR) ^ Tile::swz(r);
+  for (int x = 0; x < GX; ++x) {
+    const bool is_q = (x * NW + wave) / LT == 0;
+    fill[x] = is_q ? qrow : dorow;
+    const int64_t stride = is_q ? a.sq.j : a.sdo.j;
+    fill_step[x] = 32 * stride;
+    fill_row[x] = (uint32_t)stride * (uint32_t)sizeof(T);
+  }
+  int fill_rows = N - 1;  // the last row of the pair row, counted from them
+  auto issue_stage = [&](int buf) {
+    asm volatile("" : "+v"(lane_o));
+    const uint32_t ln = (uint32_t)lane_o;
+#pragma unroll
+    for (int x = 0; x < GX; ++x) {
+      const int gi = x * NW + wave;
+      const uint32_t r = (uint32_t)(gi % LT * (64 / Tile::CPR)) + ln / Tile::CPR, cc = (ln % Tile::CPR) ^ (uint32_t)Tile::swz((int)r);
       // a 64-bit base per tile (scalar registers) and a 32-bit byte offset per lane; rows past
       // the end of the pair row (last tile only) read the last row again
-      const T* base = rows + (int64_t)jrow * stride;
-      const uint32_t voff = (uint32_t)(min(r & 31, N - 1 - jrow) * (int)stride + cc * Tile::VEC) * (uint32_t)sizeof(T);
-      const uint32_t dst = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(TRI_L3 unsigned char*)(st + gi * 1024));
-      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(dst), "v"(voff), "s"(base) : "memory", "m0");
+      const uint32_t voff = __umul24((uint32_t)min((int)r, fill_rows), fill_row[x]) + 16 * cc;
+      const T* base = fill[x];
+      const uint32_t dst = __builtin_amdgcn_readfirstlane(lds0 + (uint32_t)(OFF_ST + buf * STAGE + gi * 1024));
+      // (waves without a share load with no lane; their counted wait is for nothing of theirs, the barrier behind it stands for the others')
+      if constexpr (2 * LT < NW) {
+        const int mine = __builtin_amdgcn_readfirstlane(gi < 2 * LT ? -1 : 0);
+        asm volatile("s_mov_b32 m0, %0\n\ts_mov_b32 exec_lo, %3\n\ts_mov_b32 exec_hi, %3\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b64 exec, -1" : : "s"(dst), "v"(voff), "s"(base), "s"(mine) : "memory", "m0");
+      } else {
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(dst), "v"(voff), "s"(base) : "memory", "m0");
+      }
     }
+    // (behind the last query tile the last one is requested again, into a stage nobody reads any more)
+    const int more = __builtin_amdgcn_readfirstlane(fill_rows >= 32 ? -1 : 0);
+#pragma unroll
+    for (int x = 0; x < GX; ++x) fill[x] += fill_step[x] & (int64_t)more;
+    fill_rows -= 32 & more;
   };
-  issue_stage(0, 0);
-  issue_stage(min(1, NJ - 1), 1);
+  issue_stage(0);
+  issue_stage(1);
 
   // (a fully masked row goes its own way; these words come through the scalar cache, all in flight together and apart from the
   // vector loads around them)
@@ -711,14 +739,12 @@ __global__ __launch_bounds__(kRowWaves * 64, bwd_row_two_waves(D, KT) ? 2 : 1) v
   // (a tile's address is a wave-uniform base, computed on the scalar unit, plus this lane's
   // constant 32-bit byte offset: no vector arithmetic per tile)
   uint32_t bias_lane = (uint32_t)((perm32(kl) + 32 * g) * 8 * sizeof(T));
-  asm volatile("" : "+v"(bias_lane));
   auto bias_load = [&](int jt, int t, u32x4v* dst) {
     const int kt = min(KT0 + NW * t + wave, a.NP - 1);
     const char* tile = reinterpret_cast<const char*>(pack_bh + ((int64_t)min(jt, a.NP - 1) * a.NP + kt) * 1024);
-    uint32_t vo = bias_lane;
-    asm volatile("" : "+v"(vo));  // (opaque here: the sum of the lane offset and the head's base is not hoisted as a 64-bit vector)
-    dst[0] = *reinterpret_cast<const u32x4v*>(tile + (uint64_t)vo);
-    dst[1] = *reinterpret_cast<const u32x4v*>(tile + (uint64_t)vo + 512 * sizeof(T));
+    asm volatile("" : "+v"(bias_lane));  // (opaque here: the sum of the lane offset and the head's base is not hoisted as a 64-bit vector)
+    dst[0] = *reinterpret_cast<const u32x4v*>(tile + (uint64_t)bias_lane);
+    dst[1] = *reinterpret_cast<const u32x4v*>(tile + (uint64_t)bias_lane + 512 * sizeof(T));
   };
   const float c = a.c;
 
@@ -785,8 +811,8 @@ __global__ __launch_bounds__(kRowWaves * 64, bwd_row_two_waves(D, KT) ? 2 : 1) v
     typename E::vec4 hi[DM], lo[DM];
   };
   auto fetch_carry = [&](int jt, DqCarry& cy) {
-    int ln = lane;
-    asm volatile("" : "+v"(ln));
+    asm volatile("" : "+v"(lane_o));
+    const int ln = lane_o;
     const int j = min(32 * jt + (ln & 31), N - 1);
 #pragma unroll
     for (int mt = 0; mt < DM; ++mt) {
@@ -797,8 +823,8 @@ __global__ __launch_bounds__(kRowWaves * 64, bwd_row_two_waves(D, KT) ? 2 : 1) v
   };
   // this wave's dq tile of a query tile -> LDS, a quarter for each wave that sums one
   auto store_partials = [&](int buf, const f32x16 (&acc)[DM]) {
-    int ln = lane;
-    asm volatile("" : "+v"(ln));
+    asm volatile("" : "+v"(lane_o));
+    const int ln = lane_o;
 #pragma unroll
     for (int q = 0; q < kRowWaves; ++q)
 #pragma unroll
@@ -814,8 +840,8 @@ __global__ __launch_bounds__(kRowWaves * 64, bwd_row_two_waves(D, KT) ? 2 : 1) v
     f32x4 v[4][DM];
   };
   auto load_partials = [&](int buf, DqParts& pp) {
-    int ln = lane;
-    asm volatile("" : "+v"(ln));
+    asm volatile("" : "+v"(lane_o));
+    const int ln = lane_o;
     const f32x4* own = reinterpret_cast<const f32x4*>(tri_smem + part_own) + ln;
     const f32x4* others = reinterpret_cast<const f32x4*>(tri_smem + part_rd + (buf ? RED_BYTES : 0)) + ln;
 #pragma unroll
@@ -826,14 +852,15 @@ __global__ __launch_bounds__(kRowWaves * 64, bwd_row_two_waves(D, KT) ? 2 : 1) v
     }
   };
   // Their sum (the own part first, then the others in wave order), scaled, as the stores will write it: dq, what rounding it to the
-  // element type lost (between the passes over a long row), and this lane's byte offset from
-  // the start of the query tile in dq (~0: nothing to store).  The sum is cut into pieces of a
+  // element type lost (between the passes over a long row), this lane's byte offset from
+  // the start of the query tile in dq, and which lanes store.  The sum is cut into pieces of a
   // few instructions each (piece 0 .. kSumPieces-1, in this order): they run one per MFMA of a
   // step that has no vector work of its own, in the shadow of the matrix pipe.
   struct DqOut {
     f32x4 sum[DM];
     u32x2v hi[DM], lo[DM];
     uint32_t off;
+    uint64_t live;  // the lanes that store
   };
   constexpr int kSumPieces = 6;
   auto sum_dq_piece = [&](int piece, int jt, DqParts& pp, const DqCarry& cy, DqOut& o) {
@@ -849,12 +876,10 @@ __global__ __launch_bounds__(kRowWaves * 64, bwd_row_two_waves(D, KT) ? 2 : 1) v
 #pragma unroll
         for (int e = 0; e < 4; ++e) o.sum[mt][e] *= a.scale;
       if constexpr (MULTI) {
-        if (!first_pass) {
 #pragma unroll
-          for (int mt = 0; mt < DM; ++mt)
+        for (int mt = 0; mt < DM; ++mt)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) o.sum[mt][e] += (float)cy.hi[mt][e] + (float)cy.lo[mt][e];
-        }
+          for (int e = 0; e < 4; ++e) o.sum[mt][e] += (float)cy.hi[mt][e] + (float)cy.lo[mt][e];  // (zeros in the first pass)
       }
     } else if (piece == 4) {
 #pragma unroll
@@ -869,30 +894,27 @@ __global__ __launch_bounds__(kRowWaves * 64, bwd_row_two_waves(D, KT) ? 2 : 1) v
         o.lo[mt] = __builtin_bit_cast(u32x2v, lv);
       }
     } else {
-      int ln = lane;
-      asm volatile("" : "+v"(ln));
+      asm volatile("" : "+v"(lane_o));
+      const int ln = lane_o;
       const int jl = ln & 31, d0 = 8 * wave + 4 * (ln >> 5);
-      const bool live = jt >= 0 && jl < N - 32 * jt && d0 < D;
-      // (row strides of the gradients are below 2^24 elements, like those of the inputs)
-      o.off = live ? (__umul24((uint32_t)jl, (uint32_t)a.sdq.j) + (uint32_t)d0) * (uint32_t)sizeof(T) : ~0u;
+      // (head dims that are no multiple of 32: a quarter past the end has no live lane)
+      o.live = __builtin_amdgcn_ballot_w64((int)(jl < N - 32 * jt) & (int)(d0 < D)) & (jt < 0 ? 0ull : ~0ull);
+      // (row strides of the gradients are below 2^24 bytes, like those of the inputs)
+      o.off = (__umul24((uint32_t)jl, (uint32_t)a.sdq.j) + (uint32_t)d0) * (uint32_t)sizeof(T);
     }
   };
-  // (a 64-bit base per query tile in scalar registers and the 32-bit byte offset of the lane)
+  // (a 64-bit base per query tile in scalar registers and the 32-bit byte offset of the lane; every lane of the wave is active here)
   auto store_dq = [&](int jt, const T* base, const DqOut& o) {
-    const T* base_lo = lorow + (int64_t)(32 * jt) * D;
-    if (o.off != ~0u) {
 #pragma unroll
-      for (int mt = 0; mt < DM; ++mt) {
-        if (32 * mt + 8 * wave >= D) continue;  // (wave-uniform; head dims that are no multiple of 32)
-        asm volatile("global_store_dwordx2 %0, %1, %2 offset:%3" : : "v"(o.off), "v"(o.hi[mt]), "s"(base), "n"(64 * mt) : "memory");
-        if constexpr (MULTI) {
-          if (!last_pass) {
-            int ln = lane;
-            asm volatile("" : "+v"(ln));
-            const uint32_t off_lo = (uint32_t)((ln & 31) * D + 8 * wave + 4 * (ln >> 5)) * (uint32_t)sizeof(T);
-            asm volatile("global_store_dwordx2 %0, %1, %2 offset:%3" : : "v"(off_lo), "v"(o.lo[mt]), "s"(base_lo), "n"(64 * mt) : "memory");
-          }
-        }
+    for (int mt = 0; mt < DM; ++mt) {
+      asm volatile("s_mov_b64 exec, %4\n\tglobal_store_dwordx2 %0, %1, %2 offset:%3\n\ts_mov_b64 exec, -1" : : "v"(o.off), "v"(o.hi[mt]), "s"(base), "n"(64 * mt), "s"(o.live) : "memory");
+      if constexpr (MULTI) {
+        const T* base_lo = lorow + (int64_t)(32 * jt) * D;
+        const uint64_t live_lo = last_pass ? 0ull : o.live;
+        asm volatile("" : "+v"(lane_o));
+        const int ln = lane_o;
+        const uint32_t off_lo = (uint32_t)((ln & 31) * D + 8 * wave + 4 * (ln >> 5)) * (uint32_t)sizeof(T);
+        asm volatile("s_mov_b64 exec, %4\n\tglobal_store_dwordx2 %0, %1, %2 offset:%3\n\ts_mov_b64 exec, -1" : : "v"(off_lo), "v"(o.lo[mt]), "s"(base_lo), "n"(64 * mt), "s"(live_lo) : "memory");
       }
     }
   };
@@ -908,6 +930,11 @@ __global__ __launch_bounds__(kRowWaves * 64, bwd_row_two_waves(D, KT) ? 2 : 1) v
   // MFMAs of tile t-1 (whose dS has been through LDS by then) after them.
   auto query_tiles = [&](auto masked_tag) __attribute__((always_inline)) {
     constexpr bool MASKED = decltype(masked_tag)::value;
+    int masked_bits = 0;  // bit t set: this lane's key of tile t is masked
+    if constexpr (MASKED) {
+#pragma unroll
+      for (int t = 0; t < KT; ++t) masked_bits |= (kw[t] >> kl & 1u ? 0 : 1) << t;
+    }
     // (each version has its own accumulators, from zeroing to the final stores: merging
     // the versions' accumulators where they meet would copy all of them)
     f32x16 dkacc[KT][DM], dvacc[KT][DM];
@@ -938,9 +965,15 @@ __global__ __launch_bounds__(kRowWaves * 64, bwd_row_two_waves(D, KT) ? 2 : 1) v
     };
     fetch_bias(0, 0);
     fetch_bias(0, 1);
-    uint32_t lw_next = 0u, dw_next = 0u;  // words from the global planes: those of the next query tile
-    if constexpr (!WORDS_LDS) fetch_words(0, lw_next, dw_next);
-    DqCarry carry;
+    uint32_t lw_next = 0u, dw_next = 0u;  // the words of the next query tile
+    auto load_words = [&](int jt) {
+      const int j = 32 * min(jt, NJ - 1) + perm32(kl);
+      lw_next = nl[j];
+      dw_next = nd[j];
+    };
+    if constexpr (WORDS_LDS) load_words(0);
+    else fetch_words(0, lw_next, dw_next);
+    DqCarry carry = {};
     const T* dq_base = dqrow;  // dq of the query tile before the current one (from the second on)
     // dq of a query tile is summed over the waves, and stored, during the first step of the
     // next query tile, which has no vector work of its own.
@@ -959,18 +992,8 @@ __global__ __launch_bounds__(kRowWaves * 64, bwd_row_two_waves(D, KT) ? 2 : 1) v
       const unsigned char* dot = qt + 32 * ROWB;
 
       // operand words of this lane's query (lanes 32..63 carry zeros)
-      {
-        uint32_t lw, dw;
-        if constexpr (!WORDS_LDS) {
-          lw = lw_next;
-          dw = dw_next;
-        } else {
-          lw = nl[32 * jt + perm32(kl)];
-          dw = nd[32 * jt + perm32(kl)];
-        }
-        s_off.set_raw(g ? 0u : lw);
-        d_off.v[0] = g ? 0u : dw;
-      }
+      s_off.set_raw(g ? 0u : lw_next);
+      d_off.v[0] = g ? 0u : dw_next;
       frag qn[DS], don[DS];
 #pragma unroll
       for (int s = 0; s < DS; ++s) {
@@ -987,8 +1010,8 @@ __global__ __launch_bounds__(kRowWaves * 64, bwd_row_two_waves(D, KT) ? 2 : 1) v
         for (int mt = 0; mt < DM; ++mt)
 #pragma unroll
           for (int s2 = 0; s2 < PS; ++s2) {
-            qtr[mt][s2] = ofq.transposed(qt, s2, mt);
-            dotr[mt][s2] = ofq.transposed(dot, s2, mt);
+            qtr[mt][s2] = ofq.transposed_all(qt, s2, mt);
+            dotr[mt][s2] = ofq.transposed_all(dot, s2, mt);
           }
       };
 
@@ -1024,13 +1047,15 @@ __global__ __launch_bounds__(kRowWaves * 64, bwd_row_two_waves(D, KT) ? 2 : 1) v
         constexpr bool refill = t == KT - 2;
         constexpr int refill_at = Sch::value.last_sb;
         SB();
+        frag kb = keys_op.plain();
+        if constexpr (has_next && MASKED) kb = keys_op.masked_bit(masked_bits, tn);
+        SB();
         TRI_ROW_TICK(t + 1);  // (slot 0: from the loop head to step -1; slot k: step k-2)
         // (words from the global planes: those of the next query tile, fetched before the last
         // bias tile of this one so that no wait for them is a wait for everything in flight)
         if constexpr (!WORDS_LDS && t == KT - 1) fetch_words(jt + 1, lw_next, dw_next);
+        if constexpr (WORDS_LDS && t == KT) load_words(jt + 1);  // (in front of the barrier: not another trip to LDS behind it)
         if constexpr (valu && !refill) fetch_bias(jt, t + 2);
-        frag kb = keys_op.plain();
-        if constexpr (has_next && MASKED) kb = keys_op.masked(kw[tn]);
         SB();
         auto unit = [&](int u) __attribute__((always_inline)) {
           if (u < 8) {
@@ -1086,7 +1111,7 @@ __global__ __launch_bounds__(kRowWaves * 64, bwd_row_two_waves(D, KT) ? 2 : 1) v
               if ((piece + 3 < NM ? piece + 3 : NM - 1) == x) sum_dq_piece(piece, jt - 1, parts, carry, dq_words);
             if constexpr (x == NM - 1) {
               store_dq(jt - 1, dq_base, dq_words);
-              if (jt > 0) dq_base += 32 * a.sdq.j;
+              dq_base += jt > 0 ? 32 * a.sdq.j : 0;
               if constexpr (MULTI) {
                 if (!first_pass) fetch_carry(jt, carry);
               }
@@ -1100,12 +1125,11 @@ __global__ __launch_bounds__(kRowWaves * 64, bwd_row_two_waves(D, KT) ? 2 : 1) v
             for (int s2 = 0; s2 < PS; ++s2) {
               dst_prev[s2] = ofd.transposed(ds_tile, s2, 0);
 #pragma unroll
-              for (int mt = 0; mt < DM; ++mt) ktr_prev[mt][s2] = ofk.transposed(ktile, s2, mt);
+              for (int mt = 0; mt < DM; ++mt) ktr_prev[mt][s2] = ofk.transposed_all(ktile, s2, mt);
             }
           }
           if constexpr (refill && x == refill_at) {
-            // (the last query tiles fetch the last one again, into a stage nobody reads any more)
-            issue_stage(min(jt + 2, NJ - 1), buf_fill);
+            issue_stage(buf_fill);
             fetch_bias(jt, t + 2);
           }
           if constexpr (has_next && x == Sch::value.last_sqk && t + 2 < KT) load_kn(t + 2);

@@ -17,9 +17,9 @@
 // * nothing in a step branches: the compiler sinks what stands in front of a branch behind it, out of the schedule (a step with one took
 //   1.8 instead of 0.9 thousand clocks).  Lanes are masked with exec inside asm statements, pointers advance by masked steps.
 //
-// bf16, h = 4, d = 32, the dq + dk + dv kernel alone, against the four- and eight-wave forms before it on one card: n = 200 41.4 ->
-// 36.5 us, 256 50.6 -> 47, 300 115 -> 94, 384 170 -> 142, 449 (interleaved heads) 319 -> 279, 512 343 -> 298, 512 with padding from 397
-// on 309 -> 288.  With eight heads at n = 256, two rounds of rows per SIMD, 97 -> 100: the start and end of a row are not hidden there.
+// bf16, h = 4, d = 32, the dq + dk + dv kernel alone, against the four- and eight-wave forms before it on one card: n = 200 41.1 ->
+// 36.0 us, 256 51.2 -> 45.3, 300 115 -> 94, 384 170 -> 142, 449 (interleaved heads) 319 -> 279, 512 343 -> 297, 512 with padding from 397
+// on 309 -> 287.  With eight heads at n = 256, two rounds of rows per SIMD, 98 -> 98: the start and end of a row are not hidden there.
 //
 // What bounds it: instruction issue, as in tri_bwd_row.hpp: a step with both neighbours takes about 780 clocks for 14 to 16 MFMAs (448 to 512
 // clocks of matrix pipe), 64 vector instructions of its pair and 50 others; the three steps that carry the query tile's own work (operands of the next
@@ -324,6 +324,14 @@ __global__ __launch_bounds__(NW * 64, 1) void tri_bwd_row_short_kernel(const Bwd
   // tiles attended (no mask work) and some keys masked out.
   auto query_tiles = [&](auto masked_tag) __attribute__((always_inline)) {
     constexpr bool MASKED = decltype(masked_tag)::value;
+    // The masked operands of all key tiles are kept where the registers allow; one wave of eight tiles makes them in the step (n = 256,
+    // h = 4: 47.1 -> 45.8 us, nothing of the loop is in scratch any more; two waves lose by it: n = 512 with padding 286 -> 290).
+    constexpr bool MASK_BITS = MASKED && KT == 8 && NW == 1;
+    int masked_bits = 0;  // bit t set: this lane's key of tile t is masked
+    if constexpr (MASK_BITS) {
+#pragma unroll
+      for (int t = 0; t < KT; ++t) masked_bits |= (kw[t] >> kl & 1u ? 0 : 1) << t;
+    }
     // (each version has its own accumulators, from zeroing to the final stores: merging
     // the versions' accumulators where they meet would copy all of them)
     f32x16 dkacc[KT], dvacc[KT];
@@ -438,6 +446,11 @@ __global__ __launch_bounds__(NW * 64, 1) void tri_bwd_row_short_kernel(const Bwd
       constexpr int NU = valu ? 16 : 0;  // vector units of four instructions
       constexpr bool fetch_late = KT % 2 != 0 && (t + 2) % KT == 0;
       SB();
+      frag kb = keys_op.plain();
+      if constexpr (has_next && MASK_BITS) {
+        kb = keys_op.masked_bit(masked_bits, tn);
+        SB();
+      }
       if constexpr (valu) TRI_ROW_TICK(t);  // (slot 0: step KT-1; slot k: step k-1, less the end of step 0, see below)
       if constexpr (new_query) {
         set_lse(jt + (t < 0 ? 0 : 1));
@@ -448,8 +461,7 @@ __global__ __launch_bounds__(NW * 64, 1) void tri_bwd_row_short_kernel(const Bwd
       // wave of eight key tiles has no registers for that and would reload its V operands from scratch, which waits for every load in flight:
       // h = 8, n = 256 98.9 -> 97.1 us with the scores' product made anew.  Two waves have: n = 512 302.4, made anew 303.7.)
       if constexpr (KT == 8 && NW == 1 && has_next && !MASKED) asm volatile("" : "+v"(s_off.v[0]));
-      frag kb = keys_op.plain();
-      if constexpr (has_next && MASKED) kb = keys_op.masked(kw[tn]);
+      if constexpr (has_next && MASKED && !MASK_BITS) kb = keys_op.masked(kw[tn]);
       SB();
       auto unit = [&](int u) __attribute__((always_inline)) {
         if (u < 8) {

@@ -384,6 +384,13 @@ struct OffsetMask {
       v[1] = (keepw & bit) ? 0u : mask_dword();
       return as_frag(v);
     }
+    // the same for words that do not change inside the caller's loop: bit t of `masked_bits` set = the lane's key of tile t is masked.
+    // (Opaque here: the operands would be made before the loop and kept, four registers for every tile.)
+    TRI_DEV frag masked_bit(int& masked_bits, int t) {
+      asm volatile("" : "+v"(masked_bits));
+      v[1] = (uint32_t)(masked_bits << (31 - t) >> 31) & mask_dword();
+      return as_frag(v);
+    }
     // the same as a new value: for callers whose tiles are rarely masked (the operand in
     // place would be carried, and copied, through the unmasked path as well)
     TRI_DEV frag masked_copy(uint32_t keepw) const {

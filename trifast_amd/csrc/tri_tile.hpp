@@ -77,8 +77,8 @@ struct LdsTile {
   // step at n = 242, h = 8, d = 64 took 410 us, with 5 x 399, with the row number 399.)
   TRI_DEV static int swz(int r) {
     constexpr int B = CPR < 16 ? CPR : 16;  // (16 chunks are all banks)
-    const int x = (r / RPB) % B;
-    return B <= 4 ? x : (x + (x << 2)) % B;  // (5 x: bits 2 and 3 take what bits 0 and 1 are)
+    const unsigned x = (unsigned)r / RPB % B;  // (rows are not negative)
+    return (int)(B <= 4 ? x : (x + (x << 2)) % B);  // (5 x: bits 2 and 3 take what bits 0 and 1 are)
   }
   // byte offset, from the tile base, of byte `o` of row r (o must not straddle a chunk)
   TRI_DEV static int off(int r, int o) { return (r * CPR + ((o >> 4) ^ swz(r))) * 16 + (o & 15); }
