@@ -208,6 +208,23 @@ constexpr int64_t bwd_row_blocks(int bh, int n) {
   return (int64_t)8 * ((bh + heads - 1) / heads) * ((n + share - 1) / share);
 }
 
+// The start of a launch.  Rows take equally long, so compute units that start together fetch the K, V, dO and o of a row together, compute
+// while memory is idle, and store dk and dv together, row after row.  The workgroups of the first round (`per_cu` on each of 32 compute
+// units of each XCD) start one after the other instead, over about the time memory needs for their rows (16 bytes per element at 5
+// TB/s): 2 n d clocks.  That much later the last of them ends, so launches with few rounds take half of it, and rows that
+// compute for long, which gain least; one round has nothing to gain.  A wave sleeps at most 2 n d clocks once per launch.
+// bf16, us, this kernel alone, without -> with: d = 64, h = 8: n = 256 216.4 -> 209.1, n = 330 444 -> 419, two of n = 384 1056 -> 1032
+// (twice the time: 212.9, 409, 1015); d = 32, h = 4: n = 300 94.0 -> 88.8, n = 600 544 -> 527, n = 768 921 -> 897, n = 1024 1971
+// -> 1957; h = 5, n = 256 75.6 -> 72.2; h = 16, n = 128 39.5 -> 37.8.  Not halved: d = 64, h = 2, n = 256 58.1 -> 61.8 (halved 56.4); d = 32, h = 4,
+// n = 512 298 -> 301 (296).  Passes over longer rows: n = 1280 4211 -> 4258, so not there.
+TRI_DEV void stagger_rows(int block, int per_cu, int bh, int n, int d) {
+  const int slot = block >> 3, round = 256 * per_cu;
+  const int64_t rows = (int64_t)bh * n;
+  if (slot >= 32 * per_cu || rows <= round) return;
+  const bool half = n > 10 * d || (per_cu == 1 && rows < 4 * round);
+  for (int z = slot * (n * d >> 7) / (half ? 16 * per_cu : 8 * per_cu); z > 0; --z) __builtin_amdgcn_s_sleep(1);  // (64 clocks)
+}
+
 // LDS bytes of bwd_uniform_row: each wave's four 32-row tiles and 64 floats of delta, then the
 // sums of the row (two D x D products, three vectors)
 constexpr int bwd_uniform_lds_bytes(int D, int es, int NW) {
@@ -558,6 +575,7 @@ __global__ __launch_bounds__(kRowWaves * 64, bwd_row_two_waves(D, KT) ? 2 : 1) v
   extern __shared__ __attribute__((aligned(16))) unsigned char tri_smem[];
 
   TRI_ROW_MARK(t_entry);
+  if constexpr (!MULTI) stagger_rows(blockIdx.x, bwd_row_two_waves(D, KT) ? 2 : 1, a.BH, a.N, D);
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);

@@ -68,6 +68,7 @@ __global__ __launch_bounds__(NW * 64, 1) void tri_bwd_row_short_kernel(const Bwd
   extern __shared__ __attribute__((aligned(16))) unsigned char tri_smem[];
 
   TRI_ROW_MARK(t_entry);
+  stagger_rows(blockIdx.x, 4 / NW, a.BH, a.N, D);
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = NW > 1 ? __builtin_amdgcn_readfirstlane(tid >> 6) : 0;
