@@ -509,9 +509,9 @@ struct DeltaRows {
 #pragma unroll
     for (int x = 0; x < NB; ++x) lv[x] = lse[min(query(x, tid), n - 1)];
   }
-  // words(query, delta, lse) for every query from j0 on
+  // words(query, delta, lse) for every query
   template <typename Words>
-  TRI_DEV void finish(int tid, Words words, int j0) {
+  TRI_DEV void finish(int tid, Words words) {
     typedef T pair __attribute__((ext_vector_type(2)));
     const int c = tid % CPR;
 #pragma unroll
@@ -534,7 +534,7 @@ struct DeltaRows {
           const float keep = c & m ? s[y + m] : s[y], give = c & m ? s[y] : s[y + m];
           s[y] = keep + (m == 4 ? dpp_move<0x141>(give) : m == 2 ? dpp_move<0x4e>(give) : dpp_move<0xb1>(give));
         }
-      if ((x * CPR + c) * RPL < ROWS) words(j0 + query(x, tid), s[0], lv[x]);
+      if ((x * CPR + c) * RPL < ROWS) words(query(x, tid), s[0], lv[x]);
     }
   }
 };
@@ -706,8 +706,7 @@ __global__ __launch_bounds__(kRowWaves * 64, bwd_row_two_waves(D, KT) ? 2 : 1) v
   }
   const T* const orow = reinterpret_cast<const T*>(a.o) + ((int64_t)bh * N + i) * N * D;
   const float* const lserow = a.lse + ((int64_t)bh * N + i) * N;
-  constexpr int DROWS = WORDS_LDS ? KEYS : NW * 64;  // queries at a time
-  DeltaRows<T, D, DROWS, NW> dr;
+  DeltaRows<T, D, WORDS_LDS ? KEYS : 1, NW> dr;
   if constexpr (WORDS_LDS) dr.load(orow, dorow, (uint32_t)a.sdo.j, lserow, N, tid);
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -740,11 +739,20 @@ __global__ __launch_bounds__(kRowWaves * 64, bwd_row_two_waves(D, KT) ? 2 : 1) v
       }
     };
     if constexpr (WORDS_LDS) {
-      dr.finish(tid, query_words, 0);
+      dr.finish(tid, query_words);
     } else {
-      for (int j0 = 0; j0 < N; j0 += DROWS) {
-        dr.load(orow + (int64_t)j0 * D, dorow + (int64_t)j0 * a.sdo.j, (uint32_t)a.sdo.j, lserow + j0, N - j0, tid);
-        dr.finish(tid, query_words, j0);
+      // (rows of 1024 keys are as fast this way, and with the loads above in a loop the compiler (ROCm 7.2.0) ends with a segmentation fault
+      // in its pass over accumulator copies at d = 64 and four key tiles in bf16)
+      for (int j = tid; j < N; j += NW * 64) {
+        float dsum = 0.f;
+#pragma unroll
+        for (int x = 0; x < D / 8; ++x) {
+          const typename E::vec ov = *reinterpret_cast<const typename E::vec*>(orow + (int64_t)j * D + 8 * x);
+          const typename E::vec dv = *reinterpret_cast<const typename E::vec*>(dorow + (int64_t)j * a.sdo.j + 8 * x);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) dsum += (float)ov[e] * (float)dv[e];
+        }
+        query_words(j, dsum, lserow[j]);
       }
     }
   }
