@@ -29,7 +29,7 @@ struct BwdKVFamily {
     if constexpr (stage <= kMaxLds && (sizeof(T) == 4 ? R == 1 || (D <= 32 && NW == 4 && BJ == 32) : acc_regs <= 200 || R == 1)) {
       if (dry) return hipSuccess;
       dim3 grid((a.N + NW * 32 - 1) / (NW * 32), ((a.N + R - 1) / R + 7) / 8 * 8, bh);
-      return launch_dyn(tri_bwd_kv_kernel<T, D, NW, R, BJ, nbuf>, grid, dim3(NW * 64), nbuf * stage, st, a);
+      return launch_dyn(tri_bwd_kv_kernel<T, D, NW, R, BJ, nbuf>, grid, dim3(NW * 64), bwd_kv_lds_bytes(D, (int)sizeof(T), NW, R, BJ, nbuf), st, a);
     } else {
       return hipErrorInvalidConfiguration;
     }

@@ -5,7 +5,8 @@
 // dk, dv accumulators stay in registers, and the queries of the rows are streamed
 // through LDS in tiles of BJ (direct global->LDS loads, double-buffered, swizzled;
 // rows of Q and dO, the lse and delta operand words left by the dq kernel, and the packed
-// bias tiles).  Scores are computed UN-transposed here, S = Q K^T, so that a lane
+// bias tiles).  With one pair row per workgroup and rows of 64 bytes or more (16-bit types) the tiles are 32 queries, whatever BJ says,
+// in a ring of four.  Scores are computed UN-transposed here, S = Q K^T, so that a lane
 // owns one key (column) and 16 queries of every 32-query tile: P and dS are then
 // already in B-operand layout for the two products that contract over queries,
 //   dv^T += dO^T P,   dk^T += Q^T dS,   dk = dk^T / sqrt(d),
@@ -32,6 +33,18 @@ namespace tri {
 // (fp32: the rows as three parts, words and bias in registers)
 constexpr int bwd_kv_stage_bytes(int D, int es, int NW, int R, int BJ) {
   return 2 * R * BJ * lds_row_bytes(D, es) + (es == 4 ? 0 : 2 * R * BJ * 4 + NW * (BJ / 32) * 2048);
+}
+
+// The ring of 32-query stages (one pair row, 16-bit types; whole loads for every wave): a stage's rows and bias tiles, then lse2 and -delta
+// of its queries once per wave.
+constexpr int kBwdKVStages = 4;
+constexpr bool bwd_kv_ring(int D, int es, int R) { return es == 2 && R == 1 && D >= 32; }
+constexpr int bwd_kv_ring_stage_bytes(int D, int es, int NW) { return ring_stage_bytes(D, es, NW, 1) + NW * 256; }
+// LDS bytes of a workgroup
+constexpr int bwd_kv_lds_bytes(int D, int es, int NW, int R, int BJ, int nbuf) {
+  const int stages = nbuf * bwd_kv_stage_bytes(D, es, NW, R, BJ);
+  const int ring = bwd_kv_ring(D, es, R) ? kBwdKVStages * bwd_kv_ring_stage_bytes(D, es, NW) : 0;
+  return stages > ring ? stages : ring;
 }
 
 // Two waves per SIMD (at most 256 registers) wherever the tile fits them or nearly
@@ -346,66 +359,185 @@ __global__ __launch_bounds__(NW * 64, (bwd_kv_min_waves<T, D, R, BJ>())) void tr
     }
   };
 
-  // Stages that lie inside the query range run in the main loop; a ragged last
-  // stage runs after it with the edge handling.
-  const int nfull = N / BJ;  // whole stages
-  const bool ragged = N % BJ != 0;
-  if constexpr (NBUF == 2) {
-    issue_loads(0, 0);
-    store_loads(0);
-    wait_dma();
-    __syncthreads();
-    // (the whole loop exists twice; a wave picks its version once.  Both run the same
-    // stages and barriers.)
-    auto whole_stages = [&](auto common_tag) __attribute__((always_inline)) {
-      int s = 0;
-      for (; s + 1 < nfull; s += 2) {
-        issue_loads((s + 1) * BJ, 1);
-        compute_stage(std::false_type{}, common_tag, s * BJ, 0);
-        store_loads(1);
-        wait_dma();
-        __syncthreads();
-        if ((s + 2) * BJ < N) issue_loads((s + 2) * BJ, 0);
-        compute_stage(std::false_type{}, common_tag, (s + 1) * BJ, 1);
-        if ((s + 2) * BJ < N) store_loads(0);
-        wait_dma();
-        __syncthreads();
-      }
-      return s;
+  // The stages as a ring of four tiles of 32 queries: while a tile's sums are made the scores and dP of the tile after it start, from a stage
+  // that has landed, and the loads of the two stages behind that one are in flight, with a counted wait and one barrier per stage.
+  // What bounded the double buffer was the wait for everything in flight at the end of each stage, 20 spilled registers and
+  // the general loop that a ragged end takes; outputs are the same bits.  Whole steps, h = 4, d = 64, bf16: n = 401
+  // 779 -> 735 us, b = 2, n = 512 with 300 valid 1961 -> 1916; h = 2: n = 1000 3962 -> 3902, d = 128, n = 600 2522 -> 2506; h = 8,
+  // n = 768 in fp16 7854 -> 7844 (the chip lowers its clock there).  Without the scores a stage ahead n = 1000 takes 3924 and n = 768 7935; three
+  // stages and three waves per SIMD, which spill 12 registers, 4473 and 9054.
+  auto ring_loop = [&](auto common_tag, auto stages_tag) __attribute__((always_inline)) {
+    constexpr bool COMMON = decltype(common_tag)::value;
+    using Ring = StageRing<T, D, NW, 1, decltype(stages_tag)::value>;
+    constexpr int NS = Ring::NS, RSTAGE = bwd_kv_ring_stage_bytes(D, (int)sizeof(T), NW), NLD = Ring::NLD + 1;
+    const int ns = (N + 31) >> 5;
+    Ring ring;
+    ring.init(a.sq, a.sdo, qbh, dobh, pack_bh + (int64_t)kt * 1024, a.NP * 1024, N, i0, wave, lane, tri_smem);
+    const uint32_t* const words = reinterpret_cast<const uint32_t*>(g ? delta_bh : lse2_bh) + (int64_t)i0 * N;
+    auto issue = [&](int boff) {
+      const uint32_t* src = words + min(32 * ring.pos + kl, N - 1);
+      const uint32_t dst = __builtin_amdgcn_readfirstlane(ring.lds0 + (uint32_t)(boff + Ring::FSTAGE + wave * 256));
+      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" : : "s"(dst), "v"(src) : "memory", "m0");
+      ring.issue(boff, ns, wave, lane);
     };
-    bool common = wave_active;
+    const typename E::ofrag ones = E::osplat(1.0f);
+    auto chains = [&](int stage, int boff, f32x16& sc, f32x16& dp) __attribute__((always_inline)) {
+      const unsigned char* st = tri_smem + boff;
+      const uint32_t* w = reinterpret_cast<const uint32_t*>(st + Ring::FSTAGE + wave * 256) + perm32(kl);
+      uint32_t lw = w[0];
+      if (32 * stage + perm32(kl) >= N) lw = split_word<T>(E::kMaskElem);  // queries past the end: P = dS = 0
+      lseop.set(lw, g);
+      f32x16 bv = zero16();
+      if (COMMON || !flagged[0]) {
+        const unsigned char* src = st + Ring::FOFF_B + wave * 2048;
 #pragma unroll
-    for (int r = 0; r < R; ++r) common = common && !flagged[r] && tile_live[r];
-    const int s = common ? whole_stages(std::true_type{}) : whole_stages(std::false_type{});
-    // buffer 0 now holds stage s: the last whole one, the ragged one, or a spare
-    if (s < nfull) {
-      if (ragged) issue_loads((s + 1) * BJ, 1);
-      compute_stage(std::false_type{}, std::false_type{}, s * BJ, 0);
-      if (ragged) {
-        store_loads(1);
+        for (int r2 = 0; r2 < 2; ++r2) {
+          const frag x = *reinterpret_cast<const frag*>(src + r2 * 1024 + lane * 16);
+#pragma unroll
+          for (int pp = 0; pp < NPART; ++pp) bv = E::mfma(bsel[r2][pp], x, bv);
+        }
+      }
+      sc = E::mfma(lseop.get(), keyop[0], bv);
+      dp = E::mfma(rank1_operand<T>(w[32], g), ones, zero16());
+#pragma unroll
+      for (int sd = 0; sd < DS; ++sd) {
+        sc = E::mfma(ofs.natural(st, sd), kf[0][sd], sc);
+        dp = E::mfma(ofs.natural(st + Ring::FOFF_V, sd), vf[0][sd], dp);
+      }
+    };
+    auto sums = [&](int boff, const f32x16& sc, const f32x16& dp) __attribute__((always_inline)) {
+      const unsigned char* st = tri_smem + boff;
+      float p[16], ds[16];
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        p[v] = fast_exp2(sc[v] * c);
+        ds[v] = p[v] * dp[v];
+      }
+#pragma unroll
+      for (int s2 = 0; s2 < PS; ++s2) {
+        const frag pf = E::pack(&p[KP * s2]);
+        const frag dsf = E::pack(&ds[KP * s2]);
+#pragma unroll
+        for (int mt = 0; mt < DM; ++mt) {
+          dvacc[0][mt] = E::mfma(ofs.transposed(st + Ring::FOFF_V, s2, mt), pf, dvacc[0][mt]);
+          dkacc[0][mt] = E::mfma(ofs.transposed(st, s2, mt), dsf, dkacc[0][mt]);
+        }
+      }
+    };
+#pragma unroll
+    for (int st = 0; st < NS - 1; ++st) issue(st * RSTAGE);
+    wait_dma_known();  // (the loads of the prologue are not in flight any more as far as the compiler's own waits go)
+    auto up = [](int boff) { return boff == (NS - 1) * RSTAGE ? 0 : boff + RSTAGE; };
+    auto down = [](int boff) { return boff == 0 ? (NS - 1) * RSTAGE : boff - RSTAGE; };
+    int boff = 0;
+    // Both versions of the loop, which may run side by side in a workgroup, meet at the same barriers and use the buffers alike: behind the
+    // one of stage s the stages up to s + 1 have landed, the last reads of stage s - 1 are made, and stage s + 3 is
+    // requested into its buffer.
+    ring_sync<(NS - 2) * NLD>();
+    auto advance = [&] {
+      ring_sync<(NS - 3) * NLD>();
+      issue(down(boff));
+    };
+    int s = 0;
+    if constexpr (COMMON) {
+      f32x16 sa, da, sb, db;
+      chains(0, 0, sa, da);
+      auto trip = [&](int stage, const f32x16& s0, const f32x16& d0, f32x16& s1, f32x16& d1) __attribute__((always_inline)) {
+        advance();
+        chains(stage + 1, up(boff), s1, d1);
+        sums(boff, s0, d0);
+        boff = up(boff);
+      };
+      for (; s + 2 < ns; s += 2) {
+        trip(s, sa, da, sb, db);
+        trip(s + 1, sb, db, sa, da);
+      }
+      if (s + 1 < ns) {
+        trip(s, sa, da, sb, db);
+        sums(boff, sb, db);
+      } else {
+        sums(boff, sa, da);
+      }
+    } else {
+      for (; s < ns; ++s) {
+        if (s + 1 < ns) advance();
+        if (tile_live[0]) {
+          f32x16 sc, dp;
+          chains(s, boff, sc, dp);
+          sums(boff, sc, dp);
+        }
+        boff = up(boff);
+      }
+    }
+    wait_dma();  // (the last prefetches are still on their way into LDS)
+  };
+
+  if constexpr (bwd_kv_ring(D, (int)sizeof(T), R)) {
+    constexpr std::integral_constant<int, kBwdKVStages> stages{};
+    if (wave_active && !flagged[0] && tile_live[0]) ring_loop(std::true_type{}, stages);
+    else ring_loop(std::false_type{}, stages);
+  } else {
+    // Stages that lie inside the query range run in the main loop; a ragged last
+    // stage runs after it with the edge handling.
+    const int nfull = N / BJ;  // whole stages
+    const bool ragged = N % BJ != 0;
+    if constexpr (NBUF == 2) {
+      issue_loads(0, 0);
+      store_loads(0);
+      wait_dma();
+      __syncthreads();
+      // (the whole loop exists twice; a wave picks its version once.  Both run the same
+      // stages and barriers.)
+      auto whole_stages = [&](auto common_tag) __attribute__((always_inline)) {
+        int s = 0;
+        for (; s + 1 < nfull; s += 2) {
+          issue_loads((s + 1) * BJ, 1);
+          compute_stage(std::false_type{}, common_tag, s * BJ, 0);
+          store_loads(1);
+          wait_dma();
+          __syncthreads();
+          if ((s + 2) * BJ < N) issue_loads((s + 2) * BJ, 0);
+          compute_stage(std::false_type{}, common_tag, (s + 1) * BJ, 1);
+          if ((s + 2) * BJ < N) store_loads(0);
+          wait_dma();
+          __syncthreads();
+        }
+        return s;
+      };
+      bool common = wave_active;
+#pragma unroll
+      for (int r = 0; r < R; ++r) common = common && !flagged[r] && tile_live[r];
+      const int s = common ? whole_stages(std::true_type{}) : whole_stages(std::false_type{});
+      // buffer 0 now holds stage s: the last whole one, the ragged one, or a spare
+      if (s < nfull) {
+        if (ragged) issue_loads((s + 1) * BJ, 1);
+        compute_stage(std::false_type{}, std::false_type{}, s * BJ, 0);
+        if (ragged) {
+          store_loads(1);
+          wait_dma();
+          __syncthreads();
+          compute_stage(std::true_type{}, std::false_type{}, (s + 1) * BJ, 1);
+        }
+      } else if (ragged) {
+        compute_stage(std::true_type{}, std::false_type{}, s * BJ, 0);
+      }
+    } else {
+      // one stage only (the double buffer does not fit in LDS): load, then compute
+      for (int s = 0; s < nfull; ++s) {
+        issue_loads(s * BJ, 0);
+        store_loads(0);
         wait_dma();
         __syncthreads();
-        compute_stage(std::true_type{}, std::false_type{}, (s + 1) * BJ, 1);
+        compute_stage(std::false_type{}, std::false_type{}, s * BJ, 0);
+        __syncthreads();
       }
-    } else if (ragged) {
-      compute_stage(std::true_type{}, std::false_type{}, s * BJ, 0);
-    }
-  } else {
-    // one stage only (the double buffer does not fit in LDS): load, then compute
-    for (int s = 0; s < nfull; ++s) {
-      issue_loads(s * BJ, 0);
-      store_loads(0);
-      wait_dma();
-      __syncthreads();
-      compute_stage(std::false_type{}, std::false_type{}, s * BJ, 0);
-      __syncthreads();
-    }
-    if (ragged) {
-      issue_loads(nfull * BJ, 0);
-      store_loads(0);
-      wait_dma();
-      __syncthreads();
-      compute_stage(std::true_type{}, std::false_type{}, nfull * BJ, 0);
+      if (ragged) {
+        issue_loads(nfull * BJ, 0);
+        store_loads(0);
+        wait_dma();
+        __syncthreads();
+        compute_stage(std::true_type{}, std::false_type{}, nfull * BJ, 0);
+      }
     }
   }
 
