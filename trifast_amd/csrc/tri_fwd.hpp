@@ -182,67 +182,17 @@ __global__ __launch_bounds__(NW * 64, (R * ((BKF % kFwdFast) / 32) >= 8 || D * s
       for (int st = 0; st < Ring::NS - 1; ++st) ring.issue(st * Ring::FSTAGE, a.nwords, wave, lane);
     }
   }
-  // (the other loops start from empty buffers)
-  auto drop_ring = [&] {
-    if constexpr (FAST) {
-      wait_dma();
-      __syncthreads();
-    }
+  // (what goes another way starts from empty buffers)
+  auto drop_loads = [&] {
+    wait_dma();
+    __syncthreads();
   };
-
-  // per-row state.  A fully masked row drops the q.k and bias terms (all logits
-  // equal): its Q operand is zero and it skips the bias.
-  bool flagged[R];
-  bool any_flagged = false;
-  const uint32_t* keep_row[R];
-  frag qf[R][DS];
-  f32x16 oacc[R][DM];
-  float mref[R], mc[R], lrun[R];
-  bool all_flagged = true;
-#pragma unroll
-  for (int r = 0; r < R; ++r) {
-    flagged[r] = uniform_word(a.rowflag, b * N + min(i0 + r, N - 1)) != 0;
-    all_flagged &= flagged[r];
-  }
-  if (all_flagged) {
-    drop_ring();
-    fwd_uniform_rows<T, D, NW, R>(a, vbh, bh, i0, bx * (NW * 32), tri_smem);
-    return;
-  }
-#pragma unroll
-  for (int r = 0; r < R; ++r) {
-    const int i = min(i0 + r, N - 1);  // rows past the end repeat the last one and are not stored
-    any_flagged |= flagged[r];
-    keep_row[r] = a.keep + ((int64_t)b * N + i) * a.nwords;
-#pragma unroll
-    for (int s = 0; s < DS; ++s) {
-      if (j < N && !flagged[r])
-        qf[r][s] = E::load(qbh + i * a.sq.i + (int64_t)j * a.sq.j + 2 * KP * s + KP * g);
-      else
-        qf[r][s] = E::zero();
-    }
-    mref[r] = kNeg;
-    mc[r] = kNeg;
-    lrun[r] = 0.f;
-#pragma unroll
-    for (int mt = 0; mt < DM; ++mt) oacc[r][mt] = zero16();
-  }
-  const float c = a.c;
 
   // the key mask enters the scores through one extra MFMA: keys operand with the mask
   // element of this lane's key (patched in place per tile) against a constant queries
   // operand (see OffsetMask; its per-query offset is not used here: the word is zero)
   typename OffsetMask<T>::Keys kop;
   typename E::ofrag qzero;
-
-  KeyTileMasks masks;
-  masks.build<R, NW>(reinterpret_cast<uint64_t*>(tri_smem + LDS_MAIN), [&](int r) { return keep_row[r]; }, a.nwords, any_flagged, wave, lane,
-                      FAST && (N & 31) != 0 ? 0xffffffffu << (N & 31) : 0u);
-
-  // lane-constant LDS offsets of the operand reads: K rows as natural operands
-  // (tile row m stands for key perm32(m)), V rows through transposing reads
-  OperandOffsets<T, D> ofs;
-  ofs.init(perm32(jl), lane);
 
   // per-lane source pointers of the K and V stage tiles for keys 0..BK-1
   // (set up by the general stage loop only: the scheduled loop below has no use for them, and
@@ -321,6 +271,64 @@ __global__ __launch_bounds__(NW * 64, (R * ((BKF % kFwdFast) / 32) >= 8 || D * s
       vstream.store(tri_smem + buf * STAGE + OFF_V);
     }
   };
+  // The first stage of the other tiles' loop is requested here too, whether or not some row attends to it: its loads would otherwise wait
+  // for the row flags, the keep words behind those and the key-tile bitmaps made of them, three trips to memory (inference, bf16, us: h = 4, d = 32,
+  // n = 130 19.4 -> 18.4; d = 64, b = 2, n = 100 20.0 -> 18.7; h = 2, d = 128, n = 250 42.1 -> 40.8; d = 32, n = 400 padded 58.8 -> 58.3).
+  // In fp32 the loads would hold registers meanwhile: 16 spilled at d = 64, two waves per SIMD in place of three at d = 32.
+  constexpr bool EARLY = !FAST && sizeof(T) == 2;
+  if constexpr (EARLY) {
+    setup_general();
+    issue_loads(0, 0);
+  }
+
+  // per-row state.  A fully masked row drops the q.k and bias terms (all logits
+  // equal): its Q operand is zero and it skips the bias.
+  bool flagged[R];
+  bool any_flagged = false;
+  const uint32_t* keep_row[R];
+  frag qf[R][DS];
+  f32x16 oacc[R][DM];
+  float mref[R], mc[R], lrun[R];
+  bool all_flagged = true;
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    flagged[r] = uniform_word(a.rowflag, b * N + min(i0 + r, N - 1)) != 0;
+    all_flagged &= flagged[r];
+  }
+  if (all_flagged) {
+    if constexpr (sizeof(T) == 2) drop_loads();
+    fwd_uniform_rows<T, D, NW, R>(a, vbh, bh, i0, bx * (NW * 32), tri_smem);
+    return;
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int i = min(i0 + r, N - 1);  // rows past the end repeat the last one and are not stored
+    any_flagged |= flagged[r];
+    keep_row[r] = a.keep + ((int64_t)b * N + i) * a.nwords;
+#pragma unroll
+    for (int s = 0; s < DS; ++s) {
+      if (j < N && !flagged[r])
+        qf[r][s] = E::load(qbh + i * a.sq.i + (int64_t)j * a.sq.j + 2 * KP * s + KP * g);
+      else
+        qf[r][s] = E::zero();
+    }
+    mref[r] = kNeg;
+    mc[r] = kNeg;
+    lrun[r] = 0.f;
+#pragma unroll
+    for (int mt = 0; mt < DM; ++mt) oacc[r][mt] = zero16();
+  }
+  const float c = a.c;
+
+  KeyTileMasks masks;
+  masks.build<R, NW>(reinterpret_cast<uint64_t*>(tri_smem + LDS_MAIN), [&](int r) { return keep_row[r]; }, a.nwords, any_flagged, wave, lane,
+                      FAST && (N & 31) != 0 ? 0xffffffffu << (N & 31) : 0u);
+
+  // lane-constant LDS offsets of the operand reads: K rows as natural operands
+  // (tile row m stands for key perm32(m)), V rows through transposing reads
+  OperandOffsets<T, D> ofs;
+  ofs.init(perm32(jl), lane);
+
   // the 16 bias values of this lane for key tile u of the stage, raw-score domain
   auto bias_from_lds = [&](int buf, int u) -> f32x16 {
     const unsigned char* src = tri_smem + buf * STAGE + OFF_B + (wave * KU + u) * BIAS_B;
@@ -810,7 +818,10 @@ __global__ __launch_bounds__(NW * 64, (R * ((BKF % kFwdFast) / 32) >= 8 || D * s
     want_keep_words = !PLAIN;
     auto next = [&](int t) { return PLAIN ? min(t, ntiles) : masks.next_live<KU>(t); };
     int t0 = next(0);
-    issue_loads(min(32 * t0, N - 1), 0);
+    if (!EARLY || t0 != 0) {  // (or on its way)
+      if constexpr (EARLY) drop_loads();
+      issue_loads(min(32 * t0, N - 1), 0);
+    }
     store_loads(0);
     wait_dma();
     __syncthreads();
@@ -843,8 +854,8 @@ __global__ __launch_bounds__(NW * 64, (R * ((BKF % kFwdFast) / 32) >= 8 || D * s
   } else if (fast_masked) {
     if constexpr (FAST) fast_loop(std::true_type{});
   } else {
-    drop_ring();
-    setup_general();
+    if constexpr (FAST) drop_loads();
+    if constexpr (!EARLY) setup_general();
     if (masks.all_plain() && ntiles % KU == 0 && (N & 31) == 0) stage_loop(std::integral_constant<int, kPlain>{});
     else if (!any_flagged) stage_loop(std::integral_constant<int, kMasked>{});
     else stage_loop(std::integral_constant<int, kGeneral>{});
