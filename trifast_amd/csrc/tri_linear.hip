@@ -32,7 +32,7 @@ hipError_t fwd_run(LinearFwdArgs a, hipStream_t st) {
   for (int p = 0; p < a.nlayers; ++p) a.total_chunks += (a.n[p] + 31) / 32;
   constexpr int chunk_bytes = 32 * KD * (int)sizeof(T);
   const int64_t blocks = (a.rows + 128 * RT - 1) / (128 * RT);
-  split_chunks(blocks, a.total_chunks, kLinearFwdWeights / chunk_bytes, GATED ? 256 : 1024, a.chunks, a.groups);
+  split_chunks(blocks, a.total_chunks, 40 * 1024 / chunk_bytes, GATED ? 256 : 1024, a.chunks, a.groups);
   return launch_dyn(linear_fwd_kernel<T, KD, RT, GATED>, row_grid(a.rows, 128 * RT, a.groups), dim3(256), a.chunks * (chunk_bytes + 32 * (int)sizeof(T)), st, a);
 }
 

@@ -121,7 +121,6 @@ TRI_DEV typename Elem<T>::vec gated_piece(typename Elem<T>::vec o, typename Elem
 // before): 577 workgroups of 256 rows on 512 resident slots ran two rounds at n = 384, and 24
 // workgroups did all the work at n = 77.
 // ---------------------------------------------------------------------------------------
-constexpr int kLinearFwdWeights = 40 * 1024;  // LDS bytes of a workgroup's weights at most
 template <typename T, int KD, int RT, bool GATED>
 __global__ __launch_bounds__(256) void linear_fwd_kernel(const LinearFwdArgs a) {
   using E = Elem<T>;
@@ -149,20 +148,14 @@ __global__ __launch_bounds__(256) void linear_fwd_kernel(const LinearFwdArgs a) 
     Tile::template fill<32, 4>(lin_smem + q * CHUNK_B, [&](int r) { return w + (int64_t)min(at.col0 + r, last) * KD; }, wave, lane);
   }
   // ... and their biases (a bias loaded in front of a chunk's products waits for the stores of the chunk before:
-  // gated, K = 128, 128 outputs with bias, 40000 rows 12.0 -> 11.7 us, 147456 25.4 -> 24.0; K = 64 20.1 -> 19.7),
-  // requested here and put there behind the requests of the rows: at once, the rows waited for them, another trip to memory in every workgroup
-  // (the block in training at n = 384 520 -> 506 us, in inference at n = 77 28.4 -> 27.1)
+  // gated, K = 128, 128 outputs with bias, 40000 rows 12.0 -> 11.7 us, 147456 25.4 -> 24.0; K = 64 20.1 -> 19.7)
   T* const biases = reinterpret_cast<T*>(lin_smem + nq * CHUNK_B);
-  constexpr int NBV = (kLinearFwdWeights / CHUNK_B + 3) / 4;
-  T bv[NBV];
-#pragma unroll
-  for (int x = 0; x < NBV; ++x) {
-    bv[x] = (T)0.0f;
-    const int q = wave + 4 * x;
-    if (q >= nq) continue;
+  for (int q = wave; q < nq; q += 4) {
     const ChunkAt at = chunk_at(a, q0 + q);
     const T* bias = reinterpret_cast<const T*>(a.bias[at.p]);
-    if (bias && at.col0 + cl < a.n[at.p]) bv[x] = bias[at.col0 + cl];
+    T value = (T)0.0f;
+    if (bias && at.col0 + cl < a.n[at.p]) value = bias[at.col0 + cl];
+    biases[32 * q + cl] = value;
   }
   // the rows' fragments (rows past the end repeat the last one and are not stored)
   int64_t row[RT];
@@ -198,10 +191,6 @@ __global__ __launch_bounds__(256) void linear_fwd_kernel(const LinearFwdArgs a) 
       for (int s = 0; s < KS; ++s) xf[t][s] = *reinterpret_cast<const frag*>(x + 16 * s + 8 * g);
     }
   }
-  // (stored once the rows' loads are on their way: a store waits for the loads before it)
-#pragma unroll
-  for (int x = 0; x < NBV; ++x)
-    if (wave + 4 * x < nq) biases[32 * (wave + 4 * x) + cl] = bv[x];
   // (a wait the compiler knows: it would otherwise put one in front of every LDS read below, and wait
   // for the stores of the chunk before with it)
   wait_dma_known();
