@@ -182,9 +182,14 @@ constexpr bool bwd_row_two_waves(int D, int KT) { return D <= 32 && KT <= 2; }
 // LDS bytes of the kernel below.  dq partials: two buffers (one barrier per query tile) of
 // three quarters of a tile per wave (the quarter a wave sums itself waits in its dS tile)
 constexpr int bwd_row_red_bytes(int D) { return kRowWaves * 3 * ((D + 31) / 32) * 1024; }
+// Tiles of a stage of the query stream: Q, dO and, in rows of 128 bytes of up to 384 keys, o: delta is formed from it per query tile then, and
+// the row does not start with a trip to memory for the o and dO of all its queries, a fifth of its time there (training steps, d = 64,
+// us: h = 8, b = 2, n = 384 in fp16 2039 -> 1996; h = 8, n = 256 370 -> 351; h = 4, n = 330 419 -> 403, 384 491 -> 478).  In narrower
+// rows, whose loops are longer, the work per query tile costs as much (d = 32, n = 600 994 -> 1006, 768 1812 both, 850 2767 -> 2764; d = 16, n = 700 1261 -> 1259).
+constexpr int bwd_row_stage_tiles(int D, int KT, bool multi) { return D == 64 && KT <= 3 && !multi ? 3 : 2; }
 constexpr int bwd_row_base_lds_bytes(int D, int es, int KT, bool multi) {  // (without the per-query words)
   const int rowb = D * es, keys = kRowWaves * KT * 32;
-  return keys * rowb + 3 * (2 * 32 * rowb) + kRowWaves * 2048 + 2 * bwd_row_red_bytes(D) +
+  return keys * rowb + 3 * (bwd_row_stage_tiles(D, KT, multi) * 32 * rowb) + kRowWaves * 2048 + 2 * bwd_row_red_bytes(D) +
          kRowWaves * bwd_row_v_lds_tiles(D, KT, multi) * (D / 16) * 1024;
 }
 // The per-query operand words of the row (two planes of 4 bytes per query) live in LDS where
@@ -488,8 +493,8 @@ TRI_DEV void bwd_uniform_row(const BwdArgs& a, int bh, int i, unsigned char* sme
 
 // delta = rowsum(o * do) of up to ROWS queries by NW waves.  A load takes whole rows side by side, 16 bytes of one per lane, so that the CPR
 // lanes of a row each hold a part of its sum; they trade the parts of CPR rows in such a way that each ends with the sum of one of them.
-// (A row per lane, 16 bytes at a time, touches 64 rows with every load.  d = 64, h = 8: n = 256 228.4 -> 216.8 us, two of n = 384
-// 1141 -> 1108; d = 32 within 0.6 %.)
+// (A row per lane, 16 bytes at a time, touches 64 rows with every load.  Measured at d = 64, which forms delta per query tile now: h = 8, n = 256
+// 228.4 -> 216.8 us; d = 32 within 0.6 %.)
 template <typename T, int D, int ROWS, int NW>
 struct DeltaRows {
   using E = Elem<T>;
@@ -556,7 +561,9 @@ __global__ __launch_bounds__(kRowWaves * 64, bwd_row_two_waves(D, KT) ? 2 : 1) v
   constexpr int ROWB = Tile::ROWB;
   constexpr int KEYS = NW * KT * 32;         // keys (and queries) the workgroup can hold
   constexpr bool WORDS_LDS = bwd_row_words_in_lds(D, (int)sizeof(T), KT, MULTI);  // per-query words of the row in LDS (else from the global planes)
-  constexpr int STAGE = 2 * 32 * ROWB;        // Q tile | dO tile
+  constexpr int NT = bwd_row_stage_tiles(D, KT, MULTI);
+  constexpr bool O_STAGE = NT == 3;
+  constexpr int STAGE = NT * 32 * ROWB;       // Q tile | dO tile (| o tile)
   constexpr int OFF_K = 0;
   constexpr int OFF_ST = KEYS * ROWB;
   constexpr int OFF_DS = OFF_ST + 3 * STAGE;  // three stages: in use, ready, in flight
@@ -564,7 +571,7 @@ __global__ __launch_bounds__(kRowWaves * 64, bwd_row_two_waves(D, KT) ? 2 : 1) v
   constexpr int OFF_NL = OFF_RED + 2 * bwd_row_red_bytes(D);
   constexpr int PLANE = WORDS_LDS ? KEYS * 4 : 0;  // per-query words of the row
   constexpr int OFF_ND = OFF_NL + PLANE;
-  constexpr int G2W = (2 * 32 * (ROWB / 16) / 64 + NW - 1) / NW;  // global->LDS loads per wave and stage
+  constexpr int G2W = (NT * 32 * (ROWB / 16) / 64 + NW - 1) / NW;  // global->LDS loads per wave and stage
   constexpr int VL = bwd_row_v_lds_tiles(D, KT, MULTI);  // this wave's last VL key tiles keep V in LDS
   constexpr int VR = KT - VL;
   constexpr int OFF_V = OFF_ND + PLANE;
@@ -603,6 +610,7 @@ __global__ __launch_bounds__(kRowWaves * 64, bwd_row_two_waves(D, KT) ? 2 : 1) v
   const T* krow = reinterpret_cast<const T*>(a.k) + b * a.sk.b + h * a.sk.h + i * a.sk.i;
   const T* vrow = reinterpret_cast<const T*>(a.v) + b * a.sv.b + h * a.sv.h + i * a.sv.i;
   const T* dorow = reinterpret_cast<const T*>(a.dout) + b * a.sdo.b + h * a.sdo.h + i * a.sdo.i;
+  const T* const orow = reinterpret_cast<const T*>(a.o) + ((int64_t)bh * N + i) * N * D;
   const T* pack_bh = reinterpret_cast<const T*>(a.packq) + (int64_t)bh * a.NP * a.NP * 1024;
 
   unsigned char* const lds_k = tri_smem + OFF_K;
@@ -625,17 +633,17 @@ __global__ __launch_bounds__(kRowWaves * 64, bwd_row_two_waves(D, KT) ? 2 : 1) v
   // to the next they would be spilled, and a reload from scratch waits for every load in flight.)
   // (No branch: what stands in front of one is sunk behind it by the compiler, out of the schedule of the loop below.)
   const uint32_t lds0 = (uint32_t)(uintptr_t)(TRI_L3 unsigned char*)tri_smem;
-  // the stage is two tiles (Q rows, dO rows) of LT wave loads of 1 KiB, dealt to the waves in turn: GX loads for each, or, with fewer
-  // loads than waves (head dim 16), one each for the first; fill[] are the first rows of the next stage to request, per load
-  constexpr int LT = 32 * Tile::CPR / 64, GX = (2 * LT + NW - 1) / NW;
+  // the stage is two or three tiles (Q rows, dO rows, o rows) of LT wave loads of 1 KiB, dealt to the waves in turn: GX loads for each, or, where that
+  // does not come out even (head dim 16), some without a share; fill[] are the first rows of the next stage to request, per load
+  constexpr int LT = 32 * Tile::CPR / 64, GX = (NT * LT + NW - 1) / NW;
   const T* fill[GX];
   int64_t fill_step[GX];
   uint32_t fill_row[GX];  // bytes between rows (below 2^24: a limit of the entry points)
 #pragma unroll
   for (int x = 0; x < GX; ++x) {
-    const bool is_q = (x * NW + wave) / LT == 0;
-    fill[x] = is_q ? qrow : dorow;
-    const int64_t stride = is_q ? a.sq.j : a.sdo.j;
+    const int tile = (x * NW + wave) / LT;
+    fill[x] = tile == 0 ? qrow : O_STAGE && tile == 2 ? orow : dorow;
+    const int64_t stride = tile == 0 ? a.sq.j : O_STAGE && tile == 2 ? D : a.sdo.j;
     fill_step[x] = 32 * stride;
     fill_row[x] = (uint32_t)stride * (uint32_t)sizeof(T);
   }
@@ -653,8 +661,8 @@ __global__ __launch_bounds__(kRowWaves * 64, bwd_row_two_waves(D, KT) ? 2 : 1) v
       const T* base = fill[x];
       const uint32_t dst = __builtin_amdgcn_readfirstlane(lds0 + (uint32_t)(OFF_ST + buf * STAGE + gi * 1024));
       // (waves without a share load with no lane; their counted wait is for nothing of theirs, the barrier behind it stands for the others')
-      if constexpr (2 * LT < NW) {
-        const int mine = __builtin_amdgcn_readfirstlane(gi < 2 * LT ? -1 : 0);
+      if constexpr (NT * LT % NW != 0) {
+        const int mine = __builtin_amdgcn_readfirstlane(gi < NT * LT ? -1 : 0);
         asm volatile("s_mov_b32 m0, %0\n\ts_mov_b32 exec_lo, %3\n\ts_mov_b32 exec_hi, %3\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b64 exec, -1" : : "s"(dst), "v"(voff), "s"(base), "s"(mine) : "memory", "m0");
       } else {
         asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(dst), "v"(voff), "s"(base) : "memory", "m0");
@@ -704,10 +712,17 @@ __global__ __launch_bounds__(kRowWaves * 64, bwd_row_two_waves(D, KT) ? 2 : 1) v
 #pragma unroll
     for (int s = 0; s < DS; ++s) vx[t][s] = *reinterpret_cast<const frag*>(vrow + (int64_t)key * a.sv.j + 2 * KP * s + KP * g);
   }
-  const T* const orow = reinterpret_cast<const T*>(a.o) + ((int64_t)bh * N + i) * N * D;
   const float* const lserow = a.lse + ((int64_t)bh * N + i) * N;
+  static_assert(WORDS_LDS || !O_STAGE, "the words of a query are kept in LDS until the end of the row");
   DeltaRows<T, D, WORDS_LDS ? KEYS : 1, NW> dr;
-  if constexpr (WORDS_LDS) dr.load(orow, dorow, (uint32_t)a.sdo.j, lserow, N, tid);
+  constexpr int LSE_N = O_STAGE ? (KEYS + NW * 64 - 1) / (NW * 64) : 1;
+  float lse_x[LSE_N];
+  if constexpr (O_STAGE) {
+#pragma unroll
+    for (int x = 0; x < LSE_N; ++x) lse_x[x] = lserow[min(x * NW * 64 + tid, N - 1)];
+  } else if constexpr (WORDS_LDS) {
+    dr.load(orow, dorow, (uint32_t)a.sdo.j, lserow, N, tid);
+  }
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int t = 0; t < KT; ++t)
@@ -738,7 +753,16 @@ __global__ __launch_bounds__(kRowWaves * 64, bwd_row_two_waves(D, KT) ? 2 : 1) v
         nd[j] = dw;
       }
     };
-    if constexpr (WORDS_LDS) {
+    if constexpr (O_STAGE) {
+#pragma unroll
+      for (int x = 0; x < LSE_N; ++x) {
+        const int j = x * NW * 64 + tid;
+        if (KEYS % (NW * 64) != 0 && j >= KEYS) continue;
+        const uint32_t lw = split_word<T>(j < N ? -lse_x[x] * a.sqrt_d : E::kMaskElem);  // queries past the end: P = dS = 0
+        if (j < N) lplane[j] = lw;
+        nl[j] = lw;
+      }
+    } else if constexpr (WORDS_LDS) {
       dr.finish(tid, query_words);
     } else {
       // (rows of 1024 keys are as fast this way, and with the loads above in a loop the compiler (ROCm 7.2.0) ends with a segmentation fault
@@ -1020,7 +1044,7 @@ __global__ __launch_bounds__(kRowWaves * 64, bwd_row_two_waves(D, KT) ? 2 : 1) v
     auto load_words = [&](int jt) {
       const int j = 32 * min(jt, NJ - 1) + perm32(kl);
       lw_next = nl[j];
-      dw_next = nd[j];
+      if constexpr (!O_STAGE) dw_next = nd[j];
     };
     if constexpr (WORDS_LDS) load_words(0);
     else fetch_words(0, lw_next, dw_next);
@@ -1044,13 +1068,31 @@ __global__ __launch_bounds__(kRowWaves * 64, bwd_row_two_waves(D, KT) ? 2 : 1) v
 
       // operand words of this lane's query (lanes 32..63 carry zeros)
       s_off.set_raw(g ? 0u : lw_next);
-      d_off.v[0] = g ? 0u : dw_next;
-      frag qn[DS], don[DS];
+      if constexpr (!O_STAGE) d_off.v[0] = g ? 0u : dw_next;
+      frag qn[DS], don[DS], on[O_STAGE ? DS : 1];
 #pragma unroll
       for (int s = 0; s < DS; ++s) {
         qn[s] = ofq.natural(qt, s);
         don[s] = ofq.natural(dot, s);
+        if constexpr (O_STAGE) on[s] = ofq.natural(dot + 32 * ROWB, s);
       }
+      // delta of the query tile, of which a lane holds half a row, in four sums and their total; the word is kept for the end of
+      // the row, by every wave for itself
+      float dsum[4];
+      auto set_delta = [&](int piece) __attribute__((always_inline)) {
+        typedef T pair __attribute__((ext_vector_type(2)));
+        if (piece < 2) {
+#pragma unroll
+          for (int s = piece * DS / 2; s < (piece + 1) * DS / 2; ++s)
+#pragma unroll
+            for (int e = 0; e < 8; e += 2)
+              dsum[e / 2] = pair_dot(pair{on[s][e], on[s][e + 1]}, pair{don[s][e], don[s][e + 1]}, s == 0 ? 0.f : dsum[e / 2]);
+        } else {
+          const uint32_t word = split_word<T>(-half_sum((dsum[0] + dsum[1]) + (dsum[2] + dsum[3])));
+          nd[32 * jt + perm32(kl)] = word;
+          d_off.v[0] = word & (uint32_t)((g | (int)(perm32(kl) >= N - 32 * jt)) - 1);
+        }
+      };
       // Q^T, dO^T (A operands of dk, dv): transposing reads are the slowest LDS reads and the
       // four waves share one LDS pipe, so they are read once per query tile where registers
       // allow and again for every key tile where they do not
@@ -1146,6 +1188,7 @@ __global__ __launch_bounds__(kRowWaves * 64, bwd_row_two_waves(D, KT) ? 2 : 1) v
             else dqacc[idx % DM] = E::mfma(ktr_prev[idx % DM][idx / DM], dst_prev[idx / DM], dqacc[idx % DM]);
           }
           SB();
+          if constexpr (O_STAGE && t == -1 && x < 3) set_delta(x);
           // Q^T, dO^T of the query tile are first used by the step after next: their reads go
           // where the LDS pipe has nothing else to do
           if constexpr (QD_ONCE && t == -1 && x == 1) load_qd_tr();
@@ -1227,6 +1270,14 @@ __global__ __launch_bounds__(kRowWaves * 64, bwd_row_two_waves(D, KT) ? 2 : 1) v
     const uint64_t t_clk1 = __builtin_amdgcn_s_memtime(), t_loop1 = __builtin_amdgcn_s_memrealtime();
 #endif
 
+    // the words that the db kernel reads (each thread writes what its own wave has put there)
+    if constexpr (O_STAGE) {
+#pragma unroll
+      for (int x = 0; x < LSE_N; ++x) {
+        const int j = x * NW * 64 + tid;
+        if (j < N) dplane[j] = nd[j];
+      }
+    }
     // ---- dk, dv of this wave's keys -------------------------------------------------------
     // (the accumulators were last written by MFMAs inside asm statements, which the compiler
     // does not know to be MFMAs: each is read only after that MFMA has had time to retire)
