@@ -703,7 +703,7 @@ __global__ __launch_bounds__(kRowWaves * 64, bwd_row_two_waves(D, KT) ? 2 : 1) v
   frag vf[VR > 0 ? VR : 1][DS];
   frag* const v_lds = reinterpret_cast<frag*>(tri_smem + OFF_V + wave * VL * DS * 1024) + lane;
   // (every load of the prologue is issued before the first one is used: the V rows here, then
-  // the row's o and do for delta (queries past the end read the last one again): one trip to
+  // the row's o and do where delta comes from them (queries past the end read the last one again): one trip to
   // memory for all of them, while the K row is on its way to LDS)
   frag vx[KT][DS];
 #pragma unroll
