@@ -340,3 +340,50 @@ def test_probe_builds_of_the_kernels_compile(source, flags):
     cmd = [build._hipcc(), *build.HIPCC_FLAGS, *flags, "-DTRI_DEV_ONLY_BF16_D32", "--cuda-device-only", "-fsyntax-only", "-I", str(build.CSRC), str(build.CSRC / source)]
     res = subprocess.run(cmd, capture_output=True, text=True)
     assert res.returncode == 0, res.stderr[-2000:]
+
+
+@pytest.fixture(scope="module", params=["__bf16", "_Float16"])
+def wide_row_kernels(request, tmp_path_factory):
+    """Assembly of the row-resident backward at head dim 64: key tiles per wave -> (lines of the kernel)."""
+    import re
+    import subprocess
+
+    from trifast_amd import build
+
+    if build._compiler_flags():
+        pytest.skip("not the compiler that the kernels are laid out for")
+    tiles = (2, 3)
+    tmp = tmp_path_factory.mktemp("row")
+    source, asm = tmp / "row.hip", tmp / "row.s"
+    source.write_text('#include "tri_bwd_row.hpp"\nnamespace tri {\n' + "".join(
+        f"template __global__ void tri_bwd_row_kernel<{request.param}, 64, {kt}, false>(const BwdArgs);\n" for kt in tiles) + "}\n")
+    cmd = [build._hipcc(), *build.HIPCC_FLAGS, "--cuda-device-only", "-S", "-I", str(build.CSRC), "-o", str(asm), str(source)]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    assert res.returncode == 0, res.stderr[-2000:]
+    kernels = re.findall(r"^_Z\w*tri_bwd_row_kernel\w*Li64ELi(\d)E\w*:(.*?)^\.Lfunc_end", asm.read_text(), re.S | re.M)
+    assert sorted(int(kt) for kt, _ in kernels) == list(tiles)
+    return {int(kt): body.splitlines() for kt, body in kernels}
+
+
+def test_row_resident_loop_keeps_nothing_in_scratch(wide_row_kernels):
+    """One branch, the loop's own, and no scratch access in the loop over the query tiles: a reload waits for every load in
+    flight, those of the ring among them."""
+    import re
+
+    for kt, lines in wide_row_kernels.items():
+        label = {m.group(1): at for at, line in enumerate(lines) if (m := re.match(r"(\.LBB\w+):", line))}
+        loops = [lines[label[m.group(1)]:at + 1] for at, line in enumerate(lines)
+                 if (m := re.match(r"\s+s_c?branch\w*\s+(\.LBB\w+)", line)) and label[m.group(1)] <= at]
+        # the two versions of the loop (with and without masked keys) are the ones that request stages of the ring and take exponentials
+        loops = [x for x in loops if "Inner Loop" in x[0] and any("global_load_lds" in y for y in x) and sum("v_exp_f32" in y for y in x) == 16 * kt]
+        assert len(loops) == 2, kt
+        for loop in loops:
+            assert [y for y in loop if "scratch_" in y] == [], kt
+            assert sum(bool(re.match(r"\s+s_c?branch", y)) for y in loop) == 1, kt
+
+
+def test_fully_masked_rows_leave_nothing_in_scratch(wide_row_kernels):
+    """The sums of a fully masked row (two 64 x 64 products and three vectors) take no address per element: that filled
+    the registers of the whole kernel, and every address came back from scratch with a wait of its own."""
+    for kt, lines in wide_row_kernels.items():
+        assert [line for line in lines if "scratch_" in line] == [], kt

@@ -368,29 +368,45 @@ TRI_DEV void bwd_uniform_row(const BwdArgs& a, int bh, int i, unsigned char* sme
     }
     __builtin_amdgcn_wave_barrier();
   }
-  // the waves' parts, in wave order
+  // The waves' parts, in wave order.  A wave's turn is one run of reads, adds and writes without a branch, at immediates from two bases
+  // that are made in the turn.  (One address per element, made before the turns, took every register of the kernel: at d = 64 they came
+  // back from scratch one by one, and the loop over the query tiles of the other rows had a reload of its own.  This kernel alone, h = 4, d = 64,
+  // bf16, us: n = 256 with 60 valid 399 -> 156, 199 valid 185 -> 118, n = 384 with 300 valid 388 -> 262; without padding n = 256, h = 8 197 -> 194, n = 330
+  // 219 -> 215, b = 2, h = 8, n = 384 in fp16 1004 -> 978.)
   for (int w = 0; w < NW; ++w) {
     if (wave == w) {
+      int ln = lane;
+      asm volatile("" : "+v"(ln));
+      const int row0 = 4 * (ln >> 5), col0 = ln & 31;
+      float *const p1 = m1 + row0 * D + col0, *const pv = sk + row0;
+      auto add = [&](auto first_tag, auto vectors_tag) __attribute__((always_inline)) {
+        constexpr bool FIRST = decltype(first_tag)::value, VECTORS = decltype(vectors_tag)::value;
+        auto sum = [](float& at, float x) { at = x + (FIRST ? 0.f : at); };
 #pragma unroll
-      for (int mt = 0; mt < DM; ++mt)
+        for (int mt = 0; mt < DM; ++mt)
 #pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const int row = 32 * mt + crow(v, g);
-          if (row >= D) continue;
+          for (int v = 0; v < 16; ++v) {
+            const int row = 32 * mt + crow(v, 0);  // (the other half of the lanes: four rows on)
+            if (row + 4 >= D) continue;
+            if constexpr (VECTORS) {
+              sum(pv[row], ak[mt][v]);
+              sum(pv[D + row], aq[mt][v]);
+              sum(pv[2 * D + row], ao[mt][v]);
+            } else {
 #pragma unroll
-          for (int nt = 0; nt < DM; ++nt) {
-            const int col = 32 * nt + jl;
-            if (col < D) {
-              m1[row * D + col] = acc1[mt][nt][v] + (w ? m1[row * D + col] : 0.f);
-              m2[row * D + col] = acc2[mt][nt][v] + (w ? m2[row * D + col] : 0.f);
+              for (int nt = 0; nt < DM; ++nt) {
+                sum(p1[row * D + 32 * nt], acc1[mt][nt][v]);
+                sum(p1[D * D + row * D + 32 * nt], acc2[mt][nt][v]);
+              }
             }
           }
-          if (jl == 0) {
-            sk[row] = ak[mt][v] + (w ? sk[row] : 0.f);
-            sq[row] = aq[mt][v] + (w ? sq[row] : 0.f);
-            so[row] = ao[mt][v] + (w ? so[row] : 0.f);
-          }
-        }
+      };
+      auto turn = [&](auto first_tag) __attribute__((always_inline)) {
+        if (D % 32 == 0 || col0 < D) add(first_tag, std::false_type{});
+        if (col0 == 0) add(first_tag, std::true_type{});
+      };
+      if (w == 0) turn(std::true_type{});
+      else turn(std::false_type{});
     }
     __syncthreads();
   }
