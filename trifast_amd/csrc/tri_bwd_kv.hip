@@ -10,7 +10,7 @@ struct BwdKVFamily {
   // {NW, R, BJ}: block of NW*32 keys x R pair rows, queries streamed BJ at a time
   static constexpr int P(int tile, int which) {
     constexpr int t[kNumTiles][3] = {
-        {4, 1, 64},  // 0: 128 keys x 1 row,  64 queries per stage (fits every dtype / head dim)
+        {4, 1, 64},  // 0: 128 keys x 1 row,  64 queries per stage, or 32 in a ring (see bwd_kv_ring; fits every dtype / head dim)
         {4, 2, 32},  // 1: 128 keys x 2 rows, 32 queries per stage
         {4, 2, 64},  // 2: 128 keys x 2 rows, 64 queries per stage
         {2, 2, 32},  // 3:  64 keys x 2 rows, 32 queries per stage
@@ -29,7 +29,19 @@ struct BwdKVFamily {
     if constexpr (stage <= kMaxLds && (sizeof(T) == 4 ? R == 1 || (D <= 32 && NW == 4 && BJ == 32) : acc_regs <= 200 || R == 1)) {
       if (dry) return hipSuccess;
       dim3 grid((a.N + NW * 32 - 1) / (NW * 32), ((a.N + R - 1) / R + 7) / 8 * 8, bh);
-      return launch_dyn(tri_bwd_kv_kernel<T, D, NW, R, BJ, nbuf>, grid, dim3(NW * 64), bwd_kv_lds_bytes(D, (int)sizeof(T), NW, R, BJ, nbuf), st, a);
+      auto launch = [&](auto ring_tag) {
+        constexpr bool RING = decltype(ring_tag)::value;
+        return launch_dyn(tri_bwd_kv_kernel<T, D, NW, R, BJ, nbuf, RING>, grid, dim3(NW * 64), bwd_kv_lds_bytes(D, (int)sizeof(T), NW, R, BJ, nbuf, RING), st, a);
+      };
+      constexpr bool has_ring = bwd_kv_ring(D, (int)sizeof(T), R);
+      if constexpr (has_ring && bwd_kv_ring_always(D)) {
+        return launch(std::true_type{});
+      } else {
+        if constexpr (has_ring) {
+          if (bwd_kv_ring_pays(a.N)) return launch(std::true_type{});
+        }
+        return launch(std::false_type{});
+      }
     } else {
       return hipErrorInvalidConfiguration;
     }
@@ -54,7 +66,7 @@ int bwd_kv_num_tiles() { return BwdKVFamily::kNumTiles + kBwdRowTiles; }
 bool bwd_kv_tile_writes_dq(int tile) { return tile >= BwdKVFamily::kNumTiles && tile < bwd_kv_num_tiles(); }
 
 TileInfo bwd_kv_tile_info(int tile) {
-  // block_j = queries per LDS stage, block_k = keys per workgroup
+  // block_j = queries per LDS stage (tile 0 of the 16-bit types: of the version without the ring), block_k = keys per workgroup
   // (row-resident tiles: four waves; short rows of up to 64 bytes run on one or two with as many key tiles in all.  The numbers
   // are the tile's name in saved picks)
   if (bwd_kv_tile_writes_dq(tile)) return TileInfo{32, 128 * kRowKeyTiles[tile - BwdKVFamily::kNumTiles], 4};

@@ -5,8 +5,8 @@
 // dk, dv accumulators stay in registers, and the queries of the rows are streamed
 // through LDS in tiles of BJ (direct global->LDS loads, double-buffered, swizzled;
 // rows of Q and dO, the lse and delta operand words left by the dq kernel, and the packed
-// bias tiles).  With one pair row per workgroup and rows of 64 bytes or more (16-bit types) the tiles are 32 queries, whatever BJ says,
-// in a ring of four.  Scores are computed UN-transposed here, S = Q K^T, so that a lane
+// bias tiles).  With one pair row per workgroup the 16-bit types also have a version whose tiles are 32 queries, whatever BJ says, in
+// a ring of four (RING, see bwd_kv_ring).  Scores are computed UN-transposed here, S = Q K^T, so that a lane
 // owns one key (column) and 16 queries of every 32-query tile: P and dS are then
 // already in B-operand layout for the two products that contract over queries,
 //   dv^T += dO^T P,   dk^T += Q^T dS,   dk = dk^T / sqrt(d),
@@ -38,13 +38,18 @@ constexpr int bwd_kv_stage_bytes(int D, int es, int NW, int R, int BJ) {
 // The ring of 32-query stages (one pair row, 16-bit types; whole loads for every wave): a stage's rows and bias tiles, then lse2 and -delta
 // of its queries once per wave.
 constexpr int kBwdKVStages = 4;
+// Where there is a version with the ring, and the rows that take it: all at head dim 64. At 32 and 128 its stages, twice as many, cost
+// more than their waits where the other version's last stage of 64 queries is more than half full, and save the empty half of it where it is not
+// (this kernel alone, stages of 64 / ring, bf16, h = 4, us: d = 128, n = 100 29.9 / 31.4, 256 160.4 / 163.5, 300 293.5 / 304.3, 384 436 / 446, 500 934 / 956,
+// 768 2740 / 2790; n = 160 76.9 / 72.2, 200 124.0 / 117.9, 600 1551 / 1527; d = 32, n = 300 73.5 / 78.3, 384 111 / 114; n = 200 with padding 33.9 / 33.3; d = 64, n = 384
+// 186.2 / 182.6, 401 267 / 237, 512 387 / 386, 700 1007 / 957, 900 2148 / 2022).
 constexpr bool bwd_kv_ring(int D, int es, int R) { return es == 2 && R == 1 && D >= 32; }
+constexpr bool bwd_kv_ring_always(int D) { return D == 64; }
+constexpr bool bwd_kv_ring_pays(int n) { return (n - 1) % 64 < 32; }
 constexpr int bwd_kv_ring_stage_bytes(int D, int es, int NW) { return ring_stage_bytes(D, es, NW, 1) + NW * 256; }
 // LDS bytes of a workgroup
-constexpr int bwd_kv_lds_bytes(int D, int es, int NW, int R, int BJ, int nbuf) {
-  const int stages = nbuf * bwd_kv_stage_bytes(D, es, NW, R, BJ);
-  const int ring = bwd_kv_ring(D, es, R) ? kBwdKVStages * bwd_kv_ring_stage_bytes(D, es, NW) : 0;
-  return stages > ring ? stages : ring;
+constexpr int bwd_kv_lds_bytes(int D, int es, int NW, int R, int BJ, int nbuf, bool ring) {
+  return ring ? kBwdKVStages * bwd_kv_ring_stage_bytes(D, es, NW) : nbuf * bwd_kv_stage_bytes(D, es, NW, R, BJ);
 }
 
 // Two waves per SIMD (at most 256 registers) wherever the tile fits them or nearly
@@ -56,7 +61,7 @@ constexpr int bwd_kv_min_waves() {
   return (row_bytes >= 512 || (row_bytes == 128 && R == 1) || (row_bytes <= 64 && R * BJ <= 64)) ? 2 : 1;
 }
 
-template <typename T, int D, int NW, int R, int BJ, int NBUF>
+template <typename T, int D, int NW, int R, int BJ, int NBUF, bool RING>
 __global__ __launch_bounds__(NW * 64, (bwd_kv_min_waves<T, D, R, BJ>())) void tri_bwd_kv_kernel(const BwdArgs a) {
   using E = Elem<T>;
   using frag = typename E::frag;
@@ -472,7 +477,7 @@ __global__ __launch_bounds__(NW * 64, (bwd_kv_min_waves<T, D, R, BJ>())) void tr
     wait_dma();  // (the last prefetches are still on their way into LDS)
   };
 
-  if constexpr (bwd_kv_ring(D, (int)sizeof(T), R)) {
+  if constexpr (RING) {
     constexpr std::integral_constant<int, kBwdKVStages> stages{};
     if (wave_active && !flagged[0] && tile_live[0]) ring_loop(std::true_type{}, stages);
     else ring_loop(std::false_type{}, stages);
