@@ -65,46 +65,66 @@ constexpr int fwd_main_lds_bytes(int D, int es, int NW, int R, int BKF) {
 // R fully masked rows (the padding of a padded batch): all logits of such a row are equal, so
 // every query's output is the mean of the row's V and its log-sum-exp is ln n.  One pass over V
 // instead of a sweep of score tiles: the workgroup's threads take the 16-byte chunks of V's rows
-// in turn, add them in fp32 in a fixed order and meet in LDS.  (n = 512 of which 115 rows are
-// padding: 160 -> 136 us.)
-template <typename T, int D, int NW, int R>
+// in turn, add them in fp32 in a fixed order and meet in LDS, all rows at the same barriers.  (n = 512 of which 115 rows are
+// padding: 160 -> 136 us.  Row after row, with a barrier of its own for the dropped first stage, what that stage costs these rows
+// was not made up for: half of the rows padding, bf16, us, before the stage was requested early / with it / now: h = 4, d = 16, n = 256
+// 16.9 / 17.7 / 16.4, n = 512 63.7 / 63.4 / 57.2; h = 8, d = 64, n = 256 46.9 / 48.0 / 45.9; h = 4, d = 128, n = 300 69.5 / 71.0 / 68.2, 512
+// 232 / 236 / 219.  One row per workgroup gains nothing by meeting: d = 128, n = 128 15.5 / 15.8 / 15.9, h = 8, n = 200 56.1 / 57.6 / 57.6.)
+template <typename T, int D, int NW, int R, int LDS>
 TRI_DEV void fwd_uniform_rows(const FwdArgs& a, const T* vbh, int bh, int i0, int j_blk, unsigned char* smem) {
   using vec = typename Elem<T>::vec;
   constexpr int VEC = Elem<T>::VEC, CH = D / VEC, SLOTS = NW * 64 / CH;  // chunks per row, threads per chunk
   const int N = a.N, tid = threadIdx.x, ch = tid % CH, slot = tid / CH;
-  float (*part)[D] = reinterpret_cast<float (*)[D]>(smem);  // [SLOTS][D]
+  // rows at a time: their parts meet in the LDS of the workgroup's stages
+  constexpr int G = R * SLOTS * D * 4 <= LDS ? R : R / 2;
+  static_assert(G * SLOTS * D * 4 <= LDS);
+  float (*part)[SLOTS][D] = reinterpret_cast<float (*)[SLOTS][D]>(smem);  // [G]
   const float lse = kLn2 * fast_log2((float)N) + a.neg_inf;
 #pragma unroll 1
-  for (int r = 0; r < R; ++r) {
-    const int i = i0 + r;
-    if (i >= N) break;
-    const T* v = vbh + i * a.sv.i + ch * VEC;
-    float acc[VEC] = {};
-#pragma unroll 4
-    for (int k = slot; k < N; k += SLOTS) {
-      const vec x = *reinterpret_cast<const vec*>(v + (int64_t)k * a.sv.j);
+  for (int r0 = 0; r0 < R; r0 += G) {
+    const T* v[G];
+    float acc[G][VEC] = {};
 #pragma unroll
-      for (int e = 0; e < VEC; ++e) acc[e] += (float)x[e];
+    for (int r = 0; r < G; ++r) v[r] = vbh + min(i0 + r0 + r, N - 1) * a.sv.i + ch * VEC;  // (rows past the end are not stored)
+#pragma unroll 8 / G
+    for (int k = slot; k < N; k += SLOTS) {  // (eight loads in flight)
+      vec x[G];
+#pragma unroll
+      for (int r = 0; r < G; ++r) x[r] = *reinterpret_cast<const vec*>(v[r] + (int64_t)k * a.sv.j);
+#pragma unroll
+      for (int r = 0; r < G; ++r)
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) acc[r][e] += (float)x[r][e];
     }
-    __syncthreads();  // (the row before has been read)
+    if (r0 == 0) wait_dma();  // (the first stage, requested before the row flags were read, has landed in this LDS)
+    __syncthreads();          // (the rows before have been read)
 #pragma unroll
-    for (int e = 0; e < VEC; ++e) part[slot][ch * VEC + e] = acc[e];
+    for (int r = 0; r < G; ++r)
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) part[r][slot][ch * VEC + e] = acc[r][e];
 #pragma unroll
     for (int half = SLOTS / 2; half > 0; half /= 2) {
       __syncthreads();
       if (slot < half) {
 #pragma unroll
-        for (int e = 0; e < VEC; ++e) part[slot][ch * VEC + e] += part[slot + half][ch * VEC + e];
+        for (int r = 0; r < G; ++r)
+#pragma unroll
+          for (int e = 0; e < VEC; ++e) part[r][slot][ch * VEC + e] += part[r][slot + half][ch * VEC + e];
       }
     }
     __syncthreads();
-    vec out;
 #pragma unroll
-    for (int e = 0; e < VEC; ++e) out[e] = (T)(part[0][ch * VEC + e] / (float)N);
-    const int64_t row = ((int64_t)bh * N + i) * N;
-    T* o = reinterpret_cast<T*>(a.o) + row * D + ch * VEC;
-    for (int j = j_blk + slot; j < min(j_blk + NW * 32, N); j += SLOTS) *reinterpret_cast<vec*>(o + (int64_t)j * D) = out;
-    if (tid < NW * 32 && j_blk + tid < N) a.lse[row + j_blk + tid] = lse;
+    for (int r = 0; r < G; ++r) {
+      const int i = i0 + r0 + r;
+      if (i >= N) break;
+      vec out;
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) out[e] = (T)(part[r][0][ch * VEC + e] / (float)N);
+      const int64_t row = ((int64_t)bh * N + i) * N;
+      T* o = reinterpret_cast<T*>(a.o) + row * D + ch * VEC;
+      for (int j = j_blk + slot; j < min(j_blk + NW * 32, N); j += SLOTS) *reinterpret_cast<vec*>(o + (int64_t)j * D) = out;
+      if (tid < NW * 32 && j_blk + tid < N) a.lse[row + j_blk + tid] = lse;
+    }
   }
 }
 
@@ -303,8 +323,7 @@ __global__ __launch_bounds__(NW * 64, (R * ((BKF % kFwdFast) / 32) >= 8 || D * s
     all_flagged &= flagged[r];
   }
   if (all_flagged) {
-    if constexpr (sizeof(T) == 2) drop_loads();
-    fwd_uniform_rows<T, D, NW, R>(a, vbh, bh, i0, bx * (NW * 32), tri_smem);
+    fwd_uniform_rows<T, D, NW, R, LDS_MAIN>(a, vbh, bh, i0, bx * (NW * 32), tri_smem);
     return;
   }
 #pragma unroll
