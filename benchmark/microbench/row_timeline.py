@@ -58,10 +58,10 @@ def main():
     if not lib.trifast_bwd_kv_tile_writes_dq(tile):
         sys.exit(f"the default dk/dv tile of workload {args.workload} is not the row-resident kernel")
     kt = lib.trifast_num_tiles(_lib.KERNEL_BWD_KV)  # (only to show the tile id range)
-    rows = b * h * n
     ws = torch.zeros(lib.trifast_bwd_workspace_bytes(b, h, n, d, code), dtype=torch.uint8, device="cuda")
     dq, dk, dv = (torch.zeros_like(o) for _ in range(3))
-    rec_buf = torch.zeros(max(rows * 32, bias.numel() // 4 + 1), dtype=torch.int64, device="cuda")
+    records = b * h * (n + 7)  # (workgroups of a launch: the rows of a head rounded up to the XCDs that share it)
+    rec_buf = torch.zeros(max(records * 32, bias.numel() // 4 + 1), dtype=torch.int64, device="cuda")
     mu8 = mask.view(torch.uint8)
     S = lambda t: _lib.i64_array(tt._strides(t))
     stream = torch.cuda.current_stream().cuda_stream
@@ -81,15 +81,11 @@ def main():
     run()
     e.record()
     e.synchronize()
-    info = _lib.tile_info(_lib.KERNEL_BWD_KV, tile)
-    KT = info["BLOCK_K"] // 128
-    short = d <= 32 and n <= 512  # (tri_bwd_row_short.hpp: one wave, or two)
-    if short:
-        KT = (n + 31) // 32 if n <= 256 else ((n + 31) // 32 + 1) // 2
-    print(f"workload {args.workload}: row-resident tile {tile} of {kt} ({KT} key tiles per wave), timing build: {s.elapsed_time(e):.3f} ms per launch")
-
-    rec = rec_buf[: rows * 32].view(rows, 32).cpu()
+    rec = rec_buf[: records * 32].view(records, 32).cpu()
     rec = rec[rec[:, 0] != 0]
+    # (the kernel that ran says what it was: which one a row takes depends on its length and on the number of rows)
+    KT, waves, short = (int(x) for x in rec[0, 28:31])
+    print(f"workload {args.workload}: row-resident tile {tile} of {kt} ({'short rows, ' if short else ''}{waves} waves of {KT} key tiles), timing build: {s.elapsed_time(e):.3f} ms per launch")
     t0 = int(rec[:, 0].min())
     us = lambda a, bcol: (rec[:, bcol] - rec[:, a]).double() / 100
     stat = lambda x: f"{x.mean():7.2f} (min {x.min():.2f}, max {x.max():.2f})"

@@ -416,3 +416,28 @@ def test_fully_masked_rows_of_the_forward_load_together(tmp_path):
         # (the only loop without products that loads 16 bytes a lane into registers; the one that is left over when it is unrolled has fewer)
         passes = [x for x in loops if not any("v_mfma" in y or "s_barrier" in y for y in x) and any("global_load_dwordx4" in y for y in x)]
         assert max(sum("global_load_dwordx4" in y for y in x) for x in passes) == 8, r
+
+
+def test_row_timeline_probe_spills_no_scalars(tmp_path):
+    """The build that times the row-resident backward runs the loop of the regular one where every key is attended: its readings stay
+    in scalar registers (spilled ones made the steps 50 clocks longer than they are)."""
+    import re
+    import subprocess
+
+    from trifast_amd import build
+
+    if build._compiler_flags():
+        pytest.skip("not the compiler that the kernels are laid out for")
+    source, asm = tmp_path / "row.hip", tmp_path / "row.s"
+    source.write_text('#include "tri_bwd_row.hpp"\nnamespace tri {\ntemplate __global__ void tri_bwd_row_kernel<__bf16, 32, 8, false>(const BwdArgs);\n}\n')
+    cmd = [build._hipcc(), *build.HIPCC_FLAGS, "-DTRI_ROW_TIMING", "--cuda-device-only", "-S", "-I", str(build.CSRC), "-o", str(asm), str(source)]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    assert res.returncode == 0, res.stderr[-2000:]
+    lines = asm.read_text().splitlines()
+    label = {m.group(1): at for at, line in enumerate(lines) if (m := re.match(r"(\.LBB\w+):", line))}
+    loops = [lines[label[m.group(1)]:at + 1] for at, line in enumerate(lines)
+             if (m := re.match(r"\s+s_c?branch\w*\s+(\.LBB\w+)", line)) and label[m.group(1)] <= at]
+    # (16 exponentials of every key tile, and the clock once per step; the loops over fully masked rows have neither)
+    loops = [x for x in loops if "Inner Loop" in x[0] and sum("v_exp_f32" in y for y in x) == 128 and any("s_memtime" in y for y in x)]
+    assert len(loops) == 2
+    assert min(sum(bool(re.match(r"\s+v_(read|write)lane", y)) for y in x) for x in loops) == 0

@@ -65,16 +65,18 @@
 // -DTRI_ROW_TIMING builds the kernel as a probe of itself (benchmark/microbench/row_timeline.py):
 // wave 0 of every workgroup reads the 100 MHz counter at the marks below and the shader clock
 // between the steps of the query-tile loop, and leaves the readings where the db argument
-// points (a buffer of the caller's; db itself is not computed by this kernel).
+// points (a buffer of the caller's; db itself is not computed by this kernel).  Of a reading only the low
+// word is kept, and what is known before the loop is written before it: with all of them held to the end the
+// loop spilled scalar registers, and its steps took 60 clocks longer (n = 1024, d = 32: 7910 clocks per query tile, now 7380).
 #ifdef TRI_ROW_TIMING
 #define TRI_ROW_MARK(var)               \
   __builtin_amdgcn_sched_barrier(0);    \
-  const uint64_t var = __builtin_amdgcn_s_memrealtime(); \
+  const uint32_t var = (uint32_t)__builtin_amdgcn_s_memrealtime(); \
   __builtin_amdgcn_sched_barrier(0)
 #define TRI_ROW_TICK(k)                                      \
   do {                                                       \
     __builtin_amdgcn_sched_barrier(0);                       \
-    const uint64_t now_ = __builtin_amdgcn_s_memtime();      \
+    const uint32_t now_ = (uint32_t)__builtin_amdgcn_s_memtime(); \
     tacc[k] += now_ - tprev;                                 \
     tprev = now_;                                            \
     __builtin_amdgcn_sched_barrier(0);                       \
@@ -1011,6 +1013,15 @@ __global__ __launch_bounds__(kRowWaves * 64, bwd_row_two_waves(D, KT) ? 2 : 1) v
   };
 
   TRI_ROW_MARK(t_p4);
+#ifdef TRI_ROW_TIMING
+  // one record of 32 words per workgroup (first wave), at the start of what db points to
+  uint64_t* const rec = reinterpret_cast<uint64_t*>(a.db) + (int64_t)L * 32;
+  if (wave == 0 && lane == 0) {
+    const uint64_t t = __builtin_amdgcn_s_memrealtime();
+    const uint32_t marks[5] = {t_entry, t_p1, t_p2, t_p3, t_p4};  // 100 MHz
+    for (int x = 0; x < 5; ++x) rec[x] = t - ((uint32_t)t - marks[x]);
+  }
+#endif
   wait_dma_known();
   __syncthreads();
 
@@ -1070,9 +1081,9 @@ __global__ __launch_bounds__(kRowWaves * 64, bwd_row_two_waves(D, KT) ? 2 : 1) v
     // next query tile, which has no vector work of its own.
     int buf = 0;  // jt % 3: the stage of this query tile
 #ifdef TRI_ROW_TIMING
-    uint64_t tacc[KT + 5] = {};  // shader clocks per step, summed over the query tiles
-    const uint64_t t_clk0 = __builtin_amdgcn_s_memtime(), t_loop0 = __builtin_amdgcn_s_memrealtime();
-    uint64_t tprev = t_clk0;
+    uint32_t tacc[KT + 5] = {};  // shader clocks per step, summed over the query tiles
+    const uint32_t t_clk0 = (uint32_t)__builtin_amdgcn_s_memtime(), t_loop0 = (uint32_t)__builtin_amdgcn_s_memrealtime();
+    uint32_t tprev = t_clk0;
 #endif
     for (int jt = 0; jt < NJ; ++jt) {
       const int buf_fill = buf == 0 ? 2 : buf - 1;  // (jt + 2) % 3: the stage to refill
@@ -1283,7 +1294,7 @@ __global__ __launch_bounds__(kRowWaves * 64, bwd_row_two_waves(D, KT) ? 2 : 1) v
       store_dq(NJ - 1, dq_base, dq_words);
     }
 #ifdef TRI_ROW_TIMING
-    const uint64_t t_clk1 = __builtin_amdgcn_s_memtime(), t_loop1 = __builtin_amdgcn_s_memrealtime();
+    const uint32_t t_clk1 = (uint32_t)__builtin_amdgcn_s_memtime(), t_loop1 = (uint32_t)__builtin_amdgcn_s_memrealtime();
 #endif
 
     // the words that the db kernel reads (each thread writes what its own wave has put there)
@@ -1315,16 +1326,18 @@ __global__ __launch_bounds__(kRowWaves * 64, bwd_row_two_waves(D, KT) ? 2 : 1) v
       store_rows_wide<T, D, DM>(dvrow + (int64_t)key * a.sdv.j, dvacc[t], 1.0f, g, key < N);
     }
 #ifdef TRI_ROW_TIMING
-    // one record of 32 words per workgroup (wave 0), at the start of what db points to
     if (wave == 0 && lane == 0) {
-      uint64_t* rec = reinterpret_cast<uint64_t*>(a.db) + (int64_t)L * 32;
       const uint64_t t_end = __builtin_amdgcn_s_memrealtime();
-      const uint64_t marks[8] = {t_entry, t_p1, t_p2, t_p3, t_p4, t_loop0, t_loop1, t_end};  // 100 MHz
-      for (int x = 0; x < 8; ++x) rec[x] = marks[x];
+      rec[5] = t_end - ((uint32_t)t_end - t_loop0);
+      rec[6] = t_end - ((uint32_t)t_end - t_loop1);
+      rec[7] = t_end;
       rec[8] = __builtin_amdgcn_s_getreg(4 | (0 << 6) | (31 << 11));   // HW_ID
       rec[9] = __builtin_amdgcn_s_getreg(20 | (0 << 6) | (31 << 11));  // XCC_ID
-      rec[10] = t_clk1 - t_clk0;                                        // shader clocks of the loop
+      rec[10] = (uint32_t)(t_clk1 - t_clk0);                            // shader clocks of the loop
       for (int x = 0; x < KT + 5; ++x) rec[11 + x] = tacc[x];
+      rec[28] = KT;  // what the record is of: key tiles per wave, waves per row, kernel (0: this one, 1: short rows)
+      rec[29] = NW;
+      rec[30] = 0;
     }
 #endif
   };

@@ -22,8 +22,13 @@ hipError_t bwd_row_run_short(const BwdArgs& a, int bh, hipStream_t st, bool dry)
 template <typename T, int D, int KT>
 hipError_t bwd_row_run_four(const BwdArgs& a, int bh, hipStream_t st, bool dry) {
   constexpr int DM = (D + 31) / 32, lds = bwd_row_lds_bytes(D, (int)sizeof(T), KT, false);
+#ifdef TRI_ROW_TIMING
+  constexpr bool builds = D < 64 || KT < 4;  // (the compiler (ROCm 7.2.0) ends with a segmentation fault in its pass over accumulator copies)
+#else
+  constexpr bool builds = true;
+#endif
   // the dk, dv accumulators of a wave's key tiles stay in registers (half of the file at most)
-  if constexpr (2 * KT * DM * 16 <= 256 && lds <= kMaxLds) {
+  if constexpr (builds && 2 * KT * DM * 16 <= 256 && lds <= kMaxLds) {
     if (dry) return hipSuccess;
     const dim3 grid((unsigned)bwd_row_blocks(bh, a.N));
     return launch_dyn(tri_bwd_row_kernel<T, D, KT>, grid, dim3(kRowWaves * 64), lds, st, a);

@@ -317,6 +317,15 @@ __global__ __launch_bounds__(NW * 64, 1) void tri_bwd_row_short_kernel(const Bwd
 
   TRI_ROW_MARK(t_p3);
   TRI_ROW_MARK(t_p4);
+#ifdef TRI_ROW_TIMING
+  // one record of 32 words per workgroup (first wave), at the start of what db points to
+  uint64_t* const rec = reinterpret_cast<uint64_t*>(a.db) + (int64_t)L * 32;
+  if (wave == 0 && lane == 0) {
+    const uint64_t t = __builtin_amdgcn_s_memrealtime();
+    const uint32_t marks[5] = {t_entry, t_p1, t_p2, t_p3, t_p4};  // 100 MHz
+    for (int x = 0; x < 5; ++x) rec[x] = t - ((uint32_t)t - marks[x]);
+  }
+#endif
   wait_dma_known();
   __syncthreads();
 
@@ -357,9 +366,9 @@ __global__ __launch_bounds__(NW * 64, 1) void tri_bwd_row_short_kernel(const Bwd
     int buf = 0;               // jt % 2: the stage of this query tile
     int jt = 0;
 #ifdef TRI_ROW_TIMING
-    uint64_t tacc[KT + 5] = {};  // shader clocks per step, summed over the query tiles
-    const uint64_t t_clk0 = __builtin_amdgcn_s_memtime(), t_loop0 = __builtin_amdgcn_s_memrealtime();
-    uint64_t tprev = t_clk0;
+    uint32_t tacc[KT + 5] = {};  // shader clocks per step, summed over the query tiles
+    const uint32_t t_clk0 = (uint32_t)__builtin_amdgcn_s_memtime(), t_loop0 = (uint32_t)__builtin_amdgcn_s_memrealtime();
+    uint32_t tprev = t_clk0;
 #endif
 
     // ---- the state that moves from step to step --------------------------------------
@@ -585,7 +594,7 @@ __global__ __launch_bounds__(NW * 64, 1) void tri_bwd_row_short_kernel(const Bwd
     static_for<kSumPieces>([&](auto pc) __attribute__((always_inline)) { sum_dq_piece(pc, (NJ - 1) & 1, NJ - 1, dqacc, dq_out); });
     store_dq(dq_base, dq_out);
 #ifdef TRI_ROW_TIMING
-    const uint64_t t_clk1 = __builtin_amdgcn_s_memtime(), t_loop1 = __builtin_amdgcn_s_memrealtime();
+    const uint32_t t_clk1 = (uint32_t)__builtin_amdgcn_s_memtime(), t_loop1 = (uint32_t)__builtin_amdgcn_s_memrealtime();
 #endif
 
     // ---- dk, dv of this wave's keys -------------------------------------------------------
@@ -604,16 +613,18 @@ __global__ __launch_bounds__(NW * 64, 1) void tri_bwd_row_short_kernel(const Bwd
       store_rows_wide<T, D, 1>(dvrow + (int64_t)key * a.sdv.j, &dvacc[t], 1.0f, g, key < N);
     }
 #ifdef TRI_ROW_TIMING
-    // one record of 32 words per workgroup (first wave), at the start of what db points to
     if (wave == 0 && lane == 0) {
-      uint64_t* rec = reinterpret_cast<uint64_t*>(a.db) + (int64_t)L * 32;
       const uint64_t t_end = __builtin_amdgcn_s_memrealtime();
-      const uint64_t marks[8] = {t_entry, t_p1, t_p2, t_p3, t_p4, t_loop0, t_loop1, t_end};  // 100 MHz
-      for (int x = 0; x < 8; ++x) rec[x] = marks[x];
+      rec[5] = t_end - ((uint32_t)t_end - t_loop0);
+      rec[6] = t_end - ((uint32_t)t_end - t_loop1);
+      rec[7] = t_end;
       rec[8] = __builtin_amdgcn_s_getreg(4 | (0 << 6) | (31 << 11));   // HW_ID
       rec[9] = __builtin_amdgcn_s_getreg(20 | (0 << 6) | (31 << 11));  // XCC_ID
-      rec[10] = t_clk1 - t_clk0;                                        // shader clocks of the loop
+      rec[10] = (uint32_t)(t_clk1 - t_clk0);                            // shader clocks of the loop
       for (int x = 0; x < KT + 3; ++x) rec[11 + x] = tacc[x];
+      rec[28] = KT;
+      rec[29] = NW;
+      rec[30] = 1;
     }
 #endif
   };
