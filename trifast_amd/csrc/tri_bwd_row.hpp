@@ -39,9 +39,11 @@
 // The prologue also computes delta = rowsum(o * do) of the row and leaves it, with
 // the row's log-sum-exp, in the per-query planes the db kernel reads.
 //
-// The loop over the query tiles has no branch: the compiler sinks what stands in front of one behind it, out of the schedule.  Lanes
-// and waves without a share are masked with exec inside asm statements, pointers advance by masked steps, transposing reads past the
-// columns of a short row return bytes nobody uses; nothing of the loop lies in scratch (a reload waits for every load in flight), which
+// In rows of one pass the loop over the query tiles has no branch: the compiler sinks what stands in front of one behind it, out of the schedule.
+// Lanes and waves without a share are masked with exec inside asm statements, pointers advance by masked steps, transposing reads past the
+// columns of a short row return bytes nobody uses; nothing of the loop lies in scratch (a reload waits for every load in flight).  (Not so
+// in rows of 128 bytes with four key tiles per wave, which the tuner alone takes: 11 reloads per query tile and a branch around the words; rows of several
+// passes branch on the first one; of the short rows 32 wide those of two waves with eight key tiles reload 16 bytes.)  It
 // is why masked key operands are made in the step and not kept.  Before that, on one card, this kernel alone, h = 4: d = 16, n = 700
 // 786 -> 652 us, n = 1024 1964 -> 1607; d = 32, n = 600 546 -> 530, n = 768 951 -> 939, n = 1024 1995 -> 1980 (bound by issue and clock);
 // d = 64, n = 300 219 -> 195, h = 8, n = 256 240 -> 228, fp16, two of n = 384 with half of the keys masked 1172 -> 1140.
@@ -220,10 +222,12 @@ constexpr int64_t bwd_row_blocks(int bh, int n) {
 // units of each XCD) start one after the other instead, over about the time memory needs for their rows (16 bytes per element at 5
 // TB/s): 2 n d clocks.  That much later the last of them ends, so launches with few rounds take half of it, and rows that
 // compute for long, which gain least; one round has nothing to gain.  A wave sleeps at most 2 n d clocks once per launch.
-// bf16, us, this kernel alone, without -> with: d = 64, h = 8: n = 256 216.4 -> 209.1, n = 330 444 -> 419, two of n = 384 1056 -> 1032
-// (twice the time: 212.9, 409, 1015); d = 32, h = 4: n = 300 94.0 -> 88.8, n = 600 544 -> 527, n = 768 921 -> 897, n = 1024 1971
-// -> 1957; h = 5, n = 256 75.6 -> 72.2; h = 16, n = 128 39.5 -> 37.8.  Not halved: d = 64, h = 2, n = 256 58.1 -> 61.8 (halved 56.4); d = 32, h = 4,
-// n = 512 298 -> 301 (296).  Passes over longer rows: n = 1280 4211 -> 4258, so not there.
+// This kernel or that of the short rows alone, us, without -> with, h = 4 where not said: d = 16: h = 8, n = 160 35.8 -> 34.8; n = 300 83.4 -> 81.2, 384
+// 110.9 -> 108.3, 700 649 -> 643, 1024 1583 -> 1572; d = 32: h = 16, n = 128 39.2 -> 37.9; h = 3, n = 256 41.1 -> 40.0; n = 300 94.2 -> 89.0, 449
+// 264 -> 259, 600 533 -> 515, 1024 1917 -> 1890; d = 64 (fp16): h = 8, n = 256 209 -> 195; n = 200 87.4 -> 82.4, 300 183 -> 174, 384 265 -> 252.
+// In 118 launches of n = 90 to 1024 (46, 46 and 26 by head dim, half of them with padding) none lost more than its scatter.  Not
+// halved: d = 64, h = 2, n = 256 58.1 -> 61.8 (halved 56.4); d = 32, n = 512 298 -> 301 (296); twice the time: d = 64, h = 8, n = 256 216 -> 213.
+// Passes over longer rows: n = 1280 4211 -> 4258, so not there.
 TRI_DEV void stagger_rows(int block, int per_cu, int bh, int n, int d) {
   const int slot = block >> 3, round = 256 * per_cu;
   const int64_t rows = (int64_t)bh * n;
@@ -535,6 +539,7 @@ struct DeltaRows {
   // words(query, delta, lse) for every query
   template <typename Words>
   TRI_DEV void finish(int tid, Words words) {
+    static_assert(CPR <= 4, "the lanes of a row trade their parts within a quad");
     typedef T pair __attribute__((ext_vector_type(2)));
     const int c = tid % CPR;
 #pragma unroll
@@ -549,13 +554,12 @@ struct DeltaRows {
           for (int e = 0; e < 8; e += 2) s[y] = pair_dot(pair{ov[ld][e], ov[ld][e + 1]}, pair{dv[ld][e], dv[ld][e + 1]}, s[y]);
         }
       }
-      // (the partner across four lanes is lane 7 - c: any lane of the other four will do, the quad's parts are summed after it)
 #pragma unroll
       for (int m = CPR / 2; m > 0; m /= 2)
 #pragma unroll
         for (int y = 0; y < m; ++y) {
           const float keep = c & m ? s[y + m] : s[y], give = c & m ? s[y] : s[y + m];
-          s[y] = keep + (m == 4 ? dpp_move<0x141>(give) : m == 2 ? dpp_move<0x4e>(give) : dpp_move<0xb1>(give));
+          s[y] = keep + (m == 2 ? dpp_move<0x4e>(give) : dpp_move<0xb1>(give));
         }
       if ((x * CPR + c) * RPL < ROWS) words(query(x, tid), s[0], lv[x]);
     }
@@ -714,7 +718,6 @@ __global__ __launch_bounds__(kRowWaves * 64, bwd_row_two_waves(D, KT) ? 2 : 1) v
   for (int t = 0; t < KT; ++t)
     if (KT0 + NW * t + wave >= NJ) kw[t] = 0u;
   TRI_ROW_MARK(t_p1);
-  const uint32_t lanebit = 1u << kl;
 
   // V rows of this lane's keys as B operands: in registers for the wave's first VR key
   // tiles, in a private piece of LDS (operand by operand, 16 bytes per lane) for the rest

@@ -7,7 +7,7 @@
 // few key tiles per wave, is summed from the parts of all waves behind a barrier, and the start and the end of a row (K, V, o and do arrive;
 // dk and dv leave) had the compute unit to themselves.  Here
 // * a wave holds up to eight key tiles, as at n = 1024: rows of up to 256 keys are one wave's (four rows share a compute unit, nothing
-//   is exchanged, no barrier), rows of up to 512 two waves' (two rows share it).  Rows of a compute unit run apart, so one's loads and stores
+//   is exchanged, no barrier; few of them are spread, see bwd_row_run), rows of up to 512 two waves' (two rows share it).  Rows of a compute unit run apart, so one's loads and stores
 //   go on beside the other's arithmetic.
 // * the (query tile, key tile) pairs of a wave are one software pipeline that does not end with a query tile: a step holds the
 //   exponentials of its pair, the score and dP MFMAs of the pair after it and the dv, dk and dq MFMAs of the pair before it, the next
@@ -21,9 +21,9 @@
 // 36.0 us, 256 51.2 -> 45.3, 300 115 -> 94, 384 170 -> 142, 449 (interleaved heads) 319 -> 279, 512 343 -> 297, 512 with padding from 397
 // on 309 -> 287.  With eight heads at n = 256, two rounds of rows per SIMD, 98 -> 98: the start and end of a row are not hidden there.
 //
-// What bounds it: instruction issue, as in tri_bwd_row.hpp: a step with both neighbours takes about 780 clocks for 14 to 16 MFMAs (448 to 512
-// clocks of matrix pipe), 64 vector instructions of its pair and 50 others; the three steps that carry the query tile's own work (operands of the next
-// one, its delta, the requests and stores) 300 to 900 more.
+// What bounds it: instruction issue, as in tri_bwd_row.hpp: a step with both neighbours takes about 740 clocks for 14 to 16 MFMAs (448 to 512
+// clocks of matrix pipe), 64 vector instructions of its pair and 50 others (two waves, beside another row's on the same LDS: 820 to 880); the four
+// steps that carry the query tile's own work (operands of the next one, its delta, the requests and stores) 50 to 850 more.
 #pragma once
 #include "tri_bwd_row.hpp"
 
@@ -34,7 +34,7 @@ constexpr int bwd_short_red_bytes(int NW) { return 4 * (NW - 1) * 1024; }   // d
 constexpr int bwd_short_own_bytes(int NW) { return NW > 1 ? 4 * 1024 : 0; }  // ... and those a wave sums itself
 constexpr int bwd_short_stage_bytes(int D, int es) { return 3 * 32 * D * es; }
 // Key tiles per wave whose V operands live in LDS instead of registers (eight tiles: as many as LDS has room for)
-constexpr int bwd_short_v_lds_tiles(int D, int KT) { return KT * (D / 16) < 16 ? 0 : KT - (KT == 8 ? 3 : 2); }
+constexpr int bwd_short_v_lds_tiles(int D, int KT) { return KT * (D / 16) < 16 ? 0 : KT - 3; }
 constexpr int bwd_short_lds_bytes(int D, int es, int KT, int NW) {
   const int row = NW * KT * 32 * D * es + 2 * bwd_short_stage_bytes(D, es) + NW * 2048 + 2 * bwd_short_red_bytes(NW) + bwd_short_own_bytes(NW) +
                   NW * bwd_short_v_lds_tiles(D, KT) * (D / 16) * 1024;

@@ -471,7 +471,7 @@ TRI_DEV float pair_sum(f16x2 w, f16x2 ones, float acc) { return __builtin_amdgcn
 TRI_DEV float pair_dot(bf16x2 x, bf16x2 y, float acc) { return __builtin_amdgcn_fdot2_f32_bf16(x, y, acc, false); }
 TRI_DEV float pair_dot(f16x2 x, f16x2 y, float acc) { return __builtin_fmaf((float)x[1], (float)y[1], __builtin_fmaf((float)x[0], (float)y[0], acc)); }
 
-// the value of another lane of the row of 16 (CTRL: the hardware's lane pattern, 0xb1 = lane ^ 1, 0x4e = lane ^ 2, 0x141 = lane ^ 7)
+// the value of another lane of the quad (CTRL: the hardware's lane pattern, 0xb1 = lane ^ 1, 0x4e = lane ^ 2)
 template <int CTRL>
 TRI_DEV float dpp_move(float x) {
   return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xf, 0xf, true));
