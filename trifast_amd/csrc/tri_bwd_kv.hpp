@@ -41,8 +41,8 @@ constexpr int kBwdKVStages = 4;
 // Where there is a version with the ring, and the rows that take it: all at head dim 64. At 32 and 128 its stages, twice as many, cost
 // more than their waits where the other version's last stage of 64 queries is more than half full, and save the empty half of it where it is not
 // (this kernel alone, stages of 64 / ring, bf16, h = 4, us: d = 128, n = 100 29.9 / 31.4, 256 160.4 / 163.5, 300 293.5 / 304.3, 384 436 / 446, 500 934 / 956,
-// 768 2740 / 2790; n = 160 76.9 / 72.2, 200 124.0 / 117.9, 600 1551 / 1527; d = 32, n = 300 73.5 / 78.3, 384 111 / 114; n = 200 with padding 33.9 / 33.3; d = 64, n = 384
-// 186.2 / 182.6, 401 267 / 237, 512 387 / 386, 700 1007 / 957, 900 2148 / 2022).
+// 768 2740 / 2790; n = 160 76.9 / 72.2, 200 124.0 / 117.9, 600 1551 / 1527; d = 32, n = 300 73.5 / 78.3, 384 111 / 114; h = 8, n = 96 14.6 / 13.9; h = 2, n = 600 211 / 211,
+// with padding 195 / 184, 850 562 / 570, with padding 505 / 479; d = 64, n = 384 186.2 / 182.6, 401 267 / 237, 512 387 / 386, 700 1007 / 957, 900 2148 / 2022).
 constexpr bool bwd_kv_ring(int D, int es, int R) { return es == 2 && R == 1 && D >= 32; }
 constexpr bool bwd_kv_ring_always(int D) { return D == 64; }
 constexpr bool bwd_kv_ring_pays(int n) { return (n - 1) % 64 < 32; }
