@@ -441,3 +441,26 @@ def test_row_timeline_probe_spills_no_scalars(tmp_path):
     loops = [x for x in loops if "Inner Loop" in x[0] and sum("v_exp_f32" in y for y in x) == 128 and any("s_memtime" in y for y in x)]
     assert len(loops) == 2
     assert min(sum(bool(re.match(r"\s+v_(read|write)lane", y)) for y in x) for x in loops) == 0
+
+
+# (key tiles, head dim, rows per XCD): the form of the row-resident backward that was measured to be at least 4 % faster there than the other
+ROW_FORMS = {
+    "kOneWave": [(5, 32, 65), (5, 16, 140), (5, 32, 260), (6, 32, 66), (6, 16, 110), (6, 32, 215), (6, 16, 384), (7, 32, 100), (7, 16, 250), (7, 32, 252),
+                 (8, 32, 115), (8, 16, 128), (3, 32, 70), (4, 16, 84), (4, 32, 140)],
+    "kTwoWaves": [(4, 32, 64), (9, 16, 65), (10, 32, 75), (11, 32, 42), (11, 16, 126), (12, 32, 144), (13, 16, 150), (16, 32, 64)],
+    "kFourWaves": [(3, 32, 9), (5, 16, 54), (6, 32, 43), (6, 32, 129), (6, 16, 144), (7, 32, 140), (7, 16, 175), (7, 32, 280), (7, 16, 400), (7, 32, 450), (8, 32, 64), (8, 16, 145),
+                   (8, 32, 160), (8, 16, 192), (8, 32, 261), (8, 16, 288), (8, 32, 384), (8, 16, 416), (8, 32, 768), (11, 32, 83)],
+}
+
+
+def test_waves_of_a_row_where_one_form_is_faster(tmp_path):
+    import subprocess
+
+    from trifast_amd import build
+
+    checks = "".join(f"static_assert(tri::bwd_row_form({w}, {d}, {r}) == tri::RowForm::{form}, \"{w} key tiles, head dim {d}, {r} rows\");\n"
+                     for form, launches in ROW_FORMS.items() for w, d, r in launches)
+    source = tmp_path / "rule.cpp"
+    source.write_text('#include "tri_bwd_row_rule.hpp"\n' + checks)
+    res = subprocess.run(["g++", "-std=c++17", "-fsyntax-only", "-I", str(build.CSRC), str(source)], capture_output=True, text=True)
+    assert res.returncode == 0, res.stderr[-2000:]

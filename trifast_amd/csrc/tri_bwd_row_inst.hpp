@@ -2,6 +2,7 @@
 // (one translation unit per type, so that they compile in parallel).
 #pragma once
 #include "tri_bwd_row.hpp"
+#include "tri_bwd_row_rule.hpp"
 #include "tri_bwd_row_short.hpp"
 #include "tri_dispatch.hpp"
 
@@ -40,36 +41,30 @@ hipError_t bwd_row_run_four(const BwdArgs& a, int bh, hipStream_t st, bool dry) 
 template <typename T, int D, int KT>
 hipError_t bwd_row_run(const BwdArgs& a, int bh, hipStream_t st, bool dry) {
   if (a.N > kRowWaves * KT * 32) return hipErrorInvalidConfiguration;
-  if constexpr (D <= 32 && KT == 2) {
-    // Up to 256 keys: one wave with as many key tiles as the row has, four rows to a compute unit.  Launches whose rows do not fill the
-    // SIMDs that way spread a row over more of them, as long as no XCD (32 compute units) gets a second round by it: two waves per row with three and four
-    // key tiles and up to 64 rows per XCD, the four waves of the other kernel with up to 32 (one row to a compute unit), and with five and more
-    // up to 64 (eight: 96, where one wave would take its row for longest).  This kernel alone, bf16, d = 32, us, one wave / two / four: rows per XCD
-    // 9 (h = 1, n = 70) 13.3 / 12.9 / 12.6, 27 (h = 3, n = 70) 13.6 / 13.2 / 12.8, 32 (h = 2, n = 128) 15.8 / 13.9 / 14.0, 35 (h = 4, n = 70) 14.0 / 13.6 / 14.9,
-    // 64 (h = 4, n = 128) 18.3 / 16.5 / 18.3, 65 (h = 5, n = 100) 18.4 / 23.9 / 24.3; one wave / four: six key tiles 43 (h = 2, n = 170) 26.4 / 22.2, 66 (h = 3) 28.4 /
-    // 31.4, seven 75 (h = 3, n = 200) 33.9 / 34.1, eight 64 (h = 2, n = 256) 38.6 / 29.7, 87 (h = 3, n = 230) 41.4 / 38.9, 96 (n = 256) 41.0 / 39.9, 128 (h = 4) 45.4 / 48.1.
-    const int64_t per_xcd = bwd_row_blocks(bh, a.N) / 8;
-    if (a.nwords > 2 && a.nwords <= 4) {
-      if (per_xcd <= 32) return bwd_row_run_four<T, D, 2>(a, bh, st, dry);
-      if (per_xcd <= 64) return bwd_row_run_short<T, D, 2, 2>(a, bh, st, dry);
-    } else if (a.nwords > 4 && per_xcd <= (a.nwords == 8 ? 96 : 64)) {
-      return bwd_row_run_four<T, D, 2>(a, bh, st, dry);
-    }
-    switch (a.nwords) {
-      case 1:
-      case 2: return bwd_row_run_short<T, D, 2, 1>(a, bh, st, dry);
-      case 3: return bwd_row_run_short<T, D, 3, 1>(a, bh, st, dry);
-      case 4: return bwd_row_run_short<T, D, 4, 1>(a, bh, st, dry);
-      case 5: return bwd_row_run_short<T, D, 5, 1>(a, bh, st, dry);
-      case 6: return bwd_row_run_short<T, D, 6, 1>(a, bh, st, dry);
-      case 7: return bwd_row_run_short<T, D, 7, 1>(a, bh, st, dry);
-      default: return bwd_row_run_short<T, D, 8, 1>(a, bh, st, dry);
-    }
-  } else if constexpr (D <= 32 && KT <= 4) {
-    // up to 384 and 512 keys: two waves, in two sizes each
+  if constexpr (D <= 32 && KT <= 4) {
     static_assert(kRowWaves * 4 * 32 == kShortRowKeys);
-    if (a.nwords <= 4 * KT - 2) return bwd_row_run_short<T, D, 2 * KT - 1, 2>(a, bh, st, dry);
-    return bwd_row_run_short<T, D, 2 * KT, 2>(a, bh, st, dry);
+    const RowForm form = bwd_row_form(a.nwords, D, bwd_row_blocks(bh, a.N) / 8);
+    if constexpr (KT <= 3) {
+      // (a tile made for longer rows takes the waves that those would)
+      if (form == RowForm::kFourWaves && (KT == 2 || a.nwords > 8)) return bwd_row_run_four<T, D, KT>(a, bh, st, dry);
+    }
+    if constexpr (KT > 2) {
+      // up to 384 and 512 keys, in two sizes each
+      if (a.nwords <= 4 * KT - 2) return bwd_row_run_short<T, D, 2 * KT - 1, 2>(a, bh, st, dry);
+      return bwd_row_run_short<T, D, 2 * KT, 2>(a, bh, st, dry);
+    } else {
+      if (form == RowForm::kTwoWaves) return bwd_row_run_short<T, D, 2, 2>(a, bh, st, dry);
+      switch (a.nwords) {
+        case 1:
+        case 2: return bwd_row_run_short<T, D, 2, 1>(a, bh, st, dry);
+        case 3: return bwd_row_run_short<T, D, 3, 1>(a, bh, st, dry);
+        case 4: return bwd_row_run_short<T, D, 4, 1>(a, bh, st, dry);
+        case 5: return bwd_row_run_short<T, D, 5, 1>(a, bh, st, dry);
+        case 6: return bwd_row_run_short<T, D, 6, 1>(a, bh, st, dry);
+        case 7: return bwd_row_run_short<T, D, 7, 1>(a, bh, st, dry);
+        default: return bwd_row_run_short<T, D, 8, 1>(a, bh, st, dry);
+      }
+    }
   } else {
     return bwd_row_run_four<T, D, KT>(a, bh, st, dry);
   }
