@@ -69,7 +69,9 @@ constexpr int fwd_main_lds_bytes(int D, int es, int NW, int R, int BKF) {
 // padding: 160 -> 136 us.  Row after row, with a barrier of its own for the dropped first stage, what that stage costs these rows
 // was not made up for: half of the rows padding, bf16, us, before the stage was requested early / with it / now: h = 4, d = 16, n = 256
 // 16.9 / 17.7 / 16.4, n = 512 63.7 / 63.4 / 57.2; h = 8, d = 64, n = 256 46.9 / 48.0 / 45.9; h = 4, d = 128, n = 300 69.5 / 71.0 / 68.2, 512
-// 232 / 236 / 219.  One row per workgroup gains nothing by meeting: d = 128, n = 128 15.5 / 15.8 / 15.9, h = 8, n = 200 56.1 / 57.6 / 57.6.)
+// 232 / 236 / 219.  One row per workgroup gains nothing by meeting: d = 128, n = 128 16.0 / 16.2 / 16.2.  Keys that do
+// not fill the last round of loads: taken one after the other they cost a trip to memory each, d = 128, h = 8, n = 77 17.9 us, now 16.8, n = 230 83.7 / 77.9, n = 450
+// 377 / 367; d = 32, h = 8, n = 230 33.2 / 32.2.)
 template <typename T, int D, int NW, int R, int LDS>
 TRI_DEV void fwd_uniform_rows(const FwdArgs& a, const T* vbh, int bh, int i0, int j_blk, unsigned char* smem) {
   using vec = typename Elem<T>::vec;
@@ -86,15 +88,25 @@ TRI_DEV void fwd_uniform_rows(const FwdArgs& a, const T* vbh, int bh, int i0, in
     float acc[G][VEC] = {};
 #pragma unroll
     for (int r = 0; r < G; ++r) v[r] = vbh + min(i0 + r0 + r, N - 1) * a.sv.i + ch * VEC;  // (rows past the end are not stored)
-#pragma unroll 8 / G
-    for (int k = slot; k < N; k += SLOTS) {  // (eight loads in flight)
-      vec x[G];
+    constexpr int U = 8 / G;  // (eight loads in flight, the last ones too: past the last key the last one is read again and counts as zero)
+#pragma unroll 1
+    for (int k0 = 0; k0 < N; k0 += U * SLOTS) {
+      typedef uint32_t words __attribute__((ext_vector_type(4)));
+      words x[U][G];
 #pragma unroll
-      for (int r = 0; r < G; ++r) x[r] = *reinterpret_cast<const vec*>(v[r] + (int64_t)k * a.sv.j);
+      for (int u = 0; u < U; ++u)
 #pragma unroll
-      for (int r = 0; r < G; ++r)
+        for (int r = 0; r < G; ++r) x[u][r] = *reinterpret_cast<const words*>(v[r] + (int64_t)min(k0 + u * SLOTS + slot, N - 1) * a.sv.j);
 #pragma unroll
-        for (int e = 0; e < VEC; ++e) acc[r][e] += (float)x[r][e];
+      for (int u = 0; u < U; ++u) {
+        const uint32_t live = (uint32_t)-(int)(k0 + u * SLOTS + slot < N);
+#pragma unroll
+        for (int r = 0; r < G; ++r) {
+          const vec y = __builtin_bit_cast(vec, x[u][r] & live);
+#pragma unroll
+          for (int e = 0; e < VEC; ++e) acc[r][e] += (float)y[e];
+        }
+      }
     }
     if (r0 == 0) wait_dma();  // (the first stage, requested before the row flags were read, has landed in this LDS)
     __syncthreads();          // (the rows before have been read)
