@@ -67,7 +67,7 @@ bool bwd_kv_tile_writes_dq(int tile) { return tile >= BwdKVFamily::kNumTiles && 
 
 TileInfo bwd_kv_tile_info(int tile) {
   // block_j = queries per LDS stage (tile 0 of the 16-bit types: of the version without the ring), block_k = keys per workgroup
-  // (row-resident tiles: four waves; short rows of up to 64 bytes run on one or two with as many key tiles in all.  The numbers
+  // (row-resident tiles: four waves; short rows of up to 64 bytes run on one, two or four with as many key tiles in all.  The numbers
   // are the tile's name in saved picks)
   if (bwd_kv_tile_writes_dq(tile)) return TileInfo{32, 128 * kRowKeyTiles[tile - BwdKVFamily::kNumTiles], 4};
   return TileInfo{BwdKVFamily::P(tile, 2), BwdKVFamily::P(tile, 0) * 32, BwdKVFamily::P(tile, 0)};

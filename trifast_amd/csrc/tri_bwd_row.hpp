@@ -181,7 +181,7 @@ struct RowSchedOf {
 // LDS the room, and the dq carried between the passes takes registers)
 constexpr int bwd_row_v_lds_tiles(int D, int KT, bool multi = false) { return KT * (D / 16) < 16 ? 0 : D <= 32 ? KT - (multi ? 2 : 3) : 1; }
 // Two waves per SIMD (256 registers each, the accumulators among the ordinary ones), of two workgroups, where a wave holds two key
-// tiles of rows of up to 64 bytes (launches of few rows, and the last pass over a long row).
+// tiles of rows of up to 64 bytes (the launches of short rows that tri_bwd_row_rule.hpp gives four waves, and the last pass over a long row).
 constexpr bool bwd_row_two_waves(int D, int KT) { return D <= 32 && KT <= 2; }
 // LDS bytes of the kernel below.  dq partials: two buffers (one barrier per query tile) of
 // three quarters of a tile per wave (the quarter a wave sums itself waits in its dS tile)

@@ -7,7 +7,7 @@
 // few key tiles per wave, is summed from the parts of all waves behind a barrier, and the start and the end of a row (K, V, o and do arrive;
 // dk and dv leave) had the compute unit to themselves.  Here
 // * a wave holds up to eight key tiles, as at n = 1024: rows of up to 256 keys are one wave's (four rows share a compute unit, nothing
-//   is exchanged, no barrier; few of them are spread, see bwd_row_run), rows of up to 512 two waves' (two rows share it).  Rows of a compute unit run apart, so one's loads and stores
+//   is exchanged, no barrier; tri_bwd_row_rule.hpp says which launches spread them over more), rows of up to 512 two waves' (two rows share it).  Rows of a compute unit run apart, so one's loads and stores
 //   go on beside the other's arithmetic.
 // * the (query tile, key tile) pairs of a wave are one software pipeline that does not end with a query tile: a step holds the
 //   exponentials of its pair, the score and dP MFMAs of the pair after it and the dv, dk and dq MFMAs of the pair before it, the next
